@@ -1,0 +1,39 @@
+"""Launch shapes that depend on the grid: each rule at the sizes where its
+choice changes, against the CPU oracle (FP64, <= 1e-12 relative L2)."""
+import numpy as np
+import pytest
+
+import chanflow as cf
+import oracle_lib as ol
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
+
+
+def step_parity(shape, steps, seed=5, **kw):
+    cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], stretch="tanh", dt=5e-4, nu=1.0 / 2800.0, **kw)
+    f = cf.initial_fields(cfg, seed=seed)
+    names = "uvwc" if cfg.scalar else "uvw"
+    orc = ol.OracleRun(ol.oracle_cfg(cfg, cf.grid_dz(cfg)))
+    for n in names:
+        orc.put(n, f[n])
+    orc.project_ic(1.0)
+    init = {n: orc.get(n) for n in names}
+    orc.steps(steps)
+    with cf.Run(cfg) as run:
+        for n in names:
+            run.upload(n, init[n])
+        run.step(steps)
+        run.sync()
+        errs = {n: rel(run.download(n), orc.get(n)) for n in names}
+    assert max(errs.values()) <= 1e-12, errs
+
+
+# z-chunks of the fused RHS: one level each (also nz = 2, all walls), two
+# levels with a shorter last chunk, four, five, and the 16-level cap
+@pytest.mark.parametrize("shape", [(8, 6, 2), (16, 12, 17), (64, 64, 49), (200, 90, 35), (96, 96, 41), (256, 256, 97)])
+def test_rhs_chunk_lengths(shape):
+    step_parity(shape, 2)

@@ -608,6 +608,8 @@ static void free_run(cf_run *r)
 
 /* ------------------------------------------------------------ create */
 
+static long rhs_tiles(int nx, int ny) { return (long) ((nx + CF_RT_X - 1) / CF_RT_X) * ((ny + CF_RT_Y - 1) / CF_RT_Y); }
+
 /* balanced z-chunks of the fused RHS for a target length: levels per
  * chunk and the launch's workgroup count (also its CFL partials) */
 static void rhs_chunks(int nx, int ny, int nz, int target, int *kc, int *blocks)
@@ -615,7 +617,40 @@ static void rhs_chunks(int nx, int ny, int nz, int target, int *kc, int *blocks)
     int nchunk = (nz + target - 1) / target;
     *kc = (nz + nchunk - 1) / nchunk;
     nchunk = (nz + *kc - 1) / *kc;
-    *blocks = ((nx + CF_RT_X - 1) / CF_RT_X) * ((ny + CF_RT_Y - 1) / CF_RT_Y) * nchunk;
+    *blocks = (int) (rhs_tiles(nx, ny) * nchunk);
+}
+
+/* The target length of the fused RHS's z-chunks for a launch over the
+ * given grids.  A workgroup marches its chunk's levels one after another,
+ * about 1 us each at low occupancy, behind a start-up worth three more, so
+ * a launch that leaves CUs idle is faster with shorter chunks, while one
+ * that fills the GPU wants long ones (two levels re-read per chunk).  Where
+ * the cap's chunks already give two rounds of the CF_RHS_SLOTS workgroups
+ * the GPU holds (three of 256 threads per CU, by LDS), the cap stands;
+ * otherwise the length with the least rounds x (levels + 3), the longer on
+ * a tie.  FP64 step, 16-level chunks against this rule's: 182 -> 135 us at
+ * 32x33x24 (1 level), 245 -> 198 us at 64x65x64 (2), 335 -> 306 us at
+ * 200x35x90 (4), 304 -> 281 us at 96x97x96 (5 and 6 alike), 647 -> 613 us at
+ * 160x121x160 (9 and 12 alike); 256x193x256 keeps its 15 (8: 4% slower). */
+#define CF_RHS_SLOTS 768
+static int rhs_target(const std::vector<const Grid *> &grids, int cap)
+{
+    int best = cap;
+    long bestcost = -1;
+    for (int t = cap; t >= 1; t--) {
+        long blocks = 0;
+        int longest = 1;
+        for (const Grid *g : grids) {
+            int kc, nb;
+            rhs_chunks(g->nx, g->ny, g->nz, t, &kc, &nb);
+            blocks += nb;
+            longest = std::max(longest, kc);
+        }
+        if (t == cap && blocks >= 2 * CF_RHS_SLOTS) return cap;
+        const long cost = (blocks + CF_RHS_SLOTS - 1) / CF_RHS_SLOTS * (longest + 3);
+        if (bestcost < 0 || cost < bestcost) { bestcost = cost; best = t; }
+    }
+    return best;
 }
 
 /* Every table of a run that depends on dt (the z-solve factors and spikes,
@@ -1134,14 +1169,15 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     size_t npart = std::max((size_t) r->nb_plane * (2 * nz + 2), (size_t) ((r->P + 63) / 64) * nz);
     if (npart < (size_t) r->nb_red) npart = r->nb_red;
     ok = ok && dalloc(&r->part, npart) && dalloc(&r->lsum, (size_t) nz + 2);
-    rhs_chunks(nx, ny, nz, CF_RHS_KC, &r->rhs_kc, &r->rhs_blocks);
+    rhs_chunks(nx, ny, nz, rhs_target({ &r->g }, CF_RHS_KC), &r->rhs_kc, &r->rhs_blocks);
     r->gblocks = ((nx + 63) / 64) * ((ny + 3) / 4) * nz;
     if (cfg->order == 4 && nx % CF_R4_X == 0 && ny % CF_R4_Y == 0
         && (size_t) nx * ny * nz * r->esz < ((size_t) 1 << 32)) {   /* 32-bit byte offsets */
         r->r4_nch = std::max(1, (nz + CF_R4_KC / 2) / CF_R4_KC);
         r->r4_blocks = (nx / CF_R4_X) * (ny / CF_R4_Y) * r->r4_nch;
     }
-    ok = ok && dalloc(&r->cflpart, (size_t) std::max(std::max(r->rhs_blocks, r->gblocks), r->r4_blocks));
+    /* a batch may cut the run's z-chunks otherwise, down to one level */
+    ok = ok && dalloc(&r->cflpart, (size_t) std::max({ (int) (rhs_tiles(nx, ny) * nz), r->gblocks, r->r4_blocks }));
     if (cfg->cflmode == 1) ok = ok && dalloc(&r->h1prev, (size_t) nz + 2);
     if (r->prec == CF_FP32 && !r->general) ok = ok && dalloc(&r->uoffd, (size_t) nz + 2 + 3 * (size_t) nz);
     if (!ok) { free_run(r); cf_set_error("device allocation failed"); return CF_ERR_NOMEM; }
@@ -2341,6 +2377,9 @@ template <typename T>
 static void batch_fill_args(cf_batch *b, std::vector<GArgs<T>> &A)
 {
     A.assign(b->n, GArgs<T>());
+    std::vector<const Grid *> grids;
+    for (const cf_run *r : b->runs) grids.push_back(&r->g);
+    const int kct = rhs_target(grids, CF_RHS_KC_BATCH);
     for (int q = 0; q < b->n; q++) {
         cf_run *r = b->runs[q];
         GArgs<T> &a = A[q];
@@ -2355,10 +2394,10 @@ static void batch_fill_args(cf_batch *b, std::vector<GArgs<T>> &A)
         a.dt = r->cfg.dt;
         a.dt_adhoc = r->pt_dt;
         a.nb_plane = r->nb_plane;
-        /* a batch has workgroups to spare: longer RHS z-chunks (fewer halo
+        /* a batch that fills the GPU takes longer RHS z-chunks (fewer halo
          * re-reads) than a run alone; the chunking does not change results */
         int bkc = 1, bblocks = 0;
-        rhs_chunks((int) r->g.nx, (int) r->g.ny, (int) r->g.nz, CF_RHS_KC_BATCH, &bkc, &bblocks);
+        rhs_chunks((int) r->g.nx, (int) r->g.ny, (int) r->g.nz, kct, &bkc, &bblocks);
         a.gblocks = b->fast ? bblocks : r->gblocks;
         a.rhs_kc = bkc;
         for (int t = 0; t < 4; t++) { a.pt[t] = r->pt[t]; a.pt4[t] = r->pt4[t]; }
