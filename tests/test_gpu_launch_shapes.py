@@ -37,3 +37,33 @@ def step_parity(shape, steps, seed=5, **kw):
 @pytest.mark.parametrize("shape", [(8, 6, 2), (16, 12, 17), (64, 64, 49), (200, 90, 35), (96, 96, 41), (256, 256, 97)])
 def test_rhs_chunk_lengths(shape):
     step_parity(shape, 2)
+
+
+# every field of the general right-hand side in one launch, and the
+# constraint from weighted sums of the right-hand side beside the z solve:
+# blocks with idle lanes and rows, one level a block, the nz = 257 system
+# that Thomas solves, the order-4 tiles and the per-field order-4 kernels
+@pytest.mark.parametrize("shape,kw", [((6, 6, 3), dict(scalar=1)), ((64, 9, 4), dict(scalar=1, betg_z=0.1)),
+                                      ((16, 6, 257), dict()), ((16, 6, 257), dict(scalar=1)),
+                                      ((32, 8, 9), dict(order=4, scalar=1)), ((30, 9, 7), dict(order=4, scalar=1))])
+def test_constraint_beside_the_solve(shape, kw):
+    cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], stretch="tanh", dt=1e-3, nu=1.0 / 500.0, uframe=0.3,
+                    want_cvolavg=0.1, cvolavgmode=kw.get("scalar", 0), **kw)
+    f = cf.initial_fields(cfg, seed=9)
+    names = "uvwc" if cfg.scalar else "uvw"
+    orc = ol.OracleRun(ol.oracle_cfg(cfg, cf.grid_dz(cfg)))
+    for n in names:
+        orc.put(n, f[n])
+    orc.project_ic(1.0)
+    init = {n: orc.get(n) for n in names}
+    want = orc.steps(4)
+    with cf.Run(cfg) as run:
+        for n in names:
+            run.upload(n, init[n])
+        run.step(4)
+        got = run.log()
+        for n in names:
+            assert rel(run.download(n), orc.get(n)) <= 1e-12, n
+    # forcings divide a cancellation by the unit response: absolute (test_gpu_parity.check_log)
+    for col in range(13):
+        assert np.allclose(got[:, col], want[:, col], rtol=1e-10, atol=1e-10), cf.LOG_COLUMNS[col]

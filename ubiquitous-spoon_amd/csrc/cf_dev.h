@@ -375,7 +375,7 @@ static __device__ __forceinline__ double wave_sum(double v)
 
 /* the maximum over a 64-lane wave of non-negative values (lanes a DPP
  * step does not reach read 0, which leaves such a maximum unchanged),
- * and over a 256-thread workgroup (sh: 4 doubles of LDS, one barrier) */
+ * and over a workgroup of NW waves (sh: NW doubles of LDS, one barrier) */
 static __device__ __forceinline__ double wave_max_nonneg(double v)
 {
     v = fmax(v, dpp_f64<0xB1, 0xf>(v));
@@ -388,23 +388,31 @@ static __device__ __forceinline__ double wave_max_nonneg(double v)
     const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
     return __hiloint2double(hi, lo);
 }
-static __device__ __forceinline__ double block_max256_nonneg(double v, double *sh)
+template <int NW>
+static __device__ __forceinline__ double block_max_nonneg(double v, double *sh)
 {
     const double w = wave_max_nonneg(v);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = w;
     __syncthreads();
-    return fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3]));
+    double m = sh[0];
+#pragma unroll
+    for (int i = 1; i < NW; i++) m = fmax(m, sh[i]);
+    return m;
 }
 
-/* the sum of one value per thread over a 256-thread workgroup: a DPP sum
- * per wave, then the four wave sums in order (one barrier, fixed order);
- * every thread returns the total.  sh: 4 doubles of LDS. */
-static __device__ __forceinline__ double block_sum256(double v, double *sh)
+/* the sum of one value per thread over a workgroup of NW waves: a DPP sum
+ * per wave, then the wave sums in order (one barrier, fixed order); every
+ * thread returns the total.  sh: NW doubles of LDS. */
+template <int NW>
+static __device__ __forceinline__ double block_sum(double v, double *sh)
 {
     const double w = wave_sum(v);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = w;
     __syncthreads();
-    return ((sh[0] + sh[1]) + sh[2]) + sh[3];
+    double t = sh[0];
+#pragma unroll
+    for (int i = 1; i < NW; i++) t += sh[i];
+    return t;
 }
 
 /* the sums over a wave's 64 lanes of each of a lane's LM <= 32 values

@@ -5,11 +5,12 @@
  * by index wrap, wall ghosts from the host-built closures (cf_tables.h).
  *
  * One substep (chanfast.c:395-656 / :1319-1580):
- *   k_grhs_{u,v,w,c}  explicit tendency f (advection, x-y diffusion,
+ *   k_grhs            explicit tendency f (advection, x-y diffusion,
  *                     buoyancy) and the implicit right-hand side
  *                     h = H(q) + gam dt f + zet dt (g + forcing) - lift
- *   k_spike / k_gsolve4  the wall-reduced z solves (order 2 / 4)
- *   k_gplane, k_gmass    plane sums and the mass-flux / scalar-mean forcing
+ *                     of u, v, w and c
+ *   k_spike / k_spike4   the wall-reduced z solves (order 2 / 4), with the
+ *                     mass-flux / scalar-mean forcing beside them (Book)
  *   k_div_fftx<.., ORD>, k_ffty, k_poisson2|4, k_ffty, k_fftx_inv  pressure
  *   k_gproject           projection + forcing correction into the state
  * Each stencil kernel reads its neighbours straight from global memory
@@ -172,17 +173,22 @@ static __device__ __forceinline__ T wall_interp(T gm2, T gm1, T x0, T x1)
 }
 
 /* block max of the CFL partials (all threads of the block call it) */
-static __device__ __forceinline__ void block_max_store(double v, double *__restrict__ out, unsigned bidx)
+/* The reductions of a 64 x 4 workgroup at one level: the sum of r (one
+ * value per thread) times the level's weight of each statistic of the
+ * substep (mwq [nz][4]) into mpart (n slots a statistic) and, where cflpart
+ * is set, the maximum of cfl (>= 0) */
+static __device__ __forceinline__ void block_store(double r, const double *__restrict__ mwq, int k, int s,
+                                                   double *__restrict__ mpart, double cfl,
+                                                   double *__restrict__ cflpart, unsigned bidx, unsigned n)
 {
-    __shared__ double red[256];
-    const int t = threadIdx.y * blockDim.x + threadIdx.x;
-    red[t] = v;
+    __shared__ double red[8];
+    const double w = wave_sum(r), c = cflpart ? wave_max_nonneg(cfl) : 0.0;
+    if (threadIdx.x == 0) { red[threadIdx.y] = w; red[4 + threadIdx.y] = c; }
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w) red[t] = fmax(red[t], red[t + w]);
-        __syncthreads();
-    }
-    if (t == 0) out[bidx] = red[0];
+    if (threadIdx.y != 0) return;
+    const int f = threadIdx.x;
+    if (f < book_stats(s)) mpart[(size_t) f * n + bidx] = mwq[4 * k + f] * (((red[0] + red[1]) + red[2]) + red[3]);
+    if (cflpart && f == 0) cflpart[bidx] = fmax(fmax(red[4], red[5]), fmax(red[6], red[7]));
 }
 
 /* ------------------------------------------------------------ u */
@@ -193,11 +199,12 @@ template <int ORD, bool SC, typename T>
 static __device__ __forceinline__ void rhsu_body(const RunDev &R, const int s,
     const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
     const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ cflpart, double cfldt, const Blk b)
+    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ cflpart, double cfldt, double *__restrict__ mpart,
+    const Blk b)
 {
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
     const int i = b.x * 64 + threadIdx.x, j = b.y * 4 + threadIdx.y, k = b.z;
-    double cflv = 0.0;
+    double cflv = 0.0, rsum = 0.0;
     if (i < nx && j < ny) {
         const size_t P = (size_t) nx * ny;
         const double *dz = R.dzt + CF_NGT;
@@ -290,23 +297,17 @@ static __device__ __forceinline__ void rhsu_body(const RunDev &R, const int s,
         if (s < 2) fo[q] = f;                 /* the last substep's tendency is never read */
         /* the z solve's right-hand side is h dvol (diffuseu.c:202); the
          * spectral solve takes h and applies dvol itself */
-        ro[q] = R.implicit ? h : h * dzk;
+        const T rr = h * dzk;
+        ro[q] = R.implicit ? h : rr;
+        rsum = (double) rr;
         if (cflpart) {                        /* get_cfl, get.c:390-417 */
             const double dzph = 0.5 * (dz[k] + dz[k + 1]);
             cflv = fmax(fmax(fabs((double) Q0) * cfldt / R.g.dx, fabs((double) v[q]) * cfldt / R.g.dy),
                         fabs((double) w[q]) * cfldt / dzph);
         }
     }
-    if (cflpart) block_max_store(cflv, cflpart, (b.z * b.ny + b.y) * b.nx + b.x);
-}
-
-template <int ORD, bool SC, typename T>
-__global__ __launch_bounds__(256) void k_grhs_u(const RunDev R, const int s,
-    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-    const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ cflpart, double cfldt)
-{
-    rhsu_body<ORD, SC, T>(R, s, u, v, w, c, g, scal, fo, ro, cflpart, cfldt, blk_native());
+    block_store(rsum, R.mwq + (size_t) (s * 2) * 4 * nz, k, s, mpart, cflv, cflpart, (b.z * b.ny + b.y) * b.nx + b.x,
+                b.nx * b.ny * b.nz);
 }
 
 /* ------------------------------------------------------------ v */
@@ -315,9 +316,9 @@ template <int ORD, bool SC, typename T>
 static __device__ __forceinline__ void rhsv_body(const RunDev &R, const int s,
     const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
     const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ cflpart, double cfldt, const Blk b)
+    T *__restrict__ fo, T *__restrict__ ro, const Blk b)
 {
-    (void) cflpart; (void) cfldt; (void) scal;
+    (void) scal;
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
     const int i = b.x * 64 + threadIdx.x, j = b.y * 4 + threadIdx.y, k = b.z;
     if (i >= nx || j >= ny) return;
@@ -410,24 +411,15 @@ static __device__ __forceinline__ void rhsv_body(const RunDev &R, const int s,
     ro[q] = R.implicit ? h : h * dzk;
 }
 
-template <int ORD, bool SC, typename T>
-__global__ __launch_bounds__(256) void k_grhs_v(const RunDev R, const int s,
-    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-    const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ cflpart, double cfldt)
-{
-    rhsv_body<ORD, SC, T>(R, s, u, v, w, c, g, scal, fo, ro, cflpart, cfldt, blk_native());
-}
-
 /* ------------------------------------------------------------ w */
 
 template <int ORD, bool SC, typename T>
 static __device__ __forceinline__ void rhsw_body(const RunDev &R, const int s,
     const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
     const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ cflpart, double cfldt, const Blk b)
+    T *__restrict__ fo, T *__restrict__ ro, const Blk b)
 {
-    (void) cflpart; (void) cfldt; (void) scal;
+    (void) scal;
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
     const int i = b.x * 64 + threadIdx.x, j = b.y * 4 + threadIdx.y, k = b.z;
     if (i >= nx || j >= ny) return;
@@ -524,15 +516,6 @@ static __device__ __forceinline__ void rhsw_body(const RunDev &R, const int s,
     ro[q] = R.implicit ? h : h * ((T) 0.5 * (DZ(k + 1) + DZ(k)));   /* times the face volume (diffusew.c:205) */
 }
 
-template <int ORD, bool SC, typename T>
-__global__ __launch_bounds__(256) void k_grhs_w(const RunDev R, const int s,
-    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-    const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ cflpart, double cfldt)
-{
-    rhsw_body<ORD, SC, T>(R, s, u, v, w, c, g, scal, fo, ro, cflpart, cfldt, blk_native());
-}
-
 /* ------------------------------------------------------------ c */
 
 /* flux_quick + advect_scalar (scalar.c:79-162), laplacexy with nu / Pr,
@@ -541,12 +524,12 @@ template <int ORD, bool SC, typename T>
 static __device__ __forceinline__ void rhsc_body(const RunDev &R, const int s,
     const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
     const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ cflpart, double cfldt, const Blk b)
+    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ mpart, const Blk b)
 {
-    (void) cflpart; (void) cfldt;
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
     const int i = b.x * 64 + threadIdx.x, j = b.y * 4 + threadIdx.y, k = b.z;
-    if (i >= nx || j >= ny) return;
+    double rsum = 0.0;
+    if (i < nx && j < ny) {
     const size_t P = (size_t) nx * ny;
     const double *dz = R.dzt + CF_NGT;
     const T A1 = (T) A1d, A2 = (T) A2d, B1 = (T) B1d, B2 = (T) B2d;
@@ -586,16 +569,40 @@ static __device__ __forceinline__ void rhsc_body(const RunDev &R, const int s,
     else h += (T) C.gamdt * f;
     h -= (T) R.liftg[((size_t) s * 4 + 3) * nz + k];
     if (s < 2) fo[q] = f;                     /* the last substep's tendency is never read */
-    ro[q] = R.implicit ? h : h * DZ(k);
+    const T rr = h * DZ(k);
+    ro[q] = R.implicit ? h : rr;
+    rsum = (double) rr;
+    }
+    block_store(rsum, R.mwq + (size_t) (s * 2 + 1) * 4 * nz, k, s, mpart, 0.0, nullptr, (b.z * b.ny + b.y) * b.nx + b.x,
+                b.nx * b.ny * b.nz);
+}
+
+/* ------------------------------------------------------------ all fields */
+
+/* One launch for every field of a substep: the z index of the grid counts
+ * (level, field), field fastest, so that the workgroups reading the same
+ * level of u, v, w and c run together.  A launch per field cost a small
+ * grid 4 us each and left most CUs idle (four of 13 us at 90x73x75). */
+template <int ORD, bool SC, typename T>
+static __device__ __forceinline__ void grhs_body(const RunDev &R, const int s, const GFields<T> &F,
+    const double *__restrict__ scal, double *__restrict__ cflpart, double cfldt, double *__restrict__ mpart, Blk b)
+{
+    constexpr unsigned nf = SC ? 4 : 3;
+    const unsigned fld = b.z % nf;
+    b.z /= nf;
+    b.nz /= nf;
+    if (fld == 0) rhsu_body<ORD, SC, T>(R, s, F.u, F.v, F.w, F.c, F.g[0], scal, F.f[0], F.r[0], cflpart, cfldt, mpart, b);
+    else if (fld == 1) rhsv_body<ORD, SC, T>(R, s, F.u, F.v, F.w, F.c, F.g[1], scal, F.f[1], F.r[1], b);
+    else if (fld == 2) rhsw_body<ORD, SC, T>(R, s, F.u, F.v, F.w, F.c, F.g[2], scal, F.f[2], F.r[2], b);
+    else if constexpr (SC)
+        rhsc_body<ORD, SC, T>(R, s, F.u, F.v, F.w, F.c, F.g[3], scal, F.f[3], F.r[3], mpart + (size_t) 4 * b.nx * b.ny * b.nz, b);
 }
 
 template <int ORD, bool SC, typename T>
-__global__ __launch_bounds__(256) void k_grhs_c(const RunDev R, const int s,
-    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-    const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ cflpart, double cfldt)
+__global__ __launch_bounds__(256) void k_grhs(const RunDev R, const int s, const GFields<T> F,
+    const double *__restrict__ scal, double *__restrict__ cflpart, double cfldt, double *__restrict__ mpart)
 {
-    rhsc_body<ORD, SC, T>(R, s, u, v, w, c, g, scal, fo, ro, cflpart, cfldt, blk_native());
+    grhs_body<ORD, SC, T>(kernarg_run(), s, F, scal, cflpart, cfldt, mpart, blk_native());
 }
 
 /* ------------------------------------------------------------ solve */
@@ -654,115 +661,15 @@ static __device__ __forceinline__ void solve4_body(const RunDev &R, const int s,
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_gsolve4(const RunDev R, const int s,
-    T *__restrict__ ru, T *__restrict__ rv, T *__restrict__ rw, T *__restrict__ rc)
+__global__ __launch_bounds__(256) void k_gsolve4(const RunDev R, const int s, const int nbx,
+    T *__restrict__ ru, T *__restrict__ rv, T *__restrict__ rw, T *__restrict__ rc, const Book B)
 {
-    solve4_body<T>(R, s, ru, rv, rw, rc, blk_native());
+    if (blockIdx.x == 0) book_body(R, B);
+    else solve4_body<T>(R, s, ru, rv, rw, rc, blk_solve(blockIdx.x - 1, nbx));
 }
 
-template __global__ void k_gsolve4<double>(const RunDev, const int, double *, double *, double *, double *);
-template __global__ void k_gsolve4<float>(const RunDev, const int, float *, float *, float *, float *);
-
-/* ------------------------------------------------------------ constraints */
-
-/* interior plane sums of u* (kind 0, blockIdx.z = 0) and c* (kind 1) for
- * get_xy_avg (get.c:281-307); deterministic fixed-order trees.
- * part[(kind * nz + k) * nb + b] */
-template <typename T>
-static __device__ __forceinline__ void plane_body(const RunDev &R, const T *__restrict__ q0,
-                                                const T *__restrict__ q1, double *__restrict__ part, int nb, const Blk b)
-{
-    __shared__ double red[4];
-    const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
-    const size_t P = (size_t) nx * ny;
-    const int lev = b.y, kind = b.z, bb = b.x;
-    const T *q = kind == 0 ? q0 : q1;
-    const size_t chunk = (P + nb - 1) / nb;
-    const size_t lo = (size_t) bb * chunk, hi = lo + chunk < P ? lo + chunk : P;
-    const T *pl = q + (size_t) lev * P;
-    double acc = 0.0;                             /* FP64 accumulation for either storage */
-    /* unrolled so that a thread's loads are in flight together */
-#pragma unroll 8
-    for (size_t e = lo + threadIdx.x; e < hi; e += 256) acc += (double) pl[e];
-    const double tot = block_sum256(acc, red);    /* DPP wave sums, then the four in order */
-    if (threadIdx.x == 0) part[((size_t) kind * nz + lev) * nb + bb] = tot;
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_gplane(const RunDev R, const T *__restrict__ q0,
-                                                const T *__restrict__ q1, double *__restrict__ part, int nb)
-{
-    plane_body<T>(R, q0, q1, part, nb, blk_native());
-}
-
-template __global__ void k_gplane<double>(const RunDev, const double *, const double *, double *, int);
-template __global__ void k_gplane<float>(const RunDev, const float *, const float *, double *, int);
-
-/* mass-flux (kind 0, chanfast.c:485-530) and scalar-mean (kind 1,
- * :572-617) constraints: plane averages, their wall ghosts from the
- * closures, bulk value, wall gradients of order 2 or 4 (:489-494,
- * :1413-1418), centreline; forcing from the unit-forcing response. */
-static __device__ __forceinline__ void mass_body(const RunDev &R, const int s, const double *__restrict__ part, int nb,
-                                               double *__restrict__ scal, double *__restrict__ logbuf, const Blk b)
-{
-    extern __shared__ double avg[];               /* nz + 6: level k at k + 3 */
-    const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz, ord = R.g.order;
-    const int kind = b.x;
-    const double *dz = R.dzt + CF_NGT;
-    const double scale = 1.0 / ((double) nx * (double) ny);
-    for (int l = threadIdx.x; l < nz; l += blockDim.x) {
-        double acc = 0.0;
-        for (int b = 0; b < nb; b++) acc += part[((size_t) kind * nz + l) * nb + b];
-        avg[l + 3] = acc * scale;
-    }
-    __syncthreads();
-    double *A = avg + 3;
-    /* the volume integral and the height as fixed-order block sums */
-    __shared__ double shv[4], shl[4];
-    double pv = 0.0, pl = 0.0;
-    for (int k = threadIdx.x; k < nz; k += blockDim.x) { pv += A[k] * dz[k]; pl += dz[k]; }
-    const double volsum = block_sum256(pv, shv), lzsum = block_sum256(pl, shl);
-    if (threadIdx.x != 0) return;
-    const double bcb = kind == 0 ? R.ubc : R.cbot, bct = kind == 0 ? R.ubc : R.ctop;
-    for (int m = 0; m < 3; m++) {
-        const Clos1 &B = R.cl.cell[0], &T = R.cl.cell[1];
-        const double b1 = nz > 1 ? A[1] : 0.0, b2 = nz > 2 ? A[2] : 0.0;
-        const double t1 = nz > 1 ? A[nz - 2] : 0.0, t2 = nz > 2 ? A[nz - 3] : 0.0;
-        A[-1 - m] = B.G[m][0] * A[0] + B.G[m][1] * b1 + B.G[m][2] * b2 + B.B[m] * bcb;
-        A[nz + m] = T.G[m][0] * A[nz - 1] + T.G[m][1] * t1 + T.G[m][2] * t2 + T.B[m] * bct;
-    }
-    double vol = volsum / lzsum;
-    const double kap = kind == 0 ? R.nu : R.kap;
-    double nb_, nt_;
-    if (ord == 2) {
-        nb_ = A[0] - A[-1];
-        nt_ = A[nz] - A[nz - 1];
-    } else {
-        nb_ = A1d * (A[0] - A[-1]) + A2d * (A[1] - A[-2]);
-        nt_ = A1d * (A[nz] - A[nz - 1]) + A2d * (A[nz + 1] - A[nz - 2]);
-    }
-    double bot = kap * (nb_ / (0.5 * (dz[0] + dz[-1])));
-    double top = kap * (nt_ / (0.5 * (dz[nz] + dz[nz - 1])));
-    double cl = nz % 2 == 0 ? 0.5 * (A[nz / 2 - 1] + A[nz / 2]) : A[nz / 2];
-    const double *s1 = R.stat1 + (size_t) (s * 2 + kind) * 4;   /* vol1, bot1, top1, cl1 */
-    double m = R.cmode[kind] == 1 ? (R.ctarget[kind] - vol) / s1[0] : R.cfixed[kind];
-    vol += s1[0] * m;
-    bot += s1[1] * m;
-    top += s1[2] * m;
-    cl += s1[3] * m;
-    scal[(kind == 0 ? SC_M0 : SC_MC0) + s] = m;
-    if (s == 2) {
-        long idx = (long) scal[SC_STEP] % R.logcap;
-        double *lg = logbuf + (size_t) idx * 13 + (kind == 0 ? 3 : 8);
-        lg[0] = m; lg[1] = bot; lg[2] = top; lg[3] = vol; lg[4] = cl;
-    }
-}
-
-__global__ __launch_bounds__(256) void k_gmass(const RunDev R, const int s, const double *__restrict__ part, int nb,
-                                               double *__restrict__ scal, double *__restrict__ logbuf)
-{
-    mass_body(R, s, part, nb, scal, logbuf, blk_native());
-}
+template __global__ void k_gsolve4<double>(const RunDev, const int, const int, double *, double *, double *, double *, const Book);
+template __global__ void k_gsolve4<float>(const RunDev, const int, const int, float *, float *, float *, float *, const Book);
 
 /* ------------------------------------------------------------ Poisson, order 4 */
 
@@ -1145,10 +1052,7 @@ __global__ __launch_bounds__(256) void k_gproject(const RunDev R, const T *us,
 template <typename T> struct GPick {
     template <int ORD, bool SC> static void fill(GSel<T> &S)
     {
-        S.u = k_grhs_u<ORD, SC, T>;
-        S.v = k_grhs_v<ORD, SC, T>;
-        S.w = k_grhs_w<ORD, SC, T>;
-        S.c = SC ? k_grhs_c<ORD, true, T> : nullptr;
+        S.rhs = k_grhs<ORD, SC, T>;
         S.proj = k_gproject<ORD, T>;
     }
 };
@@ -1177,7 +1081,7 @@ template GSel<float> pick_general<float>(int, int);
  * parameter block and buffers from the GArgs table.  Substep index s in
  * 0..2; s == 3 is a stand-alone projection of the state (dt = dt_adhoc). */
 
-template <int ORD, bool SC, typename T, int F>
+template <int ORD, bool SC, typename T>
 __global__ __launch_bounds__(256) void kb_rhs(const GArgs<T> *__restrict__ A, const unsigned *__restrict__ vs,
                                               int nrun, int s)
 {
@@ -1185,16 +1089,12 @@ __global__ __launch_bounds__(256) void kb_rhs(const GArgs<T> *__restrict__ A, co
         const GArgs<T> &a = A[r];
         T *const *fnew = (s % 2 == 0) ? a.fa : a.fb;
         T *const *gold = (s % 2 == 0) ? a.fb : a.fa;
-        const Blk b = blk_of(a, ST_CELL, lb);
-        if (F == 0)
-            rhsu_body<ORD, SC, T>(a.R, s, a.u, a.v, a.w, a.c, gold[0], a.scal, fnew[0], a.ru,
-                                  s == 0 ? a.cflpart : (double *) nullptr, a.dt, b);
-        else if (F == 1)
-            rhsv_body<ORD, SC, T>(a.R, s, a.u, a.v, a.w, a.c, gold[1], a.scal, fnew[1], a.rv, nullptr, a.dt, b);
-        else if (F == 2)
-            rhsw_body<ORD, SC, T>(a.R, s, a.u, a.v, a.w, a.c, gold[2], a.scal, fnew[2], a.rw, nullptr, a.dt, b);
-        else
-            rhsc_body<ORD, SC, T>(a.R, s, a.u, a.v, a.w, a.c, gold[3], a.scal, fnew[3], a.rc, nullptr, a.dt, b);
+        GFields<T> F;
+        F.u = a.u; F.v = a.v; F.w = a.w; F.c = a.c;
+        for (int t = 0; t < 4; t++) { F.g[t] = gold[t]; F.f[t] = fnew[t]; }
+        F.r[0] = a.ru; F.r[1] = a.rv; F.r[2] = a.rw; F.r[3] = a.rc;
+        grhs_body<ORD, SC, T>(a.R, s, F, a.scal, s == 0 ? a.cflpart : (double *) nullptr, a.dt, a.part,
+                              blk_of(a, ST_RHSG, lb));
     });
 }
 
@@ -1229,21 +1129,19 @@ __global__ __launch_bounds__(256) void kb_solve4(const GArgs<T> *__restrict__ a_
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void kb_plane(const GArgs<T> *__restrict__ a_, const unsigned *__restrict__ vs, int nrun, int s)
-{
-    (void) s;
-    batch_loop(vs, nrun, [&](int r, unsigned lb) {
-        const GArgs<T> &a = a_[r];
-        plane_body<T>(a.R, a.ru, a.rc, a.part, a.nb_plane, blk_of(a, ST_PLANE, lb));
-    });
-}
-
-template <typename T>
 __global__ __launch_bounds__(256) void kb_mass(const GArgs<T> *__restrict__ a_, const unsigned *__restrict__ vs, int nrun, int s)
 {
     batch_loop(vs, nrun, [&](int r, unsigned lb) {
+        (void) lb;
         const GArgs<T> &a = a_[r];
-        mass_body(a.R, s, a.part, a.nb_plane, a.scal, a.logbuf, blk_of(a, ST_MASS, lb));
+        Book B;
+        B.s = s;
+        B.n = a.gblocks;
+        B.part = a.part;
+        B.cflpart = s == 0 ? a.cflpart : nullptr;
+        B.scal = a.scal; B.logbuf = a.logbuf;
+        B.dt = a.dt;
+        book_body(a.R, B);
     });
 }
 
@@ -1258,7 +1156,6 @@ __global__ __launch_bounds__(256) void kb_poisson4(const GArgs<T> *__restrict__ 
 
 #define CF_INST_B(T)                                                                                              \
     template __global__ void kb_solve4<T>(const GArgs<T> *, const unsigned *, int, int);                          \
-    template __global__ void kb_plane<T>(const GArgs<T> *, const unsigned *, int, int);                           \
     template __global__ void kb_mass<T>(const GArgs<T> *, const unsigned *, int, int);                            \
     template __global__ void kb_poisson4<T>(const GArgs<T> *, const unsigned *, int, int);
 CF_INST_B(double)
@@ -1268,10 +1165,7 @@ CF_INST_B(float)
 template <typename T> struct BPick {
     template <int ORD, bool SC> static void fill(BSel<T> &S)
     {
-        S.u = kb_rhs<ORD, SC, T, 0>;
-        S.v = kb_rhs<ORD, SC, T, 1>;
-        S.w = kb_rhs<ORD, SC, T, 2>;
-        S.c = SC ? kb_rhs<ORD, true, T, 3> : nullptr;
+        S.rhs = kb_rhs<ORD, SC, T>;
         S.proj = kb_proj<ORD, T>;
         S.divx = pick_batched_divx<T>(ORD);
     }

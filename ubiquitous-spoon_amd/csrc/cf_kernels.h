@@ -16,7 +16,7 @@ enum {
     SC_CFL = 7,     /* cfl at the start of the current step */
     SC_ZERO = 8,    /* always 0 */
     SC_CFL0 = 9,    /* cflmode 1: cfl of the state at the start of a step, with the previous dt */
-    SC_TICKET = 10, /* k_level_mass: workgroups done, as a 64-bit counter (0 between launches) */
+    SC_TICKET = 10, /* kb_level_mass: workgroups done, a 32-bit counter (0 between launches) */
     SC_N = 16
 };
 
@@ -104,6 +104,12 @@ struct RunDev {
     double rdx, rdy, rdxdy;
     const double *stat1;        /* [s][kind][vol1, bot1, top1, cl1] */
     const double *h1;           /* [s][kind][nz + 2] unit-forcing profile, level k at k + 1 */
+    /* the constraint's statistics of the solved field (bulk value, bottom and
+     * top wall gradient, centreline) as weighted sums: over the plane means A
+     * of the solution, l . A + mcf with l = mlf [kind][4][nz]; over the means
+     * of the solve's right-hand side, with mwq = (solve)^-T l [s][kind][nz][4] */
+    const double *mwq, *mlf;
+    double mcf[2][4];
     int cmode[2];
     double ctarget[2], cfixed[2];
     int logcap;
@@ -145,8 +151,20 @@ static __device__ __forceinline__ Blk blk_native()
     return b;
 }
 
+/* the column block of workgroup b (nbx of them a field) of a z solve */
+static __device__ __forceinline__ Blk blk_solve(unsigned b, unsigned nbx)
+{
+    Blk r;
+    r.y = 0;
+    while (b >= nbx) { b -= nbx; r.y++; }   /* at most three times */
+    r.x = b;
+    r.z = 0;
+    r.nx = nbx; r.ny = 4; r.nz = 1;
+    return r;
+}
+
 /* launch stages of a batched step; each run's grid per stage is dims[stage] */
-enum { ST_CELL = 0, ST_SOLVE, ST_PLANE, ST_MASS, ST_ONE, ST_FFTX, ST_FFTY, ST_MODE, ST_RHS2, ST_LEVEL, CF_NST };
+enum { ST_CELL = 0, ST_RHSG, ST_SOLVE, ST_ONE, ST_FFTX, ST_FFTY, ST_MODE, ST_RHS2, ST_LEVEL, CF_NST };
 #define CF_BATCH_MAX 256        /* runs per batched launch */
 
 /* Where a substep's projected velocity comes from: the previous
@@ -310,7 +328,7 @@ template <typename T> struct GArgs {
     double *G, *S4, *scal, *logbuf, *part, *cflpart, *lsum;
     double dt;                  /* step */
     double dt_adhoc;            /* dt of a stand-alone projection (substep index 3) */
-    int nb_plane, gblocks;      /* gblocks: CFL partials of the run's RHS launch */
+    int gblocks;                /* CFL partials of the run's RHS launch */
     int rhs_kc;                 /* levels per z-chunk of the fast-path RHS */
     PoisTab pt[4];              /* substeps 0..2, stand-alone projection */
     Pois4Tab pt4[4];
@@ -360,31 +378,221 @@ static __device__ __forceinline__ Blk blk_of(const GArgs<T> &a, int stage, unsig
     return b;
 }
 
+/* The RunDev that is a kernel's first argument, where it lies in the
+ * argument segment.  A kernel that reaches the parameter block through
+ * selected addresses (the wall closures of several fields) otherwise copies
+ * the whole of it to scratch memory first: 2.2 KB a lane. */
+static __device__ __forceinline__ const RunDev &kernarg_run()
+{
+    return *(const RunDev *) (cp<RunDev>) __builtin_amdgcn_kernarg_segment_ptr();
+}
+
+/* Values that the workgroups of one launch hand to the last of them: stored
+ * and read at device scope, so they pass the caches that the XCDs do not
+ * share, and no cache has to be written back or invalidated (a release
+ * fence per workgroup wrote the dirty L2 lines of the whole XCD back:
+ * 200 us over the 4644 workgroups of one plane sum). */
+static __device__ __forceinline__ void dev_store(double *p, double v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+static __device__ __forceinline__ double dev_load(const double *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/* True in the last of n workgroups to call it, counted with a device-scope
+ * ticket.  Thread 0 waits for its own dev_stores to complete before it
+ * counts, so the last workgroup's dev_loads see those of every other.  Only
+ * which workgroup is last is a race.  The last one ends with ticket_reset;
+ * the next launch starts from 0.  (1-D workgroups.) */
+static __device__ __forceinline__ bool last_block(double *__restrict__ scal, unsigned n)
+{
+    __shared__ int last;
+    if (threadIdx.x == 0) {
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        last = __hip_atomic_fetch_add((unsigned *) (scal + SC_TICKET), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+               == n - 1;
+    }
+    __syncthreads();
+    return last != 0;
+}
+static __device__ __forceinline__ void ticket_reset(double *__restrict__ scal)
+{
+    __hip_atomic_store((unsigned *) (scal + SC_TICKET), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/* The cfl.dat record of a step that starts with CFL number mx (one thread) */
+static __device__ __forceinline__ void cfl_record(const RunDev &R, double mx, double dt, double *__restrict__ scal,
+                                                  double *__restrict__ logbuf)
+{
+    long idx = (long) scal[SC_STEP] % R.logcap;
+    double *lg = logbuf + (size_t) idx * 13;
+    for (int t = 0; t < 13; t++) lg[t] = 0.0;
+    lg[0] = scal[SC_STEP] + 1.0;
+    lg[1] = dt;
+    lg[2] = R.cfl_log > 0.0 ? R.cfl_log : mx;
+    scal[SC_CFL] = lg[2];
+}
+
+/* The forcing of kind 0 (u, chanfast.c:485-530) or 1 (c, :572-617) of
+ * substep s from the statistics v of the solved field (bulk value, bottom
+ * and top wall gradient, centreline; the last three in the last substep
+ * only) and the unit forcing's (stat1), and in the last substep the
+ * pstat / cstat record (one thread) */
+static __device__ __forceinline__ void force_record(const RunDev &R, int s, int kind, const double v[4],
+                                                    double *__restrict__ scal, double *__restrict__ logbuf)
+{
+    const double *s1 = R.stat1 + (size_t) (s * 2 + kind) * 4;   /* vol1, bot1, top1, cl1 */
+    const double m = R.cmode[kind] == 1 ? (R.ctarget[kind] - v[0]) / s1[0] : R.cfixed[kind];
+    scal[(kind == 0 ? SC_M0 : SC_MC0) + s] = m;
+    if (s == 2) {
+        long idx = (long) scal[SC_STEP] % R.logcap;
+        double *lg = logbuf + (size_t) idx * 13 + (kind == 0 ? 3 : 8);
+        lg[0] = m; lg[1] = v[1] + s1[1] * m; lg[2] = v[2] + s1[2] * m; lg[3] = v[0] + s1[0] * m; lg[4] = v[3] + s1[3] * m;
+    }
+}
+
+/* Bookkeeping of a substep by one workgroup, from the RHS launch's partial
+ * sums, beside the z solve (whose result it does not need): the plane
+ * averages of the solved field that the constraint takes (get_xy_avg,
+ * get.c:281-307; get_z_avg, :490-502) are linear in the right-hand side,
+ * and the solve is the same for every column, so
+ *   l . mean(S^-1 r) = (S^-T l) . mean(r),
+ * a weighted sum that the RHS kernels form on the way.  Reading the solved
+ * field again, in one or two launches between the solve and the
+ * divergence, took 5 us of every substep of a small grid, 12 at
+ * 256x193x256 and 20 at 192x129x192 with the scalar.
+ * n workgroups of the RHS launch each left a partial sum per statistic:
+ * part [kind][4][n]. */
+struct Book {
+    int s, n;
+    const double *part, *cflpart;           /* cflpart: the first substep's n CFL maxima, else null */
+    double *scal, *logbuf;
+    double dt;
+};
+static __device__ __forceinline__ constexpr int book_stats(int s) { return s == 2 ? 4 : 1; }
+
+/* one thread's share: v[0..7] the statistics of u and c, v[8] the CFL
+ * maximum; NF statistics, KINDS fields at compile time, so that the loads of
+ * four rounds of every array are in flight together */
+template <int NF, int KINDS, bool CFL>
+static __device__ __forceinline__ void book_share(const Book &B, double v[9])
+{
+    const gp<const double> p = (gp<const double>) B.part, cf = (gp<const double>) B.cflpart;
+    const int nt = blockDim.x;
+    for (int e0 = threadIdx.x; e0 < B.n; e0 += 4 * nt) {
+        double x[4][NF * KINDS], c[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int e = e0 + u * nt, ec = e < B.n ? e : B.n - 1;
+#pragma unroll
+            for (int q = 0; q < NF * KINDS; q++) {
+                const double t = p[(size_t) (q / NF * 4 + q % NF) * B.n + ec];
+                x[u][q] = e < B.n ? t : 0.0;
+            }
+            c[u] = CFL ? cf[ec] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+#pragma unroll
+            for (int q = 0; q < NF * KINDS; q++) v[q / NF * 4 + q % NF] += x[u][q];
+            if (CFL) v[8] = fmax(v[8], c[u]);
+        }
+    }
+}
+
+static __device__ __forceinline__ void book_body(const RunDev &R, const Book &B)
+{
+    __shared__ double sh[9][8];             /* up to eight waves */
+    const int nt = blockDim.x, nw = nt >> 6, tid = threadIdx.x, nz = R.g.nz, s = B.s;
+    const int kinds = R.scalar ? 2 : 1, nf = book_stats(s);
+    const double scale = 1.0 / ((double) R.g.nx * (double) R.g.ny);
+    double v[9];
+#pragma unroll
+    for (int q = 0; q < 9; q++) v[q] = 0.0;
+    if (s == 2) {
+        if (kinds == 2) book_share<4, 2, false>(B, v);
+        else book_share<4, 1, false>(B, v);
+    } else if (B.cflpart) {
+        if (kinds == 2) book_share<1, 2, true>(B, v);
+        else book_share<1, 1, true>(B, v);
+    } else {
+        if (kinds == 2) book_share<1, 2, false>(B, v);
+        else book_share<1, 1, false>(B, v);
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] *= scale;
+    if (R.uoff) {                           /* stored u is u - U(z): the profile's share */
+        const cp<double> U = (cp<double>) R.uoff + 1, l = (cp<double>) R.mlf;
+        for (int k = tid; k < nz; k += nt) {
+#pragma unroll
+            for (int f = 0; f < 4; f++)
+                if (f < nf) v[f] += l[f * nz + k] * U[k];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 9; q++) {
+        const double w = q == 8 ? wave_max_nonneg(v[q]) : wave_sum(v[q]);
+        if ((tid & 63) == 0) sh[q][tid >> 6] = w;
+    }
+    __syncthreads();
+    if (tid != 0) return;
+    for (int q = 0; q < 9; q++) {
+        double t = sh[q][0];
+        for (int w = 1; w < nw; w++) t = q == 8 ? fmax(t, sh[q][w]) : t + sh[q][w];
+        v[q] = t;
+    }
+    if (B.cflpart) cfl_record(R, v[8], B.dt, B.scal, B.logbuf);
+    for (int kind = 0; kind < kinds; kind++) {
+        double a[4];
+        for (int f = 0; f < 4; f++) a[f] = v[4 * kind + f] + R.mcf[kind][f];
+        force_record(R, s, kind, a, B.scal, B.logbuf);
+    }
+    if (s == 2) B.scal[SC_STEP] += 1.0;
+}
+
+/* The statistics' partial sums (SUMS) and the CFL maximum (CFL) of one
+ * 256-thread workgroup of a marching RHS kernel, substep s: a[f] the thread's
+ * weighted sums, cfl its maximum; sh: 20 doubles of LDS. */
+template <int s, bool SUMS, bool CFL>
+static __device__ __forceinline__ void book_store(double *part_, unsigned n, unsigned blk, int tid, const double a[4],
+                                                  double *sh, double *cflpart_, double cfl)
+{
+    const gp<double> part = (gp<double>) part_, cflpart = (gp<double>) cflpart_;
+    const int wave = tid >> 6;
+    const bool lane0 = (tid & 63) == 0;
+#pragma unroll
+    for (int f = 0; f < (SUMS ? book_stats(s) : 0); f++) {
+        const double w = wave_sum(a[f]);
+        if (lane0) sh[4 * f + wave] = w;
+    }
+    if constexpr (CFL) {
+        const double w = wave_max_nonneg(cfl);
+        if (lane0) sh[16 + wave] = w;
+    }
+    __syncthreads();
+    if (SUMS && tid < book_stats(s))
+        part[(size_t) tid * n + blk] = ((sh[4 * tid] + sh[4 * tid + 1]) + sh[4 * tid + 2]) + sh[4 * tid + 3];
+    if (CFL && tid == 0) cflpart[blk] = fmax(fmax(sh[16], sh[17]), fmax(sh[18], sh[19]));
+}
+
 /* off (may be null): a per-level profile subtracted on the way in and
  * added on the way out */
 template <typename T> __global__ void k_io_to_dev(const double *io, T *dev, int nx, int ny, int nz, const double *off);
 template <typename T> __global__ void k_dev_to_io(const T *dev, double *io, int nx, int ny, int nz, const double *off);
+/* The z solves of a single run: workgroup 0 does the substep's bookkeeping,
+ * the others solve nbx column blocks of each field in turn. */
+template <typename T> using k_zsolve_t = void (*)(const RunDev, const int, const int, T *, T *, T *, T *, const Book);
 template <typename T>
-__global__ void k_rhs2t(const RunDev R, const int s, const ProjSrcT<T> S, const T *gu, const T *gv, const T *gw,
-                        const double *scal, T *fu, T *fv, T *fw, T *ru, T *rv, T *rw, double *cflpart, double cfldt,
-                        int kc);
-template <typename T> __global__ void k_thomas(const RunDev R, const int s, T *ru, T *rv, T *rw, T *rc);
-template <typename T> using k_spike_t = void (*)(const RunDev, const int, T *, T *, T *, T *);
+__global__ void k_thomas(const RunDev R, const int s, const int nbx, T *ru, T *rv, T *rw, T *rc, const Book B);
+template <typename T> using k_spike_t = k_zsolve_t<T>;
+__global__ void k_book(const RunDev R, const Book B);
 template <typename T> k_spike_t<T> pick_spike(int L);
 template <typename T> k_spike_t<T> pick_spike4(int L);
-template <typename T> using k_spike_sums_t = void (*)(const RunDev, const int, T *, T *, T *, double *);
-template <typename T> k_spike_sums_t<T> pick_spike_sums(int L);
-__global__ void k_level_sum(const double *plane, int nbx, double *lsum);
-__global__ void k_mass_finalize(const RunDev R, const int s, const double *lsum, double *scal, double *logbuf,
-                                int kind);
 template <typename T>
 __global__ void k_cfl_plain(const RunDev R, const T *u, const T *v, const T *w, double dt, double *part);
 __global__ void k_cfl_reduce(const double *part, int nb, double *scal);
-__global__ void k_level_mass(const RunDev R, const int s, const double *plane, int nbx, double *lsum, double *scal,
-                             double *logbuf, int step_end);
-__global__ void k_cfl_finish(const RunDev R, const double *part, int nb, double dt,
-                             double *scal, double *logbuf);
-__global__ void k_step_end(double *scal);
 /* kernel pointer types of the FFT passes for storage precision T */
 template <typename T> struct KSel {
     typedef typename Cplx<T>::type C;
@@ -392,8 +600,11 @@ template <typename T> struct KSel {
     typedef void (*ffty_t)(const RunDev, C *, int);
     typedef void (*fftxi_t)(const RunDev, const C *, T *);
     typedef void (*pois2_t)(const RunDev, const PoisTab, C *, double *);
+    typedef void (*rhs2_t)(const RunDev, const ProjSrcT<T>, const T *, const T *, const T *, const double *, T *, T *, T *,
+                           T *, T *, T *, double *, double, int, double *);
 };
 typedef void (*k_fftx_plain_t)(const RunDev, const double *, double2 *);
+template <typename T> typename KSel<T>::rhs2_t pick_rhs2(int s);
 template <typename T> typename KSel<T>::div_t pick_div_fftx(int nx, int order);
 k_fftx_plain_t pick_fftx_plain(int nx);
 template <typename T> typename KSel<T>::ffty_t pick_ffty(int ny);
@@ -407,12 +618,18 @@ template <typename T>
 __global__ void k_maxdiv_part(const RunDev R, const T *u, const T *v, const T *w, double *part, int nb);
 
 /* general path (cf_general.hip), storage and arithmetic precision T */
+/* the fields of one substep: state, previous tendencies, new tendencies,
+ * right-hand sides (u, v, w, c) */
+template <typename T> struct GFields {
+    const T *u, *v, *w, *c;
+    const T *g[4];
+    T *f[4], *r[4];
+};
 template <typename T> struct GSel {
-    typedef void (*rhs_t)(const RunDev, const int, const T *, const T *, const T *, const T *, const T *,
-                          const double *, T *, T *, double *, double);
+    typedef void (*rhs_t)(const RunDev, const int, const GFields<T>, const double *, double *, double, double *);
     typedef void (*proj_t)(const RunDev, const T *, const T *, const T *, const T *, const double *,
                            const double *, const double *, const double *, const T *, double, T *, T *, T *, T *);
-    rhs_t u, v, w, c;
+    rhs_t rhs;
     proj_t proj;
 };
 template <typename T> GSel<T> pick_general(int order, int scalar);
@@ -420,19 +637,22 @@ template <typename T> GSel<T> pick_general(int order, int scalar);
 /* the order-4 explicit stage (cf_rhs4.hip): u and v in one launch, w and c
  * in another; grid (nx / CF_R4_X) * (ny / CF_R4_Y) * nch blocks of 256,
  * nch z-chunks */
-template <bool SC, typename T>
-__global__ void k_rhs4_uv(const RunDev R, const int s, const T *u, const T *v, const T *w, const T *c,
-    const T *gu, const T *gv, const double *scal, T *fu, T *fv, T *ru, T *rv, double *cflpart, double cfldt, int nch);
-template <bool SC, typename T>
-__global__ void k_rhs4_wc(const RunDev R, const int s, const T *u, const T *v, const T *w, const T *c,
-    const T *gw, const T *gc, const double *scal, T *fw, T *fc, T *rw, T *rc, int nch);
+template <typename T> struct R4Sel {
+    typedef void (*uv_t)(const RunDev, const T *u, const T *v, const T *w, const T *c, const T *gu, const T *gv,
+                         const double *scal, T *fu, T *fv, T *ru, T *rv, double *cflpart, double cfldt, int nch,
+                         double *mpart);
+    typedef void (*wc_t)(const RunDev, const T *u, const T *v, const T *w, const T *c, const T *gw, const T *gc,
+                         const double *scal, T *fw, T *fc, T *rw, T *rc, int nch, double *mpart);
+};
+template <typename T> typename R4Sel<T>::uv_t pick_rhs4_uv(bool sc, int s);
+template <typename T> typename R4Sel<T>::wc_t pick_rhs4_wc(bool sc, int s);
 
 /* batched launches (cf_general.hip, cf_kernels.hip): a = device array of
  * nrun GArgs, vs = that stage's virtual-block prefix (nrun + 1) */
 template <typename T> struct BSel {
     typedef void (*divx_t_)(const GArgs<T> *, const unsigned *, int, int);
     typedef void (*rhs_t)(const GArgs<T> *, const unsigned *, int, int);
-    rhs_t u, v, w, c;
+    rhs_t rhs;
     rhs_t proj;
     divx_t_ divx;
     typedef void (*kb_t)(const GArgs<T> *, const unsigned *, int, int);
@@ -443,15 +663,11 @@ template <typename T> __global__ void kb_poisson4(const GArgs<T> *a, const unsig
 template <typename T> __global__ void kb_solve4(const GArgs<T> *a, const unsigned *vs, int nrun, int s);
 template <typename T> typename BSel<T>::kb_t pick_batched_spike(int L);
 template <typename T> __global__ void kb_thomas(const GArgs<T> *a, const unsigned *vs, int nrun, int s);
-template <typename T> __global__ void kb_plane(const GArgs<T> *a, const unsigned *vs, int nrun, int s);
 template <typename T> __global__ void kb_mass(const GArgs<T> *a, const unsigned *vs, int nrun, int s);
-template <typename T> __global__ void kb_cfl(const GArgs<T> *a, const unsigned *vs, int nrun, int s);
-template <typename T> __global__ void kb_step_end(const GArgs<T> *a, const unsigned *vs, int nrun, int s);
 /* batched order-2 fast path (FP64 or FP32 storage) */
-template <typename T> __global__ void kb_rhs2t(const GArgs<T> *a, const unsigned *vs, int nrun, int s);
+template <typename T> typename BSel<T>::kb_t pick_batched_rhs2(int s);
 template <typename T> typename BSel<T>::kb_t pick_batched_spike_sums(int L);
-template <typename T> __global__ void kb_level_sum(const GArgs<T> *a, const unsigned *vs, int nrun, int s);
-template <typename T> __global__ void kb_mass_fast(const GArgs<T> *a, const unsigned *vs, int nrun, int s);
+template <typename T> __global__ void kb_level_mass(const GArgs<T> *a, const unsigned *vs, int nrun, int s);
 /* batched FFT passes: one launch per group of runs of one length; lengths
  * in CF_BFFT_SIZES have their plan compiled in, the others share a launch
  * with the runtime plan (key 0) */
@@ -470,9 +686,8 @@ template <typename T> typename BSel<T>::kb_t pick_batched_ffty(int n);
 template <typename T> typename BSel<T>::kb_t pick_batched_fftxi(int n);
 template <typename T> typename BSel<T>::kb_t pick_batched_poisson(int L);
 BSel<float>::kb_t pick_batched_poisson_islands(int L);
-template <typename T> __global__ void k_gsolve4(const RunDev R, const int s, T *ru, T *rv, T *rw, T *rc);
-template <typename T> __global__ void k_gplane(const RunDev R, const T *q0, const T *q1, double *part, int nb);
-__global__ void k_gmass(const RunDev R, const int s, const double *part, int nb, double *scal, double *logbuf);
+template <typename T>
+__global__ void k_gsolve4(const RunDev R, const int s, const int nbx, T *ru, T *rv, T *rw, T *rc, const Book B);
 template <typename T>
 __global__ void k_poisson4(const RunDev R, const Pois4Tab T_, typename Cplx<T>::type *Y, double *S);
 /* the twisted form (nz >= 6): grid ceil(M / 64) blocks of 128 */

@@ -84,26 +84,33 @@ template __global__ void k_dev_to_io<float>(const float *, double *, int, int, i
 #define RT_NA (RT_HX * RT_HY)      /* 396 halo-tile cells */
 #define RT_NP (RT_PX * RT_PY)      /* 469 pressure cells (one more in +x, +y) */
 
-/* lb: the tile's block index within the run (ntx nty nchunk of them) */
-template <typename T>
-static __device__ __forceinline__ void rhs2t_body(const RunDev &R, const int s, const ProjSrcT<T> &S,
+/* s: the substep, at compile time: the first reads no previous tendency
+ * (zeta = 0) and reduces the CFL number, the last stores no tendency (the
+ * next step starts with zeta = 0) and weighs all four statistics, so each
+ * form holds only the pointers and weights it uses (as run-time cases they
+ * spilled 56 scalar registers into vector lanes: FP32 180 us a launch at
+ * 256x193x256 against 171).  SUMS: the weighted sums of Book into
+ * mpart.  lb: the tile's block index within the run (nlb = ntx nty nchunk of
+ * them). */
+template <typename T, int s, bool SUMS>
+static __device__ __forceinline__ void rhs2t_body(const RunDev &R, const ProjSrcT<T> &S,
     const T *__restrict__ gu_, const T *__restrict__ gv_, const T *__restrict__ gw_,
     const double *__restrict__ scal_,
     T *__restrict__ fu_, T *__restrict__ fv_, T *__restrict__ fw_,
     T *__restrict__ ru_, T *__restrict__ rv_, T *__restrict__ rw_,
-    double *__restrict__ cflpart_, double cfldt, int kc, const unsigned lb)
+    double *__restrict__ cflpart_, double cfldt, int kc, double *__restrict__ mpart, const unsigned lb, const unsigned nlb)
 {
     const gp<const T> gu = (gp<const T>) gu_, gv = (gp<const T>) gv_, gw = (gp<const T>) gw_;
     const gp<T> fu = (gp<T>) fu_, fv = (gp<T>) fv_, fw = (gp<T>) fw_;
     const gp<T> ru = (gp<T>) ru_, rv = (gp<T>) rv_, rw = (gp<T>) rw_;
-    const gp<double> cflpart = (gp<double>) cflpart_;
+    constexpr bool useg = s > 0, keepf = s < 2, want_cfl = s == 0;
     const cp<double> scal = (cp<double>) scal_;
     const gp<const T> Sus = (gp<const T>) S.us, Svs = (gp<const T>) S.vs, Sws = (gp<const T>) S.ws;
     const gp<const T> Sp = (gp<const T>) S.p;
     const cp<double> Sh1 = (cp<double>) S.h1, Sm = (cp<double>) S.m;
     __shared__ __align__(16) T SU[4][RT_HY][RT_HX], SV[4][RT_HY][RT_HX], SW[4][RT_HY][RT_HX];
     __shared__ T SP[2][2][RT_PY][RT_PX];          /* [buffer][p(L), p(L+1)] */
-    double *red = (double *) &SU[0][0][0];        /* CFL reduction after the last level (>= 256 doubles) */
+    double *red = (double *) &SU[0][0][0];        /* the reductions after the last level (20 doubles) */
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
     const size_t P = (size_t) nx * ny;
     const int ntx = (nx + RT_X - 1) / RT_X, nty = (ny + RT_Y - 1) / RT_Y;
@@ -251,17 +258,16 @@ static __device__ __forceinline__ void rhs2t_body(const RunDev &R, const int s, 
     const T nu = (T) R.nu;
     const T rdx = (T) R.rdx, rdy = (T) R.rdy;
     const T rdx2 = rdx * rdx, rdy2 = rdy * rdy;
-    const T gmprev = (T) scal[R.m_prev_slot[s]];
+    const T gmprev = useg ? (T) scal[R.m_prev_slot[s]] : (T) 0;
     const T nuadt = (T) C.nuadt, gamdt = (T) C.gamdt, zetdt = (T) C.zetdt;
     const int r0 = ly + 1, c0 = lx + 1;
     double cflm = 0.0;
+    /* this thread's weighted sums of the u right-hand side (Book) */
+    const cp<double> mwq = (cp<double>) R.mwq + (size_t) (s * 2) * 4 * nz;
+    double ms[4] = { 0.0, 0.0, 0.0, 0.0 };
     /* previous tendencies of this point, one level ahead */
     const size_t qc = (size_t) j * nx + i;
     const unsigned qcb = (unsigned) (qc * sizeof(T));
-    /* gu == nullptr: the substep's zeta is 0 (no previous tendency read);
-     * fu == nullptr: this substep's tendency is never read (the next
-     * step's first substep has zeta = 0), so it is not stored */
-    const bool useg = gu != nullptr, keepf = fu != nullptr;
     T gnu = 0, gnv = 0, gnw = 0;
     if (act && useg) {
         const unsigned o = (unsigned) k0 * Pb + qcb;
@@ -288,6 +294,9 @@ static __device__ __forceinline__ void rhs2t_body(const RunDev &R, const int s, 
             const T dzk = (T) dz[k], dzkp = (T) dz[k + 1];
             const T rzk = (T) rdz[k], rzkp = (T) rdz[k + 1];
             const T rzp = (T) rdzh[k], rzm = (T) rdzh[k - 1];
+            double mw[4] = { 0.0, 0.0, 0.0, 0.0 };
+#pragma unroll
+            for (int q = 0; q < (SUMS ? book_stats(s) : 0); q++) mw[q] = mwq[4 * k + q];
             T Uk = 0, Ukp = 0, Ukm = 0, Uh = 0;    /* U at levels k, k + 1, k - 1; U's right-hand-side share */
             if (OFF && uof) {
                 Uk = (T) uof[k + 1]; Ukp = (T) uof[k + 2]; Ukm = (T) uof[k];
@@ -298,7 +307,7 @@ static __device__ __forceinline__ void rhs2t_body(const RunDev &R, const int s, 
 #define LW(sl, dr, dc) SW[sl][r0 + (dr)][c0 + (dc)]
 /* keeps each component's LDS reads next to their use (register pressure) */
 #define SEQ() asm volatile("" ::: "memory")
-            if (cflpart) {
+            if (want_cfl) {
                 double c;
                 if (cflm < (c = fabs(F(LU(s0, 0, 0), Uk)) * cfldt * rdx)) cflm = c;
                 if (cflm < (c = fabs(LV(s0, 0, 0)) * cfldt * rdy)) cflm = c;
@@ -321,12 +330,17 @@ static __device__ __forceinline__ void rhs2t_body(const RunDev &R, const int s, 
                 T f = adv + nu * (((uip - u0) - (u0 - uim)) * rdx2 + ((ujp - u0) - (u0 - ujm)) * rdy2);
                 T h = u0 + nuadt * (((ukp - u0) * rzp - (u0 - ukm) * rzm) * rzk);
                 if constexpr (OFF) h += Uh;
-                T g = gcu + gmprev;
-                h += gamdt * f + zetdt * g;
+                if constexpr (useg) h += gamdt * f + zetdt * (gcu + gmprev);
+                else h += gamdt * f;
                 if (k == 0) h -= (T) R.lift[s][0];
                 if (k == nz - 1) h -= (T) R.lift[s][1];
                 if (keepf) stb(fu, qb, f);
-                stb(ru, qb, h * dzk);
+                const T rr = h * dzk;
+                stb(ru, qb, rr);
+                if constexpr (SUMS) {
+#pragma unroll
+                    for (int q = 0; q < book_stats(s); q++) ms[q] += mw[q] * (double) rr;
+                }
             }
             SEQ();
             {   /* v */
@@ -340,7 +354,8 @@ static __device__ __forceinline__ void rhs2t_body(const RunDev &R, const int s, 
                                      + ((w0 + wjp) * (v0 + vkp) - (wkm + wjpkm) * (v0 + vkm)) * rzk);
                 T f = adv + nu * (((vip - v0) - (v0 - vim)) * rdx2 + ((vjp - v0) - (v0 - vjm)) * rdy2);
                 T h = v0 + nuadt * (((vkp - v0) * rzp - (v0 - vkm) * rzm) * rzk);
-                h += gamdt * f + zetdt * gcv;
+                if constexpr (useg) h += gamdt * f + zetdt * gcv;
+                else h += gamdt * f;
                 if (k == 0) h -= (T) R.lift[s][2];
                 if (k == nz - 1) h -= (T) R.lift[s][3];
                 if (keepf) stb(fv, qb, f);
@@ -360,7 +375,8 @@ static __device__ __forceinline__ void rhs2t_body(const RunDev &R, const int s, 
                                            + (szp * szp - szm * szm));
                 T f = adv + nu * (((wip - w0) - (w0 - wim)) * rdx2 + ((wjp - w0) - (w0 - wjm)) * rdy2);
                 T h = w0 + nuadt * (((wkp - w0) * rzkp - (w0 - wkm) * rzk) * rzp);
-                h += gamdt * f + zetdt * gcw;
+                if constexpr (useg) h += gamdt * f + zetdt * gcw;
+                else h += gamdt * f;
                 if (keepf) stb(fw, qb, f);
                 stb(rw, qb, h * dzp1h);
             } else {
@@ -380,31 +396,27 @@ static __device__ __forceinline__ void rhs2t_body(const RunDev &R, const int s, 
         level(k, A, B);
         if (k + 1 < k1) level(k + 1, B, A);
     }
-    if (cflpart) {
-        red[tid] = cflm;
-        __syncthreads();
-        for (int w = 128; w > 0; w >>= 1) {
-            if (tid < w) red[tid] = fmax(red[tid], red[tid + w]);
-            __syncthreads();
-        }
-        if (tid == 0) cflpart[lb] = red[0];
-    }
+    if constexpr (SUMS || want_cfl) book_store<s, SUMS, want_cfl>(mpart, nlb, lb, tid, ms, red, cflpart_, cflm);
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_RHS_WAVES, 8))) void k_rhs2t(const RunDev R, const int s, const ProjSrcT<T> S,
+template <typename T, int S>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_RHS_WAVES, 8))) void k_rhs2t(const RunDev R, const ProjSrcT<T> P,
     const T *__restrict__ gu, const T *__restrict__ gv, const T *__restrict__ gw,
     const double *__restrict__ scal,
     T *__restrict__ fu, T *__restrict__ fv, T *__restrict__ fw,
     T *__restrict__ ru, T *__restrict__ rv, T *__restrict__ rw,
-    double *__restrict__ cflpart, double cfldt, int kc)
+    double *__restrict__ cflpart, double cfldt, int kc, double *__restrict__ mpart)
 {
-    rhs2t_body<T>(R, s, S, gu, gv, gw, scal, fu, fv, fw, ru, rv, rw, cflpart, cfldt, kc, xcd_block(blockIdx.x, gridDim.x));
+    rhs2t_body<T, S, true>(R, P, gu, gv, gw, scal, fu, fv, fw, ru, rv, rw, cflpart, cfldt, kc, mpart,
+                           xcd_block(blockIdx.x, gridDim.x), gridDim.x);
 }
-template __global__ void k_rhs2t<double>(const RunDev, const int, const ProjSrcT<double>, const double *, const double *,
-    const double *, const double *, double *, double *, double *, double *, double *, double *, double *, double, int);
-template __global__ void k_rhs2t<float>(const RunDev, const int, const ProjSrcT<float>, const float *, const float *,
-    const float *, const double *, float *, float *, float *, float *, float *, float *, double *, double, int);
+template <typename T>
+typename KSel<T>::rhs2_t pick_rhs2(int s)
+{
+    return s == 0 ? k_rhs2t<T, 0> : (s == 1 ? k_rhs2t<T, 1> : k_rhs2t<T, 2>);
+}
+template KSel<double>::rhs2_t pick_rhs2<double>(int);
+template KSel<float>::rhs2_t pick_rhs2<float>(int);
 
 /* ---------------------------------------------------------------------
  * Batched constant-coefficient Thomas solve, one thread per (column,
@@ -467,14 +479,19 @@ static __device__ __forceinline__ void thomas_body(const RunDev &R, const int s,
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_thomas(const RunDev R, const int s,
-    T *__restrict__ ru, T *__restrict__ rv, T *__restrict__ rw, T *__restrict__ rc)
+__global__ __launch_bounds__(256) void k_thomas(const RunDev R, const int s, const int nbx,
+    T *__restrict__ ru, T *__restrict__ rv, T *__restrict__ rw, T *__restrict__ rc, const Book B)
 {
-    thomas_body<T>(R, s, ru, rv, rw, rc, blk_native());
+    if (blockIdx.x == 0) book_body(R, B);
+    else thomas_body<T>(R, s, ru, rv, rw, rc, blk_solve(blockIdx.x - 1, nbx));
 }
 
-template __global__ void k_thomas<double>(const RunDev, const int, double *, double *, double *, double *);
-template __global__ void k_thomas<float>(const RunDev, const int, float *, float *, float *, float *);
+template __global__ void k_thomas<double>(const RunDev, const int, const int, double *, double *, double *, double *, const Book);
+template __global__ void k_thomas<float>(const RunDev, const int, const int, float *, float *, float *, float *, const Book);
+
+/* the bookkeeping on its own, where no solve launch carries it (the fully
+ * implicit driver) */
+__global__ __launch_bounds__(256) void k_book(const RunDev R, const Book B) { book_body(R, B); }
 
 /* ---------------------------------------------------------------------
  * The same constant-coefficient tridiagonal solves as k_thomas, as a
@@ -581,22 +598,11 @@ static __device__ __forceinline__ void spike_body(const RunDev &R, const int s,
 }
 
 template <typename T, int LM>
-__global__ __launch_bounds__(512) void k_spike(const RunDev R, const int s,
-    T *__restrict__ ru, T *__restrict__ rv, T *__restrict__ rw, T *__restrict__ rc)
+__global__ __launch_bounds__(512) void k_spike(const RunDev R, const int s, const int nbx,
+    T *__restrict__ ru, T *__restrict__ rv, T *__restrict__ rw, T *__restrict__ rc, const Book B)
 {
-    spike_body<T, LM>(R, s, ru, rv, rw, rc, blk_native());
-}
-
-/* the fast path's solve: k_spike with the plane sums of u* fused in
- * (accumulated in FP64 whatever the storage) */
-#ifndef CF_SPIKE_WPE
-#define CF_SPIKE_WPE 1
-#endif
-template <typename T, int LM>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(CF_SPIKE_WPE, 8))) void k_spike_sums(const RunDev R, const int s, T *__restrict__ ru,
-    T *__restrict__ rv, T *__restrict__ rw, double *__restrict__ plane)
-{
-    spike_body<T, LM>(R, s, ru, rv, rw, nullptr, blk_native(), plane);
+    if (blockIdx.x == 0) book_body(R, B);
+    else spike_body<T, LM>(R, s, ru, rv, rw, rc, blk_solve(blockIdx.x - 1, nbx));
 }
 
 template <typename T>
@@ -612,20 +618,7 @@ k_spike_t<T> pick_spike(int L)
 template k_spike_t<double> pick_spike<double>(int);
 template k_spike_t<float> pick_spike<float>(int);
 
-template <typename T>
-k_spike_sums_t<T> pick_spike_sums(int L)
-{
-    switch (L) {
-#define X_(N) case N: return k_spike_sums<T, N>;
-    CF_SPIKE_LSET(X_)
-#undef X_
-    default: return nullptr;
-    }
-}
-template k_spike_sums_t<double> pick_spike_sums<double>(int);
-template k_spike_sums_t<float> pick_spike_sums<float>(int);
-
-/* second stage of the plane sums: level blockIdx.x, nbx partials in a
+/* second stage of a batched run's plane sums: level l, nbx partials in a
  * fixed tree */
 static __device__ __forceinline__ void level_sum_body(const double *__restrict__ plane, int nbx,
                                                       double *__restrict__ lsum, const int l)
@@ -633,34 +626,23 @@ static __device__ __forceinline__ void level_sum_body(const double *__restrict__
     __shared__ double red[4];
     double acc = 0.0;
     for (int q = threadIdx.x; q < nbx; q += 256) acc += plane[(size_t) l * nbx + q];
-    const double tot = block_sum256(acc, red);
-    if (threadIdx.x == 0) lsum[l] = tot;
+    const double tot = block_sum<4>(acc, red);
+    if (threadIdx.x == 0) dev_store(lsum + l, tot);
 }
 
-__global__ __launch_bounds__(256) void k_level_sum(const double *__restrict__ plane, int nbx,
-                                                   double *__restrict__ lsum)
-{
-    level_sum_body(plane, nbx, lsum, blockIdx.x);
-}
-
-
-
-
-/* ---------------------------------------------------------------------
- * Mass-flux constraint (chanfast.c:485-530): plane averages -> bulk
- * velocity (get_z_avg, get.c:490-502), wall shear, centreline; forcing
- * mdpdx = (Ub - uframe - U0) / U1 with U1 from the column-independent
- * unit-forcing solution h1 (host-precomputed per substep).  Input: the
- * per-level plane sums of the solved field (k_spike_sums, k_level_sum);
- * the wall-ghost averages are 2 bc - the adjacent level (apply_bc_u2).
- * Writes the forcing into scal[slot]; on the last substep writes the
- * pstat record.  One block of 256 threads.
- * ------------------------------------------------------------------- */
+/* Mass-flux constraint (chanfast.c:485-530) of a batched run on the fast
+ * path, from the per-level plane sums of its solved field: plane averages
+ * -> bulk velocity (get_z_avg, get.c:490-502), wall shear, centreline; the
+ * wall-ghost averages are 2 bc - the adjacent level (apply_bc_u2).  One
+ * workgroup of 256 threads.  (A single run's Book takes the weighted sums of
+ * the right-hand side instead; in a batch the RHS's z-chunks, and with them
+ * the order of those sums, depend on the other runs, and a run's result must
+ * not.) */
 static __device__ __forceinline__ void mass_finalize_body(const RunDev &R, const int s, const double *__restrict__ lsum,
-                                                          double *__restrict__ scal, double *__restrict__ logbuf, int kind)
+                                                          double *__restrict__ scal, double *__restrict__ logbuf)
 {
     extern __shared__ __align__(16) unsigned char smem_[];
-    double *avg = (double *) smem_;               /* nz + 2 */
+    double *A = (double *) smem_;                 /* nz */
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
     const double *dz = R.dzt + CF_NGT;
     const double scale = 1.0 / ((double) nx * (double) ny);
@@ -668,100 +650,22 @@ static __device__ __forceinline__ void mass_finalize_body(const RunDev &R, const
      * ..., then a fixed tree (deterministic, the same in every launch) */
     __shared__ double rv[4], rl[4];
     double pv = 0.0, pl = 0.0;
-    const double *uo = kind == 0 && R.uoff ? R.uoff + 1 : nullptr;   /* stored u is u - U(z) */
+    const double *uo = R.uoff ? R.uoff + 1 : nullptr;   /* stored u is u - U(z) */
     for (int l = threadIdx.x; l < nz; l += 256) {
-        const double a = uo ? lsum[l] * scale + uo[l] : lsum[l] * scale;
-        avg[l + 1] = a;
+        const double ls = dev_load(lsum + l);
+        const double a = uo ? ls * scale + uo[l] : ls * scale;
+        A[l] = a;
         pv += a * dz[l];
         pl += dz[l];
     }
-    const double volsum = block_sum256(pv, rv), hsum = block_sum256(pl, rl);
+    const double volsum = block_sum<4>(pv, rv), hsum = block_sum<4>(pl, rl);
     if (threadIdx.x != 0) return;
-    double *A = avg + 1;                          /* A[-1 .. nz] */
-    const double bc = kind == 0 ? R.ubc : R.cbot;
-    A[-1] = 2.0 * bc - A[0];                      /* apply_bc_u2 ghosts of the solved field */
-    A[nz] = 2.0 * (kind == 0 ? R.ubc : R.ctop) - A[nz - 1];
-    double vol = volsum / hsum;
-    const double kap = kind == 0 ? R.nu : R.nu / R.prandtl;
-    double bot = kap * (A[0] - A[-1]) / (0.5 * (dz[0] + dz[-1]));
-    double top = kap * (A[nz] - A[nz - 1]) / (0.5 * (dz[nz] + dz[nz - 1]));
-    double cl = nz % 2 == 0 ? 0.5 * (A[nz / 2 - 1] + A[nz / 2]) : A[nz / 2];
-    const double *s1 = R.stat1 + (size_t) (s * 2 + kind) * 4;   /* vol1, bot1, top1, cl1 */
-    double m = R.cmode[kind] == 1 ? (R.ctarget[kind] - vol) / s1[0] : R.cfixed[kind];
-    vol += s1[0] * m;
-    bot += s1[1] * m;
-    top += s1[2] * m;
-    cl += s1[3] * m;
-    scal[(kind == 0 ? SC_M0 : SC_MC0) + s] = m;
-    if (s == 2) {
-        long idx = (long) scal[SC_STEP] % R.logcap;
-        double *lg = logbuf + (size_t) idx * 13 + (kind == 0 ? 3 : 8);
-        lg[0] = m; lg[1] = bot; lg[2] = top; lg[3] = vol; lg[4] = cl;
-    }
-}
-
-/* The second stage of the plane sums and the mass-flux constraint in one
- * launch: each workgroup sums its level (level_sum_body), and the last
- * workgroup to finish -- counted with a device-scope ticket after a
- * release fence -- runs mass_finalize_body on all levels and resets the
- * ticket for the next launch.  The sums are in the same fixed order as the
- * two-launch form; only which workgroup finishes is a race, and it does
- * not enter the arithmetic.  step_end: also count the completed step
- * (the last substep). */
-__global__ __launch_bounds__(256) void k_level_mass(const RunDev R, const int s, const double *__restrict__ plane,
-                                                    int nbx, double *__restrict__ lsum, double *__restrict__ scal,
-                                                    double *__restrict__ logbuf, int step_end)
-{
-    level_sum_body(plane, nbx, lsum, blockIdx.x);
-    __shared__ int last;
-    if (threadIdx.x == 0) {
-        __threadfence();
-        unsigned long long *ticket = (unsigned long long *) (scal + SC_TICKET);
-        last = atomicAdd(ticket, 1ull) == (unsigned long long) (gridDim.x - 1);
-        __threadfence();
-    }
-    __syncthreads();
-    if (!last) return;
-    mass_finalize_body(R, s, lsum, scal, logbuf, 0);
-    if (threadIdx.x == 0) {
-        *(unsigned long long *) (scal + SC_TICKET) = 0ull;
-        if (step_end) scal[SC_STEP] += 1.0;
-    }
-}
-
-__global__ __launch_bounds__(256) void k_mass_finalize(const RunDev R, const int s, const double *__restrict__ lsum,
-                                                       double *__restrict__ scal, double *__restrict__ logbuf, int kind)
-{
-    mass_finalize_body(R, s, lsum, scal, logbuf, kind);
-}
-
-/* ---------------------------------------------------------------------
- * CFL at the start of a step (get_cfl, get.c:390-417): per-block max,
- * then a one-block finish that writes the cfl.dat record and bumps the
- * step counter at the end of the step (k_step_end).
- * ------------------------------------------------------------------- */
-static __device__ __forceinline__ void cfl_body(const RunDev &R, const double *__restrict__ part, int nb,
-                                                    double dt, double *__restrict__ scal, double *__restrict__ logbuf, const Blk b)
-{
-    __shared__ double red[4];
-    double m = 0.0;                               /* the block maxima are >= 0 */
-#pragma unroll 4
-    for (int b = threadIdx.x; b < nb; b += 256) m = fmax(m, part[b]);
-    const double mx = block_max256_nonneg(m, red);
-    if (threadIdx.x != 0) return;
-    long idx = (long) scal[SC_STEP] % R.logcap;
-    double *lg = logbuf + (size_t) idx * 13;
-    for (int t = 0; t < 13; t++) lg[t] = 0.0;
-    lg[0] = scal[SC_STEP] + 1.0;
-    lg[1] = dt;
-    lg[2] = R.cfl_log > 0.0 ? R.cfl_log : mx;
-    scal[SC_CFL] = lg[2];
-}
-
-__global__ __launch_bounds__(256) void k_cfl_finish(const RunDev R, const double *__restrict__ part, int nb,
-                                                    double dt, double *__restrict__ scal, double *__restrict__ logbuf)
-{
-    cfl_body(R, part, nb, dt, scal, logbuf, blk_native());
+    double v[4];
+    v[0] = volsum / hsum;
+    v[1] = R.nu * (A[0] - (2.0 * R.ubc - A[0])) / (0.5 * (dz[0] + dz[-1]));
+    v[2] = R.nu * ((2.0 * R.ubc - A[nz - 1]) - A[nz - 1]) / (0.5 * (dz[nz] + dz[nz - 1]));
+    v[3] = nz % 2 == 0 ? 0.5 * (A[nz / 2 - 1] + A[nz / 2]) : A[nz / 2];
+    force_record(R, s, 0, v, scal, logbuf);
 }
 
 /* cflmode 1 (chanfast.c:385-391): get_cfl (get.c:390-417) of the plain
@@ -815,11 +719,6 @@ __global__ __launch_bounds__(256) void k_cfl_reduce(const double *__restrict__ p
         __syncthreads();
     }
     if (threadIdx.x == 0) scal[SC_CFL0] = red[0];
-}
-
-__global__ void k_step_end(double *__restrict__ scal)
-{
-    if (threadIdx.x == 0) scal[SC_STEP] += 1.0;
 }
 
 /* ---------------------------------------------------------------------
@@ -2245,48 +2144,32 @@ __global__ __launch_bounds__(256) void kb_thomas(const GArgs<T> *__restrict__ a_
     });
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void kb_cfl(const GArgs<T> *__restrict__ a_, const unsigned *__restrict__ vs, int nrun, int s)
-{
-    (void) s;
-    batch_loop(vs, nrun, [&](int r, unsigned lb) {
-        const GArgs<T> &a = a_[r];
-        cfl_body(a.R, a.cflpart, a.gblocks, a.dt, a.scal, a.logbuf, blk_of(a, ST_ONE, lb));
-    });
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void kb_step_end(const GArgs<T> *__restrict__ a_, const unsigned *__restrict__ vs, int nrun, int s)
-{
-    (void) s;
-    batch_loop(vs, nrun, [&](int r, unsigned lb) {
-        (void) lb;
-        if (threadIdx.x == 0) a_[r].scal[SC_STEP] += 1.0;
-    });
-}
-
 /* ---- batched order-2 fast path (FP64 or FP32 storage): the single-run
  * kernels' bodies over the runs of a batch.  The argument table in use maps
  * u, v, w to the substep's input state set and ru, rv, rw to its output
  * set. */
-template <typename T>
+template <typename T, int S>
 __global__ __launch_bounds__(256) void kb_rhs2t(const GArgs<T> *__restrict__ a_, const unsigned *__restrict__ vs, int nrun, int s)
 {
+    (void) s;
     batch_loop(vs, nrun, [&](int r, unsigned lb) {
         const GArgs<T> &a = a_[r];
-        const int ps = (s + 2) % 3;               /* the substep whose projection is applied */
-        ProjSrcT<T> S;
-        S.us = a.u; S.vs = a.v; S.ws = a.w; S.p = a.p;
-        S.h1 = a.R.h1 + (size_t) (ps * 2) * (a.R.g.nz + 2);
-        S.m = a.scal + SC_M0 + ps;
-        S.dtp = a.R.sc[ps].abdt;
-        T *const *fnew = (s % 2 == 0) ? a.fa : a.fb;
-        T *const *gold = (s % 2 == 0) ? a.fb : a.fa;
-        const bool useg = a.R.sc[s].zetdt != 0.0, keepf = s < 2;
-        rhs2t_body<T>(a.R, s, S, useg ? gold[0] : nullptr, gold[1], gold[2], a.scal,
-                      keepf ? fnew[0] : nullptr, fnew[1], fnew[2], a.ru, a.rv, a.rw,
-                      s == 0 ? a.cflpart : nullptr, a.dt, a.rhs_kc, lb);
+        constexpr int ps = (S + 2) % 3;           /* the substep whose projection is applied */
+        ProjSrcT<T> P;
+        P.us = a.u; P.vs = a.v; P.ws = a.w; P.p = a.p;
+        P.h1 = a.R.h1 + (size_t) (ps * 2) * (a.R.g.nz + 2);
+        P.m = a.scal + SC_M0 + ps;
+        P.dtp = a.R.sc[ps].abdt;
+        T *const *fnew = (S % 2 == 0) ? a.fa : a.fb;
+        T *const *gold = (S % 2 == 0) ? a.fb : a.fa;
+        rhs2t_body<T, S, false>(a.R, P, gold[0], gold[1], gold[2], a.scal, fnew[0], fnew[1], fnew[2], a.ru, a.rv, a.rw,
+                                a.cflpart, a.dt, a.rhs_kc, nullptr, lb, 0);
     });
+}
+template <typename T>
+typename BSel<T>::kb_t pick_batched_rhs2(int s)
+{
+    return s == 0 ? kb_rhs2t<T, 0> : (s == 1 ? kb_rhs2t<T, 1> : kb_rhs2t<T, 2>);
 }
 
 template <typename T, int LM>
@@ -2309,23 +2192,30 @@ typename BSel<T>::kb_t pick_batched_spike_sums(int L)
     }
 }
 
+/* the second stage of the plane sums of a batch and the bookkeeping of the
+ * substep: a workgroup sums one level, and the run's last one to finish
+ * (last_block) forms the constraint; in the first substep it first reduces
+ * the CFL number of the RHS launch, in the last it counts the step */
 template <typename T>
-__global__ __launch_bounds__(256) void kb_level_sum(const GArgs<T> *__restrict__ a_, const unsigned *__restrict__ vs, int nrun, int s)
+__global__ __launch_bounds__(256) void kb_level_mass(const GArgs<T> *__restrict__ a_, const unsigned *__restrict__ vs, int nrun, int s)
 {
-    (void) s;
+    __shared__ double red[4];
     batch_loop(vs, nrun, [&](int r, unsigned lb) {
         const GArgs<T> &a = a_[r];
         level_sum_body(a.part, (int) a.dims[ST_SOLVE][0], a.lsum, (int) lb);
-    });
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void kb_mass_fast(const GArgs<T> *__restrict__ a_, const unsigned *__restrict__ vs, int nrun, int s)
-{
-    batch_loop(vs, nrun, [&](int r, unsigned lb) {
-        (void) lb;
-        const GArgs<T> &a = a_[r];
-        mass_finalize_body(a.R, s, a.lsum, a.scal, a.logbuf, 0);
+        if (!last_block(a.scal, a.dims[ST_LEVEL][0])) return;
+        if (s == 0) {
+            double m = 0.0;                       /* the block maxima are >= 0 */
+#pragma unroll 4
+            for (int b = threadIdx.x; b < a.gblocks; b += 256) m = fmax(m, a.cflpart[b]);
+            const double mx = block_max_nonneg<4>(m, red);
+            if (threadIdx.x == 0) cfl_record(a.R, mx, a.dt, a.scal, a.logbuf);
+        }
+        mass_finalize_body(a.R, s, a.lsum, a.scal, a.logbuf);
+        if (threadIdx.x == 0) {
+            ticket_reset(a.scal);
+            if (s == 2) a.scal[SC_STEP] += 1.0;
+        }
     });
 }
 
@@ -2336,13 +2226,10 @@ __global__ __launch_bounds__(256) void kb_mass_fast(const GArgs<T> *__restrict__
     template typename BSel<T>::kb_t pick_batched_poisson<T>(int);                                                  \
     template typename BSel<T>::kb_t pick_batched_spike<T>(int);                                                    \
     template __global__ void kb_thomas<T>(const GArgs<T> *, const unsigned *, int, int);                          \
-    template __global__ void kb_cfl<T>(const GArgs<T> *, const unsigned *, int, int);                             \
-    template __global__ void kb_step_end<T>(const GArgs<T> *, const unsigned *, int, int);                        \
     template typename BSel<T>::divx_t_ pick_batched_divx<T>(int);                                                  \
-    template __global__ void kb_rhs2t<T>(const GArgs<T> *, const unsigned *, int, int);                           \
+    template typename BSel<T>::kb_t pick_batched_rhs2<T>(int);                                                     \
     template typename BSel<T>::kb_t pick_batched_spike_sums<T>(int);                                               \
-    template __global__ void kb_level_sum<T>(const GArgs<T> *, const unsigned *, int, int);                       \
-    template __global__ void kb_mass_fast<T>(const GArgs<T> *, const unsigned *, int, int);
+    template __global__ void kb_level_mass<T>(const GArgs<T> *, const unsigned *, int, int);
 CF_INST_B(double)
 CF_INST_B(float)
 #undef CF_INST_B

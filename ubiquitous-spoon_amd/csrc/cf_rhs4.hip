@@ -225,13 +225,14 @@ struct Tile4 {
 /* advectu4 / advectv4 with massfluxx4 / massfluxy4, laplacexy, buoyancy,
  * helmholtz1d_operator_u4 and the u / v right-hand sides
  * (chanfast.c:1380-1420); CFL partials when cflpart is set */
-template <bool SC, typename T>
+/* s: the substep, at compile time (as in rhs2t_body) */
+template <bool SC, int s, typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_R4_WAVES, 8))) void k_rhs4_uv(
-    const RunDev R, const int s,
+    const RunDev R,
     const T *__restrict__ u_, const T *__restrict__ v_, const T *__restrict__ w_, const T *__restrict__ c_,
     const T *__restrict__ gu_, const T *__restrict__ gv_, const double *__restrict__ scal_,
     T *__restrict__ fu_, T *__restrict__ fv_, T *__restrict__ ru_, T *__restrict__ rv_,
-    double *__restrict__ cflpart_, double cfldt, int nch)
+    double *__restrict__ cflpart_, double cfldt, int nch, double *__restrict__ mpart)
 {
     const gp<const T> u = (gp<const T>) u_, v = (gp<const T>) v_, w = (gp<const T>) w_, c = (gp<const T>) c_;
     const gp<const T> gu = (gp<const T>) gu_, gv = (gp<const T>) gv_;
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_R4_WAVES
 
     __shared__ T Pu[PY][PX], Pv[PY][PX], Pw[PY][PX];
     __shared__ T Pc[SC ? PY : 1][SC ? PX : 1];
-    __shared__ double red[256];
+    __shared__ double red[20];
 
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
     const int P = nx * ny;
@@ -295,10 +296,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_R4_WAVES
     T hu = ld_cell(u, k0, oh), hv = ld_cell(v, k0, oh), hc = SC ? ld_cell(c, k0, oh) : (T) 0;
     T cc = SC ? ld_cell(c, k0, oc) : (T) 0;
     T wo = ld_face(k0 + 1, oc), hw = ld_face(k0 + 1, oh);
-    const bool want_cfl = cflpart_ != nullptr;
+    constexpr bool want_cfl = s == 0;
     double cflv = 0.0;
+    /* this thread's weighted sums of the u right-hand side (Book) */
+    const cp<double> mwq = (cp<double>) R.mwq + (size_t) (s * 2) * 4 * nz;
+    double ms[4] = { 0.0, 0.0, 0.0, 0.0 };
 
     for (int k = k0; k < k1; k++) {
+        double mw[4];
+#pragma unroll
+        for (int f = 0; f < book_stats(s); f++) mw[f] = mwq[4 * k + f];
         Pu[ly + H][lx + H] = Uc[3];
         Pv[ly + H][lx + H] = Vc[3];
         Pw[ly + H][lx + H] = wo;
@@ -379,7 +386,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_R4_WAVES
             if (s > 0) h += zetdt * (gu_q + mfu);
             h -= (T) lift[0 * nz + k];
             if (s < 2) sto(fu, q, f);
-            sto(ru, q, impl ? h : h * dzk);
+            const T rr = h * dzk;
+            sto(ru, q, impl ? h : rr);
+#pragma unroll
+            for (int f = 0; f < book_stats(s); f++) ms[f] += mw[f] * (double) rr;
             if (want_cfl)
                 cflv = fmax(cflv, fmax(fmax(fabs((double) Q0) * cfldt * R.rdx, fabs((double) Vc[3]) * cfldt * R.rdy),
                                        fabs((double) wq) * cfldt * rdzh[k]));
@@ -435,15 +445,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_R4_WAVES
         Uc[6] = nU; Vc[6] = nV;
         hu = nhu; hv = nhv; hc = nhc; cc = ncc; wo = nwo; hw = nhw;
     }
-    if (want_cfl) {
-        red[tid] = cflv;
-        __syncthreads();
-        for (int st = 128; st > 0; st >>= 1) {
-            if (tid < st) red[tid] = fmax(red[tid], red[tid + st]);
-            __syncthreads();
-        }
-        if (tid == 0) ((gp<double>) cflpart_)[blockIdx.x] = red[0];
-    }
+    book_store<s, true, want_cfl>(mpart, gridDim.x, blockIdx.x, tid, ms, red, cflpart_, cflv);
 }
 
 /* ------------------------------------------------------------ w and c */
@@ -452,12 +454,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_R4_WAVES
  * helmholtz1d_operator_w4 and the w right-hand side; with the scalar,
  * flux_quick + advect_scalar, laplacexy with nu / Pr and the scalar's
  * right-hand side (chanfast.c:1420-1470, :1495-1530) */
-template <bool SC, typename T>
+template <bool SC, int s, typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_R4_WAVES, 8))) void k_rhs4_wc(
-    const RunDev R, const int s,
+    const RunDev R,
     const T *__restrict__ u_, const T *__restrict__ v_, const T *__restrict__ w_, const T *__restrict__ c_,
     const T *__restrict__ gw_, const T *__restrict__ gc_, const double *__restrict__ scal_,
-    T *__restrict__ fw_, T *__restrict__ fc_, T *__restrict__ rw_, T *__restrict__ rc_, int nch)
+    T *__restrict__ fw_, T *__restrict__ fc_, T *__restrict__ rw_, T *__restrict__ rc_, int nch,
+    double *__restrict__ mpart)
 {
     const gp<const T> u = (gp<const T>) u_, v = (gp<const T>) v_, w = (gp<const T>) w_, c = (gp<const T>) c_;
     const gp<const T> gw = (gp<const T>) gw_, gc = (gp<const T>) gc_;
@@ -522,7 +525,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_R4_WAVES
     }
     T hw = ld_face(k0, oh), hc = SC ? ld_cell(c, k0, oh) : (T) 0;
 
+    /* this thread's weighted sums of the c right-hand side (Book) */
+    __shared__ double red[20];
+    const cp<double> mwq = (cp<double>) R.mwq + (size_t) (s * 2 + 1) * 4 * nz;
+    double ms[4] = { 0.0, 0.0, 0.0, 0.0 };
     for (int k = k0; k < k1; k++) {
+        double mw[4];
+#pragma unroll
+        for (int f = 0; f < book_stats(s); f++) mw[f] = mwq[4 * k + f];
         const bool wface = k <= nz - 2;                 /* w unknown at face k (uniform) */
         const T dzk = (T) dz[k];
         Pw[ly + H][lx + H] = Wc[3];
@@ -631,7 +641,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_R4_WAVES
             if (s > 0) h += zetdt * (gc_q + mfc);
             h -= (T) lift[3 * nz + k];
             if (s < 2) sto(fc, q, f);
-            sto(rc, q, impl ? h : h * dzk);
+            const T rr = h * dzk;
+            sto(rc, q, impl ? h : rr);
+#pragma unroll
+            for (int f = 0; f < book_stats(s); f++) ms[f] += mw[f] * (double) rr;
         }
         __syncthreads();
 #pragma unroll
@@ -642,14 +655,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CF_R4_WAVES
         U4[3] = nU; V4[3] = nV; Zh[3] = nZ;
         hw = nhw; hc = nhc;
     }
+    if constexpr (SC) book_store<s, true, false>(mpart, gridDim.x, blockIdx.x, tid, ms, red, nullptr, 0.0);
 }
 
-#define R4_INST(SC, T)                                                                                           \
-    template __global__ void k_rhs4_uv<SC, T>(const RunDev, const int, const T *, const T *, const T *, const T *, \
-        const T *, const T *, const double *, T *, T *, T *, T *, double *, double, int);                         \
-    template __global__ void k_rhs4_wc<SC, T>(const RunDev, const int, const T *, const T *, const T *, const T *, \
-        const T *, const T *, const double *, T *, T *, T *, T *, int);
-R4_INST(false, double)
-R4_INST(true, double)
-R4_INST(false, float)
-R4_INST(true, float)
+template <typename T>
+typename R4Sel<T>::uv_t pick_rhs4_uv(bool sc, int s)
+{
+    if (sc) return s == 0 ? k_rhs4_uv<true, 0, T> : (s == 1 ? k_rhs4_uv<true, 1, T> : k_rhs4_uv<true, 2, T>);
+    return s == 0 ? k_rhs4_uv<false, 0, T> : (s == 1 ? k_rhs4_uv<false, 1, T> : k_rhs4_uv<false, 2, T>);
+}
+template <typename T>
+typename R4Sel<T>::wc_t pick_rhs4_wc(bool sc, int s)
+{
+    if (sc) return s == 0 ? k_rhs4_wc<true, 0, T> : (s == 1 ? k_rhs4_wc<true, 1, T> : k_rhs4_wc<true, 2, T>);
+    return s == 0 ? k_rhs4_wc<false, 0, T> : (s == 1 ? k_rhs4_wc<false, 1, T> : k_rhs4_wc<false, 2, T>);
+}
+template R4Sel<double>::uv_t pick_rhs4_uv<double>(bool, int);
+template R4Sel<float>::uv_t pick_rhs4_uv<float>(bool, int);
+template R4Sel<double>::wc_t pick_rhs4_wc<double>(bool, int);
+template R4Sel<float>::wc_t pick_rhs4_wc<float>(bool, int);

@@ -85,7 +85,7 @@ struct cf_run {
     double *tab = nullptr;           /* all constant tables in one allocation */
     double *scal = nullptr, *logbuf = nullptr, *part = nullptr, *lsum = nullptr;
     size_t tab_n = 0;
-    int nb_plane = 1, nb_red = 1;
+    int nb_red = 1;
     RunDev rd;
     PoisTab pt[4];                   /* 3 substeps + ad-hoc dt */
     PoisTab hs2[3][3];               /* fully implicit driver: spectral Helmholtz tables [s][type], order 2 */
@@ -670,7 +670,8 @@ struct TabPack {
     bool spike_ok = true;
     bool spike4_ok = false, spike4_packed = false;
     size_t o_dz = 0, o_th = 0, o_st = 0, o_h1 = 0, o_twx = 0, o_twy = 0, o_twx32 = 0, o_twy32 = 0, o_lx = 0, o_ly = 0;
-    size_t o_rdz = 0, o_rdzh = 0, o_lift = 0;
+    size_t o_rdz = 0, o_rdzh = 0, o_lift = 0, o_mwq = 0, o_mlf = 0;
+    double mcf[2][4];                /* constants of the constraint's statistics (RunDev::mcf) */
     size_t o_p[4][6], o_sp[3][3][6], o_hp[3][3], o_p4[4], o_s4[3][3][3];
     size_t o_hs[3][3];               /* spectral Helmholtz z-tables (fully implicit driver) */
 };
@@ -756,6 +757,58 @@ static cf_status build_tables(const cf_config *cfg, const std::vector<double> &d
         cf_set_error("singular wall closure rows");
         return CF_ERR_NUMERIC;
     }
+    /* the constraint's statistics of the plane means A of u (kind 0) and c
+     * (kind 1): bulk value (get_z_avg), wall gradients (chanfast.c:489-494,
+     * :1413-1418) with the ghosts replaced by their closures, centreline --
+     * l . A + constant, from a trial column per unknown that the ghosts and
+     * the statistics reach */
+    std::vector<double> mlf((size_t) 2 * 4 * nz, 0.0), mwq((size_t) 3 * 2 * 4 * nz, 0.0);
+    {
+        double lzs = 0.0;
+        for (int k = 0; k < nz; k++) lzs += dzl[k];
+        for (int kind = 0; kind < 2; kind++) {
+            double *l = &mlf[(size_t) kind * 4 * nz];
+            const double kap = kind == 0 || !cfg->scalar ? nu : nu / cfg->prandtl;
+            const double bcb = kind == 0 ? 0.0 - cfg->uframe : -0.5, bct = kind == 0 ? 0.0 - cfg->uframe : 0.5;
+            const double hb = 0.5 * (dzl[0] + dzl[-1]), ht = 0.5 * (dzl[nz] + dzl[nz - 1]);
+            const double A1h = order == 2 ? 1.0 : 1.125 / 1.0, A2h = order == 2 ? 0.0 : -0.125 / 3.0;
+            for (int k = 0; k < nz; k++) l[k] = dzl[k] / lzs;
+            /* bottom: kap (A1h (x0 - g0) + A2h (x1 - g1)) / hb, g_m = G[m] . (x0, x1, x2) + B[m] bc; top mirrored */
+            double cb = 0.0, ct = 0.0;
+            for (int m = 0; m < (order == 2 ? 1 : 2); m++) {
+                const double am = m == 0 ? A1h : A2h;
+                const Clos1 &B = clo.cell[0], &Tp = clo.cell[1];
+                l[nz + m] += kap * am / hb;
+                l[2 * nz + nz - 1 - m] -= kap * am / ht;
+                for (int t = 0; t < 3 && t < nz; t++) {
+                    l[nz + t] -= kap * am * B.G[m][t] / hb;
+                    l[2 * nz + nz - 1 - t] += kap * am * Tp.G[m][t] / ht;
+                }
+                cb -= kap * am * B.B[m] * bcb / hb;
+                ct += kap * am * Tp.B[m] * bct / ht;
+            }
+            if (nz % 2 == 0) l[3 * nz + nz / 2 - 1] = l[3 * nz + nz / 2] = 0.5;
+            else l[3 * nz + nz / 2] = 1.0;
+            T.mcf[kind][0] = 0.0; T.mcf[kind][1] = cb; T.mcf[kind][2] = ct; T.mcf[kind][3] = 0.0;
+        }
+    }
+    /* their weights on the right-hand side: the transposed solves */
+    auto weights = [&](int s, int kind, auto &&solve_t) {
+        for (int f = 0; f < 4; f++) {
+            const double *l = &mlf[(size_t) (kind * 4 + f) * nz];
+            std::vector<double> lv(l, l + nz), x;
+            solve_t(lv, x);
+            for (int k = 0; k < nz; k++) mwq[((size_t) (s * 2 + kind) * nz + k) * 4 + f] = x[k];
+        }
+    };
+    if (order == 2)
+        for (int s = 0; s < 3; s++)
+            for (int kind = 0; kind < (cfg->scalar ? 2 : 1); kind++) {
+                std::vector<double> a, b, c, at(nz, 0.0), ct(nz, 0.0);
+                cell2_system(dzl, nz, kind == 0 ? -T.sc[s].nubdt : -T.sc[s].kbdt, a, b, c);
+                for (int k = 1; k < nz; k++) { at[k] = c[k - 1]; ct[k - 1] = a[k]; }
+                weights(s, kind, [&](const std::vector<double> &lv, std::vector<double> &x) { tridag_host(at, b, ct, lv, x); });
+            }
     std::vector<double> liftg((size_t) 3 * 4 * nz, 0.0);
     for (int s = 0; s < 3; s++)
         for (int f = 0; f < 4; f++) {
@@ -804,6 +857,20 @@ static cf_status build_tables(const cf_config *cfg, const std::vector<double> &d
                     S4.ok = num <= 1e-26 * den;
                 }
                 if (type == 2) continue;
+                if (type == 0 || cfg->scalar) {
+                    std::vector<cft::Row7> rt(rows.size());
+                    for (int i = 0; i < nz; i++)
+                        for (int t = 0; t < 7; t++) {
+                            const int j = i - 3 + t;
+                            rt[i].c[t] = j >= 0 && j < nz ? rows[j].c[6 - t] : 0.0;
+                        }
+                    std::vector<double> ft;
+                    if (cft::hept_factor(rt, ft)) {
+                        cf_set_error("zero pivot in the order-4 implicit z system (substep %d)", s);
+                        return CF_ERR_NUMERIC;
+                    }
+                    weights(s, type, [&](const std::vector<double> &lv, std::vector<double> &x) { cft::hept_solve(ft, nz, lv, x); });
+                }
                 /* unit-forcing profile (chanfast.c:1422-1424) and its statistics */
                 std::vector<double> rr(nz), x;
                 for (int k = 0; k < nz; k++) rr[k] = C.gamdt * dzl[k];
@@ -945,6 +1012,8 @@ static cf_status build_tables(const cf_config *cfg, const std::vector<double> &d
             o_sp[s][t][4] = put(S.wr.data(), S.wr.size()); o_sp[s][t][5] = put(S.minv.data(), S.minv.size());
         }
     T.o_lift = put(liftg.data(), liftg.size());
+    T.o_mwq = put(mwq.data(), mwq.size());
+    T.o_mlf = put(mlf.data(), mlf.size());
     size_t (&o_hp)[3][3] = T.o_hp;
     size_t (&o_p4)[4] = T.o_p4;
     memset(o_hp, 0, sizeof(T.o_hp));
@@ -993,6 +1062,9 @@ static void apply_tables(cf_run *r, const TabPack &TP)
     R.rdzh = tab + TP.o_rdzh;
     R.cl = TP.clo;
     R.liftg = tab + TP.o_lift;
+    R.mwq = tab + TP.o_mwq;
+    R.mlf = tab + TP.o_mlf;
+    memcpy(R.mcf, TP.mcf, sizeof(R.mcf));
     for (int s = 0; s < 3; s++) {
         R.sc[s] = TP.sc[s];
         for (int f = 0; f < 4; f++) R.lift[s][f] = TP.lift[s][f];
@@ -1163,12 +1235,6 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     ok = ok && falloc(&r->p, r->N) && dalloc(&r->stage, r->N) && dalloc(&r->G, r->M * glev);
     ok = ok && hipMalloc((void **) &r->X, 2 * r->esz * r->M * nz) == hipSuccess;
     ok = ok && dalloc(&r->tab, r->tab_n) && dalloc(&r->scal, SC_N) && dalloc(&r->logbuf, (size_t) LOGCAP * CF_LOG_N);
-    r->nb_plane = (int) ((r->P + 2047) / 2048);
-    if (r->nb_plane > 1024) r->nb_plane = 1024;
-    r->nb_red = 1024;
-    size_t npart = std::max((size_t) r->nb_plane * (2 * nz + 2), (size_t) ((r->P + 63) / 64) * nz);
-    if (npart < (size_t) r->nb_red) npart = r->nb_red;
-    ok = ok && dalloc(&r->part, npart) && dalloc(&r->lsum, (size_t) nz + 2);
     rhs_chunks(nx, ny, nz, rhs_target({ &r->g }, CF_RHS_KC), &r->rhs_kc, &r->rhs_blocks);
     r->gblocks = ((nx + 63) / 64) * ((ny + 3) / 4) * nz;
     if (cfg->order == 4 && nx % CF_R4_X == 0 && ny % CF_R4_Y == 0
@@ -1176,6 +1242,13 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
         r->r4_nch = std::max(1, (nz + CF_R4_KC / 2) / CF_R4_KC);
         r->r4_blocks = (nx / CF_R4_X) * (ny / CF_R4_Y) * r->r4_nch;
     }
+    r->nb_red = 1024;
+    /* part: a batch's plane sums of the solve, the RHS launch's partial sums
+     * (four statistics of u and, with the scalar, c) and the divergence
+     * check's maxima */
+    const size_t npart = std::max({ (size_t) ((r->P + 63) / 64) * nz, (size_t) r->nb_red,
+                                    (size_t) 4 * std::max({ r->gblocks, r->rhs_blocks, r->r4_blocks }) * (cfg->scalar ? 2 : 1) });
+    ok = ok && dalloc(&r->part, npart) && dalloc(&r->lsum, (size_t) nz + 2);
     /* a batch may cut the run's z-chunks otherwise, down to one level */
     ok = ok && dalloc(&r->cflpart, (size_t) std::max({ (int) (rhs_tiles(nx, ny) * nz), r->gblocks, r->r4_blocks }));
     if (cfg->cflmode == 1) ok = ok && dalloc(&r->h1prev, (size_t) nz + 2);
@@ -1397,6 +1470,37 @@ static cf_status enqueue_materialise(cf_run *r, double *u, double *v, double *w)
     return r->prec == CF_FP32 ? enqueue_materialise_t<float>(r, u, v, w) : enqueue_materialise_t<double>(r, u, v, w);
 }
 
+/* the z solves of nf fields in place, with the substep's bookkeeping */
+template <typename T>
+static cf_status enqueue_zsolve(cf_run *r, const char *name, int s, unsigned nf, T *ru, T *rv, T *rw, T *rc, const Book &B)
+{
+    const RunDev &R = r->rd;
+    const unsigned nb64 = (unsigned) ((r->P + 63) / 64), nb256 = (unsigned) ((r->P + 255) / 256);
+    if (r->g.order == 4 && r->use_spike4)
+        KLAUNCH(name, pick_spike4<T>(r->s4_L), dim3(nb64 * nf + 1), dim3(64 * r->s4_waves), 0, R, s, (int) nb64, ru, rv, rw, rc, B);
+    else if (r->g.order == 4)
+        KLAUNCH(name, k_gsolve4<T>, dim3(nb256 * nf + 1), dim3(256), 0, R, s, (int) nb256, ru, rv, rw, rc, B);
+    else if (r->use_spike)
+        KLAUNCH(name, pick_spike<T>(r->sp_L), dim3(nb64 * nf + 1), dim3(64 * r->spike_waves), 0, R, s, (int) nb64, ru, rv, rw, rc, B);
+    else
+        KLAUNCH(name, k_thomas<T>, dim3(nb256 * nf + 1), dim3(256), 0, R, s, (int) nb256, ru, rv, rw, rc, B);
+    return CF_OK;
+}
+
+/* the bookkeeping of substep s after an RHS launch of n workgroups */
+static Book make_book(const cf_run *r, int s, int n, double dt)
+{
+    Book B;
+    B.s = s;
+    B.n = n;
+    B.part = r->part;
+    B.cflpart = s == 0 ? r->cflpart : nullptr;
+    B.scal = r->scal;
+    B.logbuf = r->logbuf;
+    B.dt = dt;
+    return B;
+}
+
 /* one RK3 step from state set `from` to the other set */
 template <typename T>
 static cf_status enqueue_step_t(cf_run *r, int from)
@@ -1421,41 +1525,15 @@ static cf_status enqueue_step_t(cf_run *r, int from)
             S.h1 = r->h1prev;
             S.dtp = r->dtp_prev;
         }
-        /* zeta = 0 (first substep): no previous tendency; the last substep's
-         * tendency is never read (the next step starts with zeta = 0) */
-        const bool useg = RK_ZET[s] != 0.0, keepf = s < 2;
-        KLAUNCH("rhs", k_rhs2t<T>, dim3(r->rhs_blocks), dim3(256), 0, R, s, S,
-                (const T *) (useg ? tv<T>(gold[0]) : nullptr), (const T *) tv<T>(gold[1]), (const T *) tv<T>(gold[2]),
-                (const double *) r->scal, keepf ? tv<T>(fnew[0]) : nullptr, tv<T>(fnew[1]), tv<T>(fnew[2]), ou, ov, ow,
-                s == 0 ? r->cflpart : (double *) nullptr, dt, r->rhs_kc);
-        if (s == 0)
-            KLAUNCH("cfl_finish", k_cfl_finish, dim3(1), dim3(256), 0, R, (const double *) r->cflpart,
-                    r->rhs_blocks, dt, r->scal, r->logbuf);
-        const int nbx = (int) ((r->P + 63) / 64);
-        if (r->use_spike) {
-            /* the solve with the first stage of the plane sums of u* fused in */
-            KLAUNCH("spike", pick_spike_sums<T>(r->sp_L), dim3((unsigned) nbx, 3), dim3(64 * r->spike_waves), 0, R, s,
-                    ou, ov, ow, r->part);
-            /* the level sums and the constraint in one launch (its last
-             * workgroup finishes); the last substep also counts the step */
-            KLAUNCH("plane_sum", k_level_mass, dim3((unsigned) nz), dim3(256), sizeof(double) * (nz + 2), R, s,
-                    (const double *) r->part, nbx, r->lsum, r->scal, r->logbuf, s == 2 ? 1 : 0);
-        } else {
-            KLAUNCH("thomas", k_thomas<T>, dim3((unsigned) ((r->P + 255) / 256), 3), dim3(256), 0, R, s, ou, ov, ow,
-                    (T *) nullptr);
-            KLAUNCH("plane_sum", k_gplane<T>, dim3(r->nb_plane, nz, 1), dim3(256), 0, R, (const T *) ou,
-                    (const T *) nullptr, r->part, r->nb_plane);
-            KLAUNCH("plane_sum", k_level_sum, dim3((unsigned) nz), dim3(256), 0, (const double *) r->part, r->nb_plane,
-                    r->lsum);
-        }
-        if (!r->use_spike)
-            KLAUNCH("mass", k_mass_finalize, dim3(1), dim3(256), sizeof(double) * (nz + 2), R, s,
-                    (const double *) r->lsum, r->scal, r->logbuf, 0);
+        KLAUNCH("rhs", pick_rhs2<T>(s), dim3(r->rhs_blocks), dim3(256), 0, R, S, (const T *) tv<T>(gold[0]),
+                (const T *) tv<T>(gold[1]), (const T *) tv<T>(gold[2]), (const double *) r->scal, tv<T>(fnew[0]),
+                tv<T>(fnew[1]), tv<T>(fnew[2]), ou, ov, ow, r->cflpart, dt, r->rhs_kc, r->part);
+        cf_status st = enqueue_zsolve<T>(r, "spike", s, 3, ou, ov, ow, nullptr, make_book(r, s, r->rhs_blocks, dt));
+        if (st != CF_OK) return st;
         const double *h1 = R.h1 + (size_t) (s * 2 + 0) * (nz + 2);
-        cf_status st = enqueue_pressure<T>(r, ou, ov, ow, h1, r->scal + SC_M0 + s, s);
+        st = enqueue_pressure<T>(r, ou, ov, ow, h1, r->scal + SC_M0 + s, s);
         if (st != CF_OK) return st;
     }
-    if (!r->use_spike) KLAUNCH("step_end", k_step_end, dim3(1), dim3(64), 0, r->scal);
     return CF_OK;
 }
 
@@ -1520,74 +1598,44 @@ static cf_status enqueue_step_general_t(cf_run *r)
         if (r->r4_nch > 0) {
             /* order 4 on tiles that divide the grid: two z-marching launches */
             const dim3 g4((unsigned) r->r4_blocks);
-            if (sc) {
-                KLAUNCH("rhs", (k_rhs4_uv<true, T>), g4, dim3(256), 0, R, s, (const T *) u, (const T *) v, (const T *) w,
-                        (const T *) c, (const T *) tv<T>(gold[0]), (const T *) tv<T>(gold[1]), (const double *) r->scal,
-                        tv<T>(fnew[0]), tv<T>(fnew[1]), ru, rv, s == 0 ? r->cflpart : (double *) nullptr, dt, r->r4_nch);
-                KLAUNCH("rhs", (k_rhs4_wc<true, T>), g4, dim3(256), 0, R, s, (const T *) u, (const T *) v, (const T *) w,
-                        (const T *) c, (const T *) tv<T>(gold[2]), (const T *) tv<T>(gold[3]), (const double *) r->scal,
-                        tv<T>(fnew[2]), tv<T>(fnew[3]), rw, rc, r->r4_nch);
-            } else {
-                KLAUNCH("rhs", (k_rhs4_uv<false, T>), g4, dim3(256), 0, R, s, (const T *) u, (const T *) v, (const T *) w,
-                        (const T *) nullptr, (const T *) tv<T>(gold[0]), (const T *) tv<T>(gold[1]), (const double *) r->scal,
-                        tv<T>(fnew[0]), tv<T>(fnew[1]), ru, rv, s == 0 ? r->cflpart : (double *) nullptr, dt, r->r4_nch);
-                KLAUNCH("rhs", (k_rhs4_wc<false, T>), g4, dim3(256), 0, R, s, (const T *) u, (const T *) v, (const T *) w,
-                        (const T *) nullptr, (const T *) tv<T>(gold[2]), (const T *) nullptr, (const double *) r->scal,
-                        tv<T>(fnew[2]), (T *) nullptr, rw, (T *) nullptr, r->r4_nch);
-            }
-            if (s == 0)
-                KLAUNCH("cfl_finish", k_cfl_finish, dim3(1), dim3(256), 0, R, (const double *) r->cflpart, r->r4_blocks,
-                        dt, r->scal, r->logbuf);
+            const T *cs = sc ? (const T *) c : nullptr;
+            KLAUNCH("rhs", pick_rhs4_uv<T>(sc, s), g4, dim3(256), 0, R, (const T *) u, (const T *) v, (const T *) w, cs,
+                    (const T *) tv<T>(gold[0]), (const T *) tv<T>(gold[1]), (const double *) r->scal, tv<T>(fnew[0]),
+                    tv<T>(fnew[1]), ru, rv, r->cflpart, dt, r->r4_nch, r->part);
+            KLAUNCH("rhs", pick_rhs4_wc<T>(sc, s), g4, dim3(256), 0, R, (const T *) u, (const T *) v, (const T *) w, cs,
+                    (const T *) tv<T>(gold[2]), (const T *) tv<T>(gold[3]), (const double *) r->scal, tv<T>(fnew[2]),
+                    tv<T>(fnew[3]), rw, rc, r->r4_nch, r->part + (size_t) 4 * r->r4_blocks);
         } else {
-            KLAUNCH("rhs", K.u, cg, cb, 0, R, s, u, v, w, c, (const T *) tv<T>(gold[0]), (const double *) r->scal,
-                    tv<T>(fnew[0]), ru, s == 0 ? r->cflpart : (double *) nullptr, dt);
-            if (s == 0)
-                KLAUNCH("cfl_finish", k_cfl_finish, dim3(1), dim3(256), 0, R, (const double *) r->cflpart, r->gblocks, dt,
-                        r->scal, r->logbuf);
-            KLAUNCH("rhs", K.v, cg, cb, 0, R, s, u, v, w, c, (const T *) tv<T>(gold[1]), (const double *) r->scal,
-                    tv<T>(fnew[1]), rv, (double *) nullptr, dt);
-            KLAUNCH("rhs", K.w, cg, cb, 0, R, s, u, v, w, c, (const T *) tv<T>(gold[2]), (const double *) r->scal,
-                    tv<T>(fnew[2]), rw, (double *) nullptr, dt);
-            if (sc)
-                KLAUNCH("rhs", K.c, cg, cb, 0, R, s, u, v, w, c, (const T *) tv<T>(gold[3]), (const double *) r->scal,
-                        tv<T>(fnew[3]), rc, (double *) nullptr, dt);
+            GFields<T> F;
+            F.u = u; F.v = v; F.w = w; F.c = c;
+            for (int t = 0; t < 4; t++) { F.g[t] = tv<T>(gold[t]); F.f[t] = tv<T>(fnew[t]); }
+            F.r[0] = ru; F.r[1] = rv; F.r[2] = rw; F.r[3] = rc;
+            KLAUNCH("rhs", K.rhs, dim3(cg.x, cg.y, cg.z * (sc ? 4 : 3)), cb, 0, R, s, F, (const double *) r->scal,
+                    s == 0 ? r->cflpart : (double *) nullptr, dt, r->part);
         }
-        const unsigned nf = (unsigned) r->nfield;
-        if constexpr (std::is_same<T, double>::value) {
-            if (R.implicit) {
-                cf_status st = enqueue_spectral_solve(r, s, 0, ru);
+        const Book B = make_book(r, s, r->r4_nch > 0 ? r->r4_blocks : r->gblocks, dt);
+        cf_status st = CF_OK;
+        if (R.implicit) {
+            if constexpr (std::is_same<T, double>::value) {
+                KLAUNCH("mass", k_book, dim3(1), dim3(256), 0, R, B);
+                st = enqueue_spectral_solve(r, s, 0, ru);
                 if (st == CF_OK) st = enqueue_spectral_solve(r, s, 0, rv);
                 if (st == CF_OK && sc) st = enqueue_spectral_solve(r, s, 1, rc);
                 if (st == CF_OK) st = enqueue_spectral_solve(r, s, 2, rw);
-                if (st != CF_OK) return st;
             }
+        } else {
+            st = enqueue_zsolve<T>(r, "solve", s, (unsigned) r->nfield, ru, rv, rw, rc, B);
         }
-        if (R.implicit) {
-            /* done above */
-        } else if (r->g.order == 4 && r->use_spike4)
-            KLAUNCH("solve", pick_spike4<T>(r->s4_L), dim3((unsigned) ((r->P + 63) / 64), nf), dim3(64 * r->s4_waves), 0,
-                    R, s, ru, rv, rw, rc);
-        else if (r->g.order == 4)
-            KLAUNCH("solve", k_gsolve4<T>, dim3((unsigned) ((r->P + 255) / 256), nf), dim3(256), 0, R, s, ru, rv, rw, rc);
-        else if (r->use_spike)
-            KLAUNCH("solve", pick_spike<T>(r->sp_L), dim3((unsigned) ((r->P + 63) / 64), nf), dim3(64 * r->spike_waves), 0, R, s,
-                    ru, rv, rw, rc);
-        else
-            KLAUNCH("solve", k_thomas<T>, dim3((unsigned) ((r->P + 255) / 256), nf), dim3(256), 0, R, s, ru, rv, rw, rc);
-        KLAUNCH("plane_sum", k_gplane<T>, dim3(r->nb_plane, nz, sc ? 2 : 1), dim3(256), 0, R, (const T *) ru,
-                (const T *) rc, r->part, r->nb_plane);
-        KLAUNCH("mass", k_gmass, dim3(sc ? 2 : 1), dim3(256), sizeof(double) * (nz + 6), R, s,
-                (const double *) r->part, r->nb_plane, r->scal, r->logbuf);
+        if (st != CF_OK) return st;
         const double *h1u = R.h1 + (size_t) (s * 2 + 0) * (nz + 2);
         const double *h1c = R.h1 + (size_t) (s * 2 + 1) * (nz + 2);
-        cf_status st = enqueue_pressure<T>(r, ru, rv, rw, h1u, r->scal + SC_M0 + s, s);
+        st = enqueue_pressure<T>(r, ru, rv, rw, h1u, r->scal + SC_M0 + s, s);
         if (st != CF_OK) return st;
         KLAUNCH("project", K.proj, cg, cb, 0, R, (const T *) ru, (const T *) rv, (const T *) rw, (const T *) rc, h1u,
                 (const double *) (r->scal + SC_M0 + s), sc ? h1c : (const double *) nullptr,
                 (const double *) (r->scal + SC_MC0 + s), (const T *) tv<T>(r->p), R.sc[s].abdt, u, v, w,
                 sc ? c : (T *) nullptr);
     }
-    KLAUNCH("step_end", k_step_end, dim3(1), dim3(64), 0, r->scal);
     return CF_OK;
 }
 
@@ -2283,14 +2331,12 @@ extern "C" cf_status cf_op_poisson(cf_run *r, double *spec, double dt)
  * state untouched).
  */
 
-enum { KB_RHS_U = 0, KB_RHS_V, KB_RHS_W, KB_RHS_C, KB_SOLVE, KB_PLANE, KB_MASS, KB_CFL, KB_DIVX, KB_FFTY,
-       KB_POIS, KB_FFTXI, KB_PROJ, KB_STEPEND, KB_FRHS, KB_FSPIKE, KB_FLEVEL, KB_FMASS, KB_N };
-static const int KB_STAGE[KB_N] = { ST_CELL, ST_CELL, ST_CELL, ST_CELL, ST_SOLVE, ST_PLANE, ST_MASS, ST_ONE,
-                                    ST_FFTX, ST_FFTY, ST_MODE, ST_FFTX, ST_CELL, ST_ONE,
-                                    ST_RHS2, ST_SOLVE, ST_LEVEL, ST_ONE };
-static const char *KB_NAME[KB_N] = { "rhs", "rhs", "rhs", "rhs", "solve", "plane_sum", "mass", "cfl_finish",
-                                     "div_fftx", "ffty", "poisson", "fftx_inv", "project", "step_end",
-                                     "rhs", "spike", "plane_sum", "mass" };
+enum { KB_RHS = 0, KB_SOLVE, KB_MASS, KB_DIVX, KB_FFTY, KB_POIS, KB_FFTXI, KB_PROJ, KB_FRHS, KB_FSPIKE, KB_FLEVEL,
+       KB_N };
+static const int KB_STAGE[KB_N] = { ST_RHSG, ST_SOLVE, ST_ONE, ST_FFTX, ST_FFTY, ST_MODE, ST_FFTX, ST_CELL,
+                                    ST_RHS2, ST_SOLVE, ST_LEVEL };
+static const char *KB_NAME[KB_N] = { "rhs", "solve", "mass", "div_fftx", "ffty", "poisson", "fftx_inv", "project",
+                                     "rhs", "spike", "plane_sum" };
 enum { SOLVE_HEPT = 0, SOLVE_SPIKE = 1, SOLVE_THOMAS = 2 };
 
 struct cf_batch {
@@ -2393,7 +2439,6 @@ static void batch_fill_args(cf_batch *b, std::vector<GArgs<T>> &A)
         a.lsum = r->lsum;
         a.dt = r->cfg.dt;
         a.dt_adhoc = r->pt_dt;
-        a.nb_plane = r->nb_plane;
         /* a batch that fills the GPU takes longer RHS z-chunks (fewer halo
          * re-reads) than a run alone; the chunking does not change results */
         int bkc = 1, bblocks = 0;
@@ -2402,13 +2447,12 @@ static void batch_fill_args(cf_batch *b, std::vector<GArgs<T>> &A)
         a.rhs_kc = bkc;
         for (int t = 0; t < 4; t++) { a.pt[t] = r->pt[t]; a.pt4[t] = r->pt4[t]; }
         const unsigned nx = r->g.nx, ny = r->g.ny, nz = r->g.nz;
-        const unsigned P = (unsigned) r->P, nf = (unsigned) r->nfield, kinds = r->cfg.scalar ? 2u : 1u;
+        const unsigned P = (unsigned) r->P, nf = (unsigned) r->nfield;
         auto set = [&](int st, unsigned x, unsigned y, unsigned z) { a.dims[st][0] = x; a.dims[st][1] = y; a.dims[st][2] = z; };
         set(ST_CELL, (nx + 63) / 64, (ny + 3) / 4, nz);
+        set(ST_RHSG, (nx + 63) / 64, (ny + 3) / 4, nz * nf);
         if (run_uses_spike(b, r)) set(ST_SOLVE, (P + 63) / 64, nf, 1);
         else set(ST_SOLVE, (P + 255) / 256, nf, 1);
-        set(ST_PLANE, (unsigned) r->nb_plane, nz, kinds);
-        set(ST_MASS, kinds, 1, 1);
         set(ST_ONE, 1, 1, 1);
         long NL = (long) ny * nz, npairs = (NL + 1) / 2;
         set(ST_FFTX, (unsigned) ((npairs + r->rd.fx_pairs - 1) / r->rd.fx_pairs), 1, 1);
@@ -2567,10 +2611,7 @@ static cf_status batch_launch(cf_batch *b, int k, int s)
     dim3 block(256);
     size_t lds = 0;
     switch (k) {
-    case KB_RHS_U: fn = S.u; block = dim3(64, 4); break;
-    case KB_RHS_V: fn = S.v; block = dim3(64, 4); break;
-    case KB_RHS_W: fn = S.w; block = dim3(64, 4); break;
-    case KB_RHS_C: fn = S.c; block = dim3(64, 4); break;
+    case KB_RHS: fn = S.rhs; block = dim3(64, 4); break;
     case KB_PROJ: fn = S.proj; block = dim3(64, 4); break;
     case KB_SOLVE:
         if (b->solve_kind == SOLVE_HEPT) { fn = kb_solve4<T>; break; }
@@ -2589,9 +2630,7 @@ static cf_status batch_launch(cf_batch *b, int k, int s)
             HIPCHK(hipGetLastError());
             return bev_end(b);
         }
-    case KB_PLANE: fn = kb_plane<T>; break;
-    case KB_MASS: fn = kb_mass<T>; lds = b->lds_mass; break;
-    case KB_CFL: fn = kb_cfl<T>; break;
+    case KB_MASS: fn = kb_mass<T>; break;
     case KB_DIVX:
         /* FP64: one runtime-plan launch over all runs (its compiled forms
          * spill beyond length 64, and split launches measured slower) */
@@ -2632,12 +2671,10 @@ static cf_status batch_launch(cf_batch *b, int k, int s)
             }
             return bev_end(b);
         }
-    case KB_STEPEND: fn = kb_step_end<T>; break;
-    case KB_FRHS: fn = kb_rhs2t<T>; break;
+    case KB_FRHS: fn = pick_batched_rhs2<T>(s); break;
     case KB_FSPIKE:
         return batch_launch_spike<T>(b, k, s, true);
-    case KB_FLEVEL: fn = kb_level_sum<T>; break;
-    case KB_FMASS: fn = kb_mass_fast<T>; lds = b->lds_mass; break;
+    case KB_FLEVEL: fn = kb_level_mass<T>; lds = b->lds_mass; break;
     default: cf_set_error("bad batch kernel slot %d", k); return CF_ERR_ARG;
     }
     if (!fn) return CF_OK;
@@ -2669,18 +2706,13 @@ static cf_status batch_enqueue_step(cf_batch *b)
 {
     cf_status st;
     for (int s = 0; s < 3; s++) {
-        if ((st = batch_launch<T>(b, KB_RHS_U, s)) != CF_OK) return st;
-        if (s == 0 && (st = batch_launch<T>(b, KB_CFL, s)) != CF_OK) return st;
-        if ((st = batch_launch<T>(b, KB_RHS_V, s)) != CF_OK) return st;
-        if ((st = batch_launch<T>(b, KB_RHS_W, s)) != CF_OK) return st;
-        if (b->scalar && (st = batch_launch<T>(b, KB_RHS_C, s)) != CF_OK) return st;
+        if ((st = batch_launch<T>(b, KB_RHS, s)) != CF_OK) return st;
         if ((st = batch_launch<T>(b, KB_SOLVE, s)) != CF_OK) return st;
-        if ((st = batch_launch<T>(b, KB_PLANE, s)) != CF_OK) return st;
         if ((st = batch_launch<T>(b, KB_MASS, s)) != CF_OK) return st;
         if ((st = batch_enqueue_pressure<T>(b, s)) != CF_OK) return st;
         if ((st = batch_launch<T>(b, KB_PROJ, s)) != CF_OK) return st;
     }
-    return batch_launch<T>(b, KB_STEPEND, 0);
+    return CF_OK;
 }
 
 /* one RK3 step of a fast batch starting from state set `from`: the fast
@@ -2692,14 +2724,12 @@ static cf_status fbatch_enqueue_step_t(cf_batch *b, int from)
     for (int s = 0; s < 3; s++) {
         b->tab = (from + s) & 1;
         if ((st = batch_launch<T>(b, KB_FRHS, s)) != CF_OK) return st;
-        if (s == 0 && (st = batch_launch<T>(b, KB_CFL, s)) != CF_OK) return st;
         if ((st = batch_launch<T>(b, KB_FSPIKE, s)) != CF_OK) return st;
         if ((st = batch_launch<T>(b, KB_FLEVEL, s)) != CF_OK) return st;
-        if ((st = batch_launch<T>(b, KB_FMASS, s)) != CF_OK) return st;
         if ((st = batch_enqueue_pressure<T>(b, s)) != CF_OK) return st;
     }
     b->tab = 0;
-    return batch_launch<T>(b, KB_STEPEND, 0);
+    return CF_OK;
 }
 
 static cf_status fbatch_enqueue_step(cf_batch *b, int from)
@@ -2769,12 +2799,10 @@ static cf_status batch_autotune(cf_batch *b)
     }
     if ((st = batch_upload_tables<T>(b)) != CF_OK) return st;
     /* slots whose repeated launch is harmless on a zero state and that do real work */
-    const int gslots[] = { KB_RHS_U, KB_RHS_V, KB_RHS_W, KB_RHS_C, KB_SOLVE, KB_PLANE, KB_DIVX, KB_FFTY, KB_POIS,
-                           KB_FFTXI, KB_PROJ };
+    const int gslots[] = { KB_RHS, KB_SOLVE, KB_DIVX, KB_FFTY, KB_POIS, KB_FFTXI, KB_PROJ };
     const int fslots[] = { KB_FRHS, KB_FSPIKE, KB_DIVX, KB_FFTY, KB_POIS, KB_FFTXI };
-    std::vector<int> slots = b->fast ? std::vector<int>(fslots, fslots + 6) : std::vector<int>(gslots, gslots + 11);
+    std::vector<int> slots = b->fast ? std::vector<int>(fslots, fslots + 6) : std::vector<int>(gslots, gslots + 7);
     for (int k : slots) {
-        if (k == KB_RHS_C && !b->scalar) continue;
         const unsigned total = batch_total(b, KB_STAGE[k]);
         std::vector<unsigned> cand = { 0 };
         for (int m : { 1, 2, 4, 8, 16 })
@@ -2793,7 +2821,6 @@ static cf_status batch_autotune(cf_batch *b)
                  bg ? bg : total, total, 1e3 * best);
         b->tuning.push_back(line);
     }
-    b->kgrid[KB_RHS_C] = b->kgrid[KB_RHS_C] ? b->kgrid[KB_RHS_C] : b->kgrid[KB_RHS_U];
     /* the tuning launches wrote forcings, log entries and (through the
      * scalar's boundary lift) state values: restore the zero state */
     for (cf_run *r : b->runs) {
@@ -2882,7 +2909,7 @@ extern "C" cf_status cf_batch_create(const cf_config *cfgs, int nrun, cf_batch *
         b->spike_waves = std::max(b->spike_waves, r->spike_waves);
         b->lds_fx = std::max(b->lds_fx, fx_lds(r));
         b->lds_fy = std::max(b->lds_fy, fy_lds(r));
-        b->lds_mass = std::max(b->lds_mass, sizeof(double) * (size_t) (r->g.nz + 6));
+        b->lds_mass = std::max(b->lds_mass, sizeof(double) * (size_t) r->g.nz);
     }
     b->p2L = batch_p2L(b->runs);
     HIPCHK(hipSetDevice(b->device));
@@ -3312,7 +3339,7 @@ static cf_status srv_regroup(cf_server *s, int k, cf_server::Group &G)
         b->spike_waves = std::max(b->spike_waves, r->spike_waves);
         b->lds_fx = std::max(b->lds_fx, fx_lds(r));
         b->lds_fy = std::max(b->lds_fy, fy_lds(r));
-        b->lds_mass = std::max(b->lds_mass, sizeof(double) * (size_t) (r->g.nz + 6));
+        b->lds_mass = std::max(b->lds_mass, sizeof(double) * (size_t) r->g.nz);
     }
     b->solve_kind = b->order == 4 ? SOLVE_HEPT : SOLVE_SPIKE;   /* per run: spike or Thomas as alone */
     b->p2L = batch_p2L(runs);

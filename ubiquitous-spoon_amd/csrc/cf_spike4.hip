@@ -22,14 +22,19 @@
 #include "cf_kernels.h"
 
 template <typename T, int LM>
-__global__ __launch_bounds__(64 * CF_SPIKE4_SMAX) void k_spike4(const RunDev R, const int s,
-    T *__restrict__ ru, T *__restrict__ rv, T *__restrict__ rw, T *__restrict__ rc)
+__global__ __launch_bounds__(64 * CF_SPIKE4_SMAX) void k_spike4(const RunDev R, const int s, const int nbx,
+    T *__restrict__ ru, T *__restrict__ rv, T *__restrict__ rw, T *__restrict__ rc, const Book B)
 {
+    if (blockIdx.x == 0) {
+        book_body(R, B);
+        return;
+    }
+    const Blk b = blk_solve(blockIdx.x - 1, nbx);
     constexpr int MP = 6 * CF_SPIKE4_SMAX;
     __shared__ T itf[MP][64];
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
     const size_t P = (size_t) nx * ny;
-    const int f = blockIdx.y;
+    const int f = b.y;
     const int type = f == 2 ? 2 : (f == 3 ? 1 : 0);
     const Spike4Tab ST = R.s4[s][type];
     const int lane = threadIdx.x & 63;
@@ -37,7 +42,7 @@ __global__ __launch_bounds__(64 * CF_SPIKE4_SMAX) void k_spike4(const RunDev R, 
      * the tables hold LM rows per chunk, identity past the system's end */
     const int chunk = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool live = chunk < ST.S;
-    const size_t col = (size_t) blockIdx.x * 64 + lane;
+    const size_t col = (size_t) b.x * 64 + lane;
     const bool act = col < P;
     const gp<T> x = (gp<T>) (f == 0 ? ru : (f == 1 ? rv : (f == 2 ? rw : rc)));
     const int lo = chunk * LM;
