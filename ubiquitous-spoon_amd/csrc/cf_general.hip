@@ -23,23 +23,59 @@ static constexpr double A2d = -0.125 / 3.0;
 static constexpr double B1d = 1.125 / 2.0;
 static constexpr double B2d = -0.125 / 2.0;
 
-/* ------------------------------------------------------------ columns */
+/* ------------------------------------------------------------ points */
 
-/* a cell field's values at levels k-3..k+3 of column cc, ghosts from the
- * closure (ghost m of a wall = G[m] . (x0, x1, x2) + B[m] bc) */
-template <int ORD, typename T>
-static __device__ __forceinline__ void cell_col7(const T *__restrict__ q, size_t P, size_t cc, int k, int nz,
-                                                 const Clos1 *C, double bcb, double bct, T o[7])
+static __device__ __forceinline__ size_t rowof(int k, int j, int nx, size_t P) { return (size_t) k * P + (size_t) j * nx; }
+
+/* One thread's point (i, j, k) of a 256-thread workgroup that takes 256
+ * consecutive cells of a level (a row's end does not idle its lanes: 90 of
+ * 128 lanes worked in 64-wide row blocks at nx = 90).  The level is
+ * uniform, so a value's address is a scalar base and a 32-bit byte offset
+ * in the plane. */
+template <typename T> struct Pt {
+    int nx, ny, nz, i, j, k;
+    size_t P;
+    bool act;
+    __device__ __forceinline__ Pt(const RunDev &R, const Blk &b)
+    {
+        nx = R.g.nx; ny = R.g.ny; nz = R.g.nz; k = b.z;
+        P = (size_t) nx * ny;
+        const int e = (int) b.x * 256 + (int) threadIdx.x;
+        act = e < (int) P;
+        const int ec = act ? e : (int) P - 1;
+        j = qdiv(ec, nx, R.rnx);
+        i = ec - j * nx;
+    }
+    /* byte offset in the plane of the point shifted by (d, e), periodic */
+    __device__ __forceinline__ unsigned off(int d, int e) const
+    {
+        return (unsigned) (wrapm(j + e, ny) * nx + wrapm(i + d, nx)) * (unsigned) sizeof(T);
+    }
+    __device__ __forceinline__ T at(gp<const T> f, int kk, unsigned o) const
+    {
+        return *(gp<const T>) ((gp<const char>) (f + (size_t) kk * P) + o);
+    }
+    __device__ __forceinline__ void put(gp<T> f, T v) const { *(gp<T>) ((gp<char>) (f + (size_t) k * P) + off(0, 0)) = v; }
+};
+
+/* a cell field's values at levels k-3..k+3 of the point's column (those
+ * within RCH of k), ghosts from the closure (ghost m of a wall = G[m] .
+ * (x0, x1, x2) + B[m] bc; order 2 has the one next to the wall) */
+template <int ORD, int RCH, typename T>
+static __device__ __forceinline__ void cell_col7(const Pt<T> &p, gp<const T> q, const Clos1 *C, double bcb, double bct, T o[7])
 {
+    const unsigned cc = p.off(0, 0);
+    const int k = p.k, nz = p.nz;
 #pragma unroll
     for (int t = 0; t < 7; t++) {
         const int kk = k - 3 + t;
-        o[t] = (kk >= 0 && kk < nz) ? q[(size_t) kk * P + cc] : (T) 0;
+        const bool reach = t - 3 <= RCH && 3 - t <= RCH;
+        o[t] = (reach && kk >= 0 && kk < nz) ? p.at(q, kk, cc) : (T) 0;
     }
     if (k < 3) {
         const Clos1 &B = C[0];
-        const T x0 = q[cc];
-        const T x1 = ORD == 4 ? q[P + cc] : (T) 0, x2 = ORD == 4 ? q[2 * P + cc] : (T) 0;
+        const T x0 = p.at(q, 0, cc);
+        const T x1 = ORD == 4 ? p.at(q, 1, cc) : (T) 0, x2 = ORD == 4 ? p.at(q, 2, cc) : (T) 0;
 #pragma unroll
         for (int m = 0; m < (ORD == 4 ? 3 : 1); m++) {
             const int t = -1 - m - k + 3;
@@ -48,9 +84,8 @@ static __device__ __forceinline__ void cell_col7(const T *__restrict__ q, size_t
     }
     if (k > nz - 4) {
         const Clos1 &Tp = C[1];
-        const T x0 = q[(size_t) (nz - 1) * P + cc];
-        const T x1 = ORD == 4 ? q[(size_t) (nz - 2) * P + cc] : (T) 0;
-        const T x2 = ORD == 4 ? q[(size_t) (nz - 3) * P + cc] : (T) 0;
+        const T x0 = p.at(q, nz - 1, cc);
+        const T x1 = ORD == 4 ? p.at(q, nz - 2, cc) : (T) 0, x2 = ORD == 4 ? p.at(q, nz - 3, cc) : (T) 0;
 #pragma unroll
         for (int m = 0; m < (ORD == 4 ? 3 : 1); m++) {
             const int t = nz + m - k + 3;
@@ -63,29 +98,31 @@ static __device__ __forceinline__ void cell_col7(const T *__restrict__ q, size_t
  * nz-1 are 0 and the ghost faces mirror oddly about them (apply_bc_w and
  * the in-place ghost rewrite of massflux*4, advect.c:100-131) */
 template <typename T>
-static __device__ __forceinline__ T wadv(const T *__restrict__ w, size_t P, size_t cc, int kk, int nz)
+static __device__ __forceinline__ T wadv(const Pt<T> &p, gp<const T> w, unsigned o, int kk)
 {
-    if (kk >= 0 && kk <= nz - 2) return w[(size_t) kk * P + cc];
-    if (kk == -1 || kk == nz - 1) return (T) 0;
-    if (kk < -1) return -w[(size_t) (-2 - kk) * P + cc];
-    return -w[(size_t) (2 * (nz - 1) - kk) * P + cc];
+    if (kk >= 0 && kk <= p.nz - 2) return p.at(w, kk, o);
+    if (kk == -1 || kk == p.nz - 1) return (T) 0;
+    if (kk < -1) return -p.at(w, -2 - kk, o);
+    return -p.at(w, 2 * (p.nz - 1) - kk, o);
 }
 
 /* w at levels k-3..k+3 for the implicit operator: closure ghosts
  * (apply_bc_w2/4 is re-applied before helmholtz1d_operator_w) */
 template <int ORD, typename T>
-static __device__ __forceinline__ void face_col7(const T *__restrict__ w, size_t P, size_t cc, int k, int nz,
-                                                 const Clos1 *C, T o[7])
+static __device__ __forceinline__ void face_col7(const Pt<T> &p, gp<const T> w, const Clos1 *C, T o[7])
 {
+    const unsigned cc = p.off(0, 0);
+    const int k = p.k, nz = p.nz;
 #pragma unroll
     for (int t = 0; t < 7; t++) {
         const int kk = k - 3 + t;
-        o[t] = (kk >= 0 && kk <= nz - 2) ? w[(size_t) kk * P + cc] : (T) 0;
+        const bool reach = ORD == 4 || (t >= 2 && t <= 4);
+        o[t] = (reach && kk >= 0 && kk <= nz - 2) ? p.at(w, kk, cc) : (T) 0;
     }
     if (k < 3) {
         const Clos1 &B = C[0];
-        const T x0 = w[cc];
-        const T x1 = ORD == 4 ? w[P + cc] : (T) 0, x2 = ORD == 4 ? w[2 * P + cc] : (T) 0;
+        const T x0 = p.at(w, 0, cc);
+        const T x1 = ORD == 4 ? p.at(w, 1, cc) : (T) 0, x2 = ORD == 4 ? p.at(w, 2, cc) : (T) 0;
 #pragma unroll
         for (int m = 0; m < (ORD == 4 ? 3 : 1); m++) {
             const int t = -1 - m - k + 3;
@@ -94,9 +131,8 @@ static __device__ __forceinline__ void face_col7(const T *__restrict__ w, size_t
     }
     if (k > nz - 5) {
         const Clos1 &Tp = C[1];
-        const T x0 = w[(size_t) (nz - 2) * P + cc];
-        const T x1 = ORD == 4 ? w[(size_t) (nz - 3) * P + cc] : (T) 0;
-        const T x2 = ORD == 4 ? w[(size_t) (nz - 4) * P + cc] : (T) 0;
+        const T x0 = p.at(w, nz - 2, cc);
+        const T x1 = ORD == 4 ? p.at(w, nz - 3, cc) : (T) 0, x2 = ORD == 4 ? p.at(w, nz - 4, cc) : (T) 0;
 #pragma unroll
         for (int m = 0; m < (ORD == 4 ? 3 : 1); m++) {
             const int t = nz - 1 + m - k + 3;
@@ -105,62 +141,53 @@ static __device__ __forceinline__ void face_col7(const T *__restrict__ w, size_t
     }
 }
 
-static __device__ __forceinline__ size_t rowof(int k, int j, int nx, size_t P) { return (size_t) k * P + (size_t) j * nx; }
+/* The stencils below divide by cell sizes through their host-computed
+ * reciprocals, with the sizes that a flux and its cell volume share
+ * cancelled: an FP64 division is a dozen instructions, and the per-field
+ * kernels were bound by their arithmetic (10 and more divisions a point;
+ * four fields at 90x73x75 in 24 us, 44 before). */
 
-/* cell/face 1-D Helmholtz operators (diffuseu.c:107-170, diffusew.c:107-172) */
+/* the second difference of a line at unit spacing, twice staggered */
 template <int ORD, typename T>
-static __device__ __forceinline__ T helm_cell(const T *Q, const double *dzd, int k, double nudtd)
+static __device__ __forceinline__ T d2(const T *X)
 {
+    if (ORD == 2) return (X[4] - X[3]) - (X[3] - X[2]);
     const T A1 = (T) A1d, A2 = (T) A2d;
-    const T nudt = (T) nudtd;
-    auto dz = [&](int kk) -> T { return (T) dzd[kk]; };
-    const T dzp1h = (T) 0.5 * (dz(k + 1) + dz(k));
-    const T dzm1h = (T) 0.5 * (dz(k - 1) + dz(k));
-    if (ORD == 2) return Q[3] + nudt * (((Q[4] - Q[3]) / dzp1h - (Q[3] - Q[2]) / dzm1h) / dz(k));
-    const T wp3h = A1 * (Q[5] - Q[4]) + A2 * (Q[6] - Q[3]);
-    const T wp1h = A1 * (Q[4] - Q[3]) + A2 * (Q[5] - Q[2]);
-    const T wm1h = A1 * (Q[3] - Q[2]) + A2 * (Q[4] - Q[1]);
-    const T wm3h = A1 * (Q[2] - Q[1]) + A2 * (Q[3] - Q[0]);
-    const T dzp3h = (T) 0.5 * (dz(k + 2) + dz(k + 1));
-    const T dzm3h = (T) 0.5 * (dz(k - 2) + dz(k - 1));
-    return Q[3] + nudt * ((A1 * (wp1h / dzp1h - wm1h / dzm1h) + A2 * (wp3h / dzp3h - wm3h / dzm3h)) / dz(k));
+    const T p3h = A1 * (X[5] - X[4]) + A2 * (X[6] - X[3]);
+    const T p1h = A1 * (X[4] - X[3]) + A2 * (X[5] - X[2]);
+    const T m1h = A1 * (X[3] - X[2]) + A2 * (X[4] - X[1]);
+    const T m3h = A1 * (X[2] - X[1]) + A2 * (X[3] - X[0]);
+    return A1 * (p1h - m1h) + A2 * (p3h - m3h);
 }
 
+/* cell/face 1-D Helmholtz operators (diffuseu.c:107-170, diffusew.c:107-172)
+ * Q + nudt d2Q/dz2: in are the reciprocal spacings between the levels (four
+ * of them about Q[3]: -3/2, -1/2, +1/2, +3/2), out the reciprocal height */
 template <int ORD, typename T>
-static __device__ __forceinline__ T helm_face(const T *Q, const double *dzd, int k, double nudtd)
+static __device__ __forceinline__ T helm(const T *Q, T rm3, T rm1, T rp1, T rp3, T rout, T nudt)
 {
+    if (ORD == 2) return Q[3] + nudt * (((Q[4] - Q[3]) * rp1 - (Q[3] - Q[2]) * rm1) * rout);
     const T A1 = (T) A1d, A2 = (T) A2d;
-    const T nudt = (T) nudtd;
-    auto dz = [&](int kk) -> T { return (T) dzd[kk]; };
-    const T dzp1 = dz(k + 1), dzm0 = dz(k);
-    const T dzp1h = (T) 0.5 * (dz(k + 1) + dz(k));
-    if (ORD == 2) return Q[3] + nudt * (((Q[4] - Q[3]) / dzp1 - (Q[3] - Q[2]) / dzm0) / dzp1h);
-    const T wp3h = A1 * (Q[5] - Q[4]) + A2 * (Q[6] - Q[3]);
-    const T wp1h = A1 * (Q[4] - Q[3]) + A2 * (Q[5] - Q[2]);
-    const T wm1h = A1 * (Q[3] - Q[2]) + A2 * (Q[4] - Q[1]);
-    const T wm3h = A1 * (Q[2] - Q[1]) + A2 * (Q[3] - Q[0]);
-    const T dzp2 = dz(k + 2), dzm1 = dz(k - 1);
-    return Q[3] + nudt * ((A1 * (wp1h / dzp1 - wm1h / dzm0) + A2 * (wp3h / dzp2 - wm3h / dzm1)) / dzp1h);
+    const T p3h = A1 * (Q[5] - Q[4]) + A2 * (Q[6] - Q[3]);
+    const T p1h = A1 * (Q[4] - Q[3]) + A2 * (Q[5] - Q[2]);
+    const T m1h = A1 * (Q[3] - Q[2]) + A2 * (Q[4] - Q[1]);
+    const T m3h = A1 * (Q[2] - Q[1]) + A2 * (Q[3] - Q[0]);
+    return Q[3] + nudt * ((A1 * (p1h * rp1 - m1h * rm1) + A2 * (p3h * rp3 - m3h * rm3)) * rout);
 }
 
-/* x-y diffusion nu (dxx + dyy) q of one point from its x and y lines
- * (add_laplacexy_operator_*, diffuseu.c:286-359) */
+/* a quantity at the middle of points 1 and 2 of four */
 template <int ORD, typename T>
-static __device__ __forceinline__ T lapxy(const T *X, const T *Y, T dx, T dy, T nu)
+static __device__ __forceinline__ T mid(T m, T a, T b, T p)
 {
-    const T A1 = (T) A1d, A2 = (T) A2d;
-    if (ORD == 2)
-        return nu * (((X[4] - X[3]) / dx - (X[3] - X[2]) / dx) / dx + ((Y[4] - Y[3]) / dy - (Y[3] - Y[2]) / dy) / dy);
-    const T up3h = A1 * (X[5] - X[4]) + A2 * (X[6] - X[3]);
-    const T up1h = A1 * (X[4] - X[3]) + A2 * (X[5] - X[2]);
-    const T um1h = A1 * (X[3] - X[2]) + A2 * (X[4] - X[1]);
-    const T um3h = A1 * (X[2] - X[1]) + A2 * (X[3] - X[0]);
-    const T vp3h = A1 * (Y[5] - Y[4]) + A2 * (Y[6] - Y[3]);
-    const T vp1h = A1 * (Y[4] - Y[3]) + A2 * (Y[5] - Y[2]);
-    const T vm1h = A1 * (Y[3] - Y[2]) + A2 * (Y[4] - Y[1]);
-    const T vm3h = A1 * (Y[2] - Y[1]) + A2 * (Y[3] - Y[0]);
-    return nu * ((A1 * (up1h / dx - um1h / dx) + A2 * (up3h / dx - um3h / dx)) / dx
-               + (A1 * (vp1h / dy - vm1h / dy) + A2 * (vp3h / dy - vm3h / dy)) / dy);
+    return ORD == 2 ? (T) 0.5 * (a + b) : (T) B1d * (a + b) + (T) B2d * (m + p);
+}
+
+/* the flux difference of one direction from the fluxes at +1/2, -1/2 and,
+ * order 4, +3/2, -3/2 */
+template <int ORD, typename T>
+static __device__ __forceinline__ T dif(T p1, T m1, T p3, T m3)
+{
+    return ORD == 2 ? p1 - m1 : (T) A1d * (p1 - m1) + (T) A2d * (p3 - m3);
 }
 
 /* wall values of u/v the advection of u/v uses on the wall faces
@@ -172,409 +199,242 @@ static __device__ __forceinline__ T wall_interp(T gm2, T gm1, T x0, T x1)
     return (T) (0.5 * A2d) * (gm2 + x1) + (T) (0.5 * (A1d + 2.0 * A2d)) * (gm1 + x0);
 }
 
-/* block max of the CFL partials (all threads of the block call it) */
-/* The reductions of a 64 x 4 workgroup at one level: the sum of r (one
- * value per thread) times the level's weight of each statistic of the
- * substep (mwq [nz][4]) into mpart (n slots a statistic) and, where cflpart
- * is set, the maximum of cfl (>= 0) */
+/* the reductions of a workgroup at one level: the sum of r (one value per
+ * thread) times the level's weight of each statistic of the substep (mwq
+ * [nz][4]) into mpart (n slots a statistic) and, where cflpart is set, the
+ * maximum of cfl (>= 0) */
 static __device__ __forceinline__ void block_store(double r, const double *__restrict__ mwq, int k, int s,
                                                    double *__restrict__ mpart, double cfl,
                                                    double *__restrict__ cflpart, unsigned bidx, unsigned n)
 {
     __shared__ double red[8];
+    const int t = threadIdx.x;
     const double w = wave_sum(r), c = cflpart ? wave_max_nonneg(cfl) : 0.0;
-    if (threadIdx.x == 0) { red[threadIdx.y] = w; red[4 + threadIdx.y] = c; }
+    if ((t & 63) == 0) { red[t >> 6] = w; red[4 + (t >> 6)] = c; }
     __syncthreads();
-    if (threadIdx.y != 0) return;
-    const int f = threadIdx.x;
-    if (f < book_stats(s)) mpart[(size_t) f * n + bidx] = mwq[4 * k + f] * (((red[0] + red[1]) + red[2]) + red[3]);
-    if (cflpart && f == 0) cflpart[bidx] = fmax(fmax(red[4], red[5]), fmax(red[6], red[7]));
+    if (t < book_stats(s)) mpart[(size_t) t * n + bidx] = mwq[4 * k + t] * (((red[0] + red[1]) + red[2]) + red[3]);
+    if (cflpart && t == 0) cflpart[bidx] = fmax(fmax(red[4], red[5]), fmax(red[6], red[7]));
 }
 
-/* ------------------------------------------------------------ u */
+/* ------------------------------------------------------------ u and v */
 
-/* advectu2/4 + laplacexy_u + buoyancy, then the u right-hand side of
- * solve_helmholtz1d_u (chanfast.c:465-477); CFL partials at s == 0 */
-template <int ORD, bool SC, typename T>
-static __device__ __forceinline__ void rhsu_body(const RunDev &R, const int s,
-    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-    const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ cflpart, double cfldt, double *__restrict__ mpart,
-    const Blk b)
+/* advectu2/4 or advectv2/4 + laplacexy + buoyancy, then the right-hand side
+ * of solve_helmholtz1d_u (chanfast.c:465-477) of u (AX = 0) or v (AX = 1):
+ * a is the advected field, the other horizontal velocity o; "along" is the
+ * direction of a.  CFL partials of u at s == 0. */
+template <int ORD, bool SC, int AX, typename T>
+static __device__ __forceinline__ void rhsuv_body(const RunDev &R, const int s, const GFields<T> &F,
+    const double *__restrict__ scal, double *__restrict__ cflpart, double cfldt, double *__restrict__ mpart, const Blk b)
 {
-    const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
-    const int i = b.x * 64 + threadIdx.x, j = b.y * 4 + threadIdx.y, k = b.z;
+    const Pt<T> p(R, b);
+    const int k = p.k, nz = p.nz;
+    const gp<const T> a = (gp<const T>) (AX == 0 ? F.u : F.v), o = (gp<const T>) (AX == 0 ? F.v : F.u);
+    const gp<const T> w = (gp<const T>) F.w, c = (gp<const T>) F.c, g = (gp<const T>) F.g[AX];
+    const cp<double> rdz = (cp<double>) R.rdz + CF_NGT, rdzh = (cp<double>) R.rdzh + CF_NGT, dz = (cp<double>) R.dzt + CF_NGT;
     double cflv = 0.0, rsum = 0.0;
-    if (i < nx && j < ny) {
-        const size_t P = (size_t) nx * ny;
-        const double *dz = R.dzt + CF_NGT;
-    const T A1 = (T) A1d, A2 = (T) A2d, B1 = (T) B1d, B2 = (T) B2d;
-    (void) A1; (void) A2; (void) B1; (void) B2;
-    auto DZ = [&](int kk) -> T { return (T) dz[kk]; };
-        const T dx = (T) R.g.dx, dy = (T) R.g.dy;
-        const size_t cc = (size_t) j * nx + i, q = (size_t) k * P + cc;
-        const size_t row = rowof(k, j, nx, P);
-        T U[7], UX[7], UY[7];
-        cell_col7<ORD>(u, P, cc, k, nz, R.cl.cell, R.ubc, R.ubc, U);
+    if (p.act) {
+        constexpr int LO = ORD == 2 ? 2 : 0, HI = ORD == 2 ? 4 : 6;
+        auto al = [&](int d) { return AX == 0 ? p.off(d, 0) : p.off(0, d); };      /* d along a's direction */
+        auto cr = [&](int d) { return AX == 0 ? p.off(0, d) : p.off(d, 0); };      /* d across it */
+        auto ac = [&](int d, int e) { return AX == 0 ? p.off(d, e) : p.off(e, d); };
+        const double bc = AX == 0 ? R.ubc : R.vbc;
+        T Z[7], A[7], C[7];
+        cell_col7<ORD, ORD == 2 ? 1 : 3>(p, a, R.cl.cell, bc, bc, Z);
 #pragma unroll
         for (int t = 0; t < 7; t++) {
-            UX[t] = (ORD == 2 && (t < 2 || t > 4)) ? (T) 0 : u[row + wrapm(i - 3 + t, nx)];
-            UY[t] = (ORD == 2 && (t < 2 || t > 4)) ? (T) 0 : u[rowof(k, wrapm(j - 3 + t, ny), nx, P) + i];
+            A[t] = t < LO || t > HI ? (T) 0 : (t == 3 ? Z[3] : p.at(a, k, al(t - 3)));
+            C[t] = t < LO || t > HI ? (T) 0 : (t == 3 ? Z[3] : p.at(a, k, cr(t - 3)));
         }
-        const T Q0 = U[3];
-        const T dzk = DZ(k);
-        /* massfluxx (advect.c:6-99): fluxes interpolated to the u-point in x */
-        auto MU = [&](int d) -> T {     /* at x-position i + d */
-            return ORD == 2 ? (T) 0.5 * (dy * dzk * UX[3 + d] + dy * dzk * UX[4 + d])
-                            : B1 * (dy * dzk * UX[3 + d] + dy * dzk * UX[4 + d])
-                            + B2 * (dy * dzk * UX[2 + d] + dy * dzk * UX[5 + d]);
+        const T Q0 = Z[3];
+        /* massfluxx / massfluxy (advect.c:6-200): velocities interpolated to
+         * a's point along its direction */
+        auto VA = [&](int d) -> T { return mid<ORD, T>(d >= -2 ? A[2 + d] : (T) 0, A[3 + d], A[4 + d], d <= 1 ? A[5 + d] : (T) 0); };
+        auto VC = [&](int e) -> T {
+            return mid<ORD, T>(ORD == 4 ? p.at(o, k, ac(-1, e)) : (T) 0, p.at(o, k, ac(0, e)), p.at(o, k, ac(1, e)),
+                               ORD == 4 ? p.at(o, k, ac(2, e)) : (T) 0);
         };
-        const int im = wrapm(i - 1, nx), ip = wrapm(i + 1, nx), ip2 = wrapm(i + 2, nx);
-        auto MV = [&](int e) -> T {     /* at y-position j + e */
-            const size_t r2 = rowof(k, wrapm(j + e, ny), nx, P);
-            if (ORD == 2) return (T) 0.5 * (dx * dzk * v[r2 + i] + dx * dzk * v[r2 + ip]);
-            return B1 * (dx * dzk * v[r2 + i] + dx * dzk * v[r2 + ip])
-                 + B2 * (dx * dzk * v[r2 + im] + dx * dzk * v[r2 + ip2]);
-        };
-        const size_t cj = (size_t) j * nx;
-        auto MW = [&](int e) -> T {     /* at face level k + e */
+        auto VZ = [&](int e) -> T {
             const int kk = k + e;
-            if (ORD == 2) return (T) 0.5 * (dx * dy * wadv(w, P, cj + i, kk, nz) + dx * dy * wadv(w, P, cj + ip, kk, nz));
-            return B1 * (dx * dy * wadv(w, P, cj + i, kk, nz) + dx * dy * wadv(w, P, cj + ip, kk, nz))
-                 + B2 * (dx * dy * wadv(w, P, cj + im, kk, nz) + dx * dy * wadv(w, P, cj + ip2, kk, nz));
+            return mid<ORD, T>(ORD == 4 ? wadv(p, w, al(-1), kk) : (T) 0, wadv(p, w, al(0), kk), wadv(p, w, al(1), kk),
+                               ORD == 4 ? wadv(p, w, al(2), kk) : (T) 0);
         };
-        T f;
-        const T den = dx * dy * dzk;
-        if (ORD == 2) {
-            T xp = MU(0) * (T) 0.5 * (Q0 + UX[4]), xm = MU(-1) * (T) 0.5 * (Q0 + UX[2]);
-            T yp = MV(0) * (T) 0.5 * (Q0 + UY[4]), ym = MV(-1) * (T) 0.5 * (Q0 + UY[2]);
-            const T mw0 = MW(0), mwm = MW(-1);
-            T zp = mw0 * (T) 0.5 * (Q0 + U[4]), zm = mwm * (T) 0.5 * (Q0 + U[2]);
-            if (k == nz - 1) zp = mw0 * wall_interp<2, T>((T) 0, U[4], U[3], (T) 0);
-            if (k == 0) zm = mwm * wall_interp<2, T>((T) 0, U[2], U[3], (T) 0);
-            f = -((xp - xm) + (yp - ym) + (zp - zm)) / den;
-        } else {
-            T xp = MU(0) * (T) 0.5 * (Q0 + UX[4]), xm = MU(-1) * (T) 0.5 * (Q0 + UX[2]);
-            T xp3 = MU(1) * (T) 0.5 * (Q0 + UX[6]), xm3 = MU(-2) * (T) 0.5 * (Q0 + UX[0]);
-            T yp = MV(0) * (T) 0.5 * (Q0 + UY[4]), ym = MV(-1) * (T) 0.5 * (Q0 + UY[2]);
-            T yp3 = MV(1) * (T) 0.5 * (Q0 + UY[6]), ym3 = MV(-2) * (T) 0.5 * (Q0 + UY[0]);
-            const T mw0 = MW(0), mwm = MW(-1), mwp = MW(1), mwm2 = MW(-2);
-            T zp = mw0 * (T) 0.5 * (Q0 + U[4]), zm = mwm * (T) 0.5 * (Q0 + U[2]);
-            T zp3 = mwp * (T) 0.5 * (Q0 + U[6]), zm3 = mwm2 * (T) 0.5 * (Q0 + U[0]);
-            /* U[t] is level k - 3 + t; wall values from levels -2..1 / nz-2..nz+1 */
-            if (k == nz - 1) {
-                const T bct = wall_interp<4>(U[5], U[4], U[3], U[2]);
-                zp = mw0 * bct;
-                zp3 = -mwm * (T) 0.5 * (U[1] + U[4]) + (T) 2.0 * mw0 * bct;
-            }
-            if (k == nz - 2) zp3 = mwp * wall_interp<4>(U[6], U[5], U[4], U[3]);
-            if (k == 0) {
-                const T bcb = wall_interp<4>(U[1], U[2], U[3], U[4]);
-                zm = mwm * bcb;
-                zm3 = -mw0 * (T) 0.5 * (U[5] + U[2]) + (T) 2.0 * mwm * bcb;
-            }
-            if (k == 1) zm3 = mwm2 * wall_interp<4>(U[0], U[1], U[2], U[3]);
-            f = -((A1 * (xp - xm) + A2 * (xp3 - xm3)) + (A1 * (yp - ym) + A2 * (yp3 - ym3))
-                  + (A1 * (zp - zm) + A2 * (zp3 - zm3))) / den;
+        const T fa = dif<ORD, T>(VA(0) * (Q0 + A[4]), VA(-1) * (Q0 + A[2]), ORD == 4 ? VA(1) * (Q0 + A[6]) : (T) 0,
+                                 ORD == 4 ? VA(-2) * (Q0 + A[0]) : (T) 0);
+        const T fc = dif<ORD, T>(VC(0) * (Q0 + C[4]), VC(-1) * (Q0 + C[2]), ORD == 4 ? VC(1) * (Q0 + C[6]) : (T) 0,
+                                 ORD == 4 ? VC(-2) * (Q0 + C[0]) : (T) 0);
+        /* Z[t] is level k - 3 + t; wall values from levels -2..1 / nz-2..nz+1 */
+        const T w0 = VZ(0), wm = VZ(-1), wp = ORD == 4 ? VZ(1) : (T) 0, wm2 = ORD == 4 ? VZ(-2) : (T) 0;
+        T zp = w0 * (Q0 + Z[4]), zm = wm * (Q0 + Z[2]), zp3 = wp * (Q0 + Z[6]), zm3 = wm2 * (Q0 + Z[0]);
+        const T two = (T) 2;
+        if (k == nz - 1) {
+            const T bct = wall_interp<ORD>(Z[5], Z[4], Z[3], Z[2]);
+            zp = w0 * (two * bct);
+            zp3 = -wm * (Z[1] + Z[4]) + two * w0 * (two * bct);
         }
+        if (ORD == 4 && k == nz - 2) zp3 = wp * (two * wall_interp<ORD>(Z[6], Z[5], Z[4], Z[3]));
+        if (k == 0) {
+            const T bcb = wall_interp<ORD>(Z[1], Z[2], Z[3], Z[4]);
+            zm = wm * (two * bcb);
+            zm3 = -w0 * (Z[5] + Z[2]) + two * wm * (two * bcb);
+        }
+        if (ORD == 4 && k == 1) zm3 = wm2 * (two * wall_interp<ORD>(Z[0], Z[1], Z[2], Z[3]));
+        const T rx = (T) R.rdx, ry = (T) R.rdy, ra = AX == 0 ? rx : ry, rc = AX == 0 ? ry : rx;
+        T f = (T) -0.5 * (fa * ra + fc * rc + dif<ORD, T>(zp, zm, zp3, zm3) * (T) rdz[k]);
         /* the x-y diffusion: explicit in f (chanfast, diffuseu.c:286-359), or
          * in the 3-D Helmholtz operator of h when every diffusion term is
          * implicit (channel, helmholtz_operator_u, diffuseu.c:362-457) */
-        const T lxy = lapxy<ORD>(UX, UY, dx, dy, (T) 1);
+        const T lxy = d2<ORD>(A) * (ra * ra) + d2<ORD>(C) * (rc * rc);
         if (!R.implicit) f += (T) R.nu * lxy;
-        if (SC && R.betg[0] != 0.0) {       /* add_buoyancy2/4, scalar.c:6-76 */
-            const size_t r0 = row;
-            const T cx = ORD == 2 ? (T) 0.5 * (c[r0 + i] + c[r0 + ip])
-                                       : B1 * (c[r0 + i] + c[r0 + ip]) + B2 * (c[r0 + im] + c[r0 + ip2]);
-            f += cx * (T) R.betg[0];
-        }
-        const SubCoef &C = R.sc[s];
-        T h = helm_cell<ORD>(U, dz, k, C.nuadt);
-        if (R.implicit) h += (T) C.nuadt * lxy;
-        if (s > 0) h += (T) C.gamdt * f + (T) C.zetdt * (g[q] + (T) scal[R.m_prev_slot[s]]);
-        else h += (T) C.gamdt * f;
-        h -= (T) R.liftg[((size_t) s * 4 + 0) * nz + k];
-        if (s < 2) fo[q] = f;                 /* the last substep's tendency is never read */
+        if (SC && R.betg[AX] != 0.0)        /* add_buoyancy2/4, scalar.c:6-76 */
+            f += mid<ORD, T>(ORD == 4 ? p.at(c, k, al(-1)) : (T) 0, p.at(c, k, al(0)), p.at(c, k, al(1)),
+                             ORD == 4 ? p.at(c, k, al(2)) : (T) 0) * (T) R.betg[AX];
+        const SubCoef &S = R.sc[s];
+        T h = helm<ORD>(Z, ORD == 4 ? (T) rdzh[k - 2] : (T) 0, (T) rdzh[k - 1], (T) rdzh[k], ORD == 4 ? (T) rdzh[k + 1] : (T) 0,
+                        (T) rdz[k], (T) S.nuadt);
+        if (R.implicit) h += (T) S.nuadt * lxy;
+        h += (T) S.gamdt * f;
+        if (s > 0) h += (T) S.zetdt * (p.at(g, k, p.off(0, 0)) + (AX == 0 ? (T) ((cp<double>) scal)[R.m_prev_slot[s]] : (T) 0));
+        h -= (T) ((cp<double>) R.liftg)[((size_t) s * 4 + AX) * nz + k];
+        if (s < 2) p.put((gp<T>) F.f[AX], f);     /* the last substep's tendency is never read */
         /* the z solve's right-hand side is h dvol (diffuseu.c:202); the
          * spectral solve takes h and applies dvol itself */
-        const T rr = h * dzk;
-        ro[q] = R.implicit ? h : rr;
+        const T rr = h * (T) dz[k];
+        p.put((gp<T>) F.r[AX], R.implicit ? h : rr);
         rsum = (double) rr;
-        if (cflpart) {                        /* get_cfl, get.c:390-417 */
-            const double dzph = 0.5 * (dz[k] + dz[k + 1]);
-            cflv = fmax(fmax(fabs((double) Q0) * cfldt / R.g.dx, fabs((double) v[q]) * cfldt / R.g.dy),
-                        fabs((double) w[q]) * cfldt / dzph);
-        }
+        if (AX == 0 && cflpart)             /* get_cfl, get.c:390-417 */
+            cflv = fmax(fmax(fabs((double) Q0) * cfldt * R.rdx, fabs((double) p.at(o, k, p.off(0, 0))) * cfldt * R.rdy),
+                        fabs((double) p.at(w, k, p.off(0, 0))) * cfldt * rdzh[k]);
     }
-    block_store(rsum, R.mwq + (size_t) (s * 2) * 4 * nz, k, s, mpart, cflv, cflpart, (b.z * b.ny + b.y) * b.nx + b.x,
-                b.nx * b.ny * b.nz);
-}
-
-/* ------------------------------------------------------------ v */
-
-template <int ORD, bool SC, typename T>
-static __device__ __forceinline__ void rhsv_body(const RunDev &R, const int s,
-    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-    const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, const Blk b)
-{
-    (void) scal;
-    const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
-    const int i = b.x * 64 + threadIdx.x, j = b.y * 4 + threadIdx.y, k = b.z;
-    if (i >= nx || j >= ny) return;
-    const size_t P = (size_t) nx * ny;
-    const double *dz = R.dzt + CF_NGT;
-    const T A1 = (T) A1d, A2 = (T) A2d, B1 = (T) B1d, B2 = (T) B2d;
-    (void) A1; (void) A2; (void) B1; (void) B2;
-    auto DZ = [&](int kk) -> T { return (T) dz[kk]; };
-    const T dx = (T) R.g.dx, dy = (T) R.g.dy;
-    const size_t cc = (size_t) j * nx + i, q = (size_t) k * P + cc;
-    const size_t row = rowof(k, j, nx, P);
-    T V[7], VX[7], VY[7];
-    cell_col7<ORD>(v, P, cc, k, nz, R.cl.cell, R.vbc, R.vbc, V);
-#pragma unroll
-    for (int t = 0; t < 7; t++) {
-        VX[t] = (ORD == 2 && (t < 2 || t > 4)) ? (T) 0 : v[row + wrapm(i - 3 + t, nx)];
-        VY[t] = (ORD == 2 && (t < 2 || t > 4)) ? (T) 0 : v[rowof(k, wrapm(j - 3 + t, ny), nx, P) + i];
-    }
-    const T Q0 = V[3];
-    const T dzk = DZ(k);
-    const int jm = wrapm(j - 1, ny), jp = wrapm(j + 1, ny), jp2 = wrapm(j + 2, ny);
-    /* massfluxy (advect.c:132-200): fluxes interpolated to the v-point in y */
-    auto MU = [&](int d) -> T {     /* at x-position i + d */
-        const int ii = wrapm(i + d, nx);
-        const T a0 = u[rowof(k, j, nx, P) + ii], a1 = u[rowof(k, jp, nx, P) + ii];
-        if (ORD == 2) return (T) 0.5 * (dy * dzk * a0 + dy * dzk * a1);
-        const T am = u[rowof(k, jm, nx, P) + ii], a2 = u[rowof(k, jp2, nx, P) + ii];
-        return B1 * (dy * dzk * a0 + dy * dzk * a1) + B2 * (dy * dzk * am + dy * dzk * a2);
-    };
-    auto MV = [&](int e) -> T {
-        return ORD == 2 ? (T) 0.5 * (dx * dzk * VY[3 + e] + dx * dzk * VY[4 + e])
-                        : B1 * (dx * dzk * VY[3 + e] + dx * dzk * VY[4 + e])
-                        + B2 * (dx * dzk * VY[2 + e] + dx * dzk * VY[5 + e]);
-    };
-    auto MW = [&](int e) -> T {
-        const int kk = k + e;
-        const T a0 = wadv(w, P, (size_t) j * nx + i, kk, nz), a1 = wadv(w, P, (size_t) jp * nx + i, kk, nz);
-        if (ORD == 2) return (T) 0.5 * (dx * dy * a0 + dx * dy * a1);
-        const T am = wadv(w, P, (size_t) jm * nx + i, kk, nz), a2 = wadv(w, P, (size_t) jp2 * nx + i, kk, nz);
-        return B1 * (dx * dy * a0 + dx * dy * a1) + B2 * (dx * dy * am + dx * dy * a2);
-    };
-    T f;
-    const T den = dx * dy * dzk;
-    if (ORD == 2) {
-        T xp = MU(0) * (T) 0.5 * (Q0 + VX[4]), xm = MU(-1) * (T) 0.5 * (Q0 + VX[2]);
-        T yp = MV(0) * (T) 0.5 * (Q0 + VY[4]), ym = MV(-1) * (T) 0.5 * (Q0 + VY[2]);
-        const T mw0 = MW(0), mwm = MW(-1);
-        T zp = mw0 * (T) 0.5 * (Q0 + V[4]), zm = mwm * (T) 0.5 * (Q0 + V[2]);
-        if (k == nz - 1) zp = mw0 * wall_interp<2, T>((T) 0, V[4], V[3], (T) 0);
-        if (k == 0) zm = mwm * wall_interp<2, T>((T) 0, V[2], V[3], (T) 0);
-        f = -((xp - xm) + (yp - ym) + (zp - zm)) / den;
-    } else {
-        T xp = MU(0) * (T) 0.5 * (Q0 + VX[4]), xm = MU(-1) * (T) 0.5 * (Q0 + VX[2]);
-        T xp3 = MU(1) * (T) 0.5 * (Q0 + VX[6]), xm3 = MU(-2) * (T) 0.5 * (Q0 + VX[0]);
-        T yp = MV(0) * (T) 0.5 * (Q0 + VY[4]), ym = MV(-1) * (T) 0.5 * (Q0 + VY[2]);
-        T yp3 = MV(1) * (T) 0.5 * (Q0 + VY[6]), ym3 = MV(-2) * (T) 0.5 * (Q0 + VY[0]);
-        const T mw0 = MW(0), mwm = MW(-1), mwp = MW(1), mwm2 = MW(-2);
-        T zp = mw0 * (T) 0.5 * (Q0 + V[4]), zm = mwm * (T) 0.5 * (Q0 + V[2]);
-        T zp3 = mwp * (T) 0.5 * (Q0 + V[6]), zm3 = mwm2 * (T) 0.5 * (Q0 + V[0]);
-        if (k == nz - 1) {
-            const T bct = wall_interp<4>(V[5], V[4], V[3], V[2]);
-            zp = mw0 * bct;
-            zp3 = -mwm * (T) 0.5 * (V[1] + V[4]) + (T) 2.0 * mw0 * bct;
-        }
-        if (k == nz - 2) zp3 = mwp * wall_interp<4>(V[6], V[5], V[4], V[3]);
-        if (k == 0) {
-            const T bcb = wall_interp<4>(V[1], V[2], V[3], V[4]);
-            zm = mwm * bcb;
-            zm3 = -mw0 * (T) 0.5 * (V[5] + V[2]) + (T) 2.0 * mwm * bcb;
-        }
-        if (k == 1) zm3 = mwm2 * wall_interp<4>(V[0], V[1], V[2], V[3]);
-        f = -((A1 * (xp - xm) + A2 * (xp3 - xm3)) + (A1 * (yp - ym) + A2 * (yp3 - ym3))
-              + (A1 * (zp - zm) + A2 * (zp3 - zm3))) / den;
-    }
-    const T lxy = lapxy<ORD>(VX, VY, dx, dy, (T) 1);
-    if (!R.implicit) f += (T) R.nu * lxy;
-    if (SC && R.betg[1] != 0.0) {
-        const T c0 = c[q], c1 = c[rowof(k, jp, nx, P) + i];
-        const T cy = ORD == 2 ? (T) 0.5 * (c0 + c1)
-                                   : B1 * (c0 + c1) + B2 * (c[rowof(k, jm, nx, P) + i] + c[rowof(k, jp2, nx, P) + i]);
-        f += cy * (T) R.betg[1];
-    }
-    const SubCoef &C = R.sc[s];
-    T h = helm_cell<ORD>(V, dz, k, C.nuadt);
-    if (R.implicit) h += (T) C.nuadt * lxy;
-    if (s > 0) h += (T) C.gamdt * f + (T) C.zetdt * g[q];
-    else h += (T) C.gamdt * f;
-    h -= (T) R.liftg[((size_t) s * 4 + 1) * nz + k];
-    if (s < 2) fo[q] = f;                     /* the last substep's tendency is never read */
-    ro[q] = R.implicit ? h : h * dzk;
+    if (AX == 0)
+        block_store(rsum, R.mwq + (size_t) (s * 2) * 4 * nz, k, s, mpart, cflv, cflpart, b.z * b.nx + b.x, b.nx * b.nz);
 }
 
 /* ------------------------------------------------------------ w */
 
 template <int ORD, bool SC, typename T>
-static __device__ __forceinline__ void rhsw_body(const RunDev &R, const int s,
-    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-    const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, const Blk b)
+static __device__ __forceinline__ void rhsw_body(const RunDev &R, const int s, const GFields<T> &F, const Blk b)
 {
-    (void) scal;
-    const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
-    const int i = b.x * 64 + threadIdx.x, j = b.y * 4 + threadIdx.y, k = b.z;
-    if (i >= nx || j >= ny) return;
-    const size_t P = (size_t) nx * ny;
-    const size_t cc = (size_t) j * nx + i, q = (size_t) k * P + cc;
+    const Pt<T> p(R, b);
+    const int k = p.k, nz = p.nz;
+    if (!p.act) return;
+    const gp<T> fo = (gp<T>) F.f[2], ro = (gp<T>) F.r[2];
     if (k == nz - 1) {                    /* top wall face: f = 0 (advect.c:301), no unknown */
-        if (s < 2) fo[q] = 0.0;
-        ro[q] = 0.0;
+        if (s < 2) p.put(fo, (T) 0);
+        p.put(ro, (T) 0);
         return;
     }
-    const double *dz = R.dzt + CF_NGT;
-    const T A1 = (T) A1d, A2 = (T) A2d, B1 = (T) B1d, B2 = (T) B2d;
-    (void) A1; (void) A2; (void) B1; (void) B2;
-    auto DZ = [&](int kk) -> T { return (T) dz[kk]; };
-    const T dx = (T) R.g.dx, dy = (T) R.g.dy;
-    const size_t row = rowof(k, j, nx, P);
+    const gp<const T> u = (gp<const T>) F.u, v = (gp<const T>) F.v, w = (gp<const T>) F.w, c = (gp<const T>) F.c;
+    const cp<double> rdz = (cp<double>) R.rdz + CF_NGT, rdzh = (cp<double>) R.rdzh + CF_NGT, dz = (cp<double>) R.dzt + CF_NGT;
+    constexpr int LO = ORD == 2 ? 2 : 0, HI = ORD == 2 ? 4 : 6;
+    const unsigned cc = p.off(0, 0);
     T WA[7], WH[7], WX[7], WY[7];
 #pragma unroll
-    for (int t = 0; t < 7; t++) WA[t] = (ORD == 2 && (t < 2 || t > 4)) ? (T) 0 : wadv(w, P, cc, k - 3 + t, nz);
-    face_col7<ORD>(w, P, cc, k, nz, R.cl.face, WH);
+    for (int t = 0; t < 7; t++) WA[t] = t < LO || t > HI ? (T) 0 : wadv(p, w, cc, k - 3 + t);
+    face_col7<ORD>(p, w, R.cl.face, WH);
 #pragma unroll
     for (int t = 0; t < 7; t++) {
-        WX[t] = (ORD == 2 && (t < 2 || t > 4)) ? (T) 0 : w[row + wrapm(i - 3 + t, nx)];
-        WY[t] = (ORD == 2 && (t < 2 || t > 4)) ? (T) 0 : w[rowof(k, wrapm(j - 3 + t, ny), nx, P) + i];
+        WX[t] = t < LO || t > HI ? (T) 0 : (t == 3 ? WA[3] : p.at(w, k, p.off(t - 3, 0)));
+        WY[t] = t < LO || t > HI ? (T) 0 : (t == 3 ? WA[3] : p.at(w, k, p.off(0, t - 3)));
     }
     const T Q0 = WA[3];
-    /* u and v at their own levels with closure ghosts, for the z-interpolated fluxes */
-    auto ucell = [&](int ii, int jj, int kk, const T *fld, double bcb, double bct) -> T {
-        const size_t c2 = (size_t) jj * nx + ii;
-        if (kk >= 0 && kk < nz) return fld[(size_t) kk * P + c2];
+    /* a cell field at level kk with closure ghosts, for the z-interpolated
+     * fluxes and the buoyancy */
+    auto cell = [&](gp<const T> fld, unsigned o, int kk, double bcb, double bct) -> T {
+        if (kk >= 0 && kk < nz) return p.at(fld, kk, o);
         const bool lo = kk < 0;
         const Clos1 &Cl = R.cl.cell[lo ? 0 : 1];
         const int m = lo ? -1 - kk : kk - nz;
-        const T x0 = fld[(size_t) (lo ? 0 : nz - 1) * P + c2];
-        const T x1 = ORD == 4 ? fld[(size_t) (lo ? 1 : nz - 2) * P + c2] : (T) 0;
-        const T x2 = ORD == 4 ? fld[(size_t) (lo ? 2 : nz - 3) * P + c2] : (T) 0;
+        const T x0 = p.at(fld, lo ? 0 : nz - 1, o);
+        const T x1 = ORD == 4 ? p.at(fld, lo ? 1 : nz - 2, o) : (T) 0;
+        const T x2 = ORD == 4 ? p.at(fld, lo ? 2 : nz - 3, o) : (T) 0;
         return (T) Cl.G[m][0] * x0 + (T) Cl.G[m][1] * x1 + (T) Cl.G[m][2] * x2 + (T) (Cl.B[m] * (lo ? bcb : bct));
     };
-    /* massfluxz (advect.c:201-283): fluxes interpolated to the w-point in z */
-    auto MUZ = [&](int d) -> T {
-        const int ii = wrapm(i + d, nx);
-        if (ORD == 2) return (T) 0.5 * (dy * DZ(k) * ucell(ii, j, k, u, R.ubc, R.ubc) + dy * DZ(k + 1) * ucell(ii, j, k + 1, u, R.ubc, R.ubc));
-        return B1 * (dy * DZ(k) * ucell(ii, j, k, u, R.ubc, R.ubc) + dy * DZ(k + 1) * ucell(ii, j, k + 1, u, R.ubc, R.ubc))
-             + B2 * (dy * DZ(k - 1) * ucell(ii, j, k - 1, u, R.ubc, R.ubc) + dy * DZ(k + 2) * ucell(ii, j, k + 2, u, R.ubc, R.ubc));
+    /* massfluxz (advect.c:201-283): volume fluxes interpolated to the w-point in z */
+    const T dm = ORD == 4 ? (T) dz[k - 1] : (T) 0, d0 = (T) dz[k], d1 = (T) dz[k + 1], d2_ = ORD == 4 ? (T) dz[k + 2] : (T) 0;
+    auto VZ = [&](gp<const T> fld, unsigned o, double bc) -> T {
+        return mid<ORD, T>(ORD == 4 ? dm * cell(fld, o, k - 1, bc, bc) : (T) 0, d0 * cell(fld, o, k, bc, bc),
+                           d1 * cell(fld, o, k + 1, bc, bc), ORD == 4 ? d2_ * cell(fld, o, k + 2, bc, bc) : (T) 0);
     };
-    auto MVZ = [&](int e) -> T {
-        const int jj = wrapm(j + e, ny);
-        if (ORD == 2) return (T) 0.5 * (dx * DZ(k) * ucell(i, jj, k, v, R.vbc, R.vbc) + dx * DZ(k + 1) * ucell(i, jj, k + 1, v, R.vbc, R.vbc));
-        return B1 * (dx * DZ(k) * ucell(i, jj, k, v, R.vbc, R.vbc) + dx * DZ(k + 1) * ucell(i, jj, k + 1, v, R.vbc, R.vbc))
-             + B2 * (dx * DZ(k - 1) * ucell(i, jj, k - 1, v, R.vbc, R.vbc) + dx * DZ(k + 2) * ucell(i, jj, k + 2, v, R.vbc, R.vbc));
+    auto UZ = [&](int d) -> T { return VZ(u, p.off(d, 0), R.ubc); };
+    auto YZ = [&](int e) -> T { return VZ(v, p.off(0, e), R.vbc); };
+    auto WZ = [&](int e) -> T {     /* at face k + e from WA[2+e..5+e] */
+        return mid<ORD, T>(e >= -2 ? WA[2 + e] : (T) 0, WA[3 + e], WA[4 + e], e <= 1 ? WA[5 + e] : (T) 0);
     };
-    auto MWZ = [&](int e) -> T {     /* at face k + e from WA[2+e..5+e] */
-        return ORD == 2 ? (T) 0.5 * (dx * dy * WA[3 + e] + dx * dy * WA[4 + e])
-                        : B1 * (dx * dy * WA[3 + e] + dx * dy * WA[4 + e])
-                        + B2 * (dx * dy * WA[2 + e] + dx * dy * WA[5 + e]);
-    };
-    T f;
-    const T den = dx * dy * ((T) 0.5 * (DZ(k + 1) + DZ(k)));
-    if (ORD == 2) {
-        T xp = MUZ(0) * (T) 0.5 * (Q0 + WX[4]), xm = MUZ(-1) * (T) 0.5 * (Q0 + WX[2]);
-        T yp = MVZ(0) * (T) 0.5 * (Q0 + WY[4]), ym = MVZ(-1) * (T) 0.5 * (Q0 + WY[2]);
-        T zp = MWZ(0) * (T) 0.5 * (Q0 + WA[4]), zm = MWZ(-1) * (T) 0.5 * (Q0 + WA[2]);
-        f = -((xp - xm) + (yp - ym) + (zp - zm)) / den;
-    } else {
-        T xp = MUZ(0) * (T) 0.5 * (Q0 + WX[4]), xm = MUZ(-1) * (T) 0.5 * (Q0 + WX[2]);
-        T xp3 = MUZ(1) * (T) 0.5 * (Q0 + WX[6]), xm3 = MUZ(-2) * (T) 0.5 * (Q0 + WX[0]);
-        T yp = MVZ(0) * (T) 0.5 * (Q0 + WY[4]), ym = MVZ(-1) * (T) 0.5 * (Q0 + WY[2]);
-        T yp3 = MVZ(1) * (T) 0.5 * (Q0 + WY[6]), ym3 = MVZ(-2) * (T) 0.5 * (Q0 + WY[0]);
-        T zp = MWZ(0) * (T) 0.5 * (Q0 + WA[4]), zm = MWZ(-1) * (T) 0.5 * (Q0 + WA[2]);
-        T zp3 = MWZ(1) * (T) 0.5 * (Q0 + WA[6]), zm3 = MWZ(-2) * (T) 0.5 * (Q0 + WA[0]);
-        f = -((A1 * (xp - xm) + A2 * (xp3 - xm3)) + (A1 * (yp - ym) + A2 * (yp3 - ym3))
-              + (A1 * (zp - zm) + A2 * (zp3 - zm3))) / den;
-    }
-    const T lxy = lapxy<ORD>(WX, WY, dx, dy, (T) 1);
+    const T fx = dif<ORD, T>(UZ(0) * (Q0 + WX[4]), UZ(-1) * (Q0 + WX[2]), ORD == 4 ? UZ(1) * (Q0 + WX[6]) : (T) 0,
+                             ORD == 4 ? UZ(-2) * (Q0 + WX[0]) : (T) 0);
+    const T fy = dif<ORD, T>(YZ(0) * (Q0 + WY[4]), YZ(-1) * (Q0 + WY[2]), ORD == 4 ? YZ(1) * (Q0 + WY[6]) : (T) 0,
+                             ORD == 4 ? YZ(-2) * (Q0 + WY[0]) : (T) 0);
+    const T fz = dif<ORD, T>(WZ(0) * (Q0 + WA[4]), WZ(-1) * (Q0 + WA[2]), ORD == 4 ? WZ(1) * (Q0 + WA[6]) : (T) 0,
+                             ORD == 4 ? WZ(-2) * (Q0 + WA[0]) : (T) 0);
+    const T rx = (T) R.rdx, ry = (T) R.rdy, rh = (T) rdzh[k];
+    T f = (T) -0.5 * ((fx * rx + fy * ry + fz) * rh);
+    const T lxy = d2<ORD>(WX) * (rx * rx) + d2<ORD>(WY) * (ry * ry);
     if (!R.implicit) f += (T) R.nu * lxy;
-    if (SC && R.betg[2] != 0.0) {
-        const T c0 = ucell(i, j, k, c, R.cbot, R.ctop), c1 = ucell(i, j, k + 1, c, R.cbot, R.ctop);
-        T cz;
-        if (ORD == 2) cz = (T) 0.5 * (c0 + c1);
-        else {
-            const T cm = ucell(i, j, k - 1, c, R.cbot, R.ctop);
-            const T c2 = ucell(i, j, k + 2, c, R.cbot, R.ctop);
-            cz = B1 * (c0 + c1) + B2 * (cm + c2);
-        }
-        f += cz * (T) R.betg[2];
-    }
-    const SubCoef &C = R.sc[s];
-    T h = helm_face<ORD>(WH, dz, k, C.nuadt);
-    if (R.implicit) h += (T) C.nuadt * lxy;
-    if (s > 0) h += (T) C.gamdt * f + (T) C.zetdt * g[q];
-    else h += (T) C.gamdt * f;
-    h -= (T) R.liftg[((size_t) s * 4 + 2) * nz + k];
-    if (s < 2) fo[q] = f;                     /* the last substep's tendency is never read */
-    ro[q] = R.implicit ? h : h * ((T) 0.5 * (DZ(k + 1) + DZ(k)));   /* times the face volume (diffusew.c:205) */
+    if (SC && R.betg[2] != 0.0)
+        f += mid<ORD, T>(ORD == 4 ? cell(c, cc, k - 1, R.cbot, R.ctop) : (T) 0, cell(c, cc, k, R.cbot, R.ctop),
+                         cell(c, cc, k + 1, R.cbot, R.ctop), ORD == 4 ? cell(c, cc, k + 2, R.cbot, R.ctop) : (T) 0)
+             * (T) R.betg[2];
+    const SubCoef &S = R.sc[s];
+    T h = helm<ORD>(WH, ORD == 4 ? (T) rdz[k - 1] : (T) 0, (T) rdz[k], (T) rdz[k + 1], ORD == 4 ? (T) rdz[k + 2] : (T) 0, rh,
+                    (T) S.nuadt);
+    if (R.implicit) h += (T) S.nuadt * lxy;
+    h += (T) S.gamdt * f;
+    if (s > 0) h += (T) S.zetdt * p.at((gp<const T>) F.g[2], k, cc);
+    h -= (T) ((cp<double>) R.liftg)[((size_t) s * 4 + 2) * nz + k];
+    if (s < 2) p.put(fo, f);                  /* the last substep's tendency is never read */
+    p.put(ro, R.implicit ? h : h * ((T) 0.5 * (d1 + d0)));    /* times the face volume (diffusew.c:205) */
 }
 
 /* ------------------------------------------------------------ c */
 
-/* flux_quick + advect_scalar (scalar.c:79-162), laplacexy with nu / Pr,
- * then the scalar's implicit right-hand side (chanfast.c:540-571) */
-template <int ORD, bool SC, typename T>
-static __device__ __forceinline__ void rhsc_body(const RunDev &R, const int s,
-    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-    const T *__restrict__ c, const T *__restrict__ g, const double *__restrict__ scal,
-    T *__restrict__ fo, T *__restrict__ ro, double *__restrict__ mpart, const Blk b)
+template <int ORD, typename T>
+static __device__ __forceinline__ void rhsc_body(const RunDev &R, const int s, const GFields<T> &F,
+    const double *__restrict__ scal, double *__restrict__ mpart, const Blk b)
 {
-    const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
-    const int i = b.x * 64 + threadIdx.x, j = b.y * 4 + threadIdx.y, k = b.z;
+    const Pt<T> p(R, b);
+    const int k = p.k, nz = p.nz;
+    const gp<const T> u = (gp<const T>) F.u, v = (gp<const T>) F.v, w = (gp<const T>) F.w, c = (gp<const T>) F.c;
+    const cp<double> rdz = (cp<double>) R.rdz + CF_NGT, rdzh = (cp<double>) R.rdzh + CF_NGT, dz = (cp<double>) R.dzt + CF_NGT;
     double rsum = 0.0;
-    if (i < nx && j < ny) {
-    const size_t P = (size_t) nx * ny;
-    const double *dz = R.dzt + CF_NGT;
-    const T A1 = (T) A1d, A2 = (T) A2d, B1 = (T) B1d, B2 = (T) B2d;
-    (void) A1; (void) A2; (void) B1; (void) B2;
-    auto DZ = [&](int kk) -> T { return (T) dz[kk]; };
-    const T dx = (T) R.g.dx, dy = (T) R.g.dy;
-    const size_t cc = (size_t) j * nx + i, q = (size_t) k * P + cc;
-    const size_t row = rowof(k, j, nx, P);
-    T Cz[7], CX[7], CY[7];
-    cell_col7<ORD>(c, P, cc, k, nz, R.cl.cell, R.cbot, R.ctop, Cz);
+    if (p.act) {
+        constexpr int LO = ORD == 2 ? 1 : 0, HI = ORD == 2 ? 5 : 6;   /* QUICK reaches two cells */
+        const unsigned cc = p.off(0, 0);
+        T Cz[7], CX[7], CY[7];
+        cell_col7<ORD, ORD == 2 ? 2 : 3>(p, c, R.cl.cell, R.cbot, R.ctop, Cz);
 #pragma unroll
-    for (int t = 0; t < 7; t++) {
-        CX[t] = (t == 0 || t == 6) && ORD == 2 ? (T) 0 : c[row + wrapm(i - 3 + t, nx)];
-        CY[t] = (t == 0 || t == 6) && ORD == 2 ? (T) 0 : c[rowof(k, wrapm(j - 3 + t, ny), nx, P) + i];
+        for (int t = 0; t < 7; t++) {
+            CX[t] = t < LO || t > HI ? (T) 0 : (t == 3 ? Cz[3] : p.at(c, k, p.off(t - 3, 0)));
+            CY[t] = t < LO || t > HI ? (T) 0 : (t == 3 ? Cz[3] : p.at(c, k, p.off(0, t - 3)));
+        }
+        const T qk = (T) -0.125;
+        /* QUICK face value upwinded by the sign of the face velocity */
+        auto quick = [&](T fl, T cm, T c0, T c1, T c2) -> T {
+            T cf = (T) 0.5 * (c0 + c1);
+            cf += fl > (T) 0 ? qk * (c1 - (T) 2.0 * c0 + cm) : qk * (c2 - (T) 2.0 * c1 + c0);
+            return fl * cf;
+        };
+        const T u0 = p.at(u, k, cc), um = p.at(u, k, p.off(-1, 0)), v0 = p.at(v, k, cc), vm = p.at(v, k, p.off(0, -1));
+        const T w0 = wadv(p, w, cc, k), wm = wadv(p, w, cc, k - 1);
+        const T fx = quick(u0, CX[2], CX[3], CX[4], CX[5]) - quick(um, CX[1], CX[2], CX[3], CX[4]);
+        const T fy = quick(v0, CY[2], CY[3], CY[4], CY[5]) - quick(vm, CY[1], CY[2], CY[3], CY[4]);
+        const T fz = quick(w0, Cz[2], Cz[3], Cz[4], Cz[5]) - quick(wm, Cz[1], Cz[2], Cz[3], Cz[4]);
+        const T rx = (T) R.rdx, ry = (T) R.rdy;
+        T f = -(fx * rx + fy * ry + fz * (T) rdz[k]);
+        const T lxy = d2<ORD>(CX) * (rx * rx) + d2<ORD>(CY) * (ry * ry);
+        if (!R.implicit) f += (T) R.kap * lxy;
+        const SubCoef &S = R.sc[s];
+        T h = helm<ORD>(Cz, ORD == 4 ? (T) rdzh[k - 2] : (T) 0, (T) rdzh[k - 1], (T) rdzh[k], ORD == 4 ? (T) rdzh[k + 1] : (T) 0,
+                        (T) rdz[k], (T) S.kadt);
+        if (R.implicit) h += (T) S.kadt * lxy;
+        h += (T) S.gamdt * f;
+        if (s > 0) h += (T) S.zetdt * (p.at((gp<const T>) F.g[3], k, cc) + (T) ((cp<double>) scal)[SC_MC0 + (s + 2) % 3]);
+        h -= (T) ((cp<double>) R.liftg)[((size_t) s * 4 + 3) * nz + k];
+        if (s < 2) p.put((gp<T>) F.f[3], f);      /* the last substep's tendency is never read */
+        const T rr = h * (T) dz[k];
+        p.put((gp<T>) F.r[3], R.implicit ? h : rr);
+        rsum = (double) rr;
     }
-    const T qk = (T) -0.125;
-    /* QUICK face value upwinded by the sign of the face volume flux */
-    auto quick = [&](T fl, T cm, T c0, T c1, T c2) -> T {
-        T cf = (T) 0.5 * (c0 + c1);
-        cf += fl > (T) 0 ? qk * (c1 - (T) 2.0 * c0 + cm) : qk * (c2 - (T) 2.0 * c1 + c0);
-        return fl * cf;
-    };
-    const int im = wrapm(i - 1, nx), jm = wrapm(j - 1, ny);
-    const T fu0 = dy * DZ(k) * u[row + i], fum = dy * DZ(k) * u[row + im];
-    const T fv0 = dx * DZ(k) * v[q], fvm = dx * DZ(k) * v[rowof(k, jm, nx, P) + i];
-    const T fw0 = dx * dy * wadv(w, P, cc, k, nz), fwm = dx * dy * wadv(w, P, cc, k - 1, nz);
-    const T mu0 = quick(fu0, CX[2], CX[3], CX[4], CX[5]), mum = quick(fum, CX[1], CX[2], CX[3], CX[4]);
-    const T mv0 = quick(fv0, CY[2], CY[3], CY[4], CY[5]), mvm = quick(fvm, CY[1], CY[2], CY[3], CY[4]);
-    const T mw0 = quick(fw0, Cz[2], Cz[3], Cz[4], Cz[5]), mwm = quick(fwm, Cz[1], Cz[2], Cz[3], Cz[4]);
-    T f = -((mu0 - mum) + (mv0 - mvm) + (mw0 - mwm)) / (dx * dy * DZ(k));
-    const T lxy = lapxy<ORD>(CX, CY, dx, dy, (T) 1);
-    if (!R.implicit) f += (T) R.kap * lxy;
-    const SubCoef &C = R.sc[s];
-    T h = helm_cell<ORD>(Cz, dz, k, C.kadt);
-    if (R.implicit) h += (T) C.kadt * lxy;
-    if (s > 0) h += (T) C.gamdt * f + (T) C.zetdt * (g[q] + (T) scal[SC_MC0 + (s + 2) % 3]);
-    else h += (T) C.gamdt * f;
-    h -= (T) R.liftg[((size_t) s * 4 + 3) * nz + k];
-    if (s < 2) fo[q] = f;                     /* the last substep's tendency is never read */
-    const T rr = h * DZ(k);
-    ro[q] = R.implicit ? h : rr;
-    rsum = (double) rr;
-    }
-    block_store(rsum, R.mwq + (size_t) (s * 2 + 1) * 4 * nz, k, s, mpart, 0.0, nullptr, (b.z * b.ny + b.y) * b.nx + b.x,
-                b.nx * b.ny * b.nz);
+    block_store(rsum, R.mwq + (size_t) (s * 2 + 1) * 4 * nz, k, s, mpart, 0.0, nullptr, b.z * b.nx + b.x, b.nx * b.nz);
 }
 
 /* ------------------------------------------------------------ all fields */
@@ -591,11 +451,10 @@ static __device__ __forceinline__ void grhs_body(const RunDev &R, const int s, c
     const unsigned fld = b.z % nf;
     b.z /= nf;
     b.nz /= nf;
-    if (fld == 0) rhsu_body<ORD, SC, T>(R, s, F.u, F.v, F.w, F.c, F.g[0], scal, F.f[0], F.r[0], cflpart, cfldt, mpart, b);
-    else if (fld == 1) rhsv_body<ORD, SC, T>(R, s, F.u, F.v, F.w, F.c, F.g[1], scal, F.f[1], F.r[1], b);
-    else if (fld == 2) rhsw_body<ORD, SC, T>(R, s, F.u, F.v, F.w, F.c, F.g[2], scal, F.f[2], F.r[2], b);
-    else if constexpr (SC)
-        rhsc_body<ORD, SC, T>(R, s, F.u, F.v, F.w, F.c, F.g[3], scal, F.f[3], F.r[3], mpart + (size_t) 4 * b.nx * b.ny * b.nz, b);
+    if (fld == 0) rhsuv_body<ORD, SC, 0>(R, s, F, scal, cflpart, cfldt, mpart, b);
+    else if (fld == 1) rhsuv_body<ORD, SC, 1>(R, s, F, scal, nullptr, cfldt, nullptr, b);
+    else if (fld == 2) rhsw_body<ORD, SC>(R, s, F, b);
+    else if constexpr (SC) rhsc_body<ORD>(R, s, F, scal, mpart + (size_t) 4 * b.nx * b.nz, b);
 }
 
 template <int ORD, bool SC, typename T>
@@ -1001,11 +860,9 @@ static __device__ __forceinline__ void proj_body(const RunDev &R, const T *us,
     T *u, T *v, T *w, T *c, const Blk b)
 {
     const T A1 = (T) A1d, A2 = (T) A2d;
-    const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
-    const int i = b.x * 64 + threadIdx.x;
-    const int j = b.y * 4 + threadIdx.y;
-    const int k = b.z;
-    if (i >= nx || j >= ny || k >= nz) return;
+    const Pt<T> pt(R, b);
+    if (!pt.act) return;
+    const int nx = pt.nx, ny = pt.ny, nz = pt.nz, i = pt.i, j = pt.j, k = pt.k;
     const size_t P = (size_t) nx * ny;
     const size_t row = rowof(k, j, nx, P), q = row + i;
     const double *rdzh = R.rdzh + CF_NGT;

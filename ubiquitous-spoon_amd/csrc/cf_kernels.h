@@ -102,6 +102,7 @@ struct RunDev {
     const double *rdz;          /* 1 / dz, level-indexed like dzt (offset CF_NGT) */
     const double *rdzh;         /* 1 / (0.5 (dz_k + dz_k+1)), offset CF_NGT */
     double rdx, rdy, rdxdy;
+    double rnx;                 /* 1 / nx, for qdiv */
     const double *stat1;        /* [s][kind][vol1, bot1, top1, cl1] */
     const double *h1;           /* [s][kind][nz + 2] unit-forcing profile, level k at k + 1 */
     /* the constraint's statistics of the solved field (bulk value, bottom and

@@ -670,19 +670,16 @@ static __device__ __forceinline__ void mass_finalize_body(const RunDev &R, const
 
 /* cflmode 1 (chanfast.c:385-391): get_cfl (get.c:390-417) of the plain
  * fields (u, v, w) with the current dt, before the step that rescales dt;
- * one workgroup of 64 x 4 per (x tile, y tile, level), its max into
- * part[block] */
+ * one workgroup per 256 cells of a level, its max into part[block] */
 template <typename T>
 __global__ __launch_bounds__(256) void k_cfl_plain(const RunDev R, const T *__restrict__ u, const T *__restrict__ v,
                                                    const T *__restrict__ w, double dt, double *__restrict__ part)
 {
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
-    const int i = blockIdx.x * 64 + threadIdx.x;
-    const int j = blockIdx.y * 4 + threadIdx.y;
-    const int k = blockIdx.z;
+    const int e = (int) blockIdx.x * 256 + (int) threadIdx.x, k = blockIdx.z;
     double m = 0.0;
-    if (i < nx && j < ny && k < nz) {
-        const size_t q = (size_t) k * nx * ny + (size_t) j * nx + i;
+    if (e < nx * ny && k < nz) {
+        const size_t q = (size_t) k * nx * ny + e;
         const double *dz = R.dzt + CF_NGT;
         const double dzph = 0.5 * (dz[k] + dz[k + 1]);
         double c;
@@ -691,15 +688,9 @@ __global__ __launch_bounds__(256) void k_cfl_plain(const RunDev R, const T *__re
         if (m < (c = fabs((double) v[q]) * dt / R.g.dy)) m = c;
         if (m < (c = fabs((double) w[q]) * dt / dzph)) m = c;
     }
-    __shared__ double red[256];
-    const int tid = threadIdx.y * 64 + threadIdx.x;
-    red[tid] = m;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (tid < s) red[tid] = fmax(red[tid], red[tid + s]);
-        __syncthreads();
-    }
-    if (tid == 0) part[((size_t) blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = red[0];
+    __shared__ double red[4];
+    const double mx = block_max_nonneg<4>(m, red);
+    if (threadIdx.x == 0) part[(size_t) blockIdx.z * gridDim.x + blockIdx.x] = mx;
 }
 template __global__ void k_cfl_plain<double>(const RunDev, const double *, const double *, const double *, double,
                                              double *);
@@ -1917,10 +1908,9 @@ __global__ __launch_bounds__(256) void k_project2(const RunDev R, const T *__res
     T *__restrict__ u, T *__restrict__ v, T *__restrict__ w)
 {
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
-    const int i = blockIdx.x * 64 + threadIdx.x;
-    const int j = blockIdx.y * 4 + threadIdx.y;
-    const int k = blockIdx.z;
-    if (i >= nx || j >= ny || k >= nz) return;
+    const int e = (int) blockIdx.x * 256 + (int) threadIdx.x, k = blockIdx.z;
+    if (e >= nx * ny || k >= nz) return;
+    const int j = qdiv(e, nx, R.rnx), i = e - j * nx;
     const size_t P = (size_t) nx * ny;
     const int ip = i + 1 < nx ? i + 1 : 0, jp = j + 1 < ny ? j + 1 : 0;
     const size_t q = (size_t) k * P + (size_t) j * nx + i;

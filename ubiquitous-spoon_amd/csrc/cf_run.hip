@@ -1236,7 +1236,7 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     ok = ok && hipMalloc((void **) &r->X, 2 * r->esz * r->M * nz) == hipSuccess;
     ok = ok && dalloc(&r->tab, r->tab_n) && dalloc(&r->scal, SC_N) && dalloc(&r->logbuf, (size_t) LOGCAP * CF_LOG_N);
     rhs_chunks(nx, ny, nz, rhs_target({ &r->g }, CF_RHS_KC), &r->rhs_kc, &r->rhs_blocks);
-    r->gblocks = ((nx + 63) / 64) * ((ny + 3) / 4) * nz;
+    r->gblocks = (int) ((r->P + 255) / 256) * nz;
     if (cfg->order == 4 && nx % CF_R4_X == 0 && ny % CF_R4_Y == 0
         && (size_t) nx * ny * nz * r->esz < ((size_t) 1 << 32)) {   /* 32-bit byte offsets */
         r->r4_nch = std::max(1, (nz + CF_R4_KC / 2) / CF_R4_KC);
@@ -1296,6 +1296,7 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     R.rdy = 1.0 / r->g.dy;
     R.rdxdy = 1.0 / (r->g.dx * r->g.dy);
     R.cmode[0] = cfg->uvolavgmode; R.ctarget[0] = cfg->want_uvolavg - cfg->uframe; R.cfixed[0] = -cfg->dpdx;
+    R.rnx = 1.0 / (double) nx;
     R.cmode[1] = cfg->cvolavgmode; R.ctarget[1] = cfg->want_cvolavg; R.cfixed[1] = 0.0;
     R.logcap = LOGCAP;
     R.fx_pairs = fx_pairs_of(nx, (int) r->esz);
@@ -1363,7 +1364,8 @@ static cf_status ev_end(cf_run *r)
         if (s_ != CF_OK) return s_;                                                 \
     } while (0)
 
-static dim3 cell_grid(const cf_run *r) { return dim3((r->g.nx + 63) / 64, (r->g.ny + 3) / 4, r->g.nz); }
+/* one thread per cell: 256 consecutive cells of a level per workgroup */
+static dim3 cell_grid(const cf_run *r) { return dim3((unsigned) ((r->P + 255) / 256), 1, r->g.nz); }
 
 static size_t fx_lds(const cf_run *r)
 {
@@ -1458,7 +1460,7 @@ template <typename T>
 static cf_status enqueue_materialise_t(cf_run *r, double *u, double *v, double *w)
 {
     ProjSrcT<T> S = current_projection<T>(r);
-    KLAUNCH("materialise", k_project2<T>, cell_grid(r), dim3(64, 4), 0, r->rd, S.us, S.vs, S.ws, S.h1, S.m,
+    KLAUNCH("materialise", k_project2<T>, cell_grid(r), dim3(256), 0, r->rd, S.us, S.vs, S.ws, S.h1, S.m,
             S.p, S.dtp, tv<T>(u), tv<T>(v), tv<T>(w));
     return CF_OK;
 }
@@ -1588,7 +1590,7 @@ static cf_status enqueue_step_general_t(cf_run *r)
     const int nz = r->g.nz;
     const double dt = r->cfg.dt;
     const bool sc = r->cfg.scalar != 0;
-    const dim3 cg = cell_grid(r), cb(64, 4);
+    const dim3 cg = cell_grid(r), cb(256);
     const GSel<T> &K = Prec<T>::gen(r);
     T *u = tv<T>(r->u), *v = tv<T>(r->v), *w = tv<T>(r->w), *c = tv<T>(r->c);
     T *ru = tv<T>(r->ru), *rv = tv<T>(r->rv), *rw = tv<T>(r->rw), *rc = tv<T>(r->rc);
@@ -1763,7 +1765,7 @@ static cf_status project_general(cf_run *r, double dt)
     T *u = tv<T>(r->u), *v = tv<T>(r->v), *w = tv<T>(r->w);
     cf_status st = enqueue_pressure<T>(r, u, v, w, nullptr, nullptr, 3);
     if (st != CF_OK) return st;
-    KLAUNCH("project", Prec<T>::gen(r).proj, cell_grid(r), dim3(64, 4), 0, r->rd, (const T *) u, (const T *) v,
+    KLAUNCH("project", Prec<T>::gen(r).proj, cell_grid(r), dim3(256), 0, r->rd, (const T *) u, (const T *) v,
             (const T *) w, (const T *) nullptr, (const double *) nullptr, (const double *) nullptr,
             (const double *) nullptr, (const double *) nullptr, (const T *) tv<T>(r->p), dt, u, v, w, (T *) nullptr);
     return CF_OK;
@@ -1803,7 +1805,7 @@ static cf_status project_fast(cf_run *r, double dt)
     if (st != CF_OK) return st;
     double *su, *sv, *sw;
     state_set(r, r->cur, &su, &sv, &sw);
-    KLAUNCH("project", k_project2<T>, cell_grid(r), dim3(64, 4), 0, r->rd, (const T *) a, (const T *) b,
+    KLAUNCH("project", k_project2<T>, cell_grid(r), dim3(256), 0, r->rd, (const T *) a, (const T *) b,
             (const T *) c, (const double *) nullptr, (const double *) nullptr, (const T *) tv<T>(r->p), dt,
             tv<T>(su), tv<T>(sv), tv<T>(sw));
     return CF_OK;
@@ -1867,10 +1869,10 @@ static cf_status adaptive_step(cf_run *r)
     }
     const dim3 cg = cell_grid(r);
     if (r->prec == CF_FP32)
-        KLAUNCH("cfl", k_cfl_plain<float>, cg, dim3(64, 4), 0, r->rd, (const float *) mu, (const float *) mv,
+        KLAUNCH("cfl", k_cfl_plain<float>, cg, dim3(256), 0, r->rd, (const float *) mu, (const float *) mv,
                 (const float *) mw, r->cfg.dt, r->cflpart);
     else
-        KLAUNCH("cfl", k_cfl_plain<double>, cg, dim3(64, 4), 0, r->rd, mu, mv, mw, r->cfg.dt, r->cflpart);
+        KLAUNCH("cfl", k_cfl_plain<double>, cg, dim3(256), 0, r->rd, mu, mv, mw, r->cfg.dt, r->cflpart);
     KLAUNCH("cfl", k_cfl_reduce, dim3(1), dim3(256), 0, (const double *) r->cflpart, (int) (cg.x * cg.y * cg.z),
             r->scal);
     double cfl = 0.0;
@@ -2446,11 +2448,11 @@ static void batch_fill_args(cf_batch *b, std::vector<GArgs<T>> &A)
         a.gblocks = b->fast ? bblocks : r->gblocks;
         a.rhs_kc = bkc;
         for (int t = 0; t < 4; t++) { a.pt[t] = r->pt[t]; a.pt4[t] = r->pt4[t]; }
-        const unsigned nx = r->g.nx, ny = r->g.ny, nz = r->g.nz;
+        const unsigned ny = r->g.ny, nz = r->g.nz;
         const unsigned P = (unsigned) r->P, nf = (unsigned) r->nfield;
         auto set = [&](int st, unsigned x, unsigned y, unsigned z) { a.dims[st][0] = x; a.dims[st][1] = y; a.dims[st][2] = z; };
-        set(ST_CELL, (nx + 63) / 64, (ny + 3) / 4, nz);
-        set(ST_RHSG, (nx + 63) / 64, (ny + 3) / 4, nz * nf);
+        set(ST_CELL, (P + 255) / 256, 1, nz);
+        set(ST_RHSG, (P + 255) / 256, 1, nz * nf);
         if (run_uses_spike(b, r)) set(ST_SOLVE, (P + 63) / 64, nf, 1);
         else set(ST_SOLVE, (P + 255) / 256, nf, 1);
         set(ST_ONE, 1, 1, 1);
@@ -2611,8 +2613,8 @@ static cf_status batch_launch(cf_batch *b, int k, int s)
     dim3 block(256);
     size_t lds = 0;
     switch (k) {
-    case KB_RHS: fn = S.rhs; block = dim3(64, 4); break;
-    case KB_PROJ: fn = S.proj; block = dim3(64, 4); break;
+    case KB_RHS: fn = S.rhs; break;
+    case KB_PROJ: fn = S.proj; break;
     case KB_SOLVE:
         if (b->solve_kind == SOLVE_HEPT) { fn = kb_solve4<T>; break; }
         {
