@@ -67,3 +67,33 @@ def test_constraint_beside_the_solve(shape, kw):
     # forcings divide a cancellation by the unit response: absolute (test_gpu_parity.check_log)
     for col in range(13):
         assert np.allclose(got[:, col], want[:, col], rtol=1e-10, atol=1e-10), cf.LOG_COLUMNS[col]
+
+
+# FFT lengths with a run-time plan (each radix alone and together, one line
+# pair a workgroup, several workgroups of a short last one) and compiled ones
+@pytest.mark.parametrize("shape", [(90, 75, 3), (45, 27, 41), (2, 3, 2), (18, 54, 200), (1215, 4, 2), (2048, 2, 3), (125, 2, 5),
+                                   (64, 50, 9), (96, 15, 7), (128, 36, 5)])
+def test_fft3d_lengths(shape):
+    cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], stretch="uniform")
+    a = np.random.default_rng(3).standard_normal(cfg.shape)
+    ref = np.fft.fft(np.fft.rfft(a, axis=0) / cfg.nx, axis=1) / cfg.ny
+    with cf.Run(cfg) as run:
+        spec = run.fft3d_fwd(a)
+        back = run.fft3d_bwd(spec)
+    assert np.abs(spec - ref).max() <= 1e-14 * np.abs(ref).max() * np.log2(cfg.nx * cfg.ny)
+    assert np.abs(back - a).max() <= 1e-13 * np.abs(a).max()
+
+
+# the divergence + x FFT at its pair counts: through the projection, which
+# leaves the velocity free of divergence
+@pytest.mark.parametrize("prec,tol", [(cf.CF_FP64, 1e-11), (cf.CF_FP32, 2e-3)])
+@pytest.mark.parametrize("shape", [(64, 6, 3), (128, 9, 4), (96, 8, 5), (90, 15, 4), (24, 40, 33), (512, 6, 4), (600, 6, 4)])
+def test_divergence_pair_counts(shape, prec, tol):
+    cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], stretch="uniform", precision=prec)
+    f = cf.initial_fields(cfg, seed=2)
+    with cf.Run(cfg) as run:
+        for n in "uvw":
+            run.upload(n, f[n])
+        before = run.max_divergence()
+        run.project(1.0)
+        assert run.max_divergence() <= tol * before

@@ -1024,7 +1024,6 @@ template <typename T> struct BPick {
     {
         S.rhs = kb_rhs<ORD, SC, T>;
         S.proj = kb_proj<ORD, T>;
-        S.divx = pick_batched_divx<T>(ORD);
     }
 };
 

@@ -120,7 +120,7 @@ struct RunDev {
     const double2 *twx, *twy;
     const float2 *twx32, *twy32;  /* the same twiddles rounded to FP32 */
     const double *lamx, *lamy;  /* modified wavenumbers 2 - 2 cos(2 pi k / n) */
-    int fx_pairs;               /* complex x lines per block */
+    int fx_pairs, dx_pairs;     /* complex x lines per block: the x FFTs, the divergence + x FFT */
     int fy_cols;                /* kx columns per y-FFT block */
     /* general path (order 4 and/or the scalar) */
     Clos cl;
@@ -165,7 +165,7 @@ static __device__ __forceinline__ Blk blk_solve(unsigned b, unsigned nbx)
 }
 
 /* launch stages of a batched step; each run's grid per stage is dims[stage] */
-enum { ST_CELL = 0, ST_RHSG, ST_SOLVE, ST_ONE, ST_FFTX, ST_FFTY, ST_MODE, ST_RHS2, ST_LEVEL, CF_NST };
+enum { ST_CELL = 0, ST_RHSG, ST_SOLVE, ST_ONE, ST_DIVX, ST_FFTX, ST_FFTY, ST_MODE, ST_RHS2, ST_LEVEL, CF_NST };
 #define CF_BATCH_MAX 256        /* runs per batched launch */
 
 /* Where a substep's projected velocity comes from: the previous
@@ -267,6 +267,36 @@ static constexpr __host__ __device__ int fx_ld(int n, int esz)
 static constexpr __host__ __device__ int fx_pairs_of(int nx, int esz)
 {
     return fxi2_on(nx, esz) ? 2048 / nx : (CF_FX_ELEMS / nx > 0 ? CF_FX_ELEMS / nx : 1);
+}
+/* ... per workgroup of the divergence + x FFT: as many elements as its 256
+ * threads gather in one round of loads (two each, three in FP32), so that a
+ * workgroup waits for memory once (64 x 65 x 64 in FP64: 8 pairs 7.3 us, 32
+ * pairs 15.3); at 256 the pair counts its register passes are built for */
+static constexpr __host__ __device__ int dx_pairs_of(int nx, int esz)
+{
+    if (divx2_on(nx, esz) || nx == 256) return fx_pairs_of(nx, esz);
+    const int e = esz == 4 ? 768 : 512;
+    return e / nx > 0 ? e / nx : 1;
+}
+
+/* lengths whose divergence + x FFT is compiled for batches of an order and
+ * element size: those without register spills */
+static inline bool bdivx_compiled(int order, int n, int esz)
+{
+    return order == 2 && (n == 32 || n == 48 || n == 64 || n == 96 || n == 128 || (n == 192 && esz == 8));
+}
+/* FFT lengths with their plan compiled in (single runs) */
+#define CF_FFT_SIZES(X) X(16) X(20) X(24) X(30) X(32) X(40) X(48) X(60) X(64) X(80) X(96) \
+    X(120) X(128) X(160) X(192) X(240) X(256) X(320) X(384) X(480) X(512)
+static inline bool fft_compiled(int n)
+{
+    switch (n) {
+#define X_(N) case N:
+    CF_FFT_SIZES(X_)
+#undef X_
+        return true;
+    default: return false;
+    }
 }
 
 #ifndef CF_P2S_NC
@@ -655,7 +685,6 @@ template <typename T> struct BSel {
     typedef void (*rhs_t)(const GArgs<T> *, const unsigned *, int, int);
     rhs_t rhs;
     rhs_t proj;
-    divx_t_ divx;
     typedef void (*kb_t)(const GArgs<T> *, const unsigned *, int, int);
 };
 template <typename T> BSel<T> pick_batched(int order, int scalar);

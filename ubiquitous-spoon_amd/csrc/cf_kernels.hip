@@ -762,8 +762,9 @@ static __device__ __forceinline__ void store_half_spectra(const C *sb, int ld, i
     const bool on = swz && fsw_on(nx);
     const int nj = 2 * nl;
     const double rny = 1.0 / (double) ny;
+    const float rnj = 1.0f / (float) nj;
     for (int e = threadIdx.x; e < nj * nkx; e += blockDim.x) {
-        const int kx = e / nj, jj = e - kx * nj;
+        const int kx = sdiv(e, rnj), jj = e - kx * nj;
         const int l = jj >> 1;
         const bool second = (jj & 1) != 0;
         const long line = 2 * (pair0 + l) + (second ? 1 : 0);
@@ -916,8 +917,8 @@ static __device__ __forceinline__ void divx_body(const RunDev &R, const T *__res
     const int ny = R.g.ny, nz = R.g.nz, nkx = R.g.nkx;
     const int ld = fft_ld(nx);
     /* compiled lengths run only on runs of element size sizeof(T), whose
-     * pair count is fx_pairs_of(NX, sizeof(T)) */
-    const int nl = NX > 0 ? fx_pairs_of(NX, sizeof(T)) : R.fx_pairs;
+     * pair count is dx_pairs_of(NX, sizeof(T)) */
+    const int nl = NX > 0 ? dx_pairs_of(NX, sizeof(T)) : R.dx_pairs;
     const int NL = ny * nz;
     const size_t P = (size_t) nx * ny;
     const double rny = 1.0 / (double) ny;
@@ -971,7 +972,7 @@ static __device__ __forceinline__ void divx_body(const RunDev &R, const T *__res
      * values go to LDS once, as the first pass's outputs (one LDS round
      * trip and two barriers fewer); the other passes follow as usual */
     constexpr int NQ = NX > 0 ? NX / 4 : 1;
-    if constexpr (NX > 0 && ORD == 2 && ct_rad_at(NX, 0) == 4 && fx_pairs_of(NX, sizeof(T)) * NQ == 256 && NQ == 64) {
+    if constexpr (NX > 0 && ORD == 2 && ct_rad_at(NX, 0) == 4 && dx_pairs_of(NX, sizeof(T)) * NQ == 256 && NQ == 64) {
         if ((ny & 1) == 0) {                      /* workgroup-uniform */
             const cp<cv<C>> twg0 = (cp<cv<C>>) twsel<C>(R.twx, R.twx32);
             C *tws0 = sb + nl * ld;
@@ -1027,13 +1028,14 @@ static __device__ __forceinline__ void divx_body(const RunDev &R, const T *__res
     C *tws = sb + nl * ld;
     const C tw0 = tw_first<NX, C>(twg, nx);
     const int tot = nl * nx;
+    const float rnx = 1.0f / (float) nx;
     for (int e0 = 0; e0 < tot; e0 += UNR * 256) {
         C res[UNR];
 #pragma unroll
         for (int u = 0; u < UNR; u++) {
             const int e = e0 + (int) threadIdx.x + u * 256;
             const int ec = e < tot ? e : tot - 1;
-            const int l = ec / nx, i = ec - l * nx;
+            const int l = NX > 0 ? ec / nx : sdiv(ec, rnx), i = ec - l * nx;
             const int pr = pair0 + l;
             if (ORD == 2 && (nx & 63) == 0 && (ny & 1) == 0) {
                 /* the pair's lines are rows j, j + 1 of one level: the
@@ -1070,7 +1072,7 @@ static __device__ __forceinline__ void divx_body(const RunDev &R, const T *__res
         for (int u = 0; u < UNR; u++) {
             const int e = e0 + (int) threadIdx.x + u * 256;
             if (e < tot) {
-                const int l = e / nx, i = e - l * nx;
+                const int l = NX > 0 ? e / nx : sdiv(e, rnx), i = e - l * nx;
                 sb[l * ld + fsw(i, fsw_on(nx))] = res[u];
             }
         }
@@ -1105,8 +1107,9 @@ __global__ __launch_bounds__(256) void k_fftx_fwd_plain(const RunDev R, const do
     const cp<cv<double2>> twg = (cp<cv<double2>>) R.twx;
     double2 *tws = sb + nl * ld;
     const double2 tw0 = tw_first<NX, double2>(twg, nx);
+    const float rnx = 1.0f / (float) nx;
     for (int e = threadIdx.x; e < nl * nx; e += blockDim.x) {
-        int l = e / nx, i = e - l * nx;
+        int l = NX > 0 ? e / nx : sdiv(e, rnx), i = e - l * nx;
         long la = 2 * (pair0 + l), lb = la + 1;
         double va = la < NL ? a[(size_t) la * nx + i] : 0.0;
         double vb = lb < NL ? a[(size_t) lb * nx + i] : 0.0;
@@ -1265,6 +1268,7 @@ static __device__ __forceinline__ void ffty_body(const RunDev &R, typename Cplx<
     C *tws = sb + TK * ld;
     const C tw0 = tw_first<NY, C>(twg, ny);
     const int tot = TK * ny, totv = nl * ny;
+    const float rny = 1.0f / (float) ny;
     for (int e0 = 0; e0 < tot; e0 += 8 * 256) {
         C v[8];
 #pragma unroll
@@ -1277,7 +1281,7 @@ static __device__ __forceinline__ void ffty_body(const RunDev &R, typename Cplx<
         for (int u = 0; u < 8; u++) {
             const int e = e0 + (int) threadIdx.x + u * 256;
             if (e < tot) {
-                const int t = e / ny, j = e - t * ny;
+                const int t = NY > 0 ? e / ny : sdiv(e, rny), j = e - t * ny;
                 sb[t * ld + fsw(j, fsw_on(ny))] = v[u];
             }
         }
@@ -1287,7 +1291,7 @@ static __device__ __forceinline__ void ffty_body(const RunDev &R, typename Cplx<
     fft_lines<NY, 8>(sb, ny, ld, TK, (cp<int>) R.rady, R.nrady, (const C *) tws, fwd ? 1.0 : -1.0);
     const T sc = fwd ? (T) (1.0 / (double) ny) : (T) 1;
     for (int e = threadIdx.x; e < nl * ny; e += blockDim.x) {
-        int t = e / ny, j = e - t * ny;
+        int t = NY > 0 ? e / ny : sdiv(e, rny), j = e - t * ny;
         C val = sb[t * ld + fsw(j, fsw_on(ny))];
         base[e] = cv_of(fwd ? cscale(val, sc) : val);
     }
@@ -1400,7 +1404,7 @@ static __device__ __forceinline__ void fftxi_body(const RunDev &R, const typenam
     const int ny = R.g.ny, nz = R.g.nz, nkx = R.g.nkx;
     const int ld = fft_ld(nx);
     const int nl = NX > 0 ? fx_pairs_of(NX, sizeof(T)) : R.fx_pairs;
-    const double rnl = 1.0 / (double) nl;
+    const float rnl = 1.0f / (float) nl, rnx = 1.0f / (float) nx;
     const long NL = (long) ny * nz;
     const long pair0 = (long) xcd_block(b.x, b.nx) * nl;
     const int half = nx / 2;
@@ -1417,7 +1421,7 @@ static __device__ __forceinline__ void fftxi_body(const RunDev &R, const typenam
         for (int u = 0; u < CF_FXI_UNR; u++) {
             const int e = e0 + (int) threadIdx.x + u * 256;
             const int ec = e < tot ? e : tot - 1;
-            const int kx = NX > 0 ? ec / nl : qdiv(ec, nl, rnl), l = ec - kx * nl;
+            const int kx = NX > 0 ? ec / nl : sdiv(ec, rnl), l = ec - kx * nl;
             const int la = 2 * ((int) pair0 + l), lb = la + 1;
             const int lac = la < NLi ? la : NLi - 1;
             const int ka = qdiv(lac, ny, rny), ja = lac - ka * ny;
@@ -1434,7 +1438,7 @@ static __device__ __forceinline__ void fftxi_body(const RunDev &R, const typenam
         for (int u = 0; u < CF_FXI_UNR; u++) {
             const int e = e0 + (int) threadIdx.x + u * 256;
             if (e < tot) {
-                const int kx = NX > 0 ? e / nl : qdiv(e, nl, rnl), l = e - kx * nl;
+                const int kx = NX > 0 ? e / nl : sdiv(e, rnl), l = e - kx * nl;
                 C a = A[u], bq = B[u];
                 if (kx == 0 || (nx % 2 == 0 && kx == half)) { a.y = (T) 0; bq.y = (T) 0; }
                 sb[l * ld + fsw(kx, fsw_on(nx))] = mkc<C>(a.x - bq.y, a.y + bq.x);
@@ -1446,7 +1450,7 @@ static __device__ __forceinline__ void fftxi_body(const RunDev &R, const typenam
     __syncthreads();
     fft_lines<NX, 8>(sb, nx, ld, nl, (cp<int>) R.radx, R.nradx, (const C *) tws, -1.0);
     for (int e = threadIdx.x; e < nl * nx; e += blockDim.x) {
-        int l = e / nx, i = e - l * nx;
+        int l = NX > 0 ? e / nx : sdiv(e, rnx), i = e - l * nx;
         long la = 2 * (pair0 + l), lb = la + 1;
         C z = sb[l * ld + fsw(i, fsw_on(nx))];
         if (la < NL) p[(size_t) la * nx + i] = z.x;
@@ -1462,9 +1466,6 @@ __global__ __launch_bounds__(256) void k_fftx_inv(const RunDev R, const typename
 }
 
 /* host-side selectors of the compile-time instances */
-#define CF_FFT_SIZES(X) X(16) X(20) X(24) X(30) X(32) X(40) X(48) X(60) X(64) X(80) X(96) \
-    X(120) X(128) X(160) X(192) X(240) X(256) X(320) X(384) X(480) X(512)
-
 template <typename T, int ORD>
 static typename KSel<T>::div_t pick_div_ord(int n)
 {
@@ -1991,15 +1992,16 @@ template __global__ void k_maxdiv_part<float>(const RunDev, const float *, const
  * compiled in; 0: any lengths, runtime plan.  Where it fits without
  * spills, the occupancy target caps them at 128 VGPRs (4 waves per SIMD). */
 /* compiled lengths gather 2 elements per thread in FP32 (not 3) so that
- * the batch loop's extra registers still fit 4 waves per SIMD */
+ * the batch loop's extra registers still fit 4 waves per SIMD (96 in FP64
+ * spills there and runs at 3) */
 template <int NX, int ORD, typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((NX > 0 && ORD == 2) ? (divx2_on(NX, sizeof(T)) ? 2 : 4) : 1, 8))) void kb_divx(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((NX > 0 && ORD == 2) ? (NX == 96 && sizeof(T) == 8 ? 3 : 4) : 1, 8))) void kb_divx(
     const GArgs<T> *__restrict__ A, const unsigned *__restrict__ vs, int nrun, int s)
 {
     constexpr int U = (NX > 0 && ORD == 2 && sizeof(T) == 4) ? 2 : 0;
     batch_loop(vs, nrun, [&](int r, unsigned lb) {
         const GArgs<T> &a = A[r];
-        const Blk b = blk_of(a, ST_FFTX, lb);
+        const Blk b = blk_of(a, ST_DIVX, lb);
         if (s < 3)
             divx_body<NX, ORD, T, U>(a.R, a.ru, a.rv, a.rw, a.R.h1 + (size_t) (s * 2) * (a.R.g.nz + 2),
                                      a.scal + SC_M0 + s, a.X, b);
@@ -2033,25 +2035,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((NX > 0 && 
     });
 }
 
-/* per-length batched FFT launches (n = bfft_key of the group's length).
- * The divergence + x-FFT has its length compiled in only where that fits
- * 4 waves per SIMD without spills inside the batch loop (order 2, n <= 128
- * in FP32, n <= 64 in FP64); other groups take the runtime plan. */
+/* the divergence + x-FFT of a batch's length group: compiled where
+ * bdivx_compiled says so (without register spills), else the run-time plan */
 template <typename T>
 typename BSel<T>::kb_t pick_batched_divx_n(int order, int n)
 {
-    constexpr int lim = sizeof(T) == 4 ? 128 : 64;
-    if (order == 2) {
-        switch (n) {
-        case 32: return kb_divx<32, 2, T>;
-        case 48: return kb_divx<48, 2, T>;
-        case 64: return kb_divx<64, 2, T>;
-        case 96: if constexpr (lim >= 96) return kb_divx<96, 2, T>; break;
-        case 128: if constexpr (lim >= 128) return kb_divx<128, 2, T>; break;
-        default: break;
-        }
+    if (!bdivx_compiled(order, n, sizeof(T))) return pick_batched_divx<T>(order);
+    switch (n) {
+    case 32: return kb_divx<32, 2, T>;
+    case 48: return kb_divx<48, 2, T>;
+    case 64: return kb_divx<64, 2, T>;
+    case 96: return kb_divx<96, 2, T>;
+    case 128: return kb_divx<128, 2, T>;
+    default:
+        if constexpr (sizeof(T) == 8) return kb_divx<192, 2, T>;
+        else return pick_batched_divx<T>(order);
     }
-    return pick_batched_divx<T>(order);
 }
 template <typename T>
 typename BSel<T>::kb_t pick_batched_ffty(int n)

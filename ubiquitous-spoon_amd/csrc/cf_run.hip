@@ -608,6 +608,10 @@ static void free_run(cf_run *r)
 
 /* ------------------------------------------------------------ create */
 
+/* y lines per workgroup: 8 elements per thread (up to 32 short lines) */
+static int fy_cols_of(int ny) { return MAXE_LINE / ny >= 32 ? 32 : (MAXE_LINE / ny > 0 ? MAXE_LINE / ny : 1); }
+#define CF_FFT_WGS 512
+
 static long rhs_tiles(int nx, int ny) { return (long) ((nx + CF_RT_X - 1) / CF_RT_X) * ((ny + CF_RT_Y - 1) / CF_RT_Y); }
 
 /* balanced z-chunks of the fused RHS for a target length: levels per
@@ -1292,19 +1296,26 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     r->kfxi = pick_fftx_inv<double>(nx);
     r->kfy32 = pick_ffty<float>(ny);
     r->kfxi32 = pick_fftx_inv<float>(nx);
+    R.rnx = 1.0 / (double) nx;
     R.rdx = 1.0 / r->g.dx;
     R.rdy = 1.0 / r->g.dy;
     R.rdxdy = 1.0 / (r->g.dx * r->g.dy);
     R.cmode[0] = cfg->uvolavgmode; R.ctarget[0] = cfg->want_uvolavg - cfg->uframe; R.cfixed[0] = -cfg->dpdx;
-    R.rnx = 1.0 / (double) nx;
     R.cmode[1] = cfg->cvolavgmode; R.ctarget[1] = cfg->want_cvolavg; R.cfixed[1] = 0.0;
     R.logcap = LOGCAP;
+    /* Lines per FFT workgroup: as many as its threads hold (fx_pairs_of,
+     * fy_cols_of), but no more than give CF_FFT_WGS workgroups -- a small grid's
+     * transforms are bound by one workgroup's chain of passes (90 x 73 x 75: y
+     * FFT 8.9 us, 11.5 with 27 lines each on 125 CUs).  Compiled x lengths
+     * have their pair count compiled in. */
+    const long npairs = ((long) ny * nz + 1) / 2;
     R.fx_pairs = fx_pairs_of(nx, (int) r->esz);
-    /* y lines per workgroup: 8 elements per thread (up to 32 short lines) */
-    R.fy_cols = MAXE_LINE / ny >= 32 ? 32 : (MAXE_LINE / ny > 0 ? MAXE_LINE / ny : 1);
+    if (!fft_compiled(nx)) R.fx_pairs = (int) std::max(1L, std::min((long) R.fx_pairs, npairs / CF_FFT_WGS));
+    R.dx_pairs = dx_pairs_of(nx, (int) r->esz);
+    R.fy_cols = (int) std::max(1L, std::min((long) fy_cols_of(ny), (long) nz * r->g.nkx / CF_FFT_WGS));
     /* the two-pass y FFT gives each of a workgroup's 256 threads at most
      * one (line, column) task per pass */
-    if (fy2_p1(ny) && R.fy_cols * std::max(fy2_p1(ny), ny / fy2_p1(ny)) > 256) {
+    if (fy2_p1(ny) && fy_cols_of(ny) * std::max(fy2_p1(ny), ny / fy2_p1(ny)) > 256) {
         free_run(r);
         cf_set_error("ny = %d: y-FFT workgroup shape", ny);
         return CF_ERR_UNSUPPORTED;
@@ -1367,14 +1378,18 @@ static cf_status ev_end(cf_run *r)
 /* one thread per cell: 256 consecutive cells of a level per workgroup */
 static dim3 cell_grid(const cf_run *r) { return dim3((unsigned) ((r->P + 255) / 256), 1, r->g.nz); }
 
-static size_t fx_lds(const cf_run *r)
+/* LDS of the x and y FFT launches: a workgroup's lines and the twiddles */
+static size_t fx_lds_n(const cf_run *r, int pairs)
 {
-    return 2 * r->esz * ((size_t) r->rd.fx_pairs * fx_ld(r->g.nx, (int) r->esz) + (size_t) r->g.nx);
+    return 2 * r->esz * ((size_t) pairs * fx_ld(r->g.nx, (int) r->esz) + (size_t) r->g.nx);
 }
-static size_t fy_lds(const cf_run *r)
+static size_t fx_lds(const cf_run *r) { return fx_lds_n(r, r->rd.fx_pairs); }
+static size_t dx_lds(const cf_run *r) { return fx_lds_n(r, r->rd.dx_pairs); }
+static size_t fy_lds_n(const cf_run *r, int cols)
 {
-    return 2 * r->esz * ((size_t) r->rd.fy_cols * fy_ld(r->g.ny) + (size_t) r->g.ny);
+    return 2 * r->esz * ((size_t) cols * fy_ld(r->g.ny) + (size_t) r->g.ny);
 }
+static size_t fy_lds(const cf_run *r) { return fy_lds_n(r, r->rd.fy_cols); }
 
 /* the kernel sets and typed views of the run's buffers for precision T */
 template <typename T> struct Prec;
@@ -1415,8 +1430,8 @@ static cf_status enqueue_pressure(cf_run *r, const T *us, const T *vs, const T *
     const RunDev &R = r->rd;
     long NL = (long) r->g.ny * r->g.nz;
     long npairs = (NL + 1) / 2;
-    unsigned gx = (unsigned) ((npairs + R.fx_pairs - 1) / R.fx_pairs);
-    KLAUNCH("div_fftx", Prec<T>::div(r), dim3(gx), dim3(256), fx_lds(r), R, us, vs, ws, h1, mptr, X);
+    const unsigned gx = (unsigned) ((npairs + R.fx_pairs - 1) / R.fx_pairs), gd = (unsigned) ((npairs + R.dx_pairs - 1) / R.dx_pairs);
+    KLAUNCH("div_fftx", Prec<T>::div(r), dim3(gd), dim3(256), dx_lds(r), R, us, vs, ws, h1, mptr, X);
     dim3 gy(fy_blocks(r));
     KLAUNCH("ffty_fwd", Prec<T>::ffty(r), gy, dim3(256), fy_lds(r), R, X, 1);
     if (r->g.order == 4)
@@ -2335,7 +2350,7 @@ extern "C" cf_status cf_op_poisson(cf_run *r, double *spec, double dt)
 
 enum { KB_RHS = 0, KB_SOLVE, KB_MASS, KB_DIVX, KB_FFTY, KB_POIS, KB_FFTXI, KB_PROJ, KB_FRHS, KB_FSPIKE, KB_FLEVEL,
        KB_N };
-static const int KB_STAGE[KB_N] = { ST_RHSG, ST_SOLVE, ST_ONE, ST_FFTX, ST_FFTY, ST_MODE, ST_FFTX, ST_CELL,
+static const int KB_STAGE[KB_N] = { ST_RHSG, ST_SOLVE, ST_ONE, ST_DIVX, ST_FFTY, ST_MODE, ST_FFTX, ST_CELL,
                                     ST_RHS2, ST_SOLVE, ST_LEVEL };
 static const char *KB_NAME[KB_N] = { "rhs", "solve", "mass", "div_fftx", "ffty", "poisson", "fftx_inv", "project",
                                      "rhs", "spike", "plane_sum" };
@@ -2354,7 +2369,7 @@ struct cf_batch {
     std::vector<int> fxK, fyK;            /* distinct x / y FFT plan keys (bfft_key), one launch each */
     unsigned kgrid[KB_N] = {0};
     int spike_waves = 1, ncu = 256;
-    size_t lds_fx = 0, lds_fy = 0, lds_mass = 0;
+    size_t lds_mass = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     /* order-2 runs (FP64 or FP32) without the scalar step on the fast path's fused
@@ -2382,7 +2397,8 @@ struct cf_batch {
 #define CF_FFT_NG 8                        /* FFT length groups: bfft_key values (7 sizes and 0) */
 #define CF_FX_ROW0 (CF_P2I_ROW0 + CF_P2_NG)      /* x-FFT groups (by nx): rows CF_FX_ROW0 + g */
 #define CF_FY_ROW0 (CF_FX_ROW0 + CF_FFT_NG)      /* y-FFT groups (by ny) */
-#define CF_TH_ROW (CF_FY_ROW0 + CF_FFT_NG)       /* order-2 runs without spike tables: Thomas */
+#define CF_DX_ROW0 (CF_FY_ROW0 + CF_FFT_NG)      /* divergence + x-FFT groups (by nx) */
+#define CF_TH_ROW (CF_DX_ROW0 + CF_FFT_NG)       /* order-2 runs without spike tables: Thomas */
 #define CF_VS_ROWS (CF_TH_ROW + 1)
 /* an order-2 run solves its z systems as it does alone: the spike where
  * its tables exist, Thomas otherwise (the two round differently) */
@@ -2421,6 +2437,16 @@ static void batch_fft_groups(cf_batch *b)
     }
 }
 
+/* line pairs per workgroup of a batched run's divergence + x FFT: one round
+ * of loads where its length is compiled (18 FP64 runs in three lengths: 231
+ * us in three launches), full workgroups on the run-time plan (the same runs:
+ * 264 us in one launch; 312 with one round of loads) */
+static int batch_dx_pairs(const cf_run *r)
+{
+    const int nx = (int) r->g.nx, esz = (int) r->esz;
+    return bdivx_compiled(r->g.order, nx, esz) ? dx_pairs_of(nx, esz) : fx_pairs_of(nx, esz);
+}
+
 template <typename T>
 static void batch_fill_args(cf_batch *b, std::vector<GArgs<T>> &A)
 {
@@ -2432,6 +2458,10 @@ static void batch_fill_args(cf_batch *b, std::vector<GArgs<T>> &A)
         cf_run *r = b->runs[q];
         GArgs<T> &a = A[q];
         a.R = r->rd;
+        /* a batch has workgroups enough: full ones */
+        a.R.fx_pairs = fx_pairs_of((int) r->g.nx, (int) r->esz);
+        a.R.fy_cols = fy_cols_of((int) r->g.ny);
+        a.R.dx_pairs = batch_dx_pairs(r);
         a.u = tv<T>(r->u); a.v = tv<T>(r->v); a.w = tv<T>(r->w); a.c = tv<T>(r->c);
         a.ru = tv<T>(r->ru); a.rv = tv<T>(r->rv); a.rw = tv<T>(r->rw); a.rc = tv<T>(r->rc);
         for (int f = 0; f < 4; f++) { a.fa[f] = tv<T>(r->fa[f]); a.fb[f] = tv<T>(r->fb[f]); }
@@ -2457,8 +2487,9 @@ static void batch_fill_args(cf_batch *b, std::vector<GArgs<T>> &A)
         else set(ST_SOLVE, (P + 255) / 256, nf, 1);
         set(ST_ONE, 1, 1, 1);
         long NL = (long) ny * nz, npairs = (NL + 1) / 2;
-        set(ST_FFTX, (unsigned) ((npairs + r->rd.fx_pairs - 1) / r->rd.fx_pairs), 1, 1);
-        set(ST_FFTY, fy_blocks(r), 1, 1);
+        set(ST_FFTX, (unsigned) ((npairs + a.R.fx_pairs - 1) / a.R.fx_pairs), 1, 1);
+        set(ST_DIVX, (unsigned) ((npairs + a.R.dx_pairs - 1) / a.R.dx_pairs), 1, 1);
+        set(ST_FFTY, (unsigned) (((long) nz * r->g.nkx + a.R.fy_cols - 1) / a.R.fy_cols), 1, 1);
         set(ST_MODE, b->order == 2 ? pois2_blocks(pois2_L(r->g.nz), r->M) : (unsigned) ((r->M + 255) / 256), 1, 1);
         set(ST_RHS2, (unsigned) std::max(bblocks, 1), 1, 1);
         set(ST_LEVEL, nz, 1, 1);
@@ -2490,12 +2521,12 @@ static cf_status batch_upload_tables(cf_batch *b)
                 continue;
             }
             if (st >= CF_FX_ROW0) {               /* FFT length group */
-                const bool y = st >= CF_FY_ROW0;
-                const int g = st - (y ? CF_FY_ROW0 : CF_FX_ROW0);
+                const bool d = st >= CF_DX_ROW0, y = !d && st >= CF_FY_ROW0;
+                const int g = st - (d ? CF_DX_ROW0 : (y ? CF_FY_ROW0 : CF_FX_ROW0));
                 const std::vector<int> &K = y ? b->fyK : b->fxK;
                 const cf_run *rq = b->runs[q];
                 if (g < (int) K.size() && bfft_key((int) (y ? rq->g.ny : rq->g.nx)) == K[g]) {
-                    const int sd2 = y ? ST_FFTY : ST_FFTX;
+                    const int sd2 = d ? ST_DIVX : (y ? ST_FFTY : ST_FFTX);
                     acc += A[q].dims[sd2][0] * A[q].dims[sd2][1] * A[q].dims[sd2][2];
                 }
                 continue;
@@ -2592,8 +2623,10 @@ static cf_status batch_launch_fft(cf_batch *b, int k, int s)
                                   : (k == KB_DIVX ? pick_batched_divx_n<T>(b->order, K[g]) : pick_batched_fftxi<T>(K[g]));
         size_t lds = 0;
         for (const cf_run *r : b->runs)
-            if (bfft_key((int) (y ? r->g.ny : r->g.nx)) == K[g]) lds = std::max(lds, y ? fy_lds(r) : fx_lds(r));
-        const int row = (y ? CF_FY_ROW0 : CF_FX_ROW0) + (int) g;
+            if (bfft_key((int) (y ? r->g.ny : r->g.nx)) == K[g])
+                lds = std::max(lds, y ? fy_lds_n(r, fy_cols_of((int) r->g.ny))
+                                  : (k == KB_DIVX ? fx_lds_n(r, batch_dx_pairs(r)) : fx_lds_n(r, fx_pairs_of((int) r->g.nx, (int) r->esz))));
+        const int row = (y ? CF_FY_ROW0 : (k == KB_DIVX ? CF_DX_ROW0 : CF_FX_ROW0)) + (int) g;
         const unsigned tg = batch_total(b, row);
         const unsigned grid = b->kgrid[k] ? std::min(b->kgrid[k], tg) : tg;
         if (grid == 0) continue;
@@ -2634,10 +2667,6 @@ static cf_status batch_launch(cf_batch *b, int k, int s)
         }
     case KB_MASS: fn = kb_mass<T>; break;
     case KB_DIVX:
-        /* FP64: one runtime-plan launch over all runs (its compiled forms
-         * spill beyond length 64, and split launches measured slower) */
-        if constexpr (std::is_same<T, double>::value) { fn = S.divx; lds = b->lds_fx; break; }
-        else return batch_launch_fft<T>(b, k, s);
     case KB_FFTY:
     case KB_FFTXI:
         return batch_launch_fft<T>(b, k, s);
@@ -2896,7 +2925,7 @@ extern "C" cf_status cf_batch_create(const cf_config *cfgs, int nrun, cf_batch *
             b->runs.clear();
             b->fast = false;
             b->spike_waves = 1;
-            b->lds_fx = b->lds_fy = b->lds_mass = 0;
+            b->lds_mass = 0;
             q = -1;
             continue;
         }
@@ -2909,8 +2938,6 @@ extern "C" cf_status cf_batch_create(const cf_config *cfgs, int nrun, cf_batch *
         }
         b->runs.push_back(r);
         b->spike_waves = std::max(b->spike_waves, r->spike_waves);
-        b->lds_fx = std::max(b->lds_fx, fx_lds(r));
-        b->lds_fy = std::max(b->lds_fy, fy_lds(r));
         b->lds_mass = std::max(b->lds_mass, sizeof(double) * (size_t) r->g.nz);
     }
     b->p2L = batch_p2L(b->runs);
@@ -3336,11 +3363,9 @@ static cf_status srv_regroup(cf_server *s, int k, cf_server::Group &G)
             if (r->cur != b->cur) swap_state_sets(r);
     }
     b->spike_waves = 1;
-    b->lds_fx = b->lds_fy = b->lds_mass = 0;
+    b->lds_mass = 0;
     for (cf_run *r : runs) {
         b->spike_waves = std::max(b->spike_waves, r->spike_waves);
-        b->lds_fx = std::max(b->lds_fx, fx_lds(r));
-        b->lds_fy = std::max(b->lds_fy, fy_lds(r));
         b->lds_mass = std::max(b->lds_mass, sizeof(double) * (size_t) r->g.nz);
     }
     b->solve_kind = b->order == 4 ? SOLVE_HEPT : SOLVE_SPIKE;   /* per run: spike or Thomas as alone */
