@@ -97,3 +97,32 @@ def test_divergence_pair_counts(shape, prec, tol):
         before = run.max_divergence()
         run.project(1.0)
         assert run.max_divergence() <= tol * before
+
+
+# rows per wave and columns per march of the spectra, levels and partials of
+# the plane sums
+@pytest.mark.parametrize("shape", [(2, 6, 3), (12, 6, 5), (16, 64, 4), (18, 135, 3), (45, 27, 7), (90, 80, 5)])
+def test_statistics_launch_shapes(shape):
+    cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], stretch="uniform")
+    nx, ny = cfg.nx, cfg.ny
+    rng = np.random.default_rng(5)
+    with cf.Run(cfg) as run:
+        f = {}
+        for n in "uv":
+            f[n] = 0.3 + rng.standard_normal(cfg.shape)
+            run.upload(n, f[n])
+        for a, b in ("uu", "uv"):
+            s = [np.fft.fft(np.fft.rfft(f[n], axis=0) / nx, axis=1) / ny for n in (a, b)]
+            q = s[0] * s[1].conj()
+            q[0, 0] = 0
+            sx, sy = run.xy_stats("spec", a, b)
+            inner = q[1:(nx + 1) // 2].sum(0)
+            mirror = np.conj(inner[-np.arange(ny // 2 + 1) % ny])
+            want = q.sum(0)[:ny // 2 + 1] + mirror
+            # sums of at most nx ny products: a few units of rounding of the largest
+            scale = 1e-13 * np.abs(q).sum(axis=(0, 1)).max()
+            assert np.abs(sx - q.sum(1)).max() <= scale and np.abs(sy - want).max() <= scale
+            d = [f[n] - f[n].mean(axis=(0, 1)) for n in (a, b)]
+            assert np.abs(run.xy_stats("corr", a, b) - (d[0] * d[1]).mean(axis=(0, 1))).max() <= 1e-13
+            assert np.abs(run.xy_stats("avg", b) - f[b].mean(axis=(0, 1))).max() <= 1e-13
+        assert np.abs(run.xy_stats("moment", "u", en=3.0) - ((f["u"] - f["u"].mean(axis=(0, 1))) ** 3).mean(axis=(0, 1))).max() <= 1e-11

@@ -725,13 +725,19 @@ template <typename T>
 __global__ void k_poisson4t(const RunDev R, const Pois4Tab T_, typename Cplx<T>::type *Y, double *S);
 
 /* plane statistics (cf_stats.hip) */
+template <typename T> __global__ void k_stat_sum(const T *a, const T *b, int P, int nbl, double *part);
 template <typename T, int MODE>
-__global__ void k_stat_plane(const T *a, const T *b, const double *ma, const double *mb, double en, int P, int nbl,
-                             double *part);
+__global__ void k_stat_central(const T *a, const T *b, const double *pa, const double *pb, double scale, double en,
+                               int P, int nbl, double *part);
 __global__ void k_stat_finish(const double *part, int nbl, int nz, double scale, double *out, const double *off);
-__global__ void k_stat_spec(const double2 *A, const double2 *B, int nx, int ny, int nkx, int nz, double *specx,
-                            double *specy);
+#define CF_SPEC_ROWS 8          /* rows kx per wave of k_stat_spec */
+__global__ void k_stat_spec(const double2 *A, const double2 *B, int nx, int ny, int nkx, int nz, double2 *specx,
+                            double2 *part);
+__global__ void k_stat_spec_finish(const double2 *specx, const double2 *part, int ny, int nkx, int nz, double2 *out);
 template <typename T> __global__ void k_stat_widen(const T *in, double *out, size_t n);
-#define CF_STAT_NBL 64          /* workgroups (partials) per level of a plane statistic */
+/* workgroups (partials) per level of a plane statistic: 8 cells a thread, up
+ * to the 64 partials that one wave sums */
+#define CF_STAT_NBL 64
+static inline int stat_nbl(size_t P) { return (int) (P / 2048 < 1 ? 1 : P / 2048 > CF_STAT_NBL ? CF_STAT_NBL : P / 2048); }
 
 #endif

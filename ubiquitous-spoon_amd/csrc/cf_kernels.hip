@@ -1091,7 +1091,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((ORD == 2 &
     divx_body<NX, ORD, T>(R, us, vs, ws, h1, mptr, X, blk_native());
 }
 
-/* the fftx_d2c stage of FFT3D_FWD on its own (no divergence), scaled 1/nx */
+/* the fftx_d2c stage of FFT3D_FWD on its own (no divergence), scaled 1/nx;
+ * the divergence + x FFT's pair counts, for its reason (128 x 97 x 128: 16
+ * pairs 12.3 us, 4 pairs 10.2) */
 template <int NX>
 __global__ __launch_bounds__(256) void k_fftx_fwd_plain(const RunDev R, const double *__restrict__ a,
                                                         double2 *__restrict__ X)
@@ -1101,19 +1103,32 @@ __global__ __launch_bounds__(256) void k_fftx_fwd_plain(const RunDev R, const do
     const int nx = NX > 0 ? NX : R.g.nx;
     const int ny = R.g.ny, nz = R.g.nz, nkx = R.g.nkx;
     const int ld = fft_ld(nx);
-    const int nl = R.fx_pairs;
-    const long NL = (long) ny * nz;
-    const long pair0 = (long) blockIdx.x * nl;
+    const int nl = R.dx_pairs;
+    const int NL = ny * nz;
+    const int pair0 = (int) blockIdx.x * nl;
     const cp<cv<double2>> twg = (cp<cv<double2>>) R.twx;
     double2 *tws = sb + nl * ld;
     const double2 tw0 = tw_first<NX, double2>(twg, nx);
     const float rnx = 1.0f / (float) nx;
-    for (int e = threadIdx.x; e < nl * nx; e += blockDim.x) {
-        int l = NX > 0 ? e / nx : sdiv(e, rnx), i = e - l * nx;
-        long la = 2 * (pair0 + l), lb = la + 1;
-        double va = la < NL ? a[(size_t) la * nx + i] : 0.0;
-        double vb = lb < NL ? a[(size_t) lb * nx + i] : 0.0;
-        sb[l * ld + fsw(i, fsw_on(nx))] = make_double2(va, vb);
+    const int tot = nl * nx;
+    for (int e0 = 0; e0 < tot; e0 += 2 * 256) {
+        double2 v[2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int e = e0 + (int) threadIdx.x + t * 256, ec = e < tot ? e : tot - 1;
+            const int l = NX > 0 ? ec / nx : sdiv(ec, rnx), i = ec - l * nx;
+            const int la = 2 * (pair0 + l), lb = la + 1;
+            const double va = a[(size_t) (la < NL ? la : NL - 1) * nx + i], vb = a[(size_t) (lb < NL ? lb : NL - 1) * nx + i];
+            v[t] = make_double2(la < NL ? va : 0.0, lb < NL ? vb : 0.0);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int e = e0 + (int) threadIdx.x + t * 256;
+            if (e < tot) {
+                const int l = NX > 0 ? e / nx : sdiv(e, rnx), i = e - l * nx;
+                sb[l * ld + fsw(i, fsw_on(nx))] = v[t];
+            }
+        }
     }
     tw_rest<NX, double2>(tws, tw0, twg, nx);
     __syncthreads();
@@ -1900,7 +1915,9 @@ KSel<float>::pois2_t pick_poisson2_islands(int L)
  * project2 (pressure.c:120-152) fused with the mass-flux correction:
  * u = (u* + h1 mdpdx) - (p_{i+1} - p_i) dt / dx, v, w likewise.  The
  * top-wall face is left at its Dirichlet value 0 (the reference subtracts
- * the Neumann-ghost difference there, which is round-off).
+ * the Neumann-ghost difference there, which is round-off).  A null output is
+ * left out: the copy in and out bounds it (128 x 97 x 128: three fields 17 us,
+ * one or two 11).
  * ------------------------------------------------------------------- */
 template <typename T>
 __global__ __launch_bounds__(256) void k_project2(const RunDev R, const T *__restrict__ us,
@@ -1918,14 +1935,12 @@ __global__ __launch_bounds__(256) void k_project2(const RunDev R, const T *__res
     const double *rdzh = R.rdzh + CF_NGT;
     const T m = mptr ? (T) *mptr : (T) 0;
     const T p0 = p[q];
-    T uc = us[q] + (h1 ? (T) h1[k + 1] * m : (T) 0);
-    u[q] = uc - (p[(size_t) k * P + (size_t) j * nx + ip] - p0) * (T) (dtp * R.rdx);
-    v[q] = vs[q] - (p[(size_t) k * P + (size_t) jp * nx + i] - p0) * (T) (dtp * R.rdy);
-    if (k < nz - 1) {
-        w[q] = ws[q] - (p[q + P] - p0) * (T) (dtp * rdzh[k]);
-    } else {
-        w[q] = (T) 0;
+    if (u) {
+        T uc = us[q] + (h1 ? (T) h1[k + 1] * m : (T) 0);
+        u[q] = uc - (p[(size_t) k * P + (size_t) j * nx + ip] - p0) * (T) (dtp * R.rdx);
     }
+    if (v) v[q] = vs[q] - (p[(size_t) k * P + (size_t) jp * nx + i] - p0) * (T) (dtp * R.rdy);
+    if (w) w[q] = k < nz - 1 ? ws[q] - (p[q + P] - p0) * (T) (dtp * rdzh[k]) : (T) 0;
 }
 template __global__ void k_project2<double>(const RunDev, const double *, const double *, const double *, const double *,
     const double *, const double *, double, double *, double *, double *);

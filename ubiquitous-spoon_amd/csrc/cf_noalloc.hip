@@ -4,8 +4,8 @@
  * their work space in a fixed device array instead of a per-call
  * allocation, for callers that cannot allocate device memory.
  *
- * The work space (CF_STAT_NBL partial sums per level, two mean profiles
- * and the result profile) lives in `scratch`, one copy per GPU for the
+ * The work space (CF_STAT_NBL partial sums per level of two fields and of
+ * their central sum, and the result profile) lives in `scratch`, one copy per GPU for the
  * life of the process.  Its device address is looked up once per device,
  * with that device current, and only that address is handed to kernels and
  * copies.  Every call on a GPU shares the GPU's array: calls that overlap
@@ -22,7 +22,7 @@
 #include <mutex>
 
 #define CF_NOALLOC_NZ_MAX 2048
-#define CF_NOALLOC_DOUBLES ((size_t) (CF_STAT_NBL + 3) * CF_NOALLOC_NZ_MAX)
+#define CF_NOALLOC_DOUBLES ((size_t) (3 * CF_STAT_NBL + 1) * CF_NOALLOC_NZ_MAX)
 #define CF_NOALLOC_DEVICES 64
 
 static __device__ __align__(256) double scratch[CF_NOALLOC_DOUBLES];
@@ -67,7 +67,7 @@ extern "C" cf_status cf_run_xy_stats_noalloc(cf_run *run, int kind, int field_a,
     }
     int nz = 0, device = 0;
     void *stream = nullptr;
-    cf_status st = cf_run_stat_plane_into(run, kind, field_a, field_b, en, nullptr, nullptr, nullptr, &nz, &stream,
+    cf_status st = cf_run_stat_plane_into(run, kind, field_a, field_b, en, nullptr, nullptr, &nz, &stream,
                                           &device);
     if (st != CF_OK) return st;
     if (nz > CF_NOALLOC_NZ_MAX) {
@@ -77,8 +77,8 @@ extern "C" cf_status cf_run_xy_stats_noalloc(cf_run *run, int kind, int field_a,
     }
     double *ws = nullptr;
     if ((st = scratch_ptr(device, &ws)) != CF_OK) return st;
-    double *part = ws, *means = ws + (size_t) CF_STAT_NBL * nz, *res = means + 2 * (size_t) nz;
-    st = cf_run_stat_plane_into(run, kind, field_a, field_b, en, part, means, res, nullptr, nullptr, nullptr);
+    double *part = ws, *res = ws + (size_t) 3 * CF_STAT_NBL * nz;
+    st = cf_run_stat_plane_into(run, kind, field_a, field_b, en, part, res, nullptr, nullptr, nullptr);
     if (st != CF_OK) return st;
     const hipStream_t s = (hipStream_t) stream;
     if (hipMemcpyAsync(out, res, sizeof(double) * (size_t) nz, hipMemcpyDeviceToHost, s) != hipSuccess

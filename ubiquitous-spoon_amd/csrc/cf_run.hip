@@ -131,6 +131,7 @@ struct cf_run {
     std::vector<double> ubar;
     double *uoffd = nullptr;
     double dtp_prev = 0.0;
+    double *statres = nullptr;       /* pinned: a plane statistic's result */
     bool prev_proj = false;
     /* profiling */
     bool profile = false;
@@ -584,7 +585,9 @@ extern "C" cf_status cf_run_footprint(const cf_config *cfg, size_t *bytes)
     size_t es = cfg->precision == CF_FP32 ? sizeof(float) : sizeof(double);
     /* state, solve output and two forcing slots per field, p: (4 nf + 1) N values;
      * X: 2 M values; FP64 stage N, G M, order-4 Poisson factors 3 M */
-    *bytes = es * ((4 * nf + 1) * N + 2 * M) + sizeof(double) * (N + (cfg->order == 4 ? 4 : 1) * M)
+    /* a tendency slot holds a spectrum: 2 M - N values more; the partial sums
+     * of the plane statistics: 192 nz */
+    *bytes = es * (4 * nf * N + 4 * M) + sizeof(double) * 192 * cfg->nz + sizeof(double) * (N + (cfg->order == 4 ? 4 : 1) * M)
            + ((size_t) 16 << 20);
     return CF_OK;
 }
@@ -601,6 +604,7 @@ static void free_run(cf_run *r)
                        r->logbuf, r->part, r->lsum, r->cflpart, r->h1prev, r->uoffd };
     for (double *b : bufs) if (b) (void) hipFree(b);
     if (r->X) (void) hipFree(r->X);
+    if (r->statres) (void) hipHostFree(r->statres);
     for (auto &pe : r->pending) { (void) hipEventDestroy(pe.second.first); (void) hipEventDestroy(pe.second.second); }
     if (r->stream) (void) hipStreamDestroy(r->stream);
     delete r;
@@ -1231,12 +1235,14 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     bool ok = true;
     ok = ok && falloc(&r->u, r->N) && falloc(&r->v, r->N) && falloc(&r->w, r->N);
     ok = ok && falloc(&r->ru, r->N) && falloc(&r->rv, r->N) && falloc(&r->rw, r->N);
-    for (int f = 0; f < 3; f++) ok = ok && falloc(&r->fa[f], r->N) && falloc(&r->fb[f], r->N);
+    /* a spectrum fits in fb[0], the partial sums of k_stat_spec in stage */
+    const size_t nst = (size_t) 2 * nz * (r->g.nkx + (size_t) 2 * ny * ((r->g.nkx + CF_SPEC_ROWS - 1) / CF_SPEC_ROWS));
+    for (int f = 0; f < 3; f++) ok = ok && falloc(&r->fa[f], r->N) && falloc(&r->fb[f], f ? r->N : 2 * r->M * nz);
     if (cfg->scalar) ok = ok && falloc(&r->c, r->N) && falloc(&r->rc, r->N) && falloc(&r->fa[3], r->N) && falloc(&r->fb[3], r->N);
     if (order == 4) ok = ok && dalloc(&r->S4, 3 * r->M * nz);
     /* G: the order-2 Poisson's chunk checkpoints (3 per chunk of 16 levels) per mode */
     const size_t glev = std::max((size_t) nz, (size_t) 3 * ((nz + 15) / 16));
-    ok = ok && falloc(&r->p, r->N) && dalloc(&r->stage, r->N) && dalloc(&r->G, r->M * glev);
+    ok = ok && falloc(&r->p, r->N) && dalloc(&r->stage, std::max(r->N, nst)) && dalloc(&r->G, r->M * glev);
     ok = ok && hipMalloc((void **) &r->X, 2 * r->esz * r->M * nz) == hipSuccess;
     ok = ok && dalloc(&r->tab, r->tab_n) && dalloc(&r->scal, SC_N) && dalloc(&r->logbuf, (size_t) LOGCAP * CF_LOG_N);
     rhs_chunks(nx, ny, nz, rhs_target({ &r->g }, CF_RHS_KC), &r->rhs_kc, &r->rhs_blocks);
@@ -1248,9 +1254,9 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     }
     r->nb_red = 1024;
     /* part: a batch's plane sums of the solve, the RHS launch's partial sums
-     * (four statistics of u and, with the scalar, c) and the divergence
-     * check's maxima */
-    const size_t npart = std::max({ (size_t) ((r->P + 63) / 64) * nz, (size_t) r->nb_red,
+     * (four statistics of u and, with the scalar, c), the divergence check's
+     * maxima and the plane statistics' partial sums */
+    const size_t npart = std::max({ (size_t) ((r->P + 63) / 64) * nz, (size_t) r->nb_red, (size_t) 3 * CF_STAT_NBL * nz,
                                     (size_t) 4 * std::max({ r->gblocks, r->rhs_blocks, r->r4_blocks }) * (cfg->scalar ? 2 : 1) });
     ok = ok && dalloc(&r->part, npart) && dalloc(&r->lsum, (size_t) nz + 2);
     /* a batch may cut the run's z-chunks otherwise, down to one level */
@@ -1385,6 +1391,13 @@ static size_t fx_lds_n(const cf_run *r, int pairs)
 }
 static size_t fx_lds(const cf_run *r) { return fx_lds_n(r, r->rd.fx_pairs); }
 static size_t dx_lds(const cf_run *r) { return fx_lds_n(r, r->rd.dx_pairs); }
+/* FP64 x FFT without a divergence: the divergence's pair count */
+static unsigned plain_blocks(const cf_run *r)
+{
+    const long npairs = ((long) r->g.ny * r->g.nz + 1) / 2;
+    return (unsigned) ((npairs + r->rd.dx_pairs - 1) / r->rd.dx_pairs);
+}
+static size_t plain_lds(const cf_run *r) { return 2 * sizeof(double) * ((size_t) r->rd.dx_pairs * fft_ld(r->g.nx) + (size_t) r->g.nx); }
 static size_t fy_lds_n(const cf_run *r, int cols)
 {
     return 2 * r->esz * ((size_t) cols * fy_ld(r->g.ny) + (size_t) r->g.ny);
@@ -1576,7 +1589,7 @@ static cf_status enqueue_spectral_solve(cf_run *r, int s, int type, double *fld)
     const long NL = (long) r->g.ny * r->g.nz, npairs = (NL + 1) / 2;
     const unsigned gx = (unsigned) ((npairs + R.fx_pairs - 1) / R.fx_pairs);
     const dim3 gy(fy_blocks(r));
-    KLAUNCH("hsolve", r->kfxp, dim3(gx), dim3(256), fx_lds(r), R, (const double *) fld, X);
+    KLAUNCH("hsolve", r->kfxp, dim3(plain_blocks(r)), dim3(256), plain_lds(r), R, (const double *) fld, X);
     KLAUNCH("hsolve", r->kfy, gy, dim3(256), fy_lds(r), R, X, 1);
     if (r->g.order == 4) {
         if (n >= 6)
@@ -2026,77 +2039,67 @@ extern "C" cf_status cf_run_max_divergence(cf_run *r, double *out)
 
 /* ------------------------------------------------------------ statistics */
 
-/* the device buffer of a field of the current state (storage precision of
- * the run); the fast path's velocity is materialised into the forcing
- * slots first, which are free between steps */
-static cf_status stat_source(cf_run *r, int field, const double **src, bool *mat)
+/* the stored fields fa and fb (or fa alone where fb < 0): the general path's
+ * state, or the fast path's velocity, materialised into the forcing slots,
+ * which are free between steps */
+static cf_status stat_sources(cf_run *r, int fa, int fb, const double **a, const double **b)
 {
-    if (field == CF_P) { *src = r->p; return CF_OK; }
-    if (field == CF_C) {
-        if (!r->c) { cf_set_error("statistics: field c needs a scalar run"); return CF_ERR_ARG; }
-        *src = r->c;
-        return CF_OK;
+    bool need[3] = { false, false, false };
+    for (int q = 0; q < 2; q++) {
+        const int f = q ? fb : fa;
+        const double **src = q ? b : a;
+        if (q && fb < 0) continue;
+        if (f == CF_P) { *src = r->p; continue; }
+        if (f == CF_C) {
+            if (!r->c) { cf_set_error("statistics: field c needs a scalar run"); return CF_ERR_ARG; }
+            *src = r->c;
+            continue;
+        }
+        if (f < CF_U || f > CF_W) { cf_set_error("statistics: bad field %d", f); return CF_ERR_ARG; }
+        if (r->general) { *src = f == CF_U ? r->u : f == CF_V ? r->v : r->w; continue; }
+        need[f] = true;
+        *src = r->fa[f];
     }
-    if (field < CF_U || field > CF_W) { cf_set_error("statistics: bad field %d", field); return CF_ERR_ARG; }
-    if (r->general) {
-        *src = field == CF_U ? r->u : field == CF_V ? r->v : r->w;
-        return CF_OK;
-    }
-    if (!*mat) {
-        cf_status st = enqueue_materialise(r, r->fa[0], r->fa[1], r->fa[2]);
-        if (st != CF_OK) return st;
-        *mat = true;
-    }
-    *src = r->fa[field];
-    return CF_OK;
+    if (!need[0] && !need[1] && !need[2]) return CF_OK;
+    return enqueue_materialise(r, need[0] ? r->fa[0] : nullptr, need[1] ? r->fa[1] : nullptr, need[2] ? r->fa[2] : nullptr);
 }
 
-/* a plane statistic of kind AVG, CORR or MOMENT into dev_out[nz], with
- * part (CF_STAT_NBL nz doubles) and means (2 nz doubles) as device work
- * space; enqueued on the run's stream */
+/* a plane statistic of kind AVG, CORR or MOMENT into res[nz], with part
+ * (3 CF_STAT_NBL nz doubles) as device work space; enqueued on the run's
+ * stream */
 template <typename T>
-static cf_status stat_plane_t(cf_run *r, int kind, const T *a, const T *b, double en, double *part, double *means,
-                              double *dev_out, const double *aoff)
+static cf_status stat_plane_t(cf_run *r, int kind, const T *a, const T *b, double en, double *part, double *res,
+                              const double *aoff)
 {
-    const int nz = r->g.nz, P = (int) r->P, nbl = CF_STAT_NBL;
-    const double scale = 1.0 / ((double) r->g.nx * (double) r->g.ny);
-    const dim3 grid(nbl, nz), fin((nz + 255) / 256);
-    double *ma = means, *mb = means + nz;
-    const double *nul = nullptr;
-    hipLaunchKernelGGL((k_stat_plane<T, 0>), grid, dim3(256), 0, r->stream, a, (const T *) nullptr, nul, nul, 0.0, P,
-                       nbl, part);
+    const int nz = r->g.nz, P = (int) r->P, nbl = stat_nbl(r->P);
+    const double scale = 1.0 / ((double) r->g.nx * (double) r->g.ny), *nul = nullptr;
+    const dim3 grid(nbl, nz), fin((nz + 3) / 4);
+    const bool two = kind == CF_STAT_CORR && a != b;
+    const double *pa = part, *pb = two ? part + (size_t) nbl * nz : part;
+    double *pc = part + (size_t) 2 * nbl * nz;
+    hipLaunchKernelGGL(k_stat_sum<T>, dim3(nbl, nz, two ? 2 : 1), dim3(256), 0, r->stream, a, b, P, nbl, part);
+    if (kind == CF_STAT_CORR)
+        hipLaunchKernelGGL((k_stat_central<T, 1>), grid, dim3(256), 0, r->stream, a, b, pa, pb, scale, 0.0, P, nbl, pc);
+    else if (kind == CF_STAT_MOMENT)
+        hipLaunchKernelGGL((k_stat_central<T, 2>), grid, dim3(256), 0, r->stream, a, b, pa, pb, scale, en, P, nbl, pc);
     /* a stored relative to a profile: the average adds it back; the
      * central statistics need only the deviations */
-    hipLaunchKernelGGL(k_stat_finish, fin, dim3(256), 0, r->stream, (const double *) part, nbl, nz, scale,
-                       kind == CF_STAT_AVG ? dev_out : ma, kind == CF_STAT_AVG ? aoff : nul);
-    if (kind == CF_STAT_CORR) {
-        hipLaunchKernelGGL((k_stat_plane<T, 0>), grid, dim3(256), 0, r->stream, b, (const T *) nullptr, nul, nul, 0.0,
-                           P, nbl, part);
-        hipLaunchKernelGGL(k_stat_finish, fin, dim3(256), 0, r->stream, (const double *) part, nbl, nz, scale, mb, nul);
-        hipLaunchKernelGGL((k_stat_plane<T, 1>), grid, dim3(256), 0, r->stream, a, b, (const double *) ma,
-                           (const double *) mb, 0.0, P, nbl, part);
-        hipLaunchKernelGGL(k_stat_finish, fin, dim3(256), 0, r->stream, (const double *) part, nbl, nz, scale, dev_out, nul);
-    } else if (kind == CF_STAT_MOMENT) {
-        hipLaunchKernelGGL((k_stat_plane<T, 2>), grid, dim3(256), 0, r->stream, a, (const T *) nullptr,
-                           (const double *) ma, nul, en, P, nbl, part);
-        hipLaunchKernelGGL(k_stat_finish, fin, dim3(256), 0, r->stream, (const double *) part, nbl, nz, scale, dev_out, nul);
-    }
+    hipLaunchKernelGGL(k_stat_finish, fin, dim3(256), 0, r->stream, kind == CF_STAT_AVG ? pa : (const double *) pc, nbl, nz,
+                       scale, res, kind == CF_STAT_AVG ? aoff : nul);
     LAUNCHCHK();
     return CF_OK;
 }
 
-static cf_status stat_plane(cf_run *r, int kind, int fa, int fb, double en, double *part, double *means,
-                            double *dev_out)
+static cf_status stat_plane(cf_run *r, int kind, int fa, int fb, double en, double *part, double *res)
 {
-    bool mat = false;
     const double *a = nullptr, *b = nullptr;
-    cf_status st = stat_source(r, fa, &a, &mat);
-    if (st == CF_OK && kind == CF_STAT_CORR) st = stat_source(r, fb, &b, &mat);
+    cf_status st = stat_sources(r, fa, kind == CF_STAT_CORR ? fb : -1, &a, &b);
+    if (st == CF_OK && kind == CF_STAT_CORR && fb < 0) { cf_set_error("statistics: bad field %d", fb); st = CF_ERR_ARG; }
     if (st != CF_OK) return st;
     const double *aoff = fa == CF_U && r->uoffd ? r->uoffd + 1 : nullptr;
     if (r->prec == CF_FP32)
-        return stat_plane_t<float>(r, kind, (const float *) a, (const float *) b, en, part, means, dev_out, aoff);
-    return stat_plane_t<double>(r, kind, a, b, en, part, means, dev_out, aoff);
+        return stat_plane_t<float>(r, kind, (const float *) a, (const float *) b, en, part, res, aoff);
+    return stat_plane_t<double>(r, kind, a, b, en, part, res, aoff);
 }
 
 /* FFT3D_FWD (1/nx, 1/ny scaled) of an FP64 field in the device layout into
@@ -2104,81 +2107,100 @@ static cf_status stat_plane(cf_run *r, int kind, int fa, int fb, double en, doub
 static cf_status stat_fft(cf_run *r, const double *src, double2 *dst)
 {
     const RunDev &R = r->rd;
-    const long NL = (long) r->g.ny * r->g.nz, npairs = (NL + 1) / 2;
-    const unsigned gx = (unsigned) ((npairs + R.fx_pairs - 1) / R.fx_pairs);
-    const size_t lx = 2 * sizeof(double) * ((size_t) R.fx_pairs * fx_ld(r->g.nx, (int) r->esz) + (size_t) r->g.nx);
     const size_t ly = 2 * sizeof(double) * ((size_t) R.fy_cols * fy_ld(r->g.ny) + (size_t) r->g.ny);
-    hipLaunchKernelGGL(r->kfxp, dim3(gx), dim3(256), lx, r->stream, R, src, dst);
+    hipLaunchKernelGGL(r->kfxp, dim3(plain_blocks(r)), dim3(256), plain_lds(r), r->stream, R, src, dst);
     hipLaunchKernelGGL(r->kfy, dim3(fy_blocks(r)), dim3(256), ly, r->stream, R, dst, 1);
     LAUNCHCHK();
     return CF_OK;
+}
+
+/* the run's pinned memory for a statistic's result, which the last kernel
+ * writes: from the run's first statistic until the run's end */
+static cf_status stat_result(cf_run *r)
+{
+    if (r->statres) return CF_OK;
+    const size_t n = (size_t) 2 * r->g.nz * (r->g.nkx + r->g.ny / 2 + 1);
+    if (hipHostMalloc((void **) &r->statres, sizeof(double) * n, hipHostMallocDefault) != hipSuccess) {
+        r->statres = nullptr;
+        cf_set_error("cf_run_xy_stats: host allocation failed");
+        return CF_ERR_NOMEM;
+    }
+    return CF_OK;
+}
+
+/* cross-spectra into the run's result memory, then out.  FP64 runs work in
+ * buffers that hold nothing between steps: the pressure spectrum, a
+ * tendency slot and the staging field; FP32 runs, whose buffers are half
+ * the size, allocate for the call. */
+static cf_status stat_spec(cf_run *r, int fa, int fb, double *out)
+{
+    const int nkx = r->g.nkx, ny = r->g.ny, nz = r->g.nz;
+    const size_t M = r->M * (size_t) nz, nout = (size_t) 2 * nz * (nkx + ny / 2 + 1);
+    const double *src[2] = { nullptr, nullptr };
+    cf_status st = stat_sources(r, fa, fb, &src[0], &src[1]);
+    if (st == CF_OK && fb < 0) { cf_set_error("statistics: bad field %d", fb); st = CF_ERR_ARG; }
+    if (st != CF_OK) return st;
+    double2 *A = r->X, *B = (double2 *) r->fb[0], *Xw = nullptr;
+    double *wide = nullptr;
+    if (r->prec == CF_FP32) {
+        if (hipMalloc((void **) &Xw, sizeof(double2) * 2 * M) != hipSuccess
+            || hipMalloc((void **) &wide, sizeof(double) * r->N) != hipSuccess) {
+            cf_set_error("cf_run_xy_stats: device allocation failed");
+            st = CF_ERR_NOMEM;
+        }
+        A = Xw;
+        B = Xw + M;
+    }
+    if (fa == fb) B = A;
+    for (int q = 0; q < (fa == fb ? 1 : 2) && st == CF_OK; q++) {
+        if (r->prec == CF_FP32) {
+            hipLaunchKernelGGL(k_stat_widen<float>, dim3((unsigned) ((r->N + 255) / 256)), dim3(256), 0, r->stream,
+                               (const float *) src[q], wide, r->N);
+            src[q] = wide;
+        }
+        st = stat_fft(r, src[q], q ? B : A);
+    }
+    if (st == CF_OK) {
+        double2 *sx = (double2 *) r->stage, *part = sx + (size_t) nkx * nz;
+        const unsigned waves = (unsigned) ((nkx + CF_SPEC_ROWS - 1) / CF_SPEC_ROWS) * nz;
+        hipLaunchKernelGGL(k_stat_spec, dim3((waves + 3) / 4), dim3(256), 0, r->stream, (const double2 *) A,
+                           (const double2 *) B, r->g.nx, ny, nkx, nz, sx, part);
+        hipLaunchKernelGGL(k_stat_spec_finish, dim3((unsigned) ((nout / 2 + 255) / 256)), dim3(256), 0, r->stream,
+                           (const double2 *) sx, (const double2 *) part, ny, nkx, nz, (double2 *) r->statres);
+        if (hipGetLastError() != hipSuccess) {
+            cf_set_error("cf_run_xy_stats: spectra failed");
+            st = CF_ERR_DEVICE;
+        }
+    }
+    const hipError_t e = hipStreamSynchronize(r->stream);
+    if (Xw) (void) hipFree(Xw);
+    if (wide) (void) hipFree(wide);
+    if (st == CF_OK) HIPCHK(e);
+    if (st == CF_OK) memcpy(out, r->statres, sizeof(double) * nout);
+    return st;
 }
 
 extern "C" cf_status cf_run_xy_stats(cf_run *r, int kind, int fa, int fb, double en, double *out)
 {
     CHECK_RUN(r);
     if (!out || kind < CF_STAT_AVG || kind > CF_STAT_SPEC) { cf_set_error("cf_run_xy_stats: bad kind or output"); return CF_ERR_ARG; }
-    const int nz = r->g.nz;
-    cf_status st;
-    if (kind != CF_STAT_SPEC) {
-        double *work = nullptr;
-        HIPCHK(hipMalloc((void **) &work, sizeof(double) * ((size_t) CF_STAT_NBL * nz + 3 * (size_t) nz)));
-        st = stat_plane(r, kind, fa, fb, en, work, work + (size_t) CF_STAT_NBL * nz,
-                        work + (size_t) CF_STAT_NBL * nz + 2 * nz);
-        if (st == CF_OK && hipMemcpyAsync(out, work + (size_t) CF_STAT_NBL * nz + 2 * nz, sizeof(double) * nz,
-                                          hipMemcpyDeviceToHost, r->stream) != hipSuccess) {
-            cf_set_error("cf_run_xy_stats: copy failed");
-            st = CF_ERR_DEVICE;
-        }
-        (void) hipStreamSynchronize(r->stream);
-        (void) hipFree(work);
-        return st;
-    }
-    /* spectra: both fields widened to FP64 (FP32 runs), transformed, the
-     * level sums of the cross-spectrum */
-    const int nkx = r->g.nkx, ny = r->g.ny;
-    const size_t M = r->M * (size_t) nz, nsx = (size_t) nkx * nz * 2, nsy = (size_t) (ny / 2 + 1) * nz * 2;
-    double2 *X2 = nullptr;
-    double *spec = nullptr, *wide = nullptr;
-    bool ok = hipMalloc((void **) &X2, sizeof(double2) * 2 * M) == hipSuccess
-           && hipMalloc((void **) &spec, sizeof(double) * (nsx + nsy)) == hipSuccess
-           && hipMalloc((void **) &wide, sizeof(double) * r->N) == hipSuccess;
-    st = ok ? CF_OK : CF_ERR_NOMEM;
-    if (!ok) cf_set_error("cf_run_xy_stats: device allocation failed");
-    bool mat = false;
-    for (int q = 0; q < 2 && st == CF_OK; q++) {
-        const double *src = nullptr;
-        st = stat_source(r, q ? fb : fa, &src, &mat);
-        if (st != CF_OK) break;
-        if (r->prec == CF_FP32) {
-            hipLaunchKernelGGL(k_stat_widen<float>, dim3((unsigned) ((r->N + 255) / 256)), dim3(256), 0, r->stream,
-                               (const float *) src, wide, r->N);
-            src = wide;
-        }
-        st = stat_fft(r, src, X2 + q * M);
-    }
-    if (st == CF_OK) {
-        hipLaunchKernelGGL(k_stat_spec, dim3(nz), dim3(256), 0, r->stream, (const double2 *) X2,
-                           (const double2 *) (X2 + M), r->g.nx, ny, nkx, nz, spec, spec + nsx);
-        if (hipGetLastError() != hipSuccess
-            || hipMemcpyAsync(out, spec, sizeof(double) * (nsx + nsy), hipMemcpyDeviceToHost, r->stream) != hipSuccess) {
-            cf_set_error("cf_run_xy_stats: spectra failed");
-            st = CF_ERR_DEVICE;
-        }
-    }
-    (void) hipStreamSynchronize(r->stream);
-    if (X2) (void) hipFree(X2);
-    if (spec) (void) hipFree(spec);
-    if (wide) (void) hipFree(wide);
-    return st;
+    cf_status st = stat_result(r);
+    if (st != CF_OK) return st;
+    if (kind == CF_STAT_SPEC) return stat_spec(r, fa, fb, out);
+    st = stat_plane(r, kind, fa, fb, en, r->part, r->statres);
+    const hipError_t e = hipStreamSynchronize(r->stream);
+    if (st != CF_OK) return st;
+    HIPCHK(e);
+    memcpy(out, r->statres, sizeof(double) * r->g.nz);
+    return CF_OK;
 }
 
 /* for entry points in other files: a plane statistic of kind AVG, CORR or
- * MOMENT into res[nz] with the caller's work space (part: CF_STAT_NBL nz
- * doubles, means: 2 nz), enqueued on the run's stream; nz, the stream and
- * the device come back for the caller */
-extern "C" cf_status cf_run_stat_plane_into(cf_run *r, int kind, int fa, int fb, double en, double *part,
-                                           double *means, double *res, int *nz, void **stream, int *device)
+ * MOMENT into res[nz] with the caller's work space (part: 3 CF_STAT_NBL nz
+ * doubles), enqueued on the run's stream; nz, the stream and the device
+ * come back for the caller */
+extern "C" cf_status cf_run_stat_plane_into(cf_run *r, int kind, int fa, int fb, double en, double *part, double *res,
+                                           int *nz, void **stream, int *device)
 {
     CHECK_RUN(r);
     if (nz) *nz = r->g.nz;
@@ -2188,7 +2210,7 @@ extern "C" cf_status cf_run_stat_plane_into(cf_run *r, int kind, int fa, int fb,
     /* profiling would create events: off for this call */
     const bool prof = r->profile;
     r->profile = false;
-    const cf_status st = stat_plane(r, kind, fa, fb, en, part, means, res);
+    const cf_status st = stat_plane(r, kind, fa, fb, en, part, res);
     r->profile = prof;
     return st;
 }
@@ -2273,9 +2295,7 @@ extern "C" cf_status cf_op_fft3d_fwd(cf_run *r, const double *in_io, double *spe
                        r->g.nx, r->g.ny, r->g.nz, (const double *) nullptr);
     LAUNCHCHK();
     const RunDev &R = r->rd;
-    long NL = (long) r->g.ny * r->g.nz, npairs = (NL + 1) / 2;
-    unsigned gx = (unsigned) ((npairs + R.fx_pairs - 1) / R.fx_pairs);
-    hipLaunchKernelGGL(r->kfxp, dim3(gx), dim3(256), fx_lds(r), r->stream, R, (const double *) r->fb[0], r->X);
+    hipLaunchKernelGGL(r->kfxp, dim3(plain_blocks(r)), dim3(256), plain_lds(r), r->stream, R, (const double *) r->fb[0], r->X);
     LAUNCHCHK();
     dim3 gy(fy_blocks(r));
     hipLaunchKernelGGL(r->kfy, gy, dim3(256), fy_lds(r), r->stream, R, r->X, 1);
