@@ -126,3 +126,28 @@ def test_statistics_launch_shapes(shape):
             assert np.abs(run.xy_stats("corr", a, b) - (d[0] * d[1]).mean(axis=(0, 1))).max() <= 1e-13
             assert np.abs(run.xy_stats("avg", b) - f[b].mean(axis=(0, 1))).max() <= 1e-13
         assert np.abs(run.xy_stats("moment", "u", en=3.0) - ((f["u"] - f["u"].mean(axis=(0, 1))) ** 3).mean(axis=(0, 1))).max() <= 1e-11
+
+
+# the fully implicit driver's solves of all fields in one launch: an odd
+# number of cells, w's faces in a shorter chunk than the cells, one thread a
+# mode (rounding grows as nz^2), and order 4's solves field by field
+@pytest.mark.parametrize("shape,kw,tol", [((9, 9, 9), dict(), 1e-12), ((15, 9, 7), dict(scalar=1), 1e-12),
+                                          ((16, 6, 33), dict(scalar=1), 1e-12), ((6, 6, 520), dict(), 4e-12),
+                                          ((16, 8, 7), dict(order=4, scalar=1), 1e-12)])
+def test_implicit_solves_together(shape, kw, tol):
+    cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], stretch="tanh", dt=1e-3, nu=1.0 / 500.0,
+                    driver=cf.CF_DRIVER_CHANNEL, **kw)
+    f = cf.initial_fields(cfg, seed=4)
+    names = "uvwc" if cfg.scalar else "uvw"
+    orc = ol.OracleRun(ol.oracle_cfg(cfg, cf.grid_dz(cfg)))
+    for n in names:
+        orc.put(n, f[n])
+    orc.project_ic(1.0)
+    init = {n: orc.get(n) for n in names}
+    orc.steps(4)
+    with cf.Run(cfg) as run:
+        for n in names:
+            run.upload(n, init[n])
+        run.step(4)
+        for n in names:
+            assert rel(run.download(n), orc.get(n)) <= tol, n

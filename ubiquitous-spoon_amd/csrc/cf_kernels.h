@@ -642,6 +642,10 @@ template <typename T> typename KSel<T>::ffty_t pick_ffty(int ny);
 template <typename T> typename KSel<T>::fftxi_t pick_fftx_inv(int nx);
 template <typename T> typename KSel<T>::pois2_t pick_poisson2(int lmax);
 KSel<float>::pois2_t pick_poisson2_islands(int lmax);
+/* levels of a field's part of G: the one-thread-per-mode solve's checkpoints */
+#define CF_P2_GLEV(nz) ((nz) > 3 * (((nz) + 15) / 16) ? (size_t) (nz) : (size_t) 3 * (((nz) + 15) / 16))
+typedef void (*k_hsolve2_t)(const RunDev, const PoisTab, const PoisTab, const PoisTab, int, double2 *, double *, const Book);
+k_hsolve2_t pick_hsolve2(int lmax);
 template <typename T>
 __global__ void k_project2(const RunDev R, const T *us, const T *vs, const T *ws, const double *h1, const double *mptr,
                            const T *p, double dtp, T *u, T *v, T *w);

@@ -1817,9 +1817,10 @@ static __device__ __forceinline__ void pois2s_run(const PoisTab &T_, typename Re
  * FP64 path's registers out of the FP32 kernel. */
 template <typename T, int L, int ISL = 2>
 static __device__ __forceinline__ void pois2_body(const RunDev &R, const PoisTab T_,
-                                                  typename Cplx<T>::type *__restrict__ Y, double *__restrict__ G, const Blk b)
+                                                  typename Cplx<T>::type *__restrict__ Y, double *__restrict__ G, const Blk b,
+                                                  const int nz)
 {
-    const int ny = R.g.ny, nz = R.g.nz, nkx = R.g.nkx;
+    const int ny = R.g.ny, nkx = R.g.nkx;
     const size_t M = (size_t) ny * nkx;
     constexpr bool f64 = sizeof(T) == sizeof(double);
     if (L > 0) {
@@ -1882,7 +1883,40 @@ template <typename T, int L, int ISL>
 __global__ __launch_bounds__(CF_P2S_THREADS) __attribute__((amdgpu_waves_per_eu(CF_P2S_WAVES(L), 8))) void k_poisson2(const RunDev R, const PoisTab T_,
                                                   typename Cplx<T>::type *__restrict__ Y, double *__restrict__ G)
 {
-    pois2_body<T, L, ISL>(R, T_, Y, G, blk_native());
+    pois2_body<T, L, ISL>(R, T_, Y, G, blk_native(), R.g.nz);
+}
+
+/* The z solves of the fully implicit driver's substep, order 2: the Poisson
+ * solve on the Helmholtz tables Hu (u, v), Hw (w: nz - 1 faces) and Hc (the
+ * scalar) over the spectra [field][nz][nkx][ny], nb workgroups a field, and
+ * the substep's bookkeeping in workgroup 0, which no solve waits for.
+ * Small grids are bound by their launches (64 x 65 x 64: 11.9 us in place of
+ * three of 8.9 and the bookkeeping's 5.7). */
+template <int L>
+__global__ __launch_bounds__(CF_P2S_THREADS) __attribute__((amdgpu_waves_per_eu(CF_P2S_WAVES(L), 8))) void k_hsolve2(
+    const RunDev R, const PoisTab Hu, const PoisTab Hw, const PoisTab Hc, const int nb, double2 *__restrict__ X,
+    double *__restrict__ G, const Book B)
+{
+    if (blockIdx.x == 0) { book_body(R, B); return; }
+    const int bx = (int) blockIdx.x - 1, f = bx / nb, nz = R.g.nz;
+    const size_t M = (size_t) R.g.ny * R.g.nkx;
+    PoisTab T_;
+#define SEL_(m) T_.m = f == 2 ? Hw.m : f == 3 ? Hc.m : Hu.m
+    SEL_(a); SEL_(c); SEL_(bz); SEL_(ex); SEL_(ey); SEL_(dvol); SEL_(db_dir); SEL_(db_neu); SEL_(db_top);
+#undef SEL_
+    Blk b = blk_native();
+    b.x = (unsigned) (bx - f * nb);
+    b.nx = (unsigned) nb;
+    pois2_body<double, L, 2>(R, T_, X + (size_t) f * M * nz, G + (size_t) f * M * CF_P2_GLEV(nz), b, f == 2 ? nz - 1 : nz);
+}
+k_hsolve2_t pick_hsolve2(int L)
+{
+    switch (L) {
+#define X_(N) case N: return k_hsolve2<N>;
+    CF_P2S_LSET(X_)
+#undef X_
+    default: return k_hsolve2<0>;
+    }
 }
 
 /* FP64: the one solve; FP32: the storage-precision modes (the islands are
@@ -2093,7 +2127,7 @@ __global__ __launch_bounds__(CF_P2S_THREADS) void kb_poisson(const GArgs<T> *__r
 {
     batch_loop(vs, nrun, [&](int r, unsigned lb) {
         const GArgs<T> &a = a_[r];
-        pois2_body<T, L, ISL>(a.R, a.pt[s], a.X, a.G, blk_of(a, ST_MODE, lb));
+        pois2_body<T, L, ISL>(a.R, a.pt[s], a.X, a.G, blk_of(a, ST_MODE, lb), a.R.g.nz);
     });
 }
 

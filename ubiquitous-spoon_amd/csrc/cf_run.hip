@@ -583,11 +583,14 @@ extern "C" cf_status cf_run_footprint(const cf_config *cfg, size_t *bytes)
     size_t M = (size_t) (cfg->nx / 2 + 1) * cfg->ny * cfg->nz;
     size_t nf = cfg->scalar ? 4 : 3;
     size_t es = cfg->precision == CF_FP32 ? sizeof(float) : sizeof(double);
-    /* state, solve output and two forcing slots per field, p: (4 nf + 1) N values;
-     * X: 2 M values; FP64 stage N, G M, order-4 Poisson factors 3 M */
-    /* a tendency slot holds a spectrum: 2 M - N values more; the partial sums
-     * of the plane statistics: 192 nz */
-    *bytes = es * (4 * nf * N + 4 * M) + sizeof(double) * 192 * cfg->nz + sizeof(double) * (N + (cfg->order == 4 ? 4 : 1) * M)
+    const bool impl = cfg->driver == CF_DRIVER_CHANNEL;
+    /* state and solve output per field, p: (2 nf + 1) N values; X: 2 M; two
+     * forcing slots per field, one of which holds a spectrum (2 M), with the
+     * fully implicit driver each; FP64 stage N, G M (fully implicit, order 2:
+     * per field), order-4 Poisson factors 3 M, partial sums of the plane
+     * statistics 192 nz */
+    *bytes = es * ((2 * nf + 1) * N + 2 * M + (impl ? 4 * nf * M : (2 * nf - 1) * N + 2 * M))
+           + sizeof(double) * (N + (cfg->order == 4 ? 4 : impl ? nf : 1) * M + (size_t) 192 * cfg->nz)
            + ((size_t) 16 << 20);
     return CF_OK;
 }
@@ -598,6 +601,10 @@ static void free_run(cf_run *r)
     for (int q = 0; q < 2; q++) {
         if (r->gexec[q]) (void) hipGraphExecDestroy(r->gexec[q]);
         if (r->graph[q]) (void) hipGraphDestroy(r->graph[q]);
+    }
+    if (r->cfg.driver == CF_DRIVER_CHANNEL) {     /* parts of ru, fa[0], fb[0] */
+        r->rv = r->rw = r->rc = nullptr;
+        for (int f = 1; f < 4; f++) r->fa[f] = r->fb[f] = nullptr;
     }
     double *bufs[] = { r->u, r->v, r->w, r->c, r->ru, r->rv, r->rw, r->rc, r->fa[0], r->fa[1], r->fa[2], r->fa[3],
                        r->fb[0], r->fb[1], r->fb[2], r->fb[3], r->p, r->G, r->S4, r->stage, r->tab, r->scal,
@@ -1234,14 +1241,28 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     auto falloc = [&](double **pp, size_t n) -> bool { return hipMalloc((void **) pp, r->esz * (n ? n : 1)) == hipSuccess; };
     bool ok = true;
     ok = ok && falloc(&r->u, r->N) && falloc(&r->v, r->N) && falloc(&r->w, r->N);
-    ok = ok && falloc(&r->ru, r->N) && falloc(&r->rv, r->N) && falloc(&r->rw, r->N);
+    if (cfg->driver == CF_DRIVER_CHANNEL) {
+        /* one block each of the right-hand sides and of the two sets of
+         * tendency slots (enqueue_spectral_solves): a block of slots holds
+         * the spectra */
+        const size_t nf = cfg->scalar ? 4 : 3;
+        ok = ok && falloc(&r->ru, nf * r->N) && falloc(&r->fa[0], nf * 2 * r->M * nz) && falloc(&r->fb[0], nf * 2 * r->M * nz);
+        double **at[4][3] = { { &r->ru, &r->fa[0], &r->fb[0] }, { &r->rv, &r->fa[1], &r->fb[1] },
+                              { &r->rw, &r->fa[2], &r->fb[2] }, { &r->rc, &r->fa[3], &r->fb[3] } };
+        for (size_t f = 1; ok && f < nf; f++)
+            for (int t = 0; t < 3; t++) *at[f][t] = *at[0][t] + f * r->N;
+        if (cfg->scalar) ok = ok && falloc(&r->c, r->N);
+    } else {
+        ok = ok && falloc(&r->ru, r->N) && falloc(&r->rv, r->N) && falloc(&r->rw, r->N);
+        for (int f = 0; f < 3; f++) ok = ok && falloc(&r->fa[f], r->N) && falloc(&r->fb[f], f ? r->N : 2 * r->M * nz);
+        if (cfg->scalar) ok = ok && falloc(&r->c, r->N) && falloc(&r->rc, r->N) && falloc(&r->fa[3], r->N) && falloc(&r->fb[3], r->N);
+    }
     /* a spectrum fits in fb[0], the partial sums of k_stat_spec in stage */
     const size_t nst = (size_t) 2 * nz * (r->g.nkx + (size_t) 2 * ny * ((r->g.nkx + CF_SPEC_ROWS - 1) / CF_SPEC_ROWS));
-    for (int f = 0; f < 3; f++) ok = ok && falloc(&r->fa[f], r->N) && falloc(&r->fb[f], f ? r->N : 2 * r->M * nz);
-    if (cfg->scalar) ok = ok && falloc(&r->c, r->N) && falloc(&r->rc, r->N) && falloc(&r->fa[3], r->N) && falloc(&r->fb[3], r->N);
     if (order == 4) ok = ok && dalloc(&r->S4, 3 * r->M * nz);
     /* G: the order-2 Poisson's chunk checkpoints (3 per chunk of 16 levels) per mode */
-    const size_t glev = std::max((size_t) nz, (size_t) 3 * ((nz + 15) / 16));
+    size_t glev = CF_P2_GLEV(nz);
+    if (cfg->driver == CF_DRIVER_CHANNEL && order == 2) glev *= cfg->scalar ? 4 : 3;     /* a part per field */
     ok = ok && falloc(&r->p, r->N) && dalloc(&r->stage, std::max(r->N, nst)) && dalloc(&r->G, r->M * glev);
     ok = ok && hipMalloc((void **) &r->X, 2 * r->esz * r->M * nz) == hipSuccess;
     ok = ok && dalloc(&r->tab, r->tab_n) && dalloc(&r->scal, SC_N) && dalloc(&r->logbuf, (size_t) LOGCAP * CF_LOG_N);
@@ -1572,39 +1593,48 @@ static cf_status enqueue_step(cf_run *r, int from)
     return r->prec == CF_FP32 ? enqueue_step_t<float>(r, from) : enqueue_step_t<double>(r, from);
 }
 
-/* The fully implicit update of one field in place (channel2/4, e.g.
- * channel.c:458-467): FFT3D_FWD of its right-hand side h, per (kx, ky) the
- * wall-reduced banded z solve with the modified wavenumbers on the
- * diagonal (solve_helmholtz_u/w, diffuseu.c:460-614, diffusew.c:466-622),
- * FFT3D_BWD.  The x-y passes are the pressure path's; the z solve is the
- * Poisson kernel of the same order on the Helmholtz tables, over nz cells
- * or the nz - 1 interior faces. */
-static cf_status enqueue_spectral_solve(cf_run *r, int s, int type, double *fld)
+/* The fully implicit update of a substep's nf fields (channel2/4, e.g.
+ * channel.c:458-467), in place: FFT3D_FWD of the right-hand sides h, per
+ * (kx, ky) the wall-reduced banded z solve with the modified wavenumbers on
+ * the diagonal (solve_helmholtz_u/w, diffuseu.c:460-614, diffusew.c:466-622),
+ * FFT3D_BWD.  The fields and their spectra are contiguous, so that a launch
+ * of the pressure path's x or y pass covers them as one grid of nf nz levels;
+ * the z solve is the Poisson solve of the same order on the Helmholtz tables,
+ * over nz cells or the nz - 1 interior faces.  X: the tendency slots that the
+ * right-hand side has just read for the last time. */
+static cf_status enqueue_spectral_solves(cf_run *r, int s, int nf, double2 *X, const Book &B)
 {
     const RunDev &R = r->rd;
     RunDev Rn = R;
-    const int n = type == 2 ? r->g.nz - 1 : r->g.nz;
-    Rn.g.nz = n;
-    double2 *X = r->X;
-    const long NL = (long) r->g.ny * r->g.nz, npairs = (NL + 1) / 2;
-    const unsigned gx = (unsigned) ((npairs + R.fx_pairs - 1) / R.fx_pairs);
-    const dim3 gy(fy_blocks(r));
-    KLAUNCH("hsolve", r->kfxp, dim3(plain_blocks(r)), dim3(256), plain_lds(r), R, (const double *) fld, X);
-    KLAUNCH("hsolve", r->kfy, gy, dim3(256), fy_lds(r), R, X, 1);
+    const int nz = r->g.nz;
+    Rn.g.nz = nf * nz;
+    const long npairs = ((long) r->g.ny * Rn.g.nz + 1) / 2;
+    const unsigned gx = (unsigned) ((npairs + R.fx_pairs - 1) / R.fx_pairs), gp = (unsigned) ((npairs + R.dx_pairs - 1) / R.dx_pairs);
+    const dim3 gy((unsigned) (((long) Rn.g.nz * r->g.nkx + R.fy_cols - 1) / R.fy_cols));
+    KLAUNCH("hsolve", r->kfxp, dim3(gp), dim3(256), plain_lds(r), Rn, (const double *) r->ru, X);
+    KLAUNCH("hsolve", r->kfy, gy, dim3(256), fy_lds(r), Rn, X, 1);
     if (r->g.order == 4) {
-        if (n >= 6)
-            KLAUNCH("hsolve", k_poisson4t<double>, dim3((unsigned) ((r->M + 63) / 64)), dim3(128), 0, Rn, r->hs4[s][type],
-                    X, r->S4);
-        else
-            KLAUNCH("hsolve", k_poisson4<double>, dim3((unsigned) ((r->M + CF_P4_THREADS - 1) / CF_P4_THREADS)),
-                    dim3(CF_P4_THREADS), 0, Rn, r->hs4[s][type], X, r->S4);
+        KLAUNCH("mass", k_book, dim3(1), dim3(256), 0, R, B);
+        for (int f = 0; f < nf; f++) {
+            const int type = f == 2 ? 2 : f == 3 ? 1 : 0;
+            Rn.g.nz = f == 2 ? nz - 1 : nz;
+            double2 *Xf = X + (size_t) f * r->M * nz;
+            if (Rn.g.nz >= 6)
+                KLAUNCH("hsolve", k_poisson4t<double>, dim3((unsigned) ((r->M + 63) / 64)), dim3(128), 0, Rn,
+                        r->hs4[s][type], Xf, r->S4);
+            else
+                KLAUNCH("hsolve", k_poisson4<double>, dim3((unsigned) ((r->M + CF_P4_THREADS - 1) / CF_P4_THREADS)),
+                        dim3(CF_P4_THREADS), 0, Rn, r->hs4[s][type], Xf, r->S4);
+        }
+        Rn.g.nz = nf * nz;
     } else {
-        const int L = pois2_L(n);
-        KLAUNCH("hsolve", pick_poisson2<double>(L), dim3(pois2_blocks(L, r->M)), dim3(CF_P2S_THREADS), pois2_lds(L, n),
-                Rn, r->hs2[s][type], X, r->G);
+        const int L = pois2_L(nz);
+        const unsigned nb = pois2_blocks(L, r->M);
+        KLAUNCH("hsolve", pick_hsolve2(L), dim3(1 + nf * nb), dim3(CF_P2S_THREADS), pois2_lds(L, nz), R, r->hs2[s][0],
+                r->hs2[s][2], r->hs2[s][1], (int) nb, X, r->G, B);
     }
-    KLAUNCH("hsolve", r->kfy, gy, dim3(256), fy_lds(r), R, X, 0);
-    KLAUNCH("hsolve", r->kfxi, dim3(gx), dim3(256), fx_lds(r), R, (const double2 *) X, fld);
+    KLAUNCH("hsolve", r->kfy, gy, dim3(256), fy_lds(r), Rn, X, 0);
+    KLAUNCH("hsolve", r->kfxi, dim3(gx), dim3(256), fx_lds(r), Rn, (const double2 *) X, r->ru);
     return CF_OK;
 }
 
@@ -1647,11 +1677,7 @@ static cf_status enqueue_step_general_t(cf_run *r)
         cf_status st = CF_OK;
         if (R.implicit) {
             if constexpr (std::is_same<T, double>::value) {
-                KLAUNCH("mass", k_book, dim3(1), dim3(256), 0, R, B);
-                st = enqueue_spectral_solve(r, s, 0, ru);
-                if (st == CF_OK) st = enqueue_spectral_solve(r, s, 0, rv);
-                if (st == CF_OK && sc) st = enqueue_spectral_solve(r, s, 1, rc);
-                if (st == CF_OK) st = enqueue_spectral_solve(r, s, 2, rw);
+                st = enqueue_spectral_solves(r, s, r->nfield, (double2 *) gold[0], B);
             }
         } else {
             st = enqueue_zsolve<T>(r, "solve", s, (unsigned) r->nfield, ru, rv, rw, rc, B);
