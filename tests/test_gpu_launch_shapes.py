@@ -1,5 +1,7 @@
 """Launch shapes that depend on the grid: each rule at the sizes where its
 choice changes, against the CPU oracle (FP64, <= 1e-12 relative L2)."""
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -151,3 +153,20 @@ def test_implicit_solves_together(shape, kw, tol):
         run.step(4)
         for n in names:
             assert rel(run.download(n), orc.get(n)) <= tol, n
+
+
+# downloads in chunks: one short chunk, a thread's two chunks and a bit, one
+# byte count over several threads; two threads downloading at once
+@pytest.mark.parametrize("shape", [(64, 64, 32), (64, 64, 33), (90, 75, 50), (256, 128, 65)])
+def test_download_chunks(shape):
+    cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], stretch="uniform")
+    rng = np.random.default_rng(6)
+    with cf.Run(cfg) as one, cf.Run(cfg) as two, ThreadPoolExecutor(2) as pool:
+        a = {n: rng.standard_normal(cfg.shape) for n in "uv"}
+        for run in (one, two):
+            for n in a:
+                run.upload(n, a[n])
+        got = list(pool.map(lambda q: [q[0].download(q[1]) for _ in range(3)], [(one, "u"), (two, "v")]))
+    for n, downloads in zip("uv", got):
+        for g in downloads:
+            assert np.array_equal(g, a[n])

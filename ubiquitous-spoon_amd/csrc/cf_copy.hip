@@ -1,0 +1,160 @@
+/*
+ * cf_copy.hip -- device-to-host copies of whole fields into pageable memory.
+ *
+ * What bounds such a copy is the host: the pages of a fresh destination are
+ * faulted in and zeroed by the one thread that stores to them (101 MB into
+ * fresh memory 24.5 ms, 4 GB/s, against 1.8 for the bus), and the stream's
+ * own copy of pageable memory waits for every chunk.  Here several threads
+ * each keep two chunks of a pinned ring in flight and copy them out: 101 MB
+ * in 5.8 ms with 8 threads (6.7 with 6, 8.3 with 4, 11.9 with 2), 7 MB in
+ * 0.3 ms with one (plain 0.4 to 3.3), 2 MB in 0.2 (plain 0.85).
+ */
+#include "chanflow.h"
+#include "cf_internal_host.h"
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <mutex>
+#include <new>
+#include <thread>
+
+#define CP_CHUNK ((size_t) 1 << 20)
+#define CP_THREADS 8
+#define CP_PER_THREAD ((size_t) 4 << 20)      /* bytes that are worth a thread */
+#define CP_MIN ((size_t) 1 << 20)             /* below: a plain copy */
+#define CP_IDLE 2                             /* rings kept for the next copies */
+
+namespace {
+
+/* pinned chunks and their events, two a thread */
+struct Ring {
+    int device = -1;
+    char *buf = nullptr;
+    hipEvent_t ev[2 * CP_THREADS] = {};
+};
+
+std::mutex g_lock;
+Ring *g_idle[CP_IDLE] = {};
+int g_users = 0;                              /* live runs; with the last one the idle rings go */
+
+void ring_free(Ring *g)
+{
+    if (!g) return;
+    for (hipEvent_t e : g->ev) if (e) (void) hipEventDestroy(e);
+    if (g->buf) (void) hipHostFree(g->buf);
+    delete g;
+}
+
+/* a ring of this device (the current one), or null */
+Ring *ring_take(int device)
+{
+    {
+        std::lock_guard<std::mutex> hold(g_lock);
+        for (Ring *&g : g_idle)
+            if (g && g->device == device) {
+                Ring *t = g;
+                g = nullptr;
+                return t;
+            }
+    }
+    Ring *g = new (std::nothrow) Ring();
+    if (!g) return nullptr;
+    g->device = device;
+    bool ok = hipHostMalloc((void **) &g->buf, 2 * CP_THREADS * CP_CHUNK, hipHostMallocDefault) == hipSuccess;
+    if (!ok) g->buf = nullptr;
+    for (hipEvent_t &e : g->ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (ok) return g;
+    (void) hipGetLastError();
+    ring_free(g);
+    return nullptr;
+}
+
+void ring_give(Ring *g)
+{
+    {
+        std::lock_guard<std::mutex> hold(g_lock);
+        if (g_users > 0)
+            for (Ring *&i : g_idle)
+                if (!i) { i = g; return; }
+    }
+    ring_free(g);
+}
+
+} // namespace
+
+extern "C" void cf_copy_users(int add)
+{
+    Ring *drop[CP_IDLE] = {};
+    {
+        std::lock_guard<std::mutex> hold(g_lock);
+        g_users += add;
+        if (g_users == 0) std::swap(drop, g_idle);
+    }
+    for (Ring *g : drop) ring_free(g);
+}
+
+extern "C" cf_status cf_copy_to_host(void *host, const void *dev, size_t bytes, int device, void *stream)
+{
+    const hipStream_t s = (hipStream_t) stream;
+    Ring *g = nullptr;
+    if (bytes >= CP_MIN) {
+        /* a destination that the runtime knows (pinned, device) is copied to
+         * directly */
+        hipPointerAttribute_t at;
+        const hipError_t e = hipPointerGetAttributes(&at, host);
+        if (e != hipSuccess) (void) hipGetLastError();
+        if (e != hipSuccess || at.type == hipMemoryTypeUnregistered) g = ring_take(device);
+    }
+    if (!g) {
+        hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e == hipSuccess) return CF_OK;
+        cf_set_error("copy to the host: %s", hipGetErrorString(e));
+        return CF_ERR_DEVICE;
+    }
+    /* what the stream still has to do is waited for once, not by every thread */
+    hipError_t first = hipStreamSynchronize(s);
+    const size_t n = (bytes + CP_CHUNK - 1) / CP_CHUNK;
+    std::atomic<size_t> next{ 0 };
+    std::atomic<int> err{ (int) first };
+    auto work = [&](int w) {
+        char *slot[2] = { g->buf + 2 * w * CP_CHUNK, g->buf + (2 * w + 1) * CP_CHUNK };
+        auto len = [&](size_t c) { return std::min(CP_CHUNK, bytes - c * CP_CHUNK); };
+        auto issue = [&](size_t c, int q) {
+            hipError_t e = hipMemcpyAsync(slot[q], (const char *) dev + c * CP_CHUNK, len(c), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipEventRecord(g->ev[2 * w + q], s);
+            if (e != hipSuccess) err = (int) e;
+        };
+        if (w > 0) (void) hipSetDevice(device);
+        size_t c = next++;
+        if (c < n && !err) issue(c, 0);
+        for (int q = 0; c < n && !err; q ^= 1) {
+            const size_t c1 = next++;
+            if (c1 < n) issue(c1, q ^ 1);
+            const hipError_t e = hipEventSynchronize(g->ev[2 * w + q]);
+            if (e != hipSuccess) { err = (int) e; break; }
+            memcpy((char *) host + c * CP_CHUNK, slot[q], len(c));
+            c = c1;
+        }
+    };
+    /* a thread that does not start leaves its chunks to the others */
+    std::thread th[CP_THREADS];
+    const int nt = (int) std::min<size_t>(CP_THREADS, std::max<size_t>(1, bytes / CP_PER_THREAD));
+    for (int w = 1; w < nt; w++) {
+        try { th[w] = std::thread(work, w); } catch (...) { break; }
+    }
+    work(0);
+    for (std::thread &t : th) if (t.joinable()) t.join();
+    if (err) {
+        /* copies of other threads may still be on their way into the ring */
+        (void) hipStreamSynchronize(s);
+        ring_free(g);
+        cf_set_error("copy to the host: %s", hipGetErrorString((hipError_t) err.load()));
+        return CF_ERR_DEVICE;
+    }
+    ring_give(g);
+    return CF_OK;
+}

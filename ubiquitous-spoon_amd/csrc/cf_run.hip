@@ -615,6 +615,7 @@ static void free_run(cf_run *r)
     for (auto &pe : r->pending) { (void) hipEventDestroy(pe.second.first); (void) hipEventDestroy(pe.second.second); }
     if (r->stream) (void) hipStreamDestroy(r->stream);
     delete r;
+    cf_copy_users(-1);
 }
 
 /* ------------------------------------------------------------ create */
@@ -1196,6 +1197,7 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     HIPCHK(hipSetDevice(cfg->device));
 
     cf_run *r = new cf_run();
+    cf_copy_users(1);
     r->cfg = *cfg;
     r->cfg.dz_user = nullptr;
     const int nx = cfg->nx, ny = cfg->ny, nz = cfg->nz;
@@ -1791,9 +1793,7 @@ static cf_status download_dev(cf_run *r, const double *src, double *host, const 
         hipLaunchKernelGGL(k_dev_to_io<double>, grid, dim3(256), 0, r->stream, src, r->stage, r->g.nx, r->g.ny, r->g.nz,
                            off);
     LAUNCHCHK();
-    HIPCHK(hipMemcpyAsync(host, r->stage, sizeof(double) * r->N, hipMemcpyDeviceToHost, r->stream));
-    HIPCHK(hipStreamSynchronize(r->stream));
-    return CF_OK;
+    return cf_copy_to_host(host, r->stage, sizeof(double) * r->N, r->cfg.device, (void *) r->stream);
 }
 
 extern "C" cf_status cf_run_download(cf_run *r, int field, double *host)

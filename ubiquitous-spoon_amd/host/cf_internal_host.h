@@ -18,6 +18,13 @@ struct cf_run;
 cf_status cf_run_stat_plane_into(struct cf_run *r, int kind, int fa, int fb, double en, double *part,
                                  double *res, int *nz, void **stream, int *device);
 
+/* a device buffer to host memory after what the stream holds, complete on
+ * return; device is current */
+cf_status cf_copy_to_host(void *host, const void *dev, size_t bytes, int device, void *stream);
+
+/* a run is made (+1) or gone (-1): what the copies keep goes with the last */
+void cf_copy_users(int add);
+
 #ifdef __cplusplus
 }
 #endif
