@@ -170,3 +170,18 @@ def test_download_chunks(shape):
     for n, downloads in zip("uv", got):
         for g in downloads:
             assert np.array_equal(g, a[n])
+
+
+# the Poisson solve's chunk lengths, with a short group of modes and a short
+# last chunk; the projection leaves what rounding times the condition leaves
+@pytest.mark.parametrize("prec,tol,per_nz2", [(cf.CF_FP64, 1e-11, 1e-15), (cf.CF_FP32, 2e-3, 1e-6)])
+@pytest.mark.parametrize("nz", [3, 17, 47, 100, 176, 193, 230, 257, 300, 400, 512, 513])
+def test_poisson_chunk_lengths(nz, prec, tol, per_nz2):
+    cfg = cf.Config(nx=12, ny=6, nz=nz, stretch="uniform", precision=prec)
+    f = cf.initial_fields(cfg, seed=2)
+    with cf.Run(cfg) as run:
+        for n in "uvw":
+            run.upload(n, f[n])
+        before = run.max_divergence()
+        run.project(1.0)
+        assert run.max_divergence() <= (tol + per_nz2 * nz * nz) * before

@@ -303,13 +303,13 @@ static inline bool fft_compiled(int n)
 #define CF_P2S_NC 16
 #endif
 #ifndef CF_P2S_MW
-#define CF_P2S_MW 8
+#define CF_P2S_MW 16
 #endif
 #ifndef CF_P2S_XCD
 #define CF_P2S_XCD 1
 #endif
 /* order-2 Poisson: the partitioned solve (at most 16 z-chunks of L rows
- * per mode, 8 modes per 256-thread workgroup), L a compiled chunk length
+ * per mode, 16 modes per 256-thread workgroup), L a compiled chunk length
  * >= nz / 16, covers nz <= 512; beyond that one thread per mode (256
  * modes per workgroup). */
 #define CF_P2S_LSET(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) \
@@ -325,11 +325,9 @@ static inline int pois2_L_of(int need)
 static inline int pois2_L(int nz) { return pois2_L_of((nz + CF_P2S_NC - 1) / CF_P2S_NC); }
 /* dynamic LDS of the partitioned solve: its six z tables */
 static inline size_t pois2_lds(int L, int nz) { return L > 0 ? 6 * sizeof(double) * (size_t) nz : 0; }
-/* workgroup shape: CF_P2S_NC z-chunks x CF_P2S_MW modes x 2 parts; a
- * z-level of the group is 2 CF_P2S_MW contiguous reals (128 B in FP64;
- * 16 modes per workgroup measured slower at 256x193x256) */
-#define CF_P2S_GW (2 * CF_P2S_MW)
-#define CF_P2S_THREADS (CF_P2S_NC * CF_P2S_GW)
+/* workgroup shape: CF_P2S_NC z-chunks x CF_P2S_MW modes; a z-level of the
+ * group is CF_P2S_MW contiguous complex values (256 B in FP64) */
+#define CF_P2S_THREADS (CF_P2S_NC * CF_P2S_MW)
 /* modes per workgroup: CF_P2S_MW partitioned, or one per thread (L = 0) */
 static inline size_t pois2_modes_per_block(int L) { return L > 0 ? CF_P2S_MW : CF_P2S_THREADS; }
 static inline unsigned pois2_blocks(int L, size_t M)

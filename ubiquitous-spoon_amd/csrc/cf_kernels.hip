@@ -1642,9 +1642,8 @@ static __device__ __forceinline__ void pois2_mode(const PoisTab &T, C *__restric
 }
 
 /* Partitioned form of the same solve, for nz <= 16 * 32.  A workgroup of
- * CF_P2S_THREADS threads owns CF_P2S_MW modes; thread t takes part t & 1
- * (real or imaginary: both parts share the matrix), mode (t >> 1) mod
- * CF_P2S_MW of the group and z-chunk t / (2 CF_P2S_MW) of L rows (L a
+ * CF_P2S_THREADS threads owns CF_P2S_MW modes; thread t takes mode t mod
+ * CF_P2S_MW of the group and z-chunk t / CF_P2S_MW of L rows (L a
  * compile-time choice >= nz / 16).  Rows
  * above nz are identity rows (x = 0), so every chunk has L - 1 interior
  * rows and a separator (its last row).  Each thread holds its chunk in
@@ -1656,67 +1655,77 @@ static __device__ __forceinline__ void pois2_mode(const PoisTab &T, C *__restric
  * per complex FP64 value), and the 16-fold parallelism over z hides the
  * latency of the level recurrences, which bounds the one-thread-per-mode
  * sweep at these mode counts.  Differs from sequential Thomas by
- * round-off. */
-/* occupancy target by chunk length: the largest without register spills */
+ * round-off.
+ *
+ * The matrix's recurrences and their divisions bound it beside the traffic,
+ * so a thread solves the real and the imaginary part together (a thread per
+ * part had every division twice), and an FP32 solve holds tables and
+ * separators in FP32 LDS, which converts each table value once a workgroup
+ * and not once a use.  256 x 193 x 256: FP64 57 -> 48 us (202 MB: 4.2 TB/s),
+ * FP32 45 -> 34.  Modes per workgroup there: 8 51 and 36 us, 16 48 and 34. */
+/* occupancy target by chunk length: the largest without register spills, or
+ * with a few (20 B at most) */
 #ifndef CF_P2S_WAVES
-#define CF_P2S_WAVES(L) ((L) == 0 ? 2 : ((L) <= 13 ? 4 : ((L) <= 20 ? 3 : 1)))
+#define CF_P2S_WAVES(L, F32) \
+    ((L) == 0 ? 2 : (F32) && (L) <= 13 ? 5 : (L) <= ((F32) ? 16 : 10) ? 4 : (L) > 24 ? 1 : (L) <= 13 || (L) == 16 ? 3 : 2)
 #endif
 
 template <int L, typename A, typename T>
-static __device__ __forceinline__ void pois2s_run(const PoisTab &T_, typename Real<typename Cplx<T>::type>::type *__restrict__ yr,
+static __device__ __forceinline__ void pois2s_run(const PoisTab &T_, typename Cplx<T>::type *__restrict__ Y,
                                                   size_t M, int nz, int nch, size_t idx, bool act,
-                                                  double lxd, double lyd, bool zero, double (*sh)[CF_P2S_NC][CF_P2S_GW],
-                                                  double (*xs)[CF_P2S_GW], double *tl)
+                                                  double lxd, double lyd, bool zero, A (*sh)[CF_P2S_NC][CF_P2S_MW],
+                                                  A (*xs)[CF_P2S_NC][CF_P2S_MW], A *tl)
 {
-    typedef typename Real<typename Cplx<T>::type>::type S;
-    const int g = threadIdx.x & (CF_P2S_GW - 1), chunk = threadIdx.x / CF_P2S_GW;
+    typedef typename Cplx<T>::type C;
+    typedef cv<C> S;
+    const int g = threadIdx.x & (CF_P2S_MW - 1), chunk = threadIdx.x / CF_P2S_MW;
     const A lx = (A) lxd, ly = (A) lyd;
     const bool live = chunk < nch;
     const int lo = chunk * L;
     const bool ld = live && act;
-    const size_t stride = 2 * M;
-    const gp<S> col = (gp<S>) yr + idx;
+    const gp<S> col = (gp<S>) Y + idx;
     const int ktop = nz - 1;
     /* the column's rows (clamped, valid reads), then the z tables into LDS
      * (tl: a, c, bz, ex, ey, dvol, nz each) with the same round trip */
-    S raw[L];
+    C raw[L];
 #pragma unroll
-    for (int t = 0; t < L; t++) raw[t] = col[(size_t) min(lo + t, ktop) * stride];
+    for (int t = 0; t < L; t++) raw[t] = cx_of<C>(col[(size_t) min(lo + t, ktop) * M]);
     {
         const cp<double> src[6] = { (cp<double>) T_.a, (cp<double>) T_.c, (cp<double>) T_.bz,
                                     (cp<double>) T_.ex, (cp<double>) T_.ey, (cp<double>) T_.dvol };
 #pragma unroll
         for (int w = 0; w < 6; w++)
-            for (int k = (int) threadIdx.x; k < nz; k += (int) blockDim.x) tl[w * nz + k] = src[w][k];
+            for (int k = (int) threadIdx.x; k < nz; k += (int) blockDim.x) tl[w * nz + k] = (A) src[w][k];
     }
     __syncthreads();
-    const double *ta = tl, *tc = tl + nz, *tbz = tl + 2 * nz, *tex = tl + 3 * nz, *tey = tl + 4 * nz,
+    const A *ta = tl, *tc = tl + nz, *tbz = tl + 2 * nz, *tex = tl + 3 * nz, *tey = tl + 4 * nz,
                  *tdv = tl + 5 * nz;
     /* row coefficients, identity beyond the top wall; every read is at a
      * clamped (valid) level and the padding is applied by selects */
     const A dbot = (A) (zero ? T_.db_dir : T_.db_neu), dtop = (A) T_.db_top;
     auto cb = [&](int k) {
         const int kc = min(k, ktop);
-        A b = (A) tbz[kc] - lx * (A) tex[kc] - ly * (A) tey[kc];
+        A b = tbz[kc] - lx * tex[kc] - ly * tey[kc];
         b -= k == 0 ? dbot : (A) 0;
         b -= k == ktop ? dtop : (A) 0;
         return k > ktop ? (A) 1 : b;
     };
-    auto ca = [&](int k) { const A v = (A) ta[min(k, ktop)]; return (k > 0 && k <= ktop) ? v : (A) 0; };
-    auto cc = [&](int k) { const A v = (A) tc[min(k, ktop)]; return k < ktop ? v : (A) 0; };
-    A d[L - 1], ph[L - 1], gm[L - 1];
-    A ds = 0;
+    auto ca = [&](int k) { const A v = ta[min(k, ktop)]; return (k > 0 && k <= ktop) ? v : (A) 0; };
+    auto cc = [&](int k) { const A v = tc[min(k, ktop)]; return k < ktop ? v : (A) 0; };
+    A d[L - 1], e[L - 1], ph[L - 1], gm[L - 1];       /* d, e: the real and imaginary part */
+    A ds = 0, es = 0;
 #pragma unroll
     for (int t = 0; t < L; t++) {
         const int k = lo + t;
-        const A v = (A) raw[t] * (A) tdv[min(k, ktop)];
-        const A r = (ld && k <= ktop) ? v : (A) 0;
-        if (t < L - 1) d[t] = r;
-        else ds = r;
+        const A dv = tdv[min(k, ktop)], v = (A) raw[t].x * dv, w = (A) raw[t].y * dv;
+        const bool in = ld && k <= ktop;
+        const A r = in ? v : (A) 0, q = in ? w : (A) 0;
+        if (t < L - 1) { d[t] = r; e[t] = q; }
+        else { ds = r; es = q; }
     }
     /* forward sweep of the interior; the separator below enters through
      * a_lo, carried as ph */
-    A ibet = 0, dp = 0, pp = 0;
+    A ibet = 0, dp = 0, ep = 0, pp = 0;
 #pragma unroll
     for (int t = 0; t < L - 1; t++) {
         const int k = lo + t;
@@ -1726,28 +1735,29 @@ static __device__ __forceinline__ void pois2s_run(const PoisTab &T_, typename Re
             b -= ca(k) * gam;
         }
         ibet = (A) 1 / b;
-        if (t == 0) { dp = d[t] * ibet; pp = -ca(k) * ibet; }
-        else { dp = (d[t] - ca(k) * dp) * ibet; pp = -ca(k) * pp * ibet; }
-        d[t] = dp; ph[t] = pp; gm[t] = gam;
+        if (t == 0) { dp = d[t] * ibet; ep = e[t] * ibet; pp = -ca(k) * ibet; }
+        else { dp = (d[t] - ca(k) * dp) * ibet; ep = (e[t] - ca(k) * ep) * ibet; pp = -ca(k) * pp * ibet; }
+        d[t] = dp; e[t] = ep; ph[t] = pp; gm[t] = gam;
     }
     /* back substitution of the particular (y), below (P) and above (Q)
      * responses, in place: d <- y, ph <- P, gm <- Q */
-    A yv = d[L - 2], pv = ph[L - 2], qv = -cc(lo + L - 2) * ibet;
-    const A yl = yv, pl = pv, ql = qv;
+    A yv = d[L - 2], zv = e[L - 2], pv = ph[L - 2], qv = -cc(lo + L - 2) * ibet;
+    const A yl = yv, zl = zv, pl = pv, ql = qv;
     A gnext = gm[L - 2];
     gm[L - 2] = qv;
 #pragma unroll
     for (int t = L - 3; t >= 0; t--) {
         yv = d[t] - gnext * yv;
+        zv = e[t] - gnext * zv;
         pv = ph[t] - gnext * pv;
         qv = -gnext * qv;
         gnext = gm[t];
-        d[t] = yv; ph[t] = pv; gm[t] = qv;
+        d[t] = yv; e[t] = zv; ph[t] = pv; gm[t] = qv;
     }
     if (live) {
-        sh[0][chunk][g] = (double) yv; sh[1][chunk][g] = (double) pv; sh[2][chunk][g] = (double) qv;
-        sh[3][chunk][g] = (double) yl; sh[4][chunk][g] = (double) pl; sh[5][chunk][g] = (double) ql;
-        sh[6][chunk][g] = (double) ds;
+        sh[0][chunk][g] = yv; sh[1][chunk][g] = pv; sh[2][chunk][g] = qv;
+        sh[3][chunk][g] = yl; sh[4][chunk][g] = pl; sh[5][chunk][g] = ql;
+        sh[6][chunk][g] = zv; sh[7][chunk][g] = zl;
     }
     __syncthreads();
     /* separator s_j = (j + 1) L - 1 above chunk j:
@@ -1755,57 +1765,64 @@ static __device__ __forceinline__ void pois2s_run(const PoisTab &T_, typename Re
      * interior row and x_{s+1} chunk j + 1's bottom one, which gives the
      * tridiagonal system sub_j X_{j-1} + dia_j X_j + sup_j X_{j+1} = rhs_j
      * over the separators; each chunk's lanes form their separator's row */
-    A sub = 0, dia = 1, sup = 0, rhs = 0;
+    A sub = 0, dia = 1, sup = 0, rhs = 0, rhi = 0;
     if (live) {
         const int j = chunk, sj = (j + 1) * L - 1;
         const bool nxt = j < nch - 1;
         const A as = ca(sj), cs = cc(sj);
-        sub = j > 0 ? as * (A) sh[4][j][g] : (A) 0;
-        dia = cb(sj) + as * (A) sh[5][j][g] + (nxt ? cs * (A) sh[1][j + 1][g] : (A) 0);
-        sup = nxt ? cs * (A) sh[2][j + 1][g] : (A) 0;
-        rhs = (A) sh[6][j][g] - as * (A) sh[3][j][g] - (nxt ? cs * (A) sh[0][j + 1][g] : (A) 0);
+        sub = j > 0 ? as * sh[4][j][g] : (A) 0;
+        dia = cb(sj) + as * sh[5][j][g] + (nxt ? cs * sh[1][j + 1][g] : (A) 0);
+        sup = nxt ? cs * sh[2][j + 1][g] : (A) 0;
+        rhs = ds - as * sh[3][j][g] - (nxt ? cs * sh[0][j + 1][g] : (A) 0);
+        rhi = es - as * sh[7][j][g] - (nxt ? cs * sh[6][j + 1][g] : (A) 0);
     }
     /* parallel cyclic reduction over the chunks (log2 nch steps, every
      * chunk's lanes at once): row j takes rows j - d and j + d out of its
-     * equation; sh[0..3] hold the rows of the current step */
+     * equation; sh[0..4] hold the rows of the current step */
     for (int d = 1; d < nch; d *= 2) {
         __syncthreads();
         if (live) {
-            sh[0][chunk][g] = (double) sub; sh[1][chunk][g] = (double) dia;
-            sh[2][chunk][g] = (double) sup; sh[3][chunk][g] = (double) rhs;
+            sh[0][chunk][g] = sub; sh[1][chunk][g] = dia;
+            sh[2][chunk][g] = sup; sh[3][chunk][g] = rhs;
+            sh[4][chunk][g] = rhi;
         }
         __syncthreads();
         if (live) {
-            A nsub = 0, nsup = 0, ndia = dia, nrhs = rhs;
+            A nsub = 0, nsup = 0, ndia = dia, nrhs = rhs, nrhi = rhi;
             if (chunk - d >= 0) {
-                const A al = -sub / (A) sh[1][chunk - d][g];
-                nsub = al * (A) sh[0][chunk - d][g];
-                ndia += al * (A) sh[2][chunk - d][g];
-                nrhs += al * (A) sh[3][chunk - d][g];
+                const A al = -sub / sh[1][chunk - d][g];
+                nsub = al * sh[0][chunk - d][g];
+                ndia += al * sh[2][chunk - d][g];
+                nrhs += al * sh[3][chunk - d][g];
+                nrhi += al * sh[4][chunk - d][g];
             }
             if (chunk + d < nch) {
-                const A ga = -sup / (A) sh[1][chunk + d][g];
-                nsup = ga * (A) sh[2][chunk + d][g];
-                ndia += ga * (A) sh[0][chunk + d][g];
-                nrhs += ga * (A) sh[3][chunk + d][g];
+                const A ga = -sup / sh[1][chunk + d][g];
+                nsup = ga * sh[2][chunk + d][g];
+                ndia += ga * sh[0][chunk + d][g];
+                nrhs += ga * sh[3][chunk + d][g];
+                nrhi += ga * sh[4][chunk + d][g];
             }
-            sub = nsub; sup = nsup; dia = ndia; rhs = nrhs;
+            sub = nsub; sup = nsup; dia = ndia; rhs = nrhs; rhi = nrhi;
         }
     }
-    if (live) xs[chunk][g] = (double) (rhs / dia);
+    if (live) { xs[0][chunk][g] = rhs / dia; xs[1][chunk][g] = rhi / dia; }
     __syncthreads();
     if (!ld) return;
-    const A XB = chunk > 0 ? (A) xs[chunk - 1][g] : (A) 0;
-    const A XA = (A) xs[chunk][g];
-    const gp<S> out = col + (size_t) lo * stride;
+    const A XB = chunk > 0 ? xs[0][chunk - 1][g] : (A) 0, ZB = chunk > 0 ? xs[1][chunk - 1][g] : (A) 0;
+    const A XA = xs[0][chunk][g], ZA = xs[1][chunk][g];
+    const gp<S> out = col + (size_t) lo * M;
+    auto put = [&](int t) {
+        out[(size_t) t * M] = cv_of(mkc<C>((T) (d[t] + ph[t] * XB + gm[t] * XA), (T) (e[t] + ph[t] * ZB + gm[t] * ZA)));
+    };
     if (lo + L - 1 <= ktop) {                     /* a full chunk */
 #pragma unroll
-        for (int t = 0; t < L - 1; t++) out[(size_t) t * stride] = (S) (d[t] + ph[t] * XB + gm[t] * XA);
-        out[(size_t) (L - 1) * stride] = (S) XA;
+        for (int t = 0; t < L - 1; t++) put(t);
+        out[(size_t) (L - 1) * M] = cv_of(mkc<C>((T) XA, (T) ZA));
     } else {
 #pragma unroll
         for (int t = 0; t < L - 1; t++)
-            if (lo + t <= ktop) out[(size_t) t * stride] = (S) (d[t] + ph[t] * XB + gm[t] * XA);
+            if (lo + t <= ktop) put(t);
     }
 }
 
@@ -1824,16 +1841,18 @@ static __device__ __forceinline__ void pois2_body(const RunDev &R, const PoisTab
     const size_t M = (size_t) ny * nkx;
     constexpr bool f64 = sizeof(T) == sizeof(double);
     if (L > 0) {
-        __shared__ double sh[7][CF_P2S_NC][CF_P2S_GW];
-        __shared__ double xs[CF_P2S_NC][CF_P2S_GW];
+        /* LDS in the arithmetic of the solve: FP64 unless all of the
+         * launch's solves are FP32 */
+        typedef typename std::conditional<f64 || ISL != 0, double, T>::type S;
+        __shared__ S shb[10][CF_P2S_NC][CF_P2S_MW];
         const int nch = (nz + L - 1) / (L > 0 ? L : 1);
-        /* FP32 rows are half a cache line per workgroup: with CF_P2S_XCD the
-         * workgroups holding neighbouring modes share an XCD (and its L2;
-         * FP32 step 1.267 -> 1.243 ms at 256x193x256); the island launch
-         * covers only the leading workgroups and keeps the plain order */
+        /* with CF_P2S_XCD the workgroups holding neighbouring modes share an
+         * XCD (and its L2: an FP32 level of the group is one cache line, at
+         * any alignment of ny); the island launch covers only the leading
+         * workgroups and keeps the plain order */
         const unsigned bx = (CF_P2S_XCD && ISL != 1) ? xcd_block(b.x, b.nx) : b.x;
         const size_t m0 = (size_t) bx * CF_P2S_MW;
-        const size_t mode = m0 + ((threadIdx.x >> 1) & (CF_P2S_MW - 1));
+        const size_t mode = m0 + (threadIdx.x & (CF_P2S_MW - 1));
         const bool act = mode < M;
         const size_t mc = act ? mode : M - 1;
         const int kx = (int) (mc / ny), ky = (int) (mc % ny);
@@ -1849,22 +1868,22 @@ static __device__ __forceinline__ void pois2_body(const RunDev &R, const PoisTab
             }
         }
         if (!f64 && ((ISL == 0 && low) || (ISL == 1 && !low))) return;   /* workgroup-uniform */
-        typename Real<typename Cplx<T>::type>::type *yr = (typename Real<typename Cplx<T>::type>::type *) Y;
         extern __shared__ __align__(16) unsigned char smem_[];
-        double *tl = (double *) smem_;            /* 6 nz doubles (pois2_lds) */
-        const size_t idx = 2 * mc + (threadIdx.x & 1);
+        /* sh: 8 planes, xs: 2; z tables: 6 nz values (pois2_lds) */
+#define LDS_(A_) (A_(*)[CF_P2S_NC][CF_P2S_MW]) shb, (A_(*)[CF_P2S_NC][CF_P2S_MW]) shb + 8, (A_ *) smem_
         const double lx = ((cp<double>) R.lamx)[kx], ly = ((cp<double>) R.lamy)[ky];
         constexpr int LL = L > 1 ? L : 2;
         if constexpr (f64 || ISL == 1) {
-            pois2s_run<LL, double, T>(T_, yr, M, nz, nch, idx, act, lx, ly, zero, sh, xs, tl);
+            pois2s_run<LL, double, T>(T_, Y, M, nz, nch, mc, act, lx, ly, zero, LDS_(double));
         } else if constexpr (ISL == 0) {
-            pois2s_run<LL, T, T>(T_, yr, M, nz, nch, idx, act, lx, ly, zero, sh, xs, tl);
+            pois2s_run<LL, T, T>(T_, Y, M, nz, nch, mc, act, lx, ly, zero, LDS_(T));
         } else {
             if (low)
-                pois2s_run<LL, double, T>(T_, yr, M, nz, nch, idx, act, lx, ly, zero, sh, xs, tl);
+                pois2s_run<LL, double, T>(T_, Y, M, nz, nch, mc, act, lx, ly, zero, LDS_(double));
             else
-                pois2s_run<LL, T, T>(T_, yr, M, nz, nch, idx, act, lx, ly, zero, sh, xs, tl);
+                pois2s_run<LL, T, T>(T_, Y, M, nz, nch, mc, act, lx, ly, zero, LDS_(T));
         }
+#undef LDS_
         return;
     }
     const size_t qm = (size_t) b.x * blockDim.x + threadIdx.x;
@@ -1880,7 +1899,7 @@ static __device__ __forceinline__ void pois2_body(const RunDev &R, const PoisTab
 }
 
 template <typename T, int L, int ISL>
-__global__ __launch_bounds__(CF_P2S_THREADS) __attribute__((amdgpu_waves_per_eu(CF_P2S_WAVES(L), 8))) void k_poisson2(const RunDev R, const PoisTab T_,
+__global__ __launch_bounds__(CF_P2S_THREADS) __attribute__((amdgpu_waves_per_eu(CF_P2S_WAVES(L, sizeof(T) == 4 && ISL == 0), 8))) void k_poisson2(const RunDev R, const PoisTab T_,
                                                   typename Cplx<T>::type *__restrict__ Y, double *__restrict__ G)
 {
     pois2_body<T, L, ISL>(R, T_, Y, G, blk_native(), R.g.nz);
@@ -1890,10 +1909,10 @@ __global__ __launch_bounds__(CF_P2S_THREADS) __attribute__((amdgpu_waves_per_eu(
  * solve on the Helmholtz tables Hu (u, v), Hw (w: nz - 1 faces) and Hc (the
  * scalar) over the spectra [field][nz][nkx][ny], nb workgroups a field, and
  * the substep's bookkeeping in workgroup 0, which no solve waits for.
- * Small grids are bound by their launches (64 x 65 x 64: 11.9 us in place of
+ * Small grids are bound by their launches (64 x 65 x 64: 10.5 us in place of
  * three of 8.9 and the bookkeeping's 5.7). */
 template <int L>
-__global__ __launch_bounds__(CF_P2S_THREADS) __attribute__((amdgpu_waves_per_eu(CF_P2S_WAVES(L), 8))) void k_hsolve2(
+__global__ __launch_bounds__(CF_P2S_THREADS) __attribute__((amdgpu_waves_per_eu(CF_P2S_WAVES(L, 0), 8))) void k_hsolve2(
     const RunDev R, const PoisTab Hu, const PoisTab Hw, const PoisTab Hc, const int nb, double2 *__restrict__ X,
     double *__restrict__ G, const Book B)
 {
