@@ -155,9 +155,9 @@ def test_implicit_solves_together(shape, kw, tol):
             assert rel(run.download(n), orc.get(n)) <= tol, n
 
 
-# downloads in chunks: one short chunk, a thread's two chunks and a bit, one
-# byte count over several threads; two threads downloading at once
-@pytest.mark.parametrize("shape", [(64, 64, 32), (64, 64, 33), (90, 75, 50), (256, 128, 65)])
+# plain downloads, and from 32 MB on in chunks by several threads, the last
+# chunk whole or short; two threads downloading at once
+@pytest.mark.parametrize("shape", [(64, 64, 32), (90, 75, 50), (256, 128, 65), (256, 128, 128), (256, 150, 125)])
 def test_download_chunks(shape):
     cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], stretch="uniform")
     rng = np.random.default_rng(6)

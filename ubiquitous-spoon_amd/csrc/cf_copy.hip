@@ -6,8 +6,12 @@
  * fresh memory 24.5 ms, 4 GB/s, against 1.8 for the bus), and the stream's
  * own copy of pageable memory waits for every chunk.  Here several threads
  * each keep two chunks of a pinned ring in flight and copy them out: 101 MB
- * in 5.8 ms with 8 threads (6.7 with 6, 8.3 with 4, 11.9 with 2), 7 MB in
- * 0.3 ms with one (plain 0.4 to 3.3), 2 MB in 0.2 (plain 0.85).
+ * in 5.8 ms with 8 threads (6.7 with 6, 8.3 with 4, 11.9 with 2).
+ *
+ * From 32 MB on: up to there an allocator hands the same pages out again, and
+ * those that the threads had faulted in made the caller's next work on them
+ * slower.  18 batched runs, whose fields are 2 to 17 MB, take 115 ms with the
+ * threads and 137 without; a server's pass after them 302 ms and 267.
  */
 #include "chanflow.h"
 #include "cf_internal_host.h"
@@ -24,7 +28,7 @@
 #define CP_CHUNK ((size_t) 1 << 20)
 #define CP_THREADS 8
 #define CP_PER_THREAD ((size_t) 4 << 20)      /* bytes that are worth a thread */
-#define CP_MIN ((size_t) 1 << 20)             /* below: a plain copy */
+#define CP_MIN ((size_t) 32 << 20)            /* below: a plain copy */
 #define CP_IDLE 2                             /* rings kept for the next copies */
 
 namespace {
