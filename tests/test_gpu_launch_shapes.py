@@ -185,3 +185,22 @@ def test_poisson_chunk_lengths(nz, prec, tol, per_nz2):
         before = run.max_divergence()
         run.project(1.0)
         assert run.max_divergence() <= (tol + per_nz2 * nz * nz) * before
+
+
+# the projection's workgroups: rows of whole waves with a short last group of
+# rows, and consecutive cells, in runs that project in place and in those
+# whose state is materialised (one component, then all)
+@pytest.mark.parametrize("shape,kw", [((64, 6, 5), dict()), ((128, 9, 6), dict(scalar=1)), ((64, 9, 7), dict(order=4, scalar=1)),
+                                      ((60, 9, 7), dict(order=4)), ((90, 10, 5), dict()), ((192, 20, 4), dict()), ((160, 9, 5), dict()),
+                                      ((120, 6, 6), dict(order=4))])
+def test_projection_workgroups(shape, kw):
+    step_parity(shape, 2, **kw)
+    cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], stretch="tanh", dt=5e-4, **kw)
+    f = cf.initial_fields(cfg, seed=3)
+    with cf.Run(cfg) as run:
+        for n in f if cfg.scalar else "uvw":
+            run.upload(n, f[n])
+        run.step(2)
+        one = {n: run.xy_stats("avg", n) for n in "uvw"}      # materialises one component
+        for n in "uvw":
+            assert np.abs(one[n] - run.download(n).mean(axis=(0, 1))).max() <= 1e-13

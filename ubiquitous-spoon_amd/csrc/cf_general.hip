@@ -867,9 +867,9 @@ static __device__ __forceinline__ void proj_body(const RunDev &R, const T *us,
     T *u, T *v, T *w, T *c, const Blk b)
 {
     const T A1 = (T) A1d, A2 = (T) A2d;
-    const Pt<T> pt(R, b);
-    if (!pt.act) return;
-    const int nx = pt.nx, ny = pt.ny, nz = pt.nz, i = pt.i, j = pt.j, k = pt.k;
+    const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz, k = b.z;
+    int i, j;
+    if (!proj_cell(R, b, i, j)) return;
     const size_t P = (size_t) nx * ny;
     const size_t row = rowof(k, j, nx, P), q = row + i;
     const double *rdzh = R.rdzh + CF_NGT;
@@ -968,7 +968,7 @@ __global__ __launch_bounds__(256) void kb_proj(const GArgs<T> *__restrict__ A, c
 {
     batch_loop(vs, nrun, [&](int r, unsigned lb) {
         const GArgs<T> &a = A[r];
-        const Blk b = blk_of(a, ST_CELL, lb);
+        const Blk b = blk_of(a, ST_PROJ, lb);
         if (s < 3) {
             const int nz = a.R.g.nz;
             const double *h1u = a.R.h1 + (size_t) (s * 2 + 0) * (nz + 2);

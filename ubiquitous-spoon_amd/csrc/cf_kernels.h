@@ -152,6 +152,43 @@ static __device__ __forceinline__ Blk blk_native()
     return b;
 }
 
+/* The cells that a projection's 256-thread workgroup takes.  Rows that start
+ * where a cache line does and leave at most one lane in five idle go in tiles
+ * of 64 x 4: p's rows above and below serve four rows (order 2 at 256x65x256
+ * 37.6 us, 256 consecutive cells of a level 41.0, at 160x97x150 26.2 and 28.1;
+ * order 4 with the scalar at 192x65x192 30.6 and 32.7, at 120x65x125 16.1 and
+ * 19.7).  Other rows go as consecutive cells (90x129x90 12.0 us, in tiles
+ * 17.1; 300x65x300 57 and 61, in FP32 30 and 39; order 4 with the scalar at
+ * 250x65x250 alone 72 and 68). */
+static inline __host__ __device__ bool proj_tiles(int nx)
+{
+    const int full = (nx + 63) & ~63;
+    return (nx & 7) == 0 && 5 * (full - nx) <= full;
+}
+struct ProjGrid { unsigned x, y; };
+static inline ProjGrid proj_blocks(int nx, int ny)
+{
+    ProjGrid g;
+    if (proj_tiles(nx)) { g.x = (unsigned) (nx + 63) / 64; g.y = (unsigned) (ny + 3) / 4; }
+    else { g.x = ((unsigned) nx * (unsigned) ny + 255) / 256; g.y = 1; }
+    return g;
+}
+/* cell (i, j) of this thread in workgroup b; false: none */
+static __device__ __forceinline__ bool proj_cell(const RunDev &R, const Blk &b, int &i, int &j)
+{
+    const int nx = R.g.nx, t = threadIdx.x;
+    if (proj_tiles(nx)) {
+        i = (int) b.x * 64 + (t & 63);
+        j = (int) b.y * 4 + (t >> 6);
+        return i < nx && j < R.g.ny;
+    }
+    const int e = (int) b.x * 256 + t;
+    if (e >= nx * R.g.ny) return false;
+    j = qdiv(e, nx, R.rnx);
+    i = e - j * nx;
+    return true;
+}
+
 /* the column block of workgroup b (nbx of them a field) of a z solve */
 static __device__ __forceinline__ Blk blk_solve(unsigned b, unsigned nbx)
 {
@@ -165,7 +202,7 @@ static __device__ __forceinline__ Blk blk_solve(unsigned b, unsigned nbx)
 }
 
 /* launch stages of a batched step; each run's grid per stage is dims[stage] */
-enum { ST_CELL = 0, ST_RHSG, ST_SOLVE, ST_ONE, ST_DIVX, ST_FFTX, ST_FFTY, ST_MODE, ST_RHS2, ST_LEVEL, CF_NST };
+enum { ST_PROJ = 0, ST_RHSG, ST_SOLVE, ST_ONE, ST_DIVX, ST_FFTX, ST_FFTY, ST_MODE, ST_RHS2, ST_LEVEL, CF_NST };
 #define CF_BATCH_MAX 256        /* runs per batched launch */
 
 /* Where a substep's projected velocity comes from: the previous
@@ -644,7 +681,8 @@ KSel<float>::pois2_t pick_poisson2_islands(int lmax);
 #define CF_P2_GLEV(nz) ((nz) > 3 * (((nz) + 15) / 16) ? (size_t) (nz) : (size_t) 3 * (((nz) + 15) / 16))
 typedef void (*k_hsolve2_t)(const RunDev, const PoisTab, const PoisTab, const PoisTab, int, double2 *, double *, const Book);
 k_hsolve2_t pick_hsolve2(int lmax);
-template <typename T>
+/* ALL: no output is null */
+template <typename T, bool ALL>
 __global__ void k_project2(const RunDev R, const T *us, const T *vs, const T *ws, const double *h1, const double *mptr,
                            const T *p, double dtp, T *u, T *v, T *w);
 template <typename T>

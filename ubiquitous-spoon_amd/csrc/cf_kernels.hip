@@ -1970,35 +1970,43 @@ KSel<float>::pois2_t pick_poisson2_islands(int L)
  * top-wall face is left at its Dirichlet value 0 (the reference subtracts
  * the Neumann-ghost difference there, which is round-off).  A null output is
  * left out: the copy in and out bounds it (128 x 97 x 128: three fields 17 us,
- * one or two 11).
+ * one or two 11); the form that writes all three has no branches for it (FP32
+ * 256 x 193 x 256: 66 us, with them 75).
  * ------------------------------------------------------------------- */
-template <typename T>
+template <typename T, bool ALL>
 __global__ __launch_bounds__(256) void k_project2(const RunDev R, const T *__restrict__ us,
     const T *__restrict__ vs, const T *__restrict__ ws, const double *__restrict__ h1,
     const double *__restrict__ mptr, const T *__restrict__ p, double dtp,
     T *__restrict__ u, T *__restrict__ v, T *__restrict__ w)
 {
     const int nx = R.g.nx, ny = R.g.ny, nz = R.g.nz;
-    const int e = (int) blockIdx.x * 256 + (int) threadIdx.x, k = blockIdx.z;
-    if (e >= nx * ny || k >= nz) return;
-    const int j = qdiv(e, nx, R.rnx), i = e - j * nx;
+    const int k = blockIdx.z;
+    int i, j;
+    if (!proj_cell(R, blk_native(), i, j)) return;
     const size_t P = (size_t) nx * ny;
     const int ip = i + 1 < nx ? i + 1 : 0, jp = j + 1 < ny ? j + 1 : 0;
     const size_t q = (size_t) k * P + (size_t) j * nx + i;
     const double *rdzh = R.rdzh + CF_NGT;
     const T m = mptr ? (T) *mptr : (T) 0;
+    /* every load before the first use, so that the branches on the outputs
+     * leave one round of them in flight */
     const T p0 = p[q];
-    if (u) {
-        T uc = us[q] + (h1 ? (T) h1[k + 1] * m : (T) 0);
-        u[q] = uc - (p[(size_t) k * P + (size_t) j * nx + ip] - p0) * (T) (dtp * R.rdx);
-    }
-    if (v) v[q] = vs[q] - (p[(size_t) k * P + (size_t) jp * nx + i] - p0) * (T) (dtp * R.rdy);
-    if (w) w[q] = k < nz - 1 ? ws[q] - (p[q + P] - p0) * (T) (dtp * rdzh[k]) : (T) 0;
+    T us0 = 0, vs0 = 0, ws0 = 0, px = 0, py = 0, pz = 0;
+    if (ALL || u) { us0 = us[q]; px = p[(size_t) k * P + (size_t) j * nx + ip]; }
+    if (ALL || v) { vs0 = vs[q]; py = p[(size_t) k * P + (size_t) jp * nx + i]; }
+    if ((ALL || w) && k < nz - 1) { ws0 = ws[q]; pz = p[q + P]; }
+    if (ALL || u) u[q] = us0 + (h1 ? (T) h1[k + 1] * m : (T) 0) - (px - p0) * (T) (dtp * R.rdx);
+    if (ALL || v) v[q] = vs0 - (py - p0) * (T) (dtp * R.rdy);
+    if (ALL || w) w[q] = k < nz - 1 ? ws0 - (pz - p0) * (T) (dtp * rdzh[k]) : (T) 0;
 }
-template __global__ void k_project2<double>(const RunDev, const double *, const double *, const double *, const double *,
-    const double *, const double *, double, double *, double *, double *);
-template __global__ void k_project2<float>(const RunDev, const float *, const float *, const float *, const double *,
-    const double *, const float *, double, float *, float *, float *);
+#define INST_(T, ALL)                                                                                                 \
+    template __global__ void k_project2<T, ALL>(const RunDev, const T *, const T *, const T *, const double *,       \
+                                                const double *, const T *, double, T *, T *, T *);
+INST_(double, true)
+INST_(double, false)
+INST_(float, true)
+INST_(float, false)
+#undef INST_
 
 /* max |div| over interior cells (case1 check, cases.c:473-486), the
  * divergence of the order in force, evaluated in FP64 whatever the

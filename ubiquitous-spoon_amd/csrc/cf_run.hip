@@ -1406,6 +1406,12 @@ static cf_status ev_end(cf_run *r)
 
 /* one thread per cell: 256 consecutive cells of a level per workgroup */
 static dim3 cell_grid(const cf_run *r) { return dim3((unsigned) ((r->P + 255) / 256), 1, r->g.nz); }
+/* ... of a projection (proj_cell) */
+static dim3 proj_grid(const cf_run *r)
+{
+    const ProjGrid g = proj_blocks(r->g.nx, r->g.ny);
+    return dim3(g.x, g.y, r->g.nz);
+}
 
 /* LDS of the x and y FFT launches: a workgroup's lines and the twiddles */
 static size_t fx_lds_n(const cf_run *r, int pairs)
@@ -1511,7 +1517,7 @@ template <typename T>
 static cf_status enqueue_materialise_t(cf_run *r, double *u, double *v, double *w)
 {
     ProjSrcT<T> S = current_projection<T>(r);
-    KLAUNCH("materialise", k_project2<T>, cell_grid(r), dim3(256), 0, r->rd, S.us, S.vs, S.ws, S.h1, S.m,
+    KLAUNCH("materialise", (u && v && w ? k_project2<T, true> : k_project2<T, false>), proj_grid(r), dim3(256), 0, r->rd, S.us, S.vs, S.ws, S.h1, S.m,
             S.p, S.dtp, tv<T>(u), tv<T>(v), tv<T>(w));
     return CF_OK;
 }
@@ -1689,7 +1695,7 @@ static cf_status enqueue_step_general_t(cf_run *r)
         const double *h1c = R.h1 + (size_t) (s * 2 + 1) * (nz + 2);
         st = enqueue_pressure<T>(r, ru, rv, rw, h1u, r->scal + SC_M0 + s, s);
         if (st != CF_OK) return st;
-        KLAUNCH("project", K.proj, cg, cb, 0, R, (const T *) ru, (const T *) rv, (const T *) rw, (const T *) rc, h1u,
+        KLAUNCH("project", K.proj, proj_grid(r), cb, 0, R, (const T *) ru, (const T *) rv, (const T *) rw, (const T *) rc, h1u,
                 (const double *) (r->scal + SC_M0 + s), sc ? h1c : (const double *) nullptr,
                 (const double *) (r->scal + SC_MC0 + s), (const T *) tv<T>(r->p), R.sc[s].abdt, u, v, w,
                 sc ? c : (T *) nullptr);
@@ -1819,7 +1825,7 @@ static cf_status project_general(cf_run *r, double dt)
     T *u = tv<T>(r->u), *v = tv<T>(r->v), *w = tv<T>(r->w);
     cf_status st = enqueue_pressure<T>(r, u, v, w, nullptr, nullptr, 3);
     if (st != CF_OK) return st;
-    KLAUNCH("project", Prec<T>::gen(r).proj, cell_grid(r), dim3(256), 0, r->rd, (const T *) u, (const T *) v,
+    KLAUNCH("project", Prec<T>::gen(r).proj, proj_grid(r), dim3(256), 0, r->rd, (const T *) u, (const T *) v,
             (const T *) w, (const T *) nullptr, (const double *) nullptr, (const double *) nullptr,
             (const double *) nullptr, (const double *) nullptr, (const T *) tv<T>(r->p), dt, u, v, w, (T *) nullptr);
     return CF_OK;
@@ -1859,7 +1865,7 @@ static cf_status project_fast(cf_run *r, double dt)
     if (st != CF_OK) return st;
     double *su, *sv, *sw;
     state_set(r, r->cur, &su, &sv, &sw);
-    KLAUNCH("project", k_project2<T>, cell_grid(r), dim3(256), 0, r->rd, (const T *) a, (const T *) b,
+    KLAUNCH("project", (k_project2<T, true>), proj_grid(r), dim3(256), 0, r->rd, (const T *) a, (const T *) b,
             (const T *) c, (const double *) nullptr, (const double *) nullptr, (const T *) tv<T>(r->p), dt,
             tv<T>(su), tv<T>(sv), tv<T>(sw));
     return CF_OK;
@@ -2396,7 +2402,7 @@ extern "C" cf_status cf_op_poisson(cf_run *r, double *spec, double dt)
 
 enum { KB_RHS = 0, KB_SOLVE, KB_MASS, KB_DIVX, KB_FFTY, KB_POIS, KB_FFTXI, KB_PROJ, KB_FRHS, KB_FSPIKE, KB_FLEVEL,
        KB_N };
-static const int KB_STAGE[KB_N] = { ST_RHSG, ST_SOLVE, ST_ONE, ST_DIVX, ST_FFTY, ST_MODE, ST_FFTX, ST_CELL,
+static const int KB_STAGE[KB_N] = { ST_RHSG, ST_SOLVE, ST_ONE, ST_DIVX, ST_FFTY, ST_MODE, ST_FFTX, ST_PROJ,
                                     ST_RHS2, ST_SOLVE, ST_LEVEL };
 static const char *KB_NAME[KB_N] = { "rhs", "solve", "mass", "div_fftx", "ffty", "poisson", "fftx_inv", "project",
                                      "rhs", "spike", "plane_sum" };
@@ -2527,7 +2533,8 @@ static void batch_fill_args(cf_batch *b, std::vector<GArgs<T>> &A)
         const unsigned ny = r->g.ny, nz = r->g.nz;
         const unsigned P = (unsigned) r->P, nf = (unsigned) r->nfield;
         auto set = [&](int st, unsigned x, unsigned y, unsigned z) { a.dims[st][0] = x; a.dims[st][1] = y; a.dims[st][2] = z; };
-        set(ST_CELL, (P + 255) / 256, 1, nz);
+        const ProjGrid pg = proj_blocks(r->g.nx, r->g.ny);
+        set(ST_PROJ, pg.x, pg.y, nz);
         set(ST_RHSG, (P + 255) / 256, 1, nz * nf);
         if (run_uses_spike(b, r)) set(ST_SOLVE, (P + 63) / 64, nf, 1);
         else set(ST_SOLVE, (P + 255) / 256, nf, 1);
