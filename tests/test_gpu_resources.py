@@ -1,0 +1,22 @@
+"""What a run holds on the device and on the host, and what it gives back."""
+import ctypes
+
+import pytest
+
+import chanflow as cf
+
+pytestmark = pytest.mark.gpu
+
+
+# a configuration that is refused after the device was found leaves no live
+# run behind: the copies' idle pinned rings go with the last one
+def test_refused_run_is_not_counted():
+    users = cf.lib().cf_copy_users
+    users.argtypes, users.restype = [ctypes.c_int], ctypes.c_int
+    live = users(0)
+    with pytest.raises(cf.ChanflowError, match="beta"):
+        cf.Run(cf.Config(nx=16, ny=6, nz=8, stretch="tanh", stretch_beta=0.0))
+    assert users(0) == live
+    with cf.Run(cf.Config(nx=16, ny=6, nz=8)):
+        assert users(0) == live + 1
+    assert users(0) == live

@@ -89,15 +89,17 @@ void ring_give(Ring *g)
 
 } // namespace
 
-extern "C" void cf_copy_users(int add)
+extern "C" int cf_copy_users(int add)
 {
     Ring *drop[CP_IDLE] = {};
+    int users;
     {
         std::lock_guard<std::mutex> hold(g_lock);
-        g_users += add;
-        if (g_users == 0) std::swap(drop, g_idle);
+        users = g_users += add;
+        if (users == 0) std::swap(drop, g_idle);
     }
     for (Ring *g : drop) ring_free(g);
+    return users;
 }
 
 extern "C" cf_status cf_copy_to_host(void *host, const void *dev, size_t bytes, int device, void *stream)

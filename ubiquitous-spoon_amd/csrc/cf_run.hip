@@ -1197,7 +1197,6 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     HIPCHK(hipSetDevice(cfg->device));
 
     cf_run *r = new cf_run();
-    cf_copy_users(1);
     r->cfg = *cfg;
     r->cfg.dz_user = nullptr;
     const int nx = cfg->nx, ny = cfg->ny, nz = cfg->nz;
@@ -1234,6 +1233,7 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     TabPack TP;
     st = build_tables(cfg, r->dz, dx, dy, cfg->dt, TP);
     if (st != CF_OK) { delete r; return st; }
+    cf_copy_users(1);                           /* from here on free_run takes it back */
     const std::vector<double> &pack = TP.pack;
     r->tab_n = pack.size();
 

@@ -22,8 +22,9 @@ cf_status cf_run_stat_plane_into(struct cf_run *r, int kind, int fa, int fb, dou
  * return; device is current */
 cf_status cf_copy_to_host(void *host, const void *dev, size_t bytes, int device, void *stream);
 
-/* a run is made (+1) or gone (-1): what the copies keep goes with the last */
-void cf_copy_users(int add);
+/* a run is made (+1) or gone (-1): what the copies keep goes with the last.
+ * The live runs come back (0 only asks) */
+int cf_copy_users(int add);
 
 #ifdef __cplusplus
 }
