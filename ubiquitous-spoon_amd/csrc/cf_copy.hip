@@ -80,9 +80,13 @@ void ring_give(Ring *g)
 {
     {
         std::lock_guard<std::mutex> hold(g_lock);
-        if (g_users > 0)
+        if (g_users > 0) {
             for (Ring *&i : g_idle)
                 if (!i) { i = g; return; }
+            /* two rings of one device do not keep another's from staying */
+            static_assert(CP_IDLE == 2, "compares the two kept rings");
+            if (g_idle[0]->device == g_idle[1]->device && g->device != g_idle[0]->device) std::swap(g, g_idle[1]);
+        }
     }
     ring_free(g);
 }
