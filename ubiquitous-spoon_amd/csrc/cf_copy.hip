@@ -2,16 +2,20 @@
  * cf_copy.hip -- device-to-host copies of whole fields into pageable memory.
  *
  * What bounds such a copy is the host: the pages of a fresh destination are
- * faulted in and zeroed by the one thread that stores to them (101 MB into
- * fresh memory 24.5 ms, 4 GB/s, against 1.8 for the bus), and the stream's
- * own copy of pageable memory waits for every chunk.  Here several threads
- * each keep two chunks of a pinned ring in flight and copy them out: 101 MB
- * in 5.8 ms with 8 threads (6.7 with 6, 8.3 with 4, 11.9 with 2).
+ * faulted in and zeroed by the one thread that stores to them, and the stream's
+ * own copy of pageable memory waits for every chunk (101 MB into fresh memory
+ * 9.5 to 24.5 ms, with the state of the host's memory; into memory in use 5.9;
+ * the bus needs 1.8).  Here several threads each keep two chunks of a pinned
+ * ring in flight and copy them out: 3.5 to 5.8 ms with 8 threads (where those
+ * took 5.8: 6.7 with 6, 8.3 with 4, 11.9 with 2).  The caller's next passes
+ * over the field take as long as after a plain copy (first read 3.7 and 3.6 ms,
+ * write 2.6 and 2.6).
  *
- * From 32 MB on: up to there an allocator hands the same pages out again, and
- * those that the threads had faulted in made the caller's next work on them
- * slower.  18 batched runs, whose fields are 2 to 17 MB, take 115 ms with the
- * threads and 137 without; a server's pass after them 302 ms and 267.
+ * From 32 MB on, by one series of measurements: with threads from 1 MB on, 18
+ * batched runs, whose fields are 2 to 17 MB, took 115 ms in place of 137, but a
+ * server's pass after them in the same process 302 in place of 267.  Another
+ * series shows the gain (101 to 117 and 137) and not the loss (260 to 320 ms
+ * with either), and a field's next passes alike, so what caused it is open.
  */
 #include "chanflow.h"
 #include "cf_internal_host.h"
@@ -27,7 +31,6 @@
 
 #define CP_CHUNK ((size_t) 1 << 20)
 #define CP_THREADS 8
-#define CP_PER_THREAD ((size_t) 4 << 20)      /* bytes that are worth a thread */
 #define CP_MIN ((size_t) 32 << 20)            /* below: a plain copy */
 #define CP_IDLE 2                             /* rings kept for the next copies */
 
@@ -152,8 +155,7 @@ extern "C" cf_status cf_copy_to_host(void *host, const void *dev, size_t bytes, 
     };
     /* a thread that does not start leaves its chunks to the others */
     std::thread th[CP_THREADS];
-    const int nt = (int) std::min<size_t>(CP_THREADS, std::max<size_t>(1, bytes / CP_PER_THREAD));
-    for (int w = 1; w < nt; w++) {
+    for (int w = 1; w < CP_THREADS; w++) {
         try { th[w] = std::thread(work, w); } catch (...) { break; }
     }
     work(0);
