@@ -46,7 +46,6 @@ def alg_bytes(kernel, N, M):
         "rhs": 88 * N,
         "spike": 48 * N,            # read r (3 fields), write solution
         "thomas": 48 * N,           # read r (3 fields), write solution
-        "plane_sum": 8 * N,         # read u*
         "div_fftx": 24 * N + 16 * M,
         "ffty_fwd": 32 * M,
         "ffty_inv": 32 * M,
@@ -98,7 +97,7 @@ def time_form(name, cfg, steps, warmup, names="uvw", bytes_per_pt=None):
         run.step(2)
         run.sync()
         kt = {}
-        for k in ("rhs", "cfl_finish", "solve", "spike", "plane_sum", "mass", "div_fftx", "ffty_fwd", "poisson",
+        for k in ("rhs", "solve", "spike", "div_fftx", "ffty_fwd", "poisson",
                   "ffty_inv", "fftx_inv", "project"):
             ms, n = run.kernel_time(k)
             if n:
@@ -341,7 +340,7 @@ def main():
     run.step(args.profile_steps)
     run.sync()
     kt = {}
-    for name in ("cfl", "rhs", "spike", "thomas", "plane_sum", "mass", "div_fftx", "ffty_fwd", "poisson",
+    for name in ("cfl", "rhs", "spike", "thomas", "div_fftx", "ffty_fwd", "poisson",
                  "ffty_inv", "fftx_inv", "project"):
         ms, n = run.kernel_time(name)
         if n:

@@ -1,4 +1,5 @@
-"""What a run holds on the device and on the host, and what it gives back."""
+"""What a run holds on the device and on the host, what it gives back, and
+where its profile keeps its time."""
 import ctypes
 
 import pytest
@@ -20,3 +21,16 @@ def test_refused_run_is_not_counted():
     with cf.Run(cf.Config(nx=16, ny=6, nz=8)):
         assert users(0) == live + 1
     assert users(0) == live
+
+
+# a solve's time is kept under the name of the solve: nz = 257 has no spike
+# tables and takes the Thomas sweep
+@pytest.mark.parametrize("nz,solve,other", [(257, "thomas", "spike"), (33, "spike", "thomas")])
+def test_solve_time_by_name(nz, solve, other):
+    with cf.Run(cf.Config(nx=16, ny=6, nz=nz)) as run:
+        run.project(1.0)
+        run.set_profiling(True)
+        run.step(2)
+        run.sync()
+        assert run.kernel_time(solve)[1] == 6
+        assert run.kernel_time(other)[1] == 0

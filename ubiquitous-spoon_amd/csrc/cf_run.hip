@@ -1587,7 +1587,8 @@ static cf_status enqueue_step_t(cf_run *r, int from)
         KLAUNCH("rhs", pick_rhs2<T>(s), dim3(r->rhs_blocks), dim3(256), 0, R, S, (const T *) tv<T>(gold[0]),
                 (const T *) tv<T>(gold[1]), (const T *) tv<T>(gold[2]), (const double *) r->scal, tv<T>(fnew[0]),
                 tv<T>(fnew[1]), tv<T>(fnew[2]), ou, ov, ow, r->cflpart, dt, r->rhs_kc, r->part);
-        cf_status st = enqueue_zsolve<T>(r, "spike", s, 3, ou, ov, ow, nullptr, make_book(r, s, r->rhs_blocks, dt));
+        cf_status st = enqueue_zsolve<T>(r, r->use_spike ? "spike" : "thomas", s, 3, ou, ov, ow, nullptr,
+                                         make_book(r, s, r->rhs_blocks, dt));
         if (st != CF_OK) return st;
         const double *h1 = R.h1 + (size_t) (s * 2 + 0) * (nz + 2);
         st = enqueue_pressure<T>(r, ou, ov, ow, h1, r->scal + SC_M0 + s, s);
