@@ -56,6 +56,7 @@ static const double RK_GAM[3] = { 8.0 / 15.0, 5.0 / 12.0, 3.0 / 4.0 };
 static const double RK_ZET[3] = { 0.0, -17.0 / 60.0, -5.0 / 12.0 };
 
 static const int LOGCAP = 4096;
+#define CF_NB_RED 1024          /* partial maxima of the divergence check */
 static const int MAXE_LINE = 2048;      /* elements per FFT block (8 per thread x 256) */
 #ifndef CF_P4_THREADS
 #define CF_P4_THREADS 64                /* order-4 Poisson: modes (threads) per workgroup of a single run */
@@ -575,26 +576,6 @@ static cf_status validate(const cf_config *c)
     return CF_OK;
 }
 
-extern "C" cf_status cf_run_footprint(const cf_config *cfg, size_t *bytes)
-{
-    cf_status st = validate(cfg);
-    if (st != CF_OK) return st;
-    size_t N = (size_t) cfg->nx * cfg->ny * cfg->nz;
-    size_t M = (size_t) (cfg->nx / 2 + 1) * cfg->ny * cfg->nz;
-    size_t nf = cfg->scalar ? 4 : 3;
-    size_t es = cfg->precision == CF_FP32 ? sizeof(float) : sizeof(double);
-    const bool impl = cfg->driver == CF_DRIVER_CHANNEL;
-    /* state and solve output per field, p: (2 nf + 1) N values; X: 2 M; two
-     * forcing slots per field, one of which holds a spectrum (2 M), with the
-     * fully implicit driver each; FP64 stage N, G M (fully implicit, order 2:
-     * per field), order-4 Poisson factors 3 M, partial sums of the plane
-     * statistics 192 nz */
-    *bytes = es * ((2 * nf + 1) * N + 2 * M + (impl ? 4 * nf * M : (2 * nf - 1) * N + 2 * M))
-           + sizeof(double) * (N + (cfg->order == 4 ? 4 : impl ? nf : 1) * M + (size_t) 192 * cfg->nz)
-           + ((size_t) 16 << 20);
-    return CF_OK;
-}
-
 static void free_run(cf_run *r)
 {
     if (!r) return;
@@ -667,6 +648,65 @@ static int rhs_target(const std::vector<const Grid *> &grids, int cap)
         if (bestcost < 0 || cost < bestcost) { bestcost = cost; best = t; }
     }
     return best;
+}
+
+/* launch shapes of a run alone, and the lengths of its work buffers */
+struct RunShape {
+    int rhs_kc, rhs_blocks;          /* fused RHS: levels per z-chunk, workgroups */
+    int gblocks;                     /* general RHS: workgroups per field */
+    int r4_nch, r4_blocks;           /* order-4 tiles (0: none): z-chunks, workgroups */
+    size_t stage, part, cflpart;     /* doubles */
+    size_t glev;                     /* levels of G, M doubles each */
+};
+static RunShape run_shape(const cf_config *cfg)
+{
+    RunShape S;
+    const int nx = cfg->nx, ny = cfg->ny, nz = cfg->nz, nkx = nx / 2 + 1;
+    const size_t P = (size_t) nx * ny, N = P * nz, esz = cfg->precision == CF_FP32 ? sizeof(float) : sizeof(double);
+    Grid g;
+    g.nx = nx; g.ny = ny; g.nz = nz;
+    rhs_chunks(nx, ny, nz, rhs_target({ &g }, CF_RHS_KC), &S.rhs_kc, &S.rhs_blocks);
+    S.gblocks = (int) ((P + 255) / 256) * nz;
+    S.r4_nch = S.r4_blocks = 0;
+    if (cfg->order == 4 && nx % CF_R4_X == 0 && ny % CF_R4_Y == 0 && N * esz < ((size_t) 1 << 32)) {   /* 32-bit byte offsets */
+        S.r4_nch = std::max(1, (nz + CF_R4_KC / 2) / CF_R4_KC);
+        S.r4_blocks = (nx / CF_R4_X) * (ny / CF_R4_Y) * S.r4_nch;
+    }
+    /* stage: a field, or the rows and partial sums of k_stat_spec (more than
+     * a field at nx = 2) */
+    S.stage = std::max(N, (size_t) 2 * nz * (nkx + (size_t) 2 * ny * ((nkx + CF_SPEC_ROWS - 1) / CF_SPEC_ROWS)));
+    /* part: a batch's plane sums of the solve, the RHS launch's partial sums
+     * (four statistics of u and, with the scalar, c), the divergence check's
+     * maxima and the plane statistics' partial sums */
+    S.part = std::max({ ((P + 63) / 64) * nz, (size_t) CF_NB_RED, (size_t) 3 * CF_STAT_NBL * nz,
+                        (size_t) 4 * std::max({ S.gblocks, S.rhs_blocks, S.r4_blocks }) * (cfg->scalar ? 2 : 1) });
+    /* a batch may cut the run's z-chunks otherwise, down to one level */
+    S.cflpart = (size_t) std::max({ (int) (rhs_tiles(nx, ny) * nz), S.gblocks, S.r4_blocks });
+    /* G: the order-2 Poisson's chunk checkpoints (3 per chunk of 16 levels) per
+     * mode, and with the fully implicit driver a part per field */
+    S.glev = CF_P2_GLEV(nz);
+    if (cfg->driver == CF_DRIVER_CHANNEL && cfg->order == 2) S.glev *= cfg->scalar ? 4 : 3;
+    return S;
+}
+
+extern "C" cf_status cf_run_footprint(const cf_config *cfg, size_t *bytes)
+{
+    cf_status st = validate(cfg);
+    if (st != CF_OK) return st;
+    const RunShape S = run_shape(cfg);
+    size_t N = (size_t) cfg->nx * cfg->ny * cfg->nz;
+    size_t M = (size_t) (cfg->nx / 2 + 1) * cfg->ny * cfg->nz;
+    size_t nf = cfg->scalar ? 4 : 3;
+    size_t es = cfg->precision == CF_FP32 ? sizeof(float) : sizeof(double);
+    const bool impl = cfg->driver == CF_DRIVER_CHANNEL;
+    /* state and solve output per field, p: (2 nf + 1) N values; X: 2 M; two
+     * forcing slots per field, one of which holds a spectrum (2 M), with the
+     * fully implicit driver each; in FP64 the work buffers, G and the order-4
+     * Poisson factors (3 M); tables, logs and the like: 16 MB */
+    *bytes = es * ((2 * nf + 1) * N + 2 * M + (impl ? 4 * nf * M : (2 * nf - 1) * N + 2 * M))
+           + sizeof(double) * (S.stage + S.part + S.cflpart + M / cfg->nz * S.glev + (cfg->order == 4 ? 3 * M : 0))
+           + ((size_t) 16 << 20);
+    return CF_OK;
 }
 
 /* Every table of a run that depends on dt (the z-solve factors and spikes,
@@ -1256,34 +1296,19 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
         if (cfg->scalar) ok = ok && falloc(&r->c, r->N);
     } else {
         ok = ok && falloc(&r->ru, r->N) && falloc(&r->rv, r->N) && falloc(&r->rw, r->N);
+        /* a statistic's spectrum fits in fb[0] */
         for (int f = 0; f < 3; f++) ok = ok && falloc(&r->fa[f], r->N) && falloc(&r->fb[f], f ? r->N : 2 * r->M * nz);
         if (cfg->scalar) ok = ok && falloc(&r->c, r->N) && falloc(&r->rc, r->N) && falloc(&r->fa[3], r->N) && falloc(&r->fb[3], r->N);
     }
-    /* a spectrum fits in fb[0], the partial sums of k_stat_spec in stage */
-    const size_t nst = (size_t) 2 * nz * (r->g.nkx + (size_t) 2 * ny * ((r->g.nkx + CF_SPEC_ROWS - 1) / CF_SPEC_ROWS));
+    const RunShape S = run_shape(cfg);
+    r->rhs_kc = S.rhs_kc; r->rhs_blocks = S.rhs_blocks; r->gblocks = S.gblocks;
+    r->r4_nch = S.r4_nch; r->r4_blocks = S.r4_blocks;
     if (order == 4) ok = ok && dalloc(&r->S4, 3 * r->M * nz);
-    /* G: the order-2 Poisson's chunk checkpoints (3 per chunk of 16 levels) per mode */
-    size_t glev = CF_P2_GLEV(nz);
-    if (cfg->driver == CF_DRIVER_CHANNEL && order == 2) glev *= cfg->scalar ? 4 : 3;     /* a part per field */
-    ok = ok && falloc(&r->p, r->N) && dalloc(&r->stage, std::max(r->N, nst)) && dalloc(&r->G, r->M * glev);
+    ok = ok && falloc(&r->p, r->N) && dalloc(&r->stage, S.stage) && dalloc(&r->G, r->M * S.glev);
     ok = ok && hipMalloc((void **) &r->X, 2 * r->esz * r->M * nz) == hipSuccess;
     ok = ok && dalloc(&r->tab, r->tab_n) && dalloc(&r->scal, SC_N) && dalloc(&r->logbuf, (size_t) LOGCAP * CF_LOG_N);
-    rhs_chunks(nx, ny, nz, rhs_target({ &r->g }, CF_RHS_KC), &r->rhs_kc, &r->rhs_blocks);
-    r->gblocks = (int) ((r->P + 255) / 256) * nz;
-    if (cfg->order == 4 && nx % CF_R4_X == 0 && ny % CF_R4_Y == 0
-        && (size_t) nx * ny * nz * r->esz < ((size_t) 1 << 32)) {   /* 32-bit byte offsets */
-        r->r4_nch = std::max(1, (nz + CF_R4_KC / 2) / CF_R4_KC);
-        r->r4_blocks = (nx / CF_R4_X) * (ny / CF_R4_Y) * r->r4_nch;
-    }
-    r->nb_red = 1024;
-    /* part: a batch's plane sums of the solve, the RHS launch's partial sums
-     * (four statistics of u and, with the scalar, c), the divergence check's
-     * maxima and the plane statistics' partial sums */
-    const size_t npart = std::max({ (size_t) ((r->P + 63) / 64) * nz, (size_t) r->nb_red, (size_t) 3 * CF_STAT_NBL * nz,
-                                    (size_t) 4 * std::max({ r->gblocks, r->rhs_blocks, r->r4_blocks }) * (cfg->scalar ? 2 : 1) });
-    ok = ok && dalloc(&r->part, npart) && dalloc(&r->lsum, (size_t) nz + 2);
-    /* a batch may cut the run's z-chunks otherwise, down to one level */
-    ok = ok && dalloc(&r->cflpart, (size_t) std::max({ (int) (rhs_tiles(nx, ny) * nz), r->gblocks, r->r4_blocks }));
+    r->nb_red = CF_NB_RED;
+    ok = ok && dalloc(&r->part, S.part) && dalloc(&r->lsum, (size_t) nz + 2) && dalloc(&r->cflpart, S.cflpart);
     if (cfg->cflmode == 1) ok = ok && dalloc(&r->h1prev, (size_t) nz + 2);
     if (r->prec == CF_FP32 && !r->general) ok = ok && dalloc(&r->uoffd, (size_t) nz + 2 + 3 * (size_t) nz);
     if (!ok) { free_run(r); cf_set_error("device allocation failed"); return CF_ERR_NOMEM; }
