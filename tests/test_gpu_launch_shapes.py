@@ -204,3 +204,52 @@ def test_projection_workgroups(shape, kw):
         one = {n: run.xy_stats("avg", n) for n in "uvw"}      # materialises one component
         for n in "uvw":
             assert np.abs(one[n] - run.download(n).mean(axis=(0, 1))).max() <= 1e-13
+
+
+# the same chunk lengths in FP32 against the FP64 solve of the same input, on
+# a grid whose modes past the FP64 ones take 18 workgroups, the last a short
+# one.  FP32 rounds the fields (three times), the transforms (log2 of 768
+# points) and the solves, whose modes past |k| = 4 have a condition of at most
+# 4 (nz / lz)^2 / 25
+@pytest.mark.parametrize("nz", [17, 33, 47, 64, 79, 95, 111, 127, 143, 159, 175, 191, 193, 223, 239, 255, 257, 321, 385, 449, 512])
+def test_poisson_fp32_against_fp64(nz):
+    got = {}
+    for prec in (cf.CF_FP64, cf.CF_FP32):
+        cfg = cf.Config(nx=32, ny=24, nz=nz, lz=2.0, stretch="uniform", precision=prec)
+        f = cf.initial_fields(cfg, seed=2)
+        with cf.Run(cfg) as run:
+            for n in "uvw":
+                run.upload(n, f[n])
+            run.project(1.0)
+            got[prec] = {n: run.download(n) for n in "uvw"}
+    tol = 2.0 ** -24 * (3 + np.log2(768) + 4 * (nz / 2.0) ** 2 / 25)
+    for n in "uvw":
+        assert rel(got[cf.CF_FP32][n], got[cf.CF_FP64][n]) <= tol, n
+
+
+# batches over lengths with a divergence + x FFT of their own (192 only in
+# FP64) and lengths on the run-time plan, an odd number of lines in the last
+# pair group: each run against the oracle
+@pytest.mark.parametrize("shapes,prec,tol", [([(192, 9, 5), (90, 15, 7), (64, 9, 6)], cf.CF_FP64, 1e-12),
+                                             ([(48, 6, 33), (96, 9, 5), (128, 9, 5), (192, 6, 17), (32, 15, 9)], cf.CF_FP64, 1e-12),
+                                             ([(192, 9, 5), (96, 9, 7), (128, 15, 9), (90, 6, 6)], cf.CF_FP32, 5e-5)])
+def test_batched_lengths(shapes, prec, tol):
+    cfgs = [cf.Config(nx=s[0], ny=s[1], nz=s[2], stretch="tanh", dt=5e-4, nu=1.0 / (2000.0 + 500.0 * q), precision=prec)
+            for q, s in enumerate(shapes)]
+    cases = []
+    for q, c in enumerate(cfgs):
+        f = cf.initial_fields(c, seed=60 + q)
+        orc = ol.OracleRun(ol.oracle_cfg(c, cf.grid_dz(c)))
+        for n in "uvw":
+            orc.put(n, f[n])
+        orc.project_ic(1.0)
+        cases.append((orc, {n: orc.get(n) for n in "uvw"}))
+    with cf.Batch(cfgs) as b:
+        for q, (orc, init) in enumerate(cases):
+            for n in "uvw":
+                b.upload(q, n, init[n])
+        b.step(8)
+        for q, (orc, _) in enumerate(cases):
+            orc.steps(8)
+            for n in "uvw":
+                assert rel(b.download(q, n), orc.get(n)) <= tol, (shapes[q], n)
