@@ -227,6 +227,25 @@ def test_poisson_fp32_against_fp64(nz):
         assert rel(got[cf.CF_FP32][n], got[cf.CF_FP64][n]) <= tol, n
 
 
+# the divergence's pair counts in FP32 against FP64, to the same roundings and
+# that of p, which its differences raise by at most max(nx, ny) / pi
+@pytest.mark.parametrize("shape", [(64, 6, 3), (128, 9, 4), (128, 10, 4), (96, 8, 5), (90, 15, 4), (24, 40, 33), (256, 6, 5), (512, 6, 4),
+                                   (600, 6, 4)])
+def test_projection_fp32_against_fp64(shape):
+    got = {}
+    for prec in (cf.CF_FP64, cf.CF_FP32):
+        cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], lz=2.0, stretch="uniform", precision=prec)
+        f = cf.initial_fields(cfg, seed=2)
+        with cf.Run(cfg) as run:
+            for n in "uvw":
+                run.upload(n, f[n])
+            run.project(1.0)
+            got[prec] = {n: run.download(n) for n in "uvw"}
+    tol = 2.0 ** -24 * (3 + np.log2(shape[0] * shape[1]) + 4 * (shape[2] / 2.0) ** 2 / 25 + max(shape[:2]) / np.pi)
+    for n in "uvw":
+        assert rel(got[cf.CF_FP32][n], got[cf.CF_FP64][n]) <= tol, n
+
+
 # batches over lengths with a divergence + x FFT of their own (192 only in
 # FP64) and lengths on the run-time plan, an odd number of lines in the last
 # pair group: each run against the oracle
