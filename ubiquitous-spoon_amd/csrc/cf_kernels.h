@@ -360,7 +360,8 @@ static inline int pois2_L_of(int need)
 }
 /* chunk length for nz (0: one thread per mode) */
 static inline int pois2_L(int nz) { return pois2_L_of((nz + CF_P2S_NC - 1) / CF_P2S_NC); }
-/* dynamic LDS of the partitioned solve: its six z tables */
+/* dynamic LDS of the partitioned solve: its six z tables in FP64 (an all-FP32
+ * launch uses half of it) */
 static inline size_t pois2_lds(int L, int nz) { return L > 0 ? 6 * sizeof(double) * (size_t) nz : 0; }
 /* workgroup shape: CF_P2S_NC z-chunks x CF_P2S_MW modes; a z-level of the
  * group is CF_P2S_MW contiguous complex values (256 B in FP64) */

@@ -1829,10 +1829,10 @@ static __device__ __forceinline__ void pois2s_run(const PoisTab &T_, typename Cp
 /* L = pois2_L(nz) (or larger): the partitioned solve with chunks of L
  * rows; L = 0: one thread per mode.  FP32 storage solves the modes with
  * |kx|, |ky| <= CF_F64_KLOW in FP64 (the islands); ISL selects what a
- * launch covers: 0 the storage-precision modes only (island workgroups
- * return at once), 1 the islands only, 2 both.  Splitting them keeps the
+ * launch covers: 0 the FP32 modes only (island workgroups return at once), 1
+ * the islands only, 2 all modes (FP64 storage).  Splitting them keeps the
  * FP64 path's registers out of the FP32 kernel. */
-template <typename T, int L, int ISL = 2>
+template <typename T, int L, int ISL>
 static __device__ __forceinline__ void pois2_body(const RunDev &R, const PoisTab T_,
                                                   typename Cplx<T>::type *__restrict__ Y, double *__restrict__ G, const Blk b,
                                                   const int nz)
@@ -1847,9 +1847,10 @@ static __device__ __forceinline__ void pois2_body(const RunDev &R, const PoisTab
         __shared__ S shb[10][CF_P2S_NC][CF_P2S_MW];
         const int nch = (nz + L - 1) / (L > 0 ? L : 1);
         /* with CF_P2S_XCD the workgroups holding neighbouring modes share an
-         * XCD (and its L2: an FP32 level of the group is one cache line, at
-         * any alignment of ny); the island launch covers only the leading
-         * workgroups and keeps the plain order */
+         * XCD (and its L2: an FP32 level of the group is 128 bytes, one cache
+         * line where nkx ny is a multiple of 16 and otherwise parts of two
+         * that the neighbouring groups share); the island launch covers only
+         * the leading workgroups and keeps the plain order */
         const unsigned bx = (CF_P2S_XCD && ISL != 1) ? xcd_block(b.x, b.nx) : b.x;
         const size_t m0 = (size_t) bx * CF_P2S_MW;
         const size_t mode = m0 + (threadIdx.x & (CF_P2S_MW - 1));
@@ -1875,13 +1876,9 @@ static __device__ __forceinline__ void pois2_body(const RunDev &R, const PoisTab
         constexpr int LL = L > 1 ? L : 2;
         if constexpr (f64 || ISL == 1) {
             pois2s_run<LL, double, T>(T_, Y, M, nz, nch, mc, act, lx, ly, zero, LDS_(double));
-        } else if constexpr (ISL == 0) {
-            pois2s_run<LL, T, T>(T_, Y, M, nz, nch, mc, act, lx, ly, zero, LDS_(T));
         } else {
-            if (low)
-                pois2s_run<LL, double, T>(T_, Y, M, nz, nch, mc, act, lx, ly, zero, LDS_(double));
-            else
-                pois2s_run<LL, T, T>(T_, Y, M, nz, nch, mc, act, lx, ly, zero, LDS_(T));
+            static_assert(f64 || ISL != 2, "an FP32 launch solves one kind of modes");
+            pois2s_run<LL, T, T>(T_, Y, M, nz, nch, mc, act, lx, ly, zero, LDS_(T));
         }
 #undef LDS_
         return;
