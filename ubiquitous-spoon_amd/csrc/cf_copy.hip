@@ -11,11 +11,18 @@
  * over the field take as long as after a plain copy (first read 3.7 and 3.6 ms,
  * write 2.6 and 2.6).
  *
- * From 32 MB on, by one series of measurements: with threads from 1 MB on, 18
- * batched runs, whose fields are 2 to 17 MB, took 115 ms in place of 137, but a
- * server's pass after them in the same process 302 in place of 267.  Another
- * series shows the gain (101 to 117 and 137) and not the loss (260 to 320 ms
- * with either), and a field's next passes alike, so what caused it is open.
+ * The threads take fresh pages from the free lists of their own CPUs.  Where a
+ * page has no memory behind it yet -- in a virtual machine, one that was never
+ * used or that was free long enough to be reported to the host -- its first
+ * touch costs a fault on the host, and a thread of its own meets more of those
+ * than the caller, which gets back what it has just freed.  So a process that
+ * begins to download by threads can pay for some copies (101 MB, each freed
+ * before the next: 4, 22, ten of 15, then 3.3 ms each; plain copies beside them
+ * 9.5 throughout), and other memory that it takes then as well: 18 batched
+ * runs, whose fields are 2 to 17 MB, took 115 ms in place of 137 with threads
+ * from 1 MB on, but a server's pass after them 302 in place of 267 (in other
+ * runs 101 to 117, and no difference after).  Hence from 32 MB on, where a
+ * field is not one of many.
  */
 #include "chanflow.h"
 #include "cf_internal_host.h"
