@@ -101,6 +101,29 @@ def test_divergence_pair_counts(shape, prec, tol):
         assert run.max_divergence() <= tol * before
 
 
+# ... and of grids with lines enough for full workgroups of them (from 512):
+# the fewest such lines and just below, an odd line and a short last
+# workgroup, compiled lengths and run-time plans
+@pytest.mark.parametrize("prec,tol", [(cf.CF_FP64, 1e-11), (cf.CF_FP32, 2e-3)])
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("shape", [(320, 32, 64), (384, 48, 43), (480, 45, 47), (512, 36, 64), (512, 30, 64), (300, 48, 64),
+                                   (300, 48, 63), (400, 75, 31), (200, 75, 69)])
+def test_divergence_pair_counts_many_lines(shape, order, prec, tol):
+    cfg = cf.Config(nx=shape[0], ny=shape[1], nz=shape[2], stretch="uniform", order=order, precision=prec)
+    f = cf.initial_fields(cfg, seed=2)
+    with cf.Run(cfg) as run:
+        for n in "uvw":
+            run.upload(n, f[n])
+        before = run.max_divergence()
+        run.project(1.0)
+        assert run.max_divergence() <= tol * before
+        if prec == cf.CF_FP64:
+            a = np.random.default_rng(3).standard_normal(cfg.shape)
+            ref = np.fft.fft(np.fft.rfft(a, axis=0) / cfg.nx, axis=1) / cfg.ny
+            got = run.fft3d_fwd(a)
+            assert np.abs(got - ref).max() <= 1e-14 * np.abs(ref).max() * np.log2(cfg.nx * cfg.ny)
+
+
 # rows per wave and columns per march of the spectra, levels and partials of
 # the plane sums
 @pytest.mark.parametrize("shape", [(2, 6, 3), (12, 6, 5), (16, 64, 4), (18, 135, 3), (45, 27, 7), (90, 80, 5)])

@@ -120,7 +120,9 @@ struct RunDev {
     const double2 *twx, *twy;
     const float2 *twx32, *twy32;  /* the same twiddles rounded to FP32 */
     const double *lamx, *lamy;  /* modified wavenumbers 2 - 2 cos(2 pi k / n) */
-    int fx_pairs, dx_pairs;     /* complex x lines per block: the x FFTs, the divergence + x FFT */
+    /* complex x lines per block: the inverse x FFT, the divergence + x FFT,
+     * the forward x FFT on its own */
+    int fx_pairs, dx_pairs, px_pairs;
     int fy_cols;                /* kx columns per y-FFT block */
     /* general path (order 4 and/or the scalar) */
     Clos cl;
@@ -334,6 +336,26 @@ static inline bool fft_compiled(int n)
         return true;
     default: return false;
     }
+}
+
+/* ... per workgroup of a single run's divergence + x FFT (paired: at
+ * order 2, whose compiled lengths have a second instance for it) and of its
+ * forward x FFT.  Few pairs are few consecutive lines, so a mode's
+ * half-spectrum values go out in short runs (one pair: 32 bytes in FP64); a
+ * grid of many lines is bound by those stores and takes full workgroups,
+ * once there are two of them for each CU.  With fewer the one round of loads
+ * counts for more (400 x 33 x 32: 14.8 us, full 16.9).  One round -> full
+ * (us): run-time plans 300 x 65 x 150 FP64 53 -> 37, 400 x 129 x 400 FP64
+ * 375 -> 298, FP32 260 -> 210; compiled lengths, which lose less to short
+ * runs and more to a second round, two pairs instead of one at order 2 (384
+ * x 129 x 384 203 -> 171, FP32 512 x 129 x 512 240 -> 189) and none at order
+ * 4 (one pair 512 x 65 x 256 80, two 89); the order-4 implicit solves,
+ * forward x FFT included, 384 x 129 x 384 1,547 -> 1,357 a substep */
+static inline int run_dx_pairs(int nx, int esz, bool paired, long npairs)
+{
+    const int one = dx_pairs_of(nx, esz), most = 1024 / nx;
+    const int full = fft_compiled(nx) ? (paired && one == 1 && most >= 2 ? 2 : one) : (one < 4 && most > one ? most : one);
+    return npairs / full >= 512 ? full : one;
 }
 
 #ifndef CF_P2S_NC
@@ -672,7 +694,7 @@ template <typename T> struct KSel {
 };
 typedef void (*k_fftx_plain_t)(const RunDev, const double *, double2 *);
 template <typename T> typename KSel<T>::rhs2_t pick_rhs2(int s);
-template <typename T> typename KSel<T>::div_t pick_div_fftx(int nx, int order);
+template <typename T> typename KSel<T>::div_t pick_div_fftx(int nx, int order, int pairs);
 k_fftx_plain_t pick_fftx_plain(int nx);
 template <typename T> typename KSel<T>::ffty_t pick_ffty(int ny);
 template <typename T> typename KSel<T>::fftxi_t pick_fftx_inv(int nx);

@@ -896,7 +896,7 @@ static __device__ __forceinline__ void divx2_body(const RunDev &R, const T *__re
  * velocity (u + h1 mdpdx, chanfast.c:519-522) fused with the forward r2c x
  * FFT scaled 1/nx (fft.c:161-177).  Order 4 sees the w ghost faces
  * mirrored oddly about the (zero) wall faces, as divergence4 sets them. */
-template <int NX, int ORD, typename T, int UNRX = 0>
+template <int NX, int ORD, typename T, int UNRX = 0, int PX = 0>
 static __device__ __forceinline__ void divx_body(const RunDev &R, const T *__restrict__ us_,
     const T *__restrict__ vs_, const T *__restrict__ ws_, const double *__restrict__ h1_,
     const double *__restrict__ mptr_, typename Cplx<T>::type *__restrict__ X_, const Blk b)
@@ -917,8 +917,8 @@ static __device__ __forceinline__ void divx_body(const RunDev &R, const T *__res
     const int ny = R.g.ny, nz = R.g.nz, nkx = R.g.nkx;
     const int ld = fft_ld(nx);
     /* compiled lengths run only on runs of element size sizeof(T), whose
-     * pair count is dx_pairs_of(NX, sizeof(T)) */
-    const int nl = NX > 0 ? dx_pairs_of(NX, sizeof(T)) : R.dx_pairs;
+     * pair count is PX, or dx_pairs_of(NX, sizeof(T)) */
+    const int nl = PX > 0 ? PX : (NX > 0 ? dx_pairs_of(NX, sizeof(T)) : R.dx_pairs);
     const int NL = ny * nz;
     const size_t P = (size_t) nx * ny;
     const double rny = 1.0 / (double) ny;
@@ -1083,12 +1083,12 @@ static __device__ __forceinline__ void divx_body(const RunDev &R, const T *__res
     store_half_spectra<C>(sb, ld, nl, nx, nkx, ny, (long) NL, (long) pair0, 0.5 / (double) nx, X);
 }
 
-template <int NX, int ORD, typename T>
+template <int NX, int ORD, typename T, int PX = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((ORD == 2 && divx2_on(NX, sizeof(T))) ? 2 : 4, 8))) void k_div_fftx(const RunDev R, const T *__restrict__ us,
     const T *__restrict__ vs, const T *__restrict__ ws, const double *__restrict__ h1,
     const double *__restrict__ mptr, typename Cplx<T>::type *__restrict__ X)
 {
-    divx_body<NX, ORD, T>(R, us, vs, ws, h1, mptr, X, blk_native());
+    divx_body<NX, ORD, T, 0, PX>(R, us, vs, ws, h1, mptr, X, blk_native());
 }
 
 /* the fftx_d2c stage of FFT3D_FWD on its own (no divergence), scaled 1/nx;
@@ -1103,7 +1103,7 @@ __global__ __launch_bounds__(256) void k_fftx_fwd_plain(const RunDev R, const do
     const int nx = NX > 0 ? NX : R.g.nx;
     const int ny = R.g.ny, nz = R.g.nz, nkx = R.g.nkx;
     const int ld = fft_ld(nx);
-    const int nl = R.dx_pairs;
+    const int nl = R.px_pairs;
     const int NL = ny * nz;
     const int pair0 = (int) blockIdx.x * nl;
     const cp<cv<double2>> twg = (cp<cv<double2>>) R.twx;
@@ -1493,8 +1493,15 @@ static typename KSel<T>::div_t pick_div_ord(int n)
 }
 
 template <typename T>
-typename KSel<T>::div_t pick_div_fftx(int n, int order)
+typename KSel<T>::div_t pick_div_fftx(int n, int order, int pairs)
 {
+    if (order == 2 && pairs == 2 && dx_pairs_of(n, sizeof(T)) == 1) {
+        switch (n) {
+#define X_(N) case N: if constexpr (dx_pairs_of(N, sizeof(T)) == 1) return k_div_fftx<N, 2, T, 2>; else break;
+        CF_FFT_SIZES(X_)
+#undef X_
+        }
+    }
     return order == 4 ? pick_div_ord<T, 4>(n) : pick_div_ord<T, 2>(n);
 }
 
@@ -1530,8 +1537,8 @@ typename KSel<T>::fftxi_t pick_fftx_inv(int n)
     }
 }
 
-template KSel<double>::div_t pick_div_fftx<double>(int, int);
-template KSel<float>::div_t pick_div_fftx<float>(int, int);
+template KSel<double>::div_t pick_div_fftx<double>(int, int, int);
+template KSel<float>::div_t pick_div_fftx<float>(int, int, int);
 template KSel<double>::ffty_t pick_ffty<double>(int);
 template KSel<float>::ffty_t pick_ffty<float>(int);
 template KSel<double>::fftxi_t pick_fftx_inv<double>(int);

@@ -1337,8 +1337,6 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     R.ubc = 0.0 - cfg->uframe;                  /* chanfast.c:59-62 */
     R.vbc = 0.0 - cfg->vframe;
     R.cbot = -0.5; R.ctop = 0.5;                /* chanfast.c:67-68 */
-    r->kdiv = pick_div_fftx<double>(nx, order);
-    r->kdiv32 = pick_div_fftx<float>(nx, order);
     r->g64 = pick_general<double>(order, cfg->scalar);
     r->g32 = pick_general<float>(order, cfg->scalar);
     R.scalar = cfg->scalar;
@@ -1365,7 +1363,10 @@ static cf_status create_run(const cf_config *cfg, bool force_general, cf_run **o
     const long npairs = ((long) ny * nz + 1) / 2;
     R.fx_pairs = fx_pairs_of(nx, (int) r->esz);
     if (!fft_compiled(nx)) R.fx_pairs = (int) std::max(1L, std::min((long) R.fx_pairs, npairs / CF_FFT_WGS));
-    R.dx_pairs = dx_pairs_of(nx, (int) r->esz);
+    R.dx_pairs = run_dx_pairs(nx, (int) r->esz, order == 2, npairs);
+    R.px_pairs = run_dx_pairs(nx, (int) r->esz, true, npairs);
+    if (r->prec == CF_FP32) r->kdiv32 = pick_div_fftx<float>(nx, order, R.dx_pairs);
+    else r->kdiv = pick_div_fftx<double>(nx, order, R.dx_pairs);
     R.fy_cols = (int) std::max(1L, std::min((long) fy_cols_of(ny), (long) nz * r->g.nkx / CF_FFT_WGS));
     /* the two-pass y FFT gives each of a workgroup's 256 threads at most
      * one (line, column) task per pass */
@@ -1445,13 +1446,13 @@ static size_t fx_lds_n(const cf_run *r, int pairs)
 }
 static size_t fx_lds(const cf_run *r) { return fx_lds_n(r, r->rd.fx_pairs); }
 static size_t dx_lds(const cf_run *r) { return fx_lds_n(r, r->rd.dx_pairs); }
-/* FP64 x FFT without a divergence: the divergence's pair count */
+/* FP64 x FFT without a divergence */
 static unsigned plain_blocks(const cf_run *r)
 {
     const long npairs = ((long) r->g.ny * r->g.nz + 1) / 2;
-    return (unsigned) ((npairs + r->rd.dx_pairs - 1) / r->rd.dx_pairs);
+    return (unsigned) ((npairs + r->rd.px_pairs - 1) / r->rd.px_pairs);
 }
-static size_t plain_lds(const cf_run *r) { return 2 * sizeof(double) * ((size_t) r->rd.dx_pairs * fft_ld(r->g.nx) + (size_t) r->g.nx); }
+static size_t plain_lds(const cf_run *r) { return 2 * sizeof(double) * ((size_t) r->rd.px_pairs * fft_ld(r->g.nx) + (size_t) r->g.nx); }
 static size_t fy_lds_n(const cf_run *r, int cols)
 {
     return 2 * r->esz * ((size_t) cols * fy_ld(r->g.ny) + (size_t) r->g.ny);
@@ -1643,7 +1644,7 @@ static cf_status enqueue_spectral_solves(cf_run *r, int s, int nf, double2 *X, c
     const int nz = r->g.nz;
     Rn.g.nz = nf * nz;
     const long npairs = ((long) r->g.ny * Rn.g.nz + 1) / 2;
-    const unsigned gx = (unsigned) ((npairs + R.fx_pairs - 1) / R.fx_pairs), gp = (unsigned) ((npairs + R.dx_pairs - 1) / R.dx_pairs);
+    const unsigned gx = (unsigned) ((npairs + R.fx_pairs - 1) / R.fx_pairs), gp = (unsigned) ((npairs + R.px_pairs - 1) / R.px_pairs);
     const dim3 gy((unsigned) (((long) Rn.g.nz * r->g.nkx + R.fy_cols - 1) / R.fy_cols));
     KLAUNCH("hsolve", r->kfxp, dim3(gp), dim3(256), plain_lds(r), Rn, (const double *) r->ru, X);
     KLAUNCH("hsolve", r->kfy, gy, dim3(256), fy_lds(r), Rn, X, 1);
